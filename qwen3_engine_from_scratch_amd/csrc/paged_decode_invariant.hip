@@ -156,7 +156,7 @@ void paged_decode_inv_stream_kernel(DecodeArgs a) {
   __shared__ int32_t s_pref[kStreamMaxB + 1];
   __shared__ int32_t s_row[kStreamMaxB];
   __shared__ int32_t s_len[kStreamMaxB];
-  __shared__ int32_t s_wsum[kWaves];
+  __shared__ int32_t s_wsum[kStreamMaxB / (kWaves * 64)][kWaves];
   // Each wave's running fold in slot order (query head g, dim d at g * kD + d)
   // and its (m, l) per query head.
   __shared__ q3::f32x4 s_f[kWaves][kMaxG * kD / 4];
@@ -171,47 +171,7 @@ void paged_decode_inv_stream_kernel(DecodeArgs a) {
   // Wave-uniform reads of the LDS tables (scalar registers and branches).
   auto pref = [&](int b) { return __builtin_amdgcn_readfirstlane(s_pref[b]); };
 
-  // ---- prologue: rows, lengths and the exclusive tile prefix of every sequence ----
-  constexpr int kPer = kStreamMaxB / (kWaves * 64);
-  int cnt[kPer];
-  int local = 0;
-#pragma unroll
-  for (int i = 0; i < kPer; ++i) {
-    const int b = tid * kPer + i;
-    int n = 0;
-    if (b < B) {
-      const int64_t row = row_of(a, b);
-      const int64_t L = row >= 0 ? clamp_len(a, a.seq_lens[row]) : 0;
-      s_row[b] = static_cast<int32_t>(row);
-      s_len[b] = static_cast<int32_t>(L);
-      n = static_cast<int>(q3::cdiv(L, kTile));
-    }
-    cnt[i] = n;
-    local += n;
-  }
-  int incl = local;
-#pragma unroll
-  for (int o = 1; o < 64; o <<= 1) {
-    const int y = __shfl_up(incl, o, 64);
-    if (lane >= o) incl += y;
-  }
-  if (lane == 63) s_wsum[wave] = incl;
-  __syncthreads();
-  int run = incl - local;
-  int total = 0;
-#pragma unroll
-  for (int w = 0; w < kWaves; ++w) {
-    if (w < wave) run += s_wsum[w];
-    total += s_wsum[w];
-  }
-#pragma unroll
-  for (int i = 0; i < kPer; ++i) {
-    const int b = tid * kPer + i;
-    if (b < B) s_pref[b] = run;
-    run += cnt[i];
-  }
-  if (tid == 0) s_pref[B] = total;
-  __syncthreads();
+  const int total = tabulate(a, s_pref, s_row, s_len, s_wsum);
 
   // empty contexts: zero rows, spread over the workgroups
   for (int b = blockIdx.x; b < B; b += gridDim.x) {

@@ -70,6 +70,81 @@ __device__ __forceinline__ int64_t clamp_len(const DecodeArgs& a, int32_t seq_le
   return L > 0 ? L : 0;
 }
 
+// Inclusive prefix sum over the 64 lanes of a wave: four shifted adds inside
+// each 16-lane DPP row, then the row totals broadcast into the rows above.
+__device__ __forceinline__ int wave_prefix_sum(int v) {
+  v += __builtin_amdgcn_update_dpp(0, v, 0x111, 0xF, 0xF, true);   // row_shr:1
+  v += __builtin_amdgcn_update_dpp(0, v, 0x112, 0xF, 0xF, true);   // row_shr:2
+  v += __builtin_amdgcn_update_dpp(0, v, 0x114, 0xF, 0xF, true);   // row_shr:4
+  v += __builtin_amdgcn_update_dpp(0, v, 0x118, 0xF, 0xF, true);   // row_shr:8
+  v += __builtin_amdgcn_update_dpp(0, v, 0x142, 0xA, 0xF, false);  // row_bcast:15
+  v += __builtin_amdgcn_update_dpp(0, v, 0x143, 0xC, 0xF, false);  // row_bcast:31
+  return v;
+}
+
+// Tabulates the batch in LDS for a persistent workgroup (kWaves waves): each
+// sequence's row and length, and the exclusive prefix of its tiles
+// (s_pref[B]: all tiles).  Returns the number of tiles.
+//
+// Every wave of the grid waits for this before its first K/V load, so it is a
+// chain of memory round trips and nothing else: thread t takes sequences t,
+// t + 256, ..., so a batch of up to 256 costs one row_ids -> seq_lens chain
+// (neighbouring sequences in one thread cost eight of them in a row), and a
+// larger one issues all its row loads, then all its length loads, before it
+// waits.
+__device__ __forceinline__ int tabulate(const DecodeArgs& a, int32_t* s_pref, int32_t* s_row,
+                                        int32_t* s_len, int32_t (*s_wsum)[kWaves]) {
+  constexpr int kThreads = kWaves * 64;
+  constexpr int kPer = kStreamMaxB / kThreads;
+  const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
+  const int B = a.B;
+  const int rounds = (B + kThreads - 1) / kThreads;  // uniform, at most kPer
+  int64_t row[kPer];
+  int32_t len[kPer];
+  int n[kPer], incl[kPer];
+#pragma unroll
+  for (int i = 0; i < kPer; ++i) {
+    if (i >= rounds) break;
+    row[i] = row_of(a, min(i * kThreads + tid, B - 1));
+  }
+#pragma unroll
+  for (int i = 0; i < kPer; ++i) {
+    if (i >= rounds) break;
+    len[i] = a.seq_lens[row[i] >= 0 ? row[i] : 0];
+  }
+#pragma unroll
+  for (int i = 0; i < kPer; ++i) {
+    if (i >= rounds) break;
+    const int b = i * kThreads + tid;
+    const int32_t L = static_cast<int32_t>(row[i] >= 0 ? clamp_len(a, len[i]) : 0);
+    n[i] = b < B ? (L + kTile - 1) / kTile : 0;
+    if (b < B) {
+      s_row[b] = static_cast<int32_t>(row[i]);
+      s_len[b] = L;
+    }
+    incl[i] = wave_prefix_sum(n[i]);
+    if (lane == 63) s_wsum[i][wave] = incl[i];
+  }
+  __syncthreads();
+  int run = 0;
+#pragma unroll
+  for (int i = 0; i < kPer; ++i) {
+    if (i >= rounds) break;
+    int before = run;
+#pragma unroll
+    for (int w = 0; w < kWaves; ++w) {
+      const int ws = s_wsum[i][w];
+      before += w < wave ? ws : 0;
+      run += ws;
+    }
+    const int b = i * kThreads + tid;
+    if (b < B) s_pref[b] = before + incl[i] - n[i];
+  }
+  if (tid == 0) s_pref[B] = run;
+  __syncthreads();
+  return run;
+}
+
 // ---------------------------------------------------------------------------
 // Tile math shared by both paths.
 

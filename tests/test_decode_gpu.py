@@ -255,3 +255,31 @@ def test_decode_garbage_workspace_same_bits(gpu, B, lo, hi):
     assert torch.equal(outs[0], outs[1]) and torch.equal(outs[0], outs[2])
     ref = gpu_dense_decode_fp32(t["q"], t["k"], t["v"], t["bt"], t["seq_lens"], t["row_ids"], 16)
     assert_close_attn(outs[0], ref, "garbage workspace")
+
+
+@pytest.mark.parametrize("invariant", [False, True])
+@pytest.mark.parametrize("B", [1, 63, 255, 256, 257, 513, 2048])
+def test_decode_batch_sizes_around_tabulation_rounds(gpu, B, invariant):
+    """The length table is built 256 sequences at a time: batches one short
+    of, at and past those edges, rows permuted and a few outside the
+    resident table (zero output)."""
+    from qwen3_engine_from_scratch_amd.kernels.paged_attention import paged_attention_decode_hip
+
+    g = torch.Generator().manual_seed(B)
+    lens = [int(x) for x in torch.randint(1, 60, (B,), generator=g)]
+    announce(f"decode tabulation B={B} invariant={invariant}")
+    t = make_device_decode(lens, 16, 8, gpu, seed=B, slack=0.1)
+    rows = torch.randperm(B, generator=g).to(torch.int32)
+    bad = torch.zeros(B, dtype=torch.bool)
+    if B > 60:
+        bad[[3, 40, B - 1]] = True
+        rows[3], rows[40], rows[B - 1] = -1, B, 1 << 30
+    rows_d = rows.to(gpu)
+    out = paged_attention_decode_hip(t["q"], t["k"], t["v"], t["bt"], t["seq_lens"], rows_d, 16,
+                                     batch_invariant=invariant)
+    torch.cuda.synchronize()
+    ok = ~bad
+    ref = gpu_dense_decode_fp32(t["q"][ok.to(gpu)], t["k"], t["v"], t["bt"], t["seq_lens"],
+                                rows_d[ok.to(gpu)], 16)
+    assert_close_attn(out[ok.to(gpu)], ref, f"B={B}")
+    assert not out[bad.to(gpu)].any()
