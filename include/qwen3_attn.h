@@ -37,6 +37,7 @@
  *   qwen3_varlen_prefill_bf16  <- flash_attention_prefill
  *                                 (qwen3/kernels/flash_attention_varlen.py:126-194)
  *                                 + flash_attention_varlen_kernel (:25-123)
+ *   qwen3_padded_prefill_bf16  <- flash_attention_prefill_batched (:197-258)
  *   qwen3_qk_norm_rope_decode_bf16 / _slots_bf16
  *                              <- q_norm, k_norm, apply_rotary_pos_emb and the
  *                                 pool write that follows them
@@ -302,6 +303,28 @@ int qwen3_varlen_prefill_bf16(const void* q, const int64_t q_strides[2],
                               int max_seqlen, int64_t total_tokens,
                               int num_heads, int num_kv_heads, int head_dim,
                               float scale, int causal, void* workspace,
+                              size_t workspace_bytes, void* stream);
+
+/* ------------------------------------------------------------------------
+ * The same attention over a right-padded batch, without packing it.
+ *
+ * Replaces flash_attention_prefill_batched
+ * (qwen3/kernels/flash_attention_varlen.py:197-258): sequence b is the first
+ * lens[b] of padded_len rows of q[b], k[b], v[b]; rows of o past lens[b] are
+ * written as zero.  The same schedules, workspace contract and output bits as
+ * qwen3_varlen_prefill_bf16 on the packed rows (per 256 sequences: larger
+ * batches go in several launches).
+ *   q          (num_seqs, padded_len, num_heads, head_dim) through strides
+ *              [batch, row, head]; k, v the same with num_kv_heads.  Row
+ *              strides from head_dim to 2^23 elements.
+ *   o          contiguous (num_seqs, padded_len, num_heads, head_dim)
+ *   lens       HOST pointer, read before the call returns; 1..padded_len each
+ * ---------------------------------------------------------------------- */
+int qwen3_padded_prefill_bf16(const void* q, const int64_t q_strides[3], const void* k,
+                              const int64_t k_strides[3], const void* v,
+                              const int64_t v_strides[3], void* o, const int32_t* lens,
+                              int num_seqs, int padded_len, int num_heads, int num_kv_heads,
+                              int head_dim, float scale, int causal, void* workspace,
                               size_t workspace_bytes, void* stream);
 
 /* ------------------------------------------------------------------------

@@ -79,6 +79,12 @@ _SIGNATURES = {
          _vp, _i, _i, _i64,
          _i, _i, _i, ctypes.c_float, _i, _vp, ctypes.c_size_t, _vp],
     ),
+    "qwen3_padded_prefill_bf16": (
+        _i,
+        [_vp, _c_i64p, _vp, _c_i64p, _vp, _c_i64p, _vp,
+         ctypes.POINTER(ctypes.c_int32), _i, _i,
+         _i, _i, _i, ctypes.c_float, _i, _vp, ctypes.c_size_t, _vp],
+    ),
     "qwen3_qk_norm_rope_decode_bf16": (
         _i,
         [_vp, _c_i64p, _vp, _c_i64p, _vp, _c_i64p, _vp, _vp, ctypes.c_float,

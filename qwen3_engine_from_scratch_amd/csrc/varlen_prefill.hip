@@ -47,6 +47,7 @@
 //    default.
 #include <cstdlib>
 #include <cstring>
+#include <initializer_list>
 
 #include "common.hpp"
 
@@ -90,16 +91,20 @@ typedef __attribute__((address_space(3))) void lds_void_t;
 typedef short i16x4 __attribute__((__vector_size__(4 * sizeof(short))));
 typedef __attribute__((address_space(3))) i16x4 lds_i16x4_t;
 
+// Strides: st one row, sh one head, sb one step of a sequence's origin -- its
+// first packed row (sb = st), or its index in the padded batch (sb = one
+// padded sequence).
 struct PrefillArgs {
   const uint16_t* q;
-  int64_t q_st, q_sh;
+  int64_t q_st, q_sh, q_sb;
   const uint16_t* k;
-  int64_t k_st, k_sh;
+  int64_t k_st, k_sh, k_sb;
   const uint16_t* v;
-  int64_t v_st, v_sh;
+  int64_t v_st, v_sh, v_sb;
   uint16_t* o;
-  int64_t o_st, o_sh;
-  const int32_t* cu;
+  int64_t o_st, o_sh, o_sb;
+  const int32_t* cu;  // packed form only
+  int pad_rows;       // padded form: rows of every sequence; 0: packed
   int num_seqs;
   int64_t total;
   int Hq, G, HG;
@@ -116,6 +121,47 @@ struct PrefillArgs {
   float* slots;       // [2 * max_ranges][slot_floats<W>()]
   int max_ranges;
 };
+
+// Lengths of the padded form, by value: they are host data, and a launch
+// argument needs no device copy to wait for.
+struct PadLens {
+  int32_t n[kMaxSeqs];
+};
+
+// Sequence t's origin and length (0: nothing of it is computed).
+__device__ __forceinline__ void seq_at(const PrefillArgs& a, const PadLens& pl, int t, int& start,
+                                       int& len) {
+  if (a.pad_rows) {
+    start = t;
+    len = pl.n[t];
+    return;
+  }
+  const int64_t s0 = a.cu[t], s1 = a.cu[t + 1];
+  const bool ok = s0 >= 0 && s1 <= a.total && s1 > s0;
+  len = ok ? static_cast<int>(s1 - s0) : 0;
+  start = ok ? static_cast<int>(s0) : 0;
+}
+
+// Padded form: the output rows past each sequence's end are zeroed, one wave
+// per row over the whole grid (heads of a row are adjacent in the output).
+// Kernels call it after their items: these stores would otherwise stand in
+// front of the first K/V tile in the memory pipeline.
+__device__ __forceinline__ void zero_pad_rows(const PrefillArgs& a, const PadLens& pl) {
+  if (!a.pad_rows) return;
+  const int lane = threadIdx.x & 63;
+  const int wpb = blockDim.x >> 6;
+  const uint32_t nw = gridDim.x * wpb;
+  const uint32_t S = a.pad_rows, rows = a.num_seqs * S;  // below 2^31
+  const int chunks = a.Hq * (kD / 8);
+  for (uint32_t r = blockIdx.x * wpb + __builtin_amdgcn_readfirstlane(threadIdx.x >> 6); r < rows;
+       r += nw) {
+    const int b = r / S, i = r - b * S;
+    if (i < pl.n[b]) continue;
+    uint16_t* o = a.o + b * a.o_sb + i * a.o_st;
+    for (int c = lane; c < chunks; c += 64)
+      *reinterpret_cast<q3::u32x4*>(o + c * 8) = q3::u32x4{0, 0, 0, 0};
+  }
+}
 
 // The staged tiles of one workgroup: two K and two V buffers.
 struct TileBufs {
@@ -164,14 +210,15 @@ __device__ __forceinline__ LaneOffsets lane_offsets(int lane, int wave, int64_t 
   return o;
 }
 
-// Issues this wave's share of the loads of key tile n0 into (sk, sv).
+// Issues this wave's share of the loads of key tile n0 into (sk, sv); k0 and
+// v0 are the sequence's first rows of the item's KV head.
 template <int W>
 __device__ __forceinline__ void tile_dma(const PrefillArgs& a, const LaneOffsets& off,
-                                         int64_t start, int len, int kvh, int n0, uint16_t* sk,
-                                         uint16_t* sv, int wave) {
+                                         const uint16_t* k0, const uint16_t* v0, int len, int n0,
+                                         uint16_t* sk, uint16_t* sv, int wave) {
   const int rows = min(kBN, len - n0);
-  const uint16_t* kb = a.k + (start + n0) * a.k_st + static_cast<int64_t>(kvh) * a.k_sh;
-  const uint16_t* vb = a.v + (start + n0) * a.v_st + static_cast<int64_t>(kvh) * a.v_sh;
+  const uint16_t* kb = k0 + n0 * a.k_st;
+  const uint16_t* vb = v0 + n0 * a.v_st;
   // Rows past `rows` are outside the descriptor and read as zero.
   const int k_bytes = static_cast<int>((rows - 1) * a.k_st * 2) + kRowBytes;
   const int v_bytes = static_cast<int>((rows - 1) * a.v_st * 2) + kRowBytes;
@@ -271,7 +318,7 @@ __device__ __forceinline__ void wait_loads() {
 // One wave's share of a work item: the sequence's rows, this wave's 32
 // query rows of one head (wave-uniform).
 struct WaveItem {
-  int64_t start;  // first row of the sequence
+  int64_t start;  // the sequence's origin (seq_at)
   int len;        // its length
   int head;       // query head of this wave
   int kvh;        // its KV head
@@ -307,7 +354,7 @@ __device__ __forceinline__ void load_q(const PrefillArgs& a, const WaveItem& wi,
                                        q3::bf16x8 (&qv)[8]) {
   const int rows = min(32, wi.len - wi.q0);
   const uint16_t* base =
-      a.q + (wi.start + wi.q0) * a.q_st + static_cast<int64_t>(wi.head) * a.q_sh;
+      a.q + wi.start * a.q_sb + wi.q0 * a.q_st + static_cast<int64_t>(wi.head) * a.q_sh;
   const int bytes = rows > 0 ? static_cast<int>((rows - 1) * a.q_st * 2) + kRowBytes : 0;
   const __amdgpu_buffer_rsrc_t qr =
       __builtin_amdgcn_make_buffer_rsrc(const_cast<uint16_t*>(base), 0, bytes, 0x00020000);
@@ -460,7 +507,8 @@ __device__ __forceinline__ void store_output(const PrefillArgs& a, const WaveIte
       *reinterpret_cast<q3::u32x2*>(stage + l32 * 256 + ((ch ^ (l32 & 15)) << 4) + hl * 8) = w;
     }
   const int rows = min(32, wi.len - wi.q0);
-  uint16_t* base = a.o + (wi.start + wi.q0) * a.o_st + static_cast<int64_t>(wi.head) * a.o_sh;
+  uint16_t* base =
+      a.o + wi.start * a.o_sb + wi.q0 * a.o_st + static_cast<int64_t>(wi.head) * a.o_sh;
   const int bytes = rows > 0 ? static_cast<int>((rows - 1) * a.o_st * 2) + kRowBytes : 0;
   const __amdgpu_buffer_rsrc_t orr = __builtin_amdgcn_make_buffer_rsrc(base, 0, bytes, 0x00020000);
   const int oc = lane & 15;  // this lane's 16-byte chunk of a row
@@ -489,7 +537,9 @@ __device__ __forceinline__ void run_tiles(const PrefillArgs& a, const LaneOffset
                                           const WaveItem& wi, int t0, int t1, const TileBufs& tb,
                                           int lane, int wave, float& m_run, float& l_run,
                                           q3::f32x16 (&acc)[4]) {
-  tile_dma<W>(a, off, wi.start, wi.len, wi.kvh, t0 * kBN, tb.k0, tb.v0, wave);
+  const uint16_t* kb = a.k + wi.start * a.k_sb + static_cast<int64_t>(wi.kvh) * a.k_sh;
+  const uint16_t* vb = a.v + wi.start * a.v_sb + static_cast<int64_t>(wi.kvh) * a.v_sh;
+  tile_dma<W>(a, off, kb, vb, wi.len, t0 * kBN, tb.k0, tb.v0, wave);
   q3::bf16x8 qv[8];
   load_q(a, wi, q_lane_offset(a, lane), qv);
   m_run = q3::kNegInf;  // running max (log2 domain) of this query
@@ -501,7 +551,7 @@ __device__ __forceinline__ void run_tiles(const PrefillArgs& a, const LaneOffset
   wait_loads();
   __syncthreads();
   auto tile = [&](int it, const uint16_t* kt, const uint16_t* vt, uint16_t* nk, uint16_t* nv) {
-    if (it + 1 < t1) tile_dma<W>(a, off, wi.start, wi.len, wi.kvh, (it + 1) * kBN, nk, nv, wave);
+    if (it + 1 < t1) tile_dma<W>(a, off, kb, vb, wi.len, (it + 1) * kBN, nk, nv, wave);
     tile_math<Prio>(a, off, wi, lane, it * kBN, kt, vt, qv, m_run, l_run, acc);
     wait_loads();
     __syncthreads();
@@ -557,17 +607,17 @@ __device__ __forceinline__ void prefill_item(const PrefillArgs& a, const LaneOff
 // heaviest first.  Items past a sequence's end exit at once.
 template <int W>
 __global__ __launch_bounds__(W * 64) __attribute__((amdgpu_waves_per_eu(2, 2)))
-void varlen_prefill_flat_kernel(PrefillArgs a) {
+void varlen_prefill_flat_kernel(PrefillArgs a, PadLens pl) {
   Q3_PREFILL_TILE_BUFFERS;
   const int64_t id = blockIdx.x;
   const int hg = static_cast<int>(id % a.groups);
   const int seq = static_cast<int>((id / a.groups) % a.num_seqs);
   const int mt =
       a.n_mtiles - 1 - static_cast<int>(id / (static_cast<int64_t>(a.groups) * a.num_seqs));
-  const int64_t start = a.cu[seq];
-  const int64_t end = a.cu[seq + 1];
-  if (start < 0 || end > a.total || end <= start) return;
-  prefill_item<W>(a, off, start, static_cast<int>(end - start), hg, mt, tb);
+  int start, len;
+  seq_at(a, pl, seq, start, len);
+  if (len > 0) prefill_item<W>(a, off, start, len, hg, mt, tb);
+  zero_pad_rows(a, pl);
 }
 
 // ---------------------------------------------------------------------------
@@ -627,7 +677,7 @@ __device__ __forceinline__ float max3_16(const q3::f32x4 (&x)[4]) {
 }
 
 __global__ __launch_bounds__(kWsWaves * 64) __attribute__((amdgpu_waves_per_eu(3, 3)))
-void varlen_prefill_ws_kernel(PrefillArgs a) {
+void varlen_prefill_ws_kernel(PrefillArgs a, PadLens pl) {
   __shared__ __attribute__((aligned(1024))) uint16_t s_k0[kTileElems];
   __shared__ __attribute__((aligned(1024))) uint16_t s_k1[kTileElems];
   __shared__ __attribute__((aligned(1024))) uint16_t s_v0[kTileElems];
@@ -643,10 +693,9 @@ void varlen_prefill_ws_kernel(PrefillArgs a) {
   const int seq = static_cast<int>((id / a.groups) % a.num_seqs);
   const int mt =
       a.n_mtiles - 1 - static_cast<int>(id / (static_cast<int64_t>(a.groups) * a.num_seqs));
-  const int64_t start = a.cu[seq];
-  const int64_t end = a.cu[seq + 1];
-  if (start < 0 || end > a.total || end <= start) return;
-  const int len = static_cast<int>(end - start);
+  int start, len;
+  seq_at(a, pl, seq, start, len);
+  zero_pad_rows(a, pl);
   if (mt * a.rows >= len) return;
   const int kend = a.causal ? min(len, mt * a.rows + a.rows) : len;
   const int n = (kend + kBN - 1) / kBN;
@@ -655,8 +704,8 @@ void varlen_prefill_ws_kernel(PrefillArgs a) {
   const int si = wave - kWsMatrix;                 // softmax wave index
   const int mi = matrix ? wave : si >> 1;          // the matrix wave served
   const WaveItem wi = wave_item<4>(a, start, len, hg, mt, mi, lane);
-  const uint16_t* kb = a.k + start * a.k_st + static_cast<int64_t>(wi.kvh) * a.k_sh;
-  const uint16_t* vb = a.v + start * a.v_st + static_cast<int64_t>(wi.kvh) * a.v_sh;
+  const uint16_t* kb = a.k + start * a.k_sb + static_cast<int64_t>(wi.kvh) * a.k_sh;
+  const uint16_t* vb = a.v + start * a.v_sb + static_cast<int64_t>(wi.kvh) * a.v_sh;
   auto kbuf = [&](int i) { return i ? s_k1 : s_k0; };
   auto vbuf = [&](int i) { return i ? s_v1 : s_v0; };
 
@@ -855,16 +904,17 @@ __device__ __forceinline__ int block_exclusive_scan(int* v, int n, int* s_wsum) 
 // outside the batch) and s_start[t] its first row.  Returns the number of items.  Called by all threads
 // of the workgroup.
 template <int W>
-__device__ __forceinline__ int build_items(const PrefillArgs& a, int* s_len, int* s_start,
-                                           int* s_sorted, int* s_first, int* s_wsum) {
+__device__ __forceinline__ int build_items(const PrefillArgs& a, const PadLens& pl, int* s_len,
+                                           int* s_start, int* s_sorted, int* s_first,
+                                           int* s_wsum) {
   const int tid = threadIdx.x;
   const int S = a.num_seqs;
   const int nm = a.n_mtiles;
   for (int t = tid; t < S; t += W * 64) {
-    const int64_t s0 = a.cu[t], s1 = a.cu[t + 1];
-    const bool ok = s0 >= 0 && s1 <= a.total && s1 > s0;
-    s_len[t] = ok ? static_cast<int>(s1 - s0) : 0;
-    s_start[t] = ok ? static_cast<int>(s0) : 0;
+    int start, len;
+    seq_at(a, pl, t, start, len);
+    s_len[t] = len;
+    s_start[t] = start;
   }
   __syncthreads();
   // Rank by length, longest first (ties by index).
@@ -925,7 +975,7 @@ __device__ __forceinline__ void item_at(const PrefillArgs& a, int64_t i64, const
 // (mirroring whole groups of 8 positions so item i stays on XCD i % 8).
 template <int W>
 __global__ __launch_bounds__(W * 64) __attribute__((amdgpu_waves_per_eu(2, 2)))
-void varlen_prefill_persistent_kernel(PrefillArgs a) {
+void varlen_prefill_persistent_kernel(PrefillArgs a, PadLens pl) {
   Q3_PREFILL_TILE_BUFFERS;
   __shared__ int s_len[kMaxSeqs];
   __shared__ int s_start[kMaxSeqs];
@@ -942,7 +992,7 @@ void varlen_prefill_persistent_kernel(PrefillArgs a) {
     asm volatile("" ::"v"(prev));  // performed before this thread reaches the barriers below
   }
 
-  const int T = build_items<W>(a, s_len, s_start, s_sorted, s_first, s_wsum);
+  const int T = build_items<W>(a, pl, s_len, s_start, s_sorted, s_first, s_wsum);
 
   auto run = [&](int64_t i64) {
     int seq, hg, mt;
@@ -1019,6 +1069,7 @@ void varlen_prefill_persistent_kernel(PrefillArgs a) {
       __syncthreads();  // the item's LDS tiles are no longer read
     }
   }
+  zero_pad_rows(a, pl);
   if (counters && tid == 0 &&
       atomicAdd(a.ctr + kPools * kPoolStride, 1u) == gridDim.x - 1) {
     // the last workgroup to finish leaves every counter at zero
@@ -1301,7 +1352,7 @@ __device__ __forceinline__ void fold_parts(const PrefillArgs& a, int vfirst, int
 // others are all in, folds without saving.  No part waits for another.
 template <int W>
 __global__ __launch_bounds__(W * 64) __attribute__((amdgpu_waves_per_eu(2, 2)))
-void varlen_prefill_range_kernel(PrefillArgs a) {
+void varlen_prefill_range_kernel(PrefillArgs a, PadLens pl) {
   Q3_PREFILL_TILE_BUFFERS;
   __shared__ int s_rlen[kMaxSeqs];
   __shared__ int s_rstart[kMaxSeqs];
@@ -1316,10 +1367,10 @@ void varlen_prefill_range_kernel(PrefillArgs a) {
   int* s_len0 = reinterpret_cast<int*>(s_k0);  // tile buffers are free until the first load
   int* s_start0 = reinterpret_cast<int*>(s_v0);
   for (int t = tid; t < S; t += W * 64) {
-    const int64_t s0 = a.cu[t], s1 = a.cu[t + 1];
-    const bool ok = s0 >= 0 && s1 <= a.total && s1 > s0;
-    s_len0[t] = ok ? static_cast<int>(s1 - s0) : 0;
-    s_start0[t] = ok ? static_cast<int>(s0) : 0;
+    int start, len;
+    seq_at(a, pl, t, start, len);
+    s_len0[t] = len;
+    s_start0[t] = start;
   }
   __syncthreads();
   for (int t = tid; t < S; t += W * 64) {
@@ -1381,12 +1432,18 @@ void varlen_prefill_range_kernel(PrefillArgs a) {
   // every workgroup busy: XCD x (workgroups w % 8 == x) holds ranges
   // x * nwg / 8 .. , adjacent items sharing its L2; fewer ranges: spread.
   const int v = rc.N == nwg && nwg % 8 == 0 ? (w % 8) * (nwg / 8) + w / 8 : w;
-  if (v >= rc.N) return;
+  if (v >= rc.N) {  // no range: only pad rows
+    zero_pad_rows(a, pl);
+    return;
+  }
   rc.v = v;
   rc.p_lo = (static_cast<int64_t>(v) * rc.U + rc.N - 1) / rc.N;
   rc.p_hi = (static_cast<int64_t>(v + 1) * rc.U + rc.N - 1) / rc.N;
   __syncthreads();  // s_ticket is reused below
-  if (rc.p_lo >= rc.p_hi) return;
+  if (rc.p_lo >= rc.p_hi) {
+    zero_pad_rows(a, pl);
+    return;
+  }
 
   const uint32_t o_lane = o_lane_offset(a, lane);
   for (RangeSeg cur = next_owned(a, rc, locate(a, rc, rc.p_lo)); cur.valid;
@@ -1441,6 +1498,7 @@ void varlen_prefill_range_kernel(PrefillArgs a) {
     }
     __syncthreads();  // the staging buffers are read before the next segment's loads refill them
   }
+  zero_pad_rows(a, pl);
 }
 
 // QWEN3_PREFILL_TILE=ws selects the wave-specialised tile (flat grid of
@@ -1468,8 +1526,8 @@ int resident_per_cu(const void* kernel, int dev, int* cache) {
 // grid (CUs x resident workgroups, from the occupancy API) or, past their
 // LDS tables, the flat grid.
 template <int W>
-int launch_prefill(PrefillArgs a, int num_seqs, int max_seqlen, int dev, int cus,
-                   hipStream_t s, const char* who) {
+int launch_prefill(PrefillArgs a, const PadLens& pl, int num_seqs, int max_seqlen, int dev,
+                   int cus, hipStream_t s, const char* who) {
   a.rows = 32 * W / a.HG;
   a.n_mtiles = static_cast<int>(q3::cdiv(max_seqlen, a.rows));
   const int64_t blocks = static_cast<int64_t>(a.groups) * num_seqs * a.n_mtiles;
@@ -1495,7 +1553,7 @@ int launch_prefill(PrefillArgs a, int num_seqs, int max_seqlen, int dev, int cus
       const int wgs = (cus * per_cu) / 8 * 8;
       a.max_ranges = a.max_ranges < wgs ? a.max_ranges : wgs;
       if (per_cu > 0 && a.max_ranges > 0 && items_max < static_cast<int64_t>(cus) * per_cu) {
-        hipLaunchKernelGGL(varlen_prefill_range_kernel<W>, dim3(wgs), dim3(W * 64), 0, s, a);
+        hipLaunchKernelGGL(varlen_prefill_range_kernel<W>, dim3(wgs), dim3(W * 64), 0, s, a, pl);
         return q3::launch_status(who);
       }
     }
@@ -1506,10 +1564,10 @@ int launch_prefill(PrefillArgs a, int num_seqs, int max_seqlen, int dev, int cus
       num_seqs <= kMaxSeqs && a.n_mtiles <= kScanMax && cus > 0 && per_cu > 0;
   if (persistent) {
     const int wgs = ((cus * per_cu + 7) / 8) * 8;  // multiple of 8 for the XCD-preserving snake
-    hipLaunchKernelGGL(varlen_prefill_persistent_kernel<W>, dim3(wgs), dim3(W * 64), 0, s, a);
+    hipLaunchKernelGGL(varlen_prefill_persistent_kernel<W>, dim3(wgs), dim3(W * 64), 0, s, a, pl);
   } else {
     hipLaunchKernelGGL(varlen_prefill_flat_kernel<W>, dim3(static_cast<unsigned>(blocks)),
-                       dim3(W * 64), 0, s, a);
+                       dim3(W * 64), 0, s, a, pl);
   }
   return q3::launch_status(who);
 }
@@ -1536,6 +1594,82 @@ int device_cus() {
   return cus;
 }
 
+// Sizes, strides and the two kernels' tables: shared by both entry points.
+bool rows_aligned16(const void* q, const void* k, const void* v, const void* o,
+                    std::initializer_list<const int64_t*> strides, int n) {
+  bool ok = q3::aligned16(q) && q3::aligned16(k) && q3::aligned16(v) && q3::aligned16(o);
+  for (const int64_t* st : strides)
+    for (int i = 0; i < n; ++i) ok = ok && st[i] % 8 == 0;
+  return ok;
+}
+
+int check_heads(int num_heads, int num_kv_heads, int head_dim, const char* who) {
+  if (head_dim != kD)
+    return q3::fail(QWEN3_EUNSUPPORTED, "%s: head_dim %d not supported (built for %d)", who,
+                    head_dim, kD);
+  if (num_kv_heads <= 0 || num_heads <= 0 || num_heads % num_kv_heads != 0 ||
+      num_heads / num_kv_heads > 16)
+    return q3::fail(QWEN3_EUNSUPPORTED, "%s: num_heads %d / num_kv_heads %d unsupported", who,
+                    num_heads, num_kv_heads);
+  return QWEN3_OK;
+}
+
+int check_workspace(const void* workspace, size_t workspace_bytes, int cus, const char* who) {
+  if (!workspace) return QWEN3_OK;
+  const size_t need = workspace_bytes_for(cus > 0 && cus <= kMaxCus ? cus : 256);
+  if (workspace_bytes < need)
+    return q3::fail(QWEN3_EWORKSPACE, "%s: workspace of %zu bytes needed, %zu given", who, need,
+                    workspace_bytes);
+  if (!q3::aligned16(workspace))
+    return q3::fail(QWEN3_EALIGN, "%s: workspace must be 16-byte aligned", who);
+  return QWEN3_OK;
+}
+
+// Completes the arguments (heads, workspace), picks the kernel and launches.
+int run_prefill(PrefillArgs a, const PadLens& pl, int max_seqlen, int num_heads, int num_kv_heads,
+                float scale, int causal, void* workspace, int cus, hipStream_t s,
+                const char* who) {
+  a.Hq = num_heads;
+  a.G = num_heads / num_kv_heads;
+  a.HG = a.G % 4 == 0 ? 4 : (a.G % 2 == 0 ? 2 : 1);
+  a.scale_log2 = scale * q3::kLog2e;
+  a.causal = causal ? 1 : 0;
+  a.groups = num_heads / a.HG;
+  q3::clear_error();
+  int dev = -1;
+  if (hipGetDevice(&dev) != hipSuccess) dev = -1;
+  // Eight-wave workgroups once the batch holds enough of their (twice as
+  // large) work items to give every CU four: they halve the K/V tile
+  // traffic per flop; smaller batches take the range schedule of four-wave
+  // workgroups, which cuts the heaviest items across workgroups.
+  const int64_t rows8 = 32 * 8 / a.HG;
+  const int64_t items8 = static_cast<int64_t>(a.groups) * q3::cdiv(a.total, rows8);
+  const bool wide = cus > 0 && items8 >= 4 * static_cast<int64_t>(cus);
+  if (workspace) {
+    char* ws = static_cast<char*>(workspace);
+    // Items handed out from the counters only on the eight-wave path: over
+    // many rounds of mixed-length items they finish 1-2% sooner.
+    if (wide) a.ctr = reinterpret_cast<uint32_t*>(ws);
+    const size_t n = ranges_for(cus > 0 && cus <= kMaxCus ? cus : 256);
+    a.tickets = reinterpret_cast<uint32_t*>(ws + kCtrBytes);
+    a.slots = reinterpret_cast<float*>(ws + kCtrBytes + ticket_bytes(n));
+    a.max_ranges = static_cast<int>(n);
+  }
+  if (ws_tile_selected()) {  // flat grid of four-wave items on the wave-specialised tile
+    a.rows = 32 * 4 / a.HG;
+    a.n_mtiles = static_cast<int>(q3::cdiv(max_seqlen, a.rows));
+    const int64_t blocks = static_cast<int64_t>(a.groups) * a.num_seqs * a.n_mtiles;
+    if (blocks > 0x7fffffff)
+      return q3::fail(QWEN3_EINVAL, "%s: grid too large (heads %d, seqs %d, max_seqlen %d)", who,
+                      a.Hq, a.num_seqs, max_seqlen);
+    hipLaunchKernelGGL(varlen_prefill_ws_kernel, dim3(static_cast<unsigned>(blocks)),
+                       dim3(kWsWaves * 64), 0, s, a, pl);
+    return q3::launch_status(who);
+  }
+  return wide ? launch_prefill<8>(a, pl, a.num_seqs, max_seqlen, dev, cus, s, who)
+              : launch_prefill<4>(a, pl, a.num_seqs, max_seqlen, dev, cus, s, who);
+}
+
 }  // namespace
 
 extern "C" size_t qwen3_varlen_prefill_workspace_bytes(void) {
@@ -1555,21 +1689,11 @@ extern "C" int qwen3_varlen_prefill_bf16(const void* q, const int64_t q_strides[
   if (!q || !k || !v || !o || !cu_seqlens || !q_strides || !k_strides || !v_strides ||
       !o_strides)
     return q3::fail(QWEN3_EINVAL, "%s: null pointer argument", who);
-  if (head_dim != kD)
-    return q3::fail(QWEN3_EUNSUPPORTED, "%s: head_dim %d not supported (built for %d)", who,
-                    head_dim, kD);
-  if (num_kv_heads <= 0 || num_heads <= 0 || num_heads % num_kv_heads != 0 ||
-      num_heads / num_kv_heads > 16)
-    return q3::fail(QWEN3_EUNSUPPORTED, "%s: num_heads %d / num_kv_heads %d unsupported", who,
-                    num_heads, num_kv_heads);
+  if (const int rc = check_heads(num_heads, num_kv_heads, head_dim, who)) return rc;
   if (num_seqs < 0 || max_seqlen < 0 || total_tokens < 0)
     return q3::fail(QWEN3_EINVAL, "%s: bad sizes", who);
   if (num_seqs == 0 || max_seqlen == 0 || total_tokens == 0) return QWEN3_OK;
-  const int64_t vec_strides[] = {q_strides[0], q_strides[1], k_strides[0], k_strides[1],
-                                 v_strides[0], v_strides[1], o_strides[0], o_strides[1]};
-  bool ok = q3::aligned16(q) && q3::aligned16(k) && q3::aligned16(v) && q3::aligned16(o);
-  for (int64_t s : vec_strides) ok = ok && s % 8 == 0;
-  if (!ok)
+  if (!rows_aligned16(q, k, v, o, {q_strides, k_strides, v_strides, o_strides}, 2))
     return q3::fail(QWEN3_EALIGN, "%s: q/k/v/o need 16-byte aligned rows (strides multiple "
                     "of 8 elements)", who);
 
@@ -1577,66 +1701,93 @@ extern "C" int qwen3_varlen_prefill_bf16(const void* q, const int64_t q_strides[
   a.q = static_cast<const uint16_t*>(q);
   a.q_st = q_strides[0];
   a.q_sh = q_strides[1];
+  a.q_sb = q_strides[0];
   a.k = static_cast<const uint16_t*>(k);
   a.k_st = k_strides[0];
   a.k_sh = k_strides[1];
+  a.k_sb = k_strides[0];
   a.v = static_cast<const uint16_t*>(v);
   a.v_st = v_strides[0];
   a.v_sh = v_strides[1];
+  a.v_sb = v_strides[0];
   a.o = static_cast<uint16_t*>(o);
   a.o_st = o_strides[0];
   a.o_sh = o_strides[1];
+  a.o_sb = o_strides[0];
   a.cu = cu_seqlens;
   a.num_seqs = num_seqs;
   a.total = total_tokens;
-  a.Hq = num_heads;
-  a.G = num_heads / num_kv_heads;
-  a.HG = a.G % 4 == 0 ? 4 : (a.G % 2 == 0 ? 2 : 1);
-  a.scale_log2 = scale * q3::kLog2e;
-  a.causal = causal ? 1 : 0;
-  a.groups = num_heads / a.HG;
   const int cus = device_cus();
-  if (workspace) {
-    const size_t need = workspace_bytes_for(cus > 0 && cus <= kMaxCus ? cus : 256);
-    if (workspace_bytes < need)
-      return q3::fail(QWEN3_EWORKSPACE, "%s: workspace of %zu bytes needed, %zu given", who,
-                      need, workspace_bytes);
-    if (!q3::aligned16(workspace))
-      return q3::fail(QWEN3_EALIGN, "%s: workspace must be 16-byte aligned", who);
-  }
+  if (const int rc = check_workspace(workspace, workspace_bytes, cus, who)) return rc;
+  return run_prefill(a, PadLens{}, max_seqlen, num_heads, num_kv_heads, scale, causal, workspace,
+                     cus, static_cast<hipStream_t>(stream), who);
+}
 
-  q3::clear_error();
-  hipStream_t s = static_cast<hipStream_t>(stream);
-  int dev = -1;
-  if (hipGetDevice(&dev) != hipSuccess) dev = -1;
-  // Eight-wave workgroups once the batch holds enough of their (twice as
-  // large) work items to give every CU four: they halve the K/V tile
-  // traffic per flop; smaller batches take the range schedule of four-wave
-  // workgroups, which cuts the heaviest items across workgroups.
-  const int64_t rows8 = 32 * 8 / a.HG;
-  const int64_t items8 = static_cast<int64_t>(a.groups) * q3::cdiv(total_tokens, rows8);
-  const bool wide = cus > 0 && items8 >= 4 * static_cast<int64_t>(cus);
-  if (workspace) {
-    char* ws = static_cast<char*>(workspace);
-    // Items handed out from the counters only on the eight-wave path: over
-    // many rounds of mixed-length items they finish 1-2% sooner.
-    if (wide) a.ctr = reinterpret_cast<uint32_t*>(ws);
-    const size_t n = ranges_for(cus > 0 && cus <= kMaxCus ? cus : 256);
-    a.tickets = reinterpret_cast<uint32_t*>(ws + kCtrBytes);
-    a.slots = reinterpret_cast<float*>(ws + kCtrBytes + ticket_bytes(n));
-    a.max_ranges = static_cast<int>(n);
+extern "C" int qwen3_padded_prefill_bf16(const void* q, const int64_t q_strides[3], const void* k,
+                                         const int64_t k_strides[3], const void* v,
+                                         const int64_t v_strides[3], void* o,
+                                         const int32_t* lens, int num_seqs, int padded_len,
+                                         int num_heads, int num_kv_heads, int head_dim,
+                                         float scale, int causal, void* workspace,
+                                         size_t workspace_bytes, void* stream) {
+  const char* who = "qwen3_padded_prefill_bf16";
+  if (!q || !k || !v || !o || !lens || !q_strides || !k_strides || !v_strides)
+    return q3::fail(QWEN3_EINVAL, "%s: null pointer argument", who);
+  if (const int rc = check_heads(num_heads, num_kv_heads, head_dim, who)) return rc;
+  if (num_seqs < 0 || padded_len < 0 ||
+      static_cast<int64_t>(kMaxSeqs) * padded_len > 0x7fffffff)
+    return q3::fail(QWEN3_EINVAL, "%s: bad sizes", who);
+  for (int i = 0; i < num_seqs; ++i)
+    if (lens[i] <= 0 || lens[i] > padded_len)
+      return q3::fail(QWEN3_EINVAL, "%s: length %d of sequence %d outside 1..%d", who, lens[i], i,
+                      padded_len);
+  if (num_seqs == 0 || padded_len == 0) return QWEN3_OK;
+  if (!rows_aligned16(q, k, v, o, {q_strides, k_strides, v_strides}, 3))
+    return q3::fail(QWEN3_EALIGN, "%s: q/k/v/o need 16-byte aligned rows (strides multiple "
+                    "of 8 elements)", who);
+  // Rows of a head apart (a tile's rows past the end must lie outside its
+  // buffer descriptor) and a 64-row tile inside 32-bit byte offsets.
+  for (const int64_t* st : {q_strides, k_strides, v_strides})
+    if (st[1] < kD || st[1] > (int64_t{1} << 23))
+      return q3::fail(QWEN3_EUNSUPPORTED, "%s: row stride %lld outside %d..2^23", who,
+                      static_cast<long long>(st[1]), kD);
+  const int cus = device_cus();
+  if (const int rc = check_workspace(workspace, workspace_bytes, cus, who)) return rc;
+
+  PrefillArgs a{};
+  a.q_sb = q_strides[0];
+  a.q_st = q_strides[1];
+  a.q_sh = q_strides[2];
+  a.k_sb = k_strides[0];
+  a.k_st = k_strides[1];
+  a.k_sh = k_strides[2];
+  a.v_sb = v_strides[0];
+  a.v_st = v_strides[1];
+  a.v_sh = v_strides[2];
+  a.o_st = static_cast<int64_t>(num_heads) * kD;
+  a.o_sh = kD;
+  a.o_sb = a.o_st * padded_len;
+  a.pad_rows = padded_len;
+  // The lengths travel as a launch argument of kMaxSeqs entries: larger
+  // batches go in several launches.
+  for (int b0 = 0; b0 < num_seqs; b0 += kMaxSeqs) {
+    const int n = num_seqs - b0 < kMaxSeqs ? num_seqs - b0 : kMaxSeqs;
+    PadLens pl{};
+    int longest = 0;
+    a.total = 0;
+    for (int i = 0; i < n; ++i) {
+      pl.n[i] = lens[b0 + i];
+      a.total += pl.n[i];
+      longest = pl.n[i] > longest ? pl.n[i] : longest;
+    }
+    a.q = static_cast<const uint16_t*>(q) + b0 * a.q_sb;
+    a.k = static_cast<const uint16_t*>(k) + b0 * a.k_sb;
+    a.v = static_cast<const uint16_t*>(v) + b0 * a.v_sb;
+    a.o = static_cast<uint16_t*>(o) + b0 * a.o_sb;
+    a.num_seqs = n;
+    if (const int rc = run_prefill(a, pl, longest, num_heads, num_kv_heads, scale, causal,
+                                   workspace, cus, static_cast<hipStream_t>(stream), who))
+      return rc;
   }
-  if (ws_tile_selected()) {  // flat grid of four-wave items on the wave-specialised tile
-    a.rows = 32 * 4 / a.HG;
-    a.n_mtiles = static_cast<int>(q3::cdiv(max_seqlen, a.rows));
-    const int64_t blocks = static_cast<int64_t>(a.groups) * num_seqs * a.n_mtiles;
-    if (blocks > 0x7fffffff)
-      return q3::fail(QWEN3_EINVAL, "%s: grid too large (heads %d, seqs %d, max_seqlen %d)", who,
-                      a.Hq, num_seqs, max_seqlen);
-    hipLaunchKernelGGL(varlen_prefill_ws_kernel, dim3(static_cast<unsigned>(blocks)),
-                       dim3(kWsWaves * 64), 0, s, a);
-    return q3::launch_status(who);
-  }
-  return wide ? launch_prefill<8>(a, num_seqs, max_seqlen, dev, cus, s, who)
-              : launch_prefill<4>(a, num_seqs, max_seqlen, dev, cus, s, who);
+  return QWEN3_OK;
 }

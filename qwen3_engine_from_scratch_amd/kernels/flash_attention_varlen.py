@@ -6,6 +6,8 @@ device work in qwen3_varlen_prefill_bf16 (include/qwen3_attn.h).
 """
 from __future__ import annotations
 
+import ctypes
+
 import torch
 
 from .. import _lib
@@ -89,34 +91,53 @@ def flash_attention_prefill(q: torch.Tensor, k: torch.Tensor, v: torch.Tensor,
     return out
 
 
+def _padded_rows(t: torch.Tensor):
+    """t (B, H, S, D) as the padded kernel reads it: (tensor, its [batch, row,
+    head] strides).  Copied to (B, S, H, D) rows where the kernel has no
+    form for it: a head_dim that is not contiguous, rows that overlap, lie
+    too far apart or are not 16-byte aligned."""
+    D = t.shape[3]
+    for x in (t, None):
+        if x is None:
+            t = t.permute(0, 2, 1, 3).clone(memory_format=torch.contiguous_format)
+            t = t.permute(0, 2, 1, 3)
+        # the stride of a dimension of one element is arbitrary
+        sb, sh, st = (t.stride(i) if t.shape[i] > 1 else 0 for i in (0, 1, 2))
+        st = st or (D if t.shape[2] == 1 else 0)
+        if (t.stride(3) == 1 and D <= st <= 1 << 23 and (sb | sh | st) % 8 == 0
+                and t.data_ptr() % 16 == 0):
+            break
+    return t, (ctypes.c_int64 * 3)(sb, st, sh)
+
+
 def flash_attention_prefill_batched(q, k, v, lens, scaling, num_heads, num_kv_heads, head_dim):
     """Right-padded batch adaptor (reference: flash_attention_prefill_batched,
     qwen3/kernels/flash_attention_varlen.py:197-258).
 
     q: (B, num_heads, S, D); k, v: (B, num_kv_heads, S, D); lens: list[int]
     valid lengths (0 < lens[i] <= S).  Returns (B, S, num_heads * D) with pad
-    rows zero.  The lengths are host data, so max_seqlen needs no device sync.
+    rows zero.  One launch on the padded tensors where they lie: packing the
+    valid rows first (boolean masks, index gathers and scatters) took 240 us
+    beside a 36 us kernel on eight prompts of 128-1024 tokens.
     """
     B, H, S, D = q.shape
-    H_kv = k.shape[1]
     assert len(lens) == B, "lens must have one entry per batch row"
     assert all(0 < l <= S for l in lens), "lens out of range (need 0 < lens_i <= S)"
-    q2 = q.permute(0, 2, 1, 3).reshape(B * S, H, D)
-    k2 = k.permute(0, 2, 1, 3).reshape(B * S, H_kv, D)
-    v2 = v.permute(0, 2, 1, 3).reshape(B * S, H_kv, D)
-    if all(l == S for l in lens):
-        cu = torch.arange(B + 1, device=q.device, dtype=torch.int32) * S
-        out_f = flash_attention_prefill(q2, k2, v2, cu, scaling, num_heads, num_kv_heads,
-                                        head_dim, max_seqlen=S)
-        return out_f.reshape(B, S, H * D)
-    s_idx = torch.arange(S, device=q.device)
-    lens_t = torch.tensor(lens, device=q.device, dtype=torch.long)
-    valid = (s_idx[None, :] < lens_t[:, None]).reshape(-1)
-    q_f, k_f, v_f = q2[valid], k2[valid], v2[valid]
-    cu = torch.zeros(B + 1, dtype=torch.int32, device=q.device)
-    torch.cumsum(torch.tensor(lens, dtype=torch.int32, device=q.device), 0, out=cu[1:])
-    out_f = flash_attention_prefill(q_f, k_f, v_f, cu, scaling, num_heads, num_kv_heads,
-                                    head_dim, max_seqlen=max(lens))
-    out = torch.zeros(B * S, H, D, dtype=q.dtype, device=q.device)
-    out[valid] = out_f
-    return out.reshape(B, S, H * D)
+    assert H == num_heads and D == head_dim
+    assert k.shape == (B, num_kv_heads, S, D) and v.shape == k.shape
+    assert q.dtype == torch.bfloat16 and k.dtype == torch.bfloat16 and v.dtype == torch.bfloat16, \
+        "HIP prefill kernel is bf16 only"
+    dev = _lib.require_hip(q, k, v)
+    out = torch.empty(B, S, H * D, dtype=q.dtype, device=q.device)
+    q, q_st = _padded_rows(q)
+    k, k_st = _padded_rows(k)
+    v, v_st = _padded_rows(v)
+    lib = _lib.load()
+    stream = _lib.stream_of(dev)
+    ws = _schedule_workspace(q.device, stream, lib)
+    rc = lib.qwen3_padded_prefill_bf16(
+        q.data_ptr(), q_st, k.data_ptr(), k_st, v.data_ptr(), v_st, out.data_ptr(),
+        (ctypes.c_int32 * B)(*[int(l) for l in lens]), B, S, num_heads, num_kv_heads, head_dim,
+        float(scaling), 1, ws.data_ptr(), ws.numel(), stream)
+    _lib.check(rc, "qwen3_padded_prefill_bf16")
+    return out

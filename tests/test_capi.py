@@ -134,6 +134,28 @@ def test_prefill_rejects_bad_arguments():
     assert call(qs=_s(2048, 129)) == -2
 
 
+def test_padded_prefill_rejects_bad_arguments():
+    lib = _lib.load()
+    q3, k3 = _s(64 * 2048, 2048, 128), _s(64 * 1024, 1024, 128)
+
+    def call(D=128, H=16, Hk=8, q=FAKE, qs=q3, ks=k3, lens=(64, 5), S=64, ws=None, wsb=0):
+        return lib.qwen3_padded_prefill_bf16(q, qs, FAKE, ks, FAKE, k3, FAKE,
+                                             (ctypes.c_int32 * len(lens))(*lens), len(lens), S,
+                                             H, Hk, D, 0.088, 1, ws, wsb, None)
+
+    assert call(D=256) == -3
+    assert call(H=12) == -3
+    assert call(q=None) == -1
+    assert call(lens=(64, 0)) == -1
+    assert call(lens=(65, 1)) == -1
+    assert call(S=1 << 24) == -1       # rows of a launch past 32 bits
+    assert call(qs=_s(64 * 2048, 2049, 128)) == -2
+    assert call(ks=_s(64, 64, 1 << 16)) == -3       # overlapping rows
+    assert call(ks=_s(64, 1 << 24, 128)) == -3      # a tile's rows past 32-bit offsets
+    assert call(ws=FAKE, wsb=lib.qwen3_varlen_prefill_workspace_bytes() - 1) == -4
+    assert call(lens=()) == 0
+
+
 def test_pre_attention_rejects_bad_arguments():
     lib = _lib.load()
     qs, ks, c4 = _s(4096, 128), _s(4096, 128), _s(1 << 16, 1 << 14, 2048, 128)

@@ -323,6 +323,62 @@ def test_prefill_batched_adaptor_pads_zero(gpu):
         assert not out[b, L:].any()
 
 
+@pytest.mark.parametrize("lens, S, hq, hkv", [
+    ([5, 48, 31], 48, 16, 8),
+    ([1], 1, 8, 8),
+    ([1, 1], 7, 8, 8),                       # mostly pad rows
+    ([700], 1000, 16, 8),                    # items cut across workgroups
+    ([129, 64, 65, 1, 1024, 333, 800, 1000], 1024, 16, 8),
+    ([1536] * 6 + [63, 1530], 1536, 32, 8),  # eight-wave workgroups
+    ([3 + i % 37 for i in range(300)], 40, 16, 8),  # past one launch's lengths
+])
+@pytest.mark.parametrize("layout", ["token", "head", "offset", "expand"])
+def test_prefill_padded_in_place_same_bits_as_packed(gpu, lens, S, hq, hkv, layout):
+    """The padded form reads the batch where it lies: the same bits as the
+    packed call on the valid rows (per 256 sequences, one launch's share),
+    zero pad rows, garbage (NaN) pad rows of q, k and v never read -- for
+    token-major and head-major tensors, and for the ones that are copied
+    (rows off 16 bytes; overlapping rows)."""
+    from qwen3_engine_from_scratch_amd.kernels.flash_attention_varlen import (
+        flash_attention_prefill, flash_attention_prefill_batched)
+
+    B = len(lens)
+    g = torch.Generator(device=gpu).manual_seed(S)
+    if layout == "expand":
+        qkv = [torch.randn(B, h, 1, 128, generator=g, device=gpu).bfloat16().expand(B, h, S, 128)
+               for h in (hq, hkv, hkv)]
+    else:
+        qkv = []
+        for h in (hq, hkv, hkv):
+            t = torch.randn(B, S, h, 128, generator=g, device=gpu).bfloat16()
+            for b, n in enumerate(lens):
+                t[b, n:] = float("nan")
+            t = t.permute(0, 2, 1, 3)
+            if layout == "head":
+                t = t.contiguous()
+            elif layout == "offset":
+                buf = torch.zeros(B, S, h * 128 + 8, dtype=t.dtype, device=gpu)
+                view = buf[:, :, 3:3 + h * 128].unflatten(2, (h, 128)).permute(0, 2, 1, 3)
+                view.copy_(t)
+                t = view
+            qkv.append(t)
+    announce(f"padded in place {layout} B={B} S={S} heads={hq}/{hkv}")
+    out = flash_attention_prefill_batched(*qkv, lens, 128 ** -0.5, hq, hkv, 128)
+    torch.cuda.synchronize()
+    assert out.shape == (B, S, hq * 128) and out.is_contiguous()
+    for b0 in range(0, B, 256):
+        part = lens[b0:b0 + 256]
+        packed = [torch.cat([t[b0 + b, :, :n].transpose(0, 1) for b, n in enumerate(part)])
+                  for t in qkv]
+        cu = torch.tensor([0] + part, dtype=torch.int32).cumsum(0, dtype=torch.int32).to(gpu)
+        ref = flash_attention_prefill(*packed, cu, 128 ** -0.5, hq, hkv, 128,
+                                      max_seqlen=max(part)).reshape(sum(part), -1)
+        got = torch.cat([out[b0 + b, :n] for b, n in enumerate(part)])
+        assert torch.equal(got, ref)
+    for b, n in enumerate(lens):
+        assert not out[b, n:].any()
+
+
 def test_prefill_golden_fixture(gpu):
     from pathlib import Path
 
