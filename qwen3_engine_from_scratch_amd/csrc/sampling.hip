@@ -185,9 +185,13 @@ struct Shared {
 // One part's results of the parallel passes (one per row and part, in the
 // workspace).
 struct alignas(16) PartOut {
-  uint32_t kmax;                  // the part's largest key (kmax, ncand: one 8-byte load)
+  uint32_t kmax;                  // the part's largest key (kmax, ncand: one 8-byte load);
+                                  // top-p alone: t_lo << 16 above it, every token with
+                                  // key >= t_lo is listed
   int32_t ncand;                  // candidates written, -1 none
-  unsigned long long best;        // greedy rows: (key + 1) << 32 | ~index, the first maximum
+  unsigned long long best;        // greedy rows: (key + 1) << 32 | ~index, the first maximum;
+                                  // rows drawn uncut: the part's draw (score, ~index);
+                                  // top-p alone: the part's mass (a double)
   unsigned long long cand[kCap];  // (key << 32) | token index
 };
 
@@ -196,6 +200,11 @@ struct alignas(16) PartOut {
 // 55 for two and 65 for eight), each part at least one round (kThreads * 8
 // tokens); 1 means the single-workgroup form.
 constexpr int kMaxParts = 8;
+// Top-p alone: tokens that the parts of a row list between them (each part
+// its share, at least; ties add to it).  Nucleus sets of language-model logits are mostly
+// below a few hundred tokens; a row whose cut lies past the listed ones is
+// streamed by one workgroup as without parts.
+constexpr int kNucleusList = 512;
 __host__ __device__ inline int parts_for(int64_t rows, int64_t vocab) {
   int p = rows <= 32 ? kMaxParts : rows <= 64 ? 4 : rows <= 128 ? 2 : 1;
   const int64_t rounds = (vocab + kThreads * 8 - 1) / (kThreads * 8);
@@ -231,6 +240,36 @@ __device__ __forceinline__ unsigned long long block_max_u64(unsigned long long v
     v = o > v ? o : v;
   }
   return __shfl(v, 0, 64);
+}
+
+// Block-wide sum in a fixed order; every thread gets the result.
+__device__ __forceinline__ double block_sum_f64(double v, Shared& sh) {
+#pragma unroll
+  for (int m = 1; m < 64; m <<= 1) v += __shfl_xor(v, m, 64);
+  __syncthreads();
+  double* part = reinterpret_cast<double*>(sh.wmass);
+  if ((threadIdx.x & 63) == 0) part[threadIdx.x >> 6] = v;
+  __syncthreads();
+  const int lane = threadIdx.x & 63;
+  v = lane < kWaves ? part[lane] : 0.0;
+#pragma unroll
+  for (int m = 1; m < kWaves; m <<= 1) v += __shfl_xor(v, m, 64);
+  return __shfl(v, 0, 64);
+}
+
+// Gumbel-max candidate of one token: (ordered score, complemented index).
+__device__ __forceinline__ unsigned long long draw_candidate(uint32_t key, int64_t idx,
+                                                             uint32_t draw, float inv_t) {
+  const float sc = key_value(key) * inv_t + gumbel_of(draw);
+  const uint32_t sb = __float_as_uint(sc);
+  const uint32_t so = (sb & 0x80000000u) ? ~sb : (sb | 0x80000000u);
+  return (static_cast<unsigned long long>(so) << 32) | (~static_cast<uint32_t>(idx));
+}
+
+// Softmax weight relative to the maximum, in fixed point.
+__device__ __forceinline__ unsigned long long fixed_weight(uint32_t key, float inv_t, float xmax) {
+  const float w = __expf(key_value(key) * inv_t - xmax);
+  return static_cast<unsigned long long>(static_cast<double>(w) * kFix + 0.5);
 }
 
 // Appends (key, index) of the lanes where q holds to the block's candidate
@@ -493,10 +532,11 @@ __device__ __forceinline__ int find_count_bin_block(const uint32_t* h, int64_t n
 // converted to double, exceeds it (there is one when top_p < 1 and the total
 // is positive).  Returns the bin, or -1, and sets `run` to the mass above
 // it.  The same block-wide scan as find_count_bin_block; the caller has
-// passed a barrier since the last read of sh.sel_bin.
+// passed a barrier since the last read of sh.sel_bin.  given_limit: the
+// limit is the caller's (the bins hold only the tokens that can be kept).
 __device__ __forceinline__ int find_mass_bin_block(const unsigned long long* m, float top_p,
                                                    double& limit, unsigned long long& run,
-                                                   Shared& sh) {
+                                                   Shared& sh, bool given_limit = false) {
   const int top = kHiBins - 1 - kBinsPerThread * static_cast<int>(threadIdx.x);
   unsigned long long mine = 0;
 #pragma unroll
@@ -504,7 +544,7 @@ __device__ __forceinline__ int find_mass_bin_block(const unsigned long long* m, 
   if (threadIdx.x == 0) sh.sel_bin = -1;  // before the scan's barriers
   unsigned long long total;
   unsigned long long r = block_scan_u64(mine, total, sh);
-  limit = static_cast<double>(fmaxf(top_p, 0.f)) * static_cast<double>(total);
+  if (!given_limit) limit = static_cast<double>(fmaxf(top_p, 0.f)) * static_cast<double>(total);
   if (static_cast<double>(r) <= limit && static_cast<double>(r + mine) > limit) {
 #pragma unroll
     for (int j = 0; j < kBinsPerThread; ++j) {
@@ -536,53 +576,85 @@ __device__ __forceinline__ void part_values(int P, T none, F&& get, T (&v)[kMaxP
 // The parallel form's first kernel, workgroup (row, part): for a greedy row
 // the part's first maximum; for a row that top-k cuts, the part's largest
 // key and its tokens at or above its own threshold (a list of -1 entries:
-// more than kCap, or nothing cut by top-k).  A part of at most 8 rounds is
-// held in registers for both of its passes.
+// more than kCap); for a row that only top-p cuts, the same with a threshold
+// that the part's share of kNucleusList tokens reach, and the part's softmax
+// mass relative to its own maximum (one pass instead of the row's maximum
+// first: the merge rescales the parts' sums, whose relative error, that of
+// the weights' 32-bit exponentials, stays); for a row that nothing cuts, the
+// draw itself over the part.  A part of at most 8 rounds is held in
+// registers for all of its passes.
+//
+// One workgroup per row is bound by the row's passes on one CU (about 20 us
+// each), which is why the uncut rows are split too: top-p 0.9 over 8 x 151,936
+// logits 88.0 -> 28.4 us; over 62 rows 104.6 -> 34.8; no cut at all, 44 rows, 178.6 -> 31.5.
 template <bool kVec>
 __global__ __launch_bounds__(kThreads) void sample_part_kernel(const uint16_t* logits,
                                                                int64_t row_s, int64_t vocab,
                                                                const float* temperature,
-                                                               const int32_t* top_k, int P,
-                                                               PartOut* parts) {
+                                                               const int32_t* top_k,
+                                                               const float* top_p, uint64_t seed,
+                                                               int P, PartOut* parts) {
   __shared__ Shared sh;
   const int64_t row = blockIdx.x / P;
   const int c = static_cast<int>(blockIdx.x % P);
   const uint16_t* p = logits + row * row_s;
-  const bool greedy = !((temperature ? temperature[row] : 0.f) > 0.f);
-  const int64_t kreq = top_k ? top_k[row] : 0;
-  const int tid = threadIdx.x;
   int64_t lo, hi;
   part_range(vocab, P, c, lo, hi);
-  PartOut& po = parts[row * P + c];
-  if (!greedy && (kreq <= 0 || kreq >= vocab)) {  // top-k cuts nothing: no list
-    if (tid == 0) po.ncand = -1;
-    return;
-  }
-  if (!greedy) {
-    for (int i = tid; i < kHiBins; i += kThreads) sh.cnt[i] = 0;
-    if (tid == 0) sh.ncand = 0;
-    __syncthreads();
-  }
-  if (greedy) {  // the part's first largest value, as the single-workgroup greedy path
-    unsigned long long best = 0;
-    for_each_round_in<kVec>(p, lo, hi, [&](int64_t i0, const uint32_t* b, auto full) {
-      const unsigned long long cb = greedy_round(i0, b, hi, full);
-      best = cb > best ? cb : best;
-    });
-    best = block_max_u64(best, sh);
-    if (tid == 0) po.best = best;
-    return;
-  }
-  // The part keeps every token whose key is >= t_lo, a key that at least
-  // kreq of the part's tokens reach: then a part token below t_lo has kreq
-  // tokens of the row strictly above it, so the list holds every token at
-  // or above the row's k-th largest key.  t_lo is the kreq-th largest of the
-  // threads' own largest keys (kreq threads reaching it are kreq distinct
-  // tokens), found on a histogram of those, one LDS atomic per thread; a
-  // kreq above the thread count takes the high bin of the kreq-th largest
-  // token from a histogram of every token instead.
   const int64_t n_part = hi - lo;
-  auto passes = [&](auto&& visit) {
+  const float temp = temperature ? temperature[row] : 0.f;
+  const bool greedy = !(temp > 0.f);
+  const float inv_t = 1.f / temp;
+  int64_t kreq = top_k ? top_k[row] : 0;
+  const bool uncut = !greedy && (kreq <= 0 || kreq >= vocab);  // top-k cuts nothing
+  const int tid = threadIdx.x;
+  PartOut& po = parts[row * P + c];
+  auto run = [&](auto&& visit) {
+    // (uncut rows are marked unlikely: their code then lies out of the way of
+    // the top-k path, whose every step already waits for cold instructions)
+    if (__builtin_expect(uncut && !((top_p ? top_p[row] : 1.f) < 1.f), 0)) {  // the part's draw
+      unsigned long long best = 0;
+      visit([&](int64_t i0, const uint32_t* b, auto full) {
+#pragma unroll
+        for (int h = 0; h < 2; ++h) {  // one Philox block per four tokens (i0 is a multiple of 8)
+          if (!full && i0 + 4 * h >= hi) break;
+          const q3::u32x4 d = draws4(seed, row, (i0 >> 2) + h);
+#pragma unroll
+          for (int j = 0; j < 4; ++j) {
+            const int64_t i = i0 + 4 * h + j;
+            const uint32_t key = okey(b[4 * h + j]);
+            const unsigned long long cd = draw_candidate(key, i, d[j], inv_t);
+            if ((full || i < hi) && key != 0 && cd > best) best = cd;
+          }
+        }
+      });
+      best = block_max_u64(best, sh);
+      if (tid == 0) po.best = best;
+      return;
+    }
+    if (uncut) kreq = kNucleusList / P;  // top-p alone: the tokens this part lists
+    if (!greedy) {
+      for (int i = tid; i < kHiBins; i += kThreads) sh.cnt[i] = 0;
+      if (tid == 0) sh.ncand = 0;
+      __syncthreads();
+    }
+    if (greedy) {  // the part's first largest value, as the single-workgroup greedy path
+      unsigned long long best = 0;
+      visit([&](int64_t i0, const uint32_t* b, auto full) {
+        const unsigned long long cb = greedy_round(i0, b, hi, full);
+        best = cb > best ? cb : best;
+      });
+      best = block_max_u64(best, sh);
+      if (tid == 0) po.best = best;
+      return;
+    }
+    // The part keeps every token whose key is >= t_lo, a key that at least
+    // kreq of the part's tokens reach: then a part token below t_lo has kreq
+    // tokens of the row strictly above it, so the list holds every token at
+    // or above the row's k-th largest key.  t_lo is the kreq-th largest of the
+    // threads' own largest keys (kreq threads reaching it are kreq distinct
+    // tokens), found on a histogram of those, one LDS atomic per thread; a
+    // kreq above the thread count takes the high bin of the kreq-th largest
+    // token from a histogram of every token instead.
     // each thread's largest key: whole rounds on raw keys, a NaN seen there
     // sends the thread through its tokens again on exact keys
     uint32_t tmax = 0, rmax = 0;
@@ -639,6 +711,31 @@ __global__ __launch_bounds__(kThreads) void sample_part_kernel(const uint16_t* l
       int64_t above = 0;
       t_lo = static_cast<uint32_t>(find_count_bin_block(sh.cnt, kreq, above, sh)) << kLoBits;
     }
+    if (__builtin_expect(uncut, 0)) {
+      // the part's mass: numbers only (a NaN's weight is 0), in doubles; a
+      // part of nothing but -inf and NaN has none, and where the maximum is
+      // not finite the row goes to the single workgroup
+      const float xm = key_value(kmax) * inv_t;
+      const bool none = kmax <= 0x7Fu;
+      double m = 0.0;
+      if (!none && xm < INFINITY && xm > -INFINITY)
+        visit([&](int64_t i0, const uint32_t* b, auto full) {
+#pragma unroll
+          for (int e = 0; e < 8; ++e) {
+            const float w = __expf(__uint_as_float(b[e] << 16) * inv_t - xm);
+            if (full || i0 + e < hi) m += static_cast<double>(fmaxf(w, 0.f));
+          }
+        });
+      m = block_sum_f64(m, sh);
+      if (tid == 0) po.best = static_cast<unsigned long long>(__double_as_longlong(m));
+      if (none || !(xm < INFINITY && xm > -INFINITY)) {
+        if (tid == 0) {
+          po.kmax = kmax;
+          po.ncand = none ? 0 : -1;
+        }
+        return;
+      }
+    }
     visit([&](int64_t i0, const uint32_t* b, auto full) {
       bool q[8], any = false;
       uint32_t keys[8];
@@ -685,29 +782,32 @@ __global__ __launch_bounds__(kThreads) void sample_part_kernel(const uint16_t* l
     const int n = sh.ncand;
     const bool ok = n <= kCap;
     if (tid == 0) {
-      po.kmax = kmax;
+      po.kmax = uncut ? kmax | (t_lo << 16) : kmax;
       po.ncand = ok ? n : -1;
     }
     if (ok)
       for (int i = tid; i < n; i += kThreads) po.cand[i] = sh.cand[i];
   };
   constexpr int kB = batch_rounds<kVec>();
-  if (n_part <= kB * kPerRound) {  // one batch: both passes over registers
+  if (n_part <= kB * kPerRound) {  // one batch: every pass over registers, loaded before
+    // the row's parameters are waited for (they decide only which passes run)
     q3::u32x4 v[kB];
     load_rounds<kVec, kB>(p + lo, n_part, 0, v);
-    passes([&](auto&& f) {
+    run([&](auto&& f) {
       visit_rounds<kB>(n_part, 0, v, [&](int64_t i0, const uint32_t* b, auto full) {
         f(lo + i0, b, full);
       });
     });
   } else {
-    passes([&](auto&& f) { for_each_round_in<kVec>(p, lo, hi, f); });
+    run([&](auto&& f) { for_each_round_in<kVec>(p, lo, hi, f); });
   }
 }
 
-// One workgroup per row.  kPre: greedy rows and, when every part kept its
-// list, passes A and B run over the parts' lists instead of the row;
-// otherwise the workgroup streams the row for them itself.
+// One workgroup per row.  kPre: greedy rows, rows drawn uncut and, when every
+// part kept its list, passes A to E run over the parts' results instead of
+// the row; otherwise the workgroup streams the row for them itself.  For
+// top-p alone the union of the lists is every token at or above the largest
+// of the parts' thresholds, and the cut must lie among those.
 template <bool kVec, bool kPre>
 __global__ __launch_bounds__(kThreads) void sample_kernel(const uint16_t* logits, int64_t row_s,
                                                           int64_t vocab, const float* temperature,
@@ -719,9 +819,29 @@ __global__ __launch_bounds__(kThreads) void sample_kernel(const uint16_t* logits
   const int64_t row = blockIdx.x;
   const uint16_t* p = logits + row * row_s;
   const float temp = temperature ? temperature[row] : 0.f;
+  const int64_t kreq = top_k ? top_k[row] : 0;
+  const float pcut = top_p ? top_p[row] : 1.f;
   const int tid = threadIdx.x;
   const int lane = tid & 63, wave = tid >> 6;
   const PartOut* rp = kPre ? parts + row * P : nullptr;
+
+  // One round trip with the row's parameters: every part's (kmax, ncand) and,
+  // ahead of knowing the counts, entry tid % L of part tid / L (L = kThreads
+  // / P entries per part: all of a short list).
+  const int L = kPre ? kThreads / P : 0;
+  const int cpart = kPre ? (tid / L < P ? tid / L : P - 1) : 0;
+  const int coff = kPre ? tid - (tid / L) * L : 0;
+  unsigned long long spec = 0;
+  unsigned long long hdr[kMaxParts];
+  if constexpr (kPre) {
+    spec = rp[cpart].cand[coff];
+    part_values(P, 0ull, [&](int c) {
+      return *reinterpret_cast<const unsigned long long*>(&rp[c].kmax);
+    }, hdr);
+    // the loads stay here (the compiler would otherwise move them into the
+    // branches that use them, after the parameters' round trip)
+    asm volatile("" ::"v"(spec), "v"(hdr[0]));
+  }
 
   // ---- greedy -----------------------------------------------------------
   if (kPre && !(temp > 0.f)) {
@@ -757,11 +877,22 @@ __global__ __launch_bounds__(kThreads) void sample_kernel(const uint16_t* logits
     return;
   }
 
-  const int64_t kreq = top_k ? top_k[row] : 0;
   const int64_t k = (kreq <= 0 || kreq > vocab) ? vocab : kreq;
-  const float pcut = top_p ? top_p[row] : 1.f;
   const bool use_p = pcut < 1.f;
   const float inv_t = 1.f / temp;
+  const bool uncut = kreq <= 0 || kreq >= vocab;  // as the part kernel
+
+  if (kPre && __builtin_expect(uncut && !use_p, 0)) {  // the best of the parts' draws
+    if (tid == 0) {
+      unsigned long long v[kMaxParts];
+      part_values(P, 0ull, [&](int c) { return rp[c].best; }, v);
+      unsigned long long b = 0;
+#pragma unroll
+      for (int c = 0; c < kMaxParts; ++c) b = v[c] > b ? v[c] : b;
+      out[row] = b ? static_cast<int64_t>(~static_cast<uint32_t>(b)) : 0;
+    }
+    return;
+  }
 
   // Appends (key, index) of the lanes where q holds to the candidate list:
   // one LDS atomic per wave.  Called by every lane of the wave.
@@ -801,21 +932,10 @@ __global__ __launch_bounds__(kThreads) void sample_kernel(const uint16_t* logits
   // ---- A: high-bin counts and the maximum key ----------------------------
   uint32_t kmax = 0;
   bool from_list = false;  // the parts' lists stand for the row in passes A, B
+  bool nucleus = false;    // ... of a row that only top-p cuts,
+  uint32_t t_all = 0;      // where the lists hold every token at or above this key
+  double nucleus_limit = 0.0;  // and this is top_p x the row's whole mass
   if constexpr (kPre) {
-    // One round trip: every part's (kmax, ncand) and, ahead of knowing the
-    // counts, entry tid % L of part tid / L (L = kThreads / P entries per
-    // part: all of a short list).
-    const int L = kThreads / P;
-    const int cpart = tid / L < P ? tid / L : P - 1;
-    const int coff = tid - (tid / L) * L;
-    const unsigned long long spec = rp[cpart].cand[coff];
-    unsigned long long hdr[kMaxParts];
-    part_values(P, 0ull, [&](int c) {
-      return *reinterpret_cast<const unsigned long long*>(&rp[c].kmax);
-    }, hdr);
-    // the entry's load stays here, in flight with the counts (the compiler
-    // would otherwise move it into the branch that uses it, after them)
-    asm volatile("" ::"v"(spec));
     int nc[kMaxParts];
     int total = 0;
     from_list = true;
@@ -823,14 +943,32 @@ __global__ __launch_bounds__(kThreads) void sample_kernel(const uint16_t* logits
 #pragma unroll
     for (int c = 0; c < kMaxParts; ++c) {
       nc[c] = static_cast<int>(hdr[c] >> 32);
-      const uint32_t km = static_cast<uint32_t>(hdr[c]);
+      const uint32_t km = static_cast<uint32_t>(hdr[c]) & 0xFFFFu;
       from_list = from_list && nc[c] >= 0;
       short_list = short_list && nc[c] <= L;
       total += nc[c] > 0 ? nc[c] : 0;
       kmax = km > kmax ? km : kmax;
     }
     from_list = from_list && total <= kCap;
-    if (from_list && short_list) {  // uniform
+    if (__builtin_expect(uncut && from_list, 0)) {  // uniform
+      unsigned long long mass[kMaxParts];
+      part_values(P, 0ull, [&](int c) { return rp[c].best; }, mass);
+      const float xm = key_value(kmax) * inv_t;
+      from_list = kmax > 0x7Fu && xm < INFINITY && xm > -INFINITY;
+      nucleus = from_list;
+      double whole = 0.0;
+#pragma unroll
+      for (int c = 0; c < kMaxParts; ++c) {
+        const uint32_t tl = static_cast<uint32_t>(hdr[c]) >> 16;
+        t_all = tl > t_all ? tl : t_all;
+        const float xc = key_value(static_cast<uint32_t>(hdr[c]) & 0xFFFFu) * inv_t;
+        const double m = __longlong_as_double(static_cast<long long>(mass[c]));
+        if (m > 0.0) whole += m * exp(static_cast<double>(xc) - static_cast<double>(xm));
+      }
+      nucleus_limit = static_cast<double>(fmaxf(pcut, 0.f)) * (whole * kFix);
+    }
+    bool sorted = from_list && short_list && (!nucleus || total <= kThreads / 4);
+    if (sorted) {  // uniform
       // A short union (the usual case: k plus a few per part): one entry
       // per thread, sorted by key (descending) and token index (ascending)
       // with a bitonic network; the top-k list is then its first k
@@ -890,35 +1028,34 @@ __global__ __launch_bounds__(kThreads) void sample_kernel(const uint16_t* logits
       }
       const uint32_t key = static_cast<uint32_t>(x >> 32);
       const uint32_t idx = ~static_cast<uint32_t>(x);
-      const bool in_k = tid < k && tid < total;
+      const bool in_k = tid < k && tid < total && key >= t_all;
       bool kept = in_k;
       if (use_p) {
-        const float xmax = key_value(kmax) * inv_t;
-        unsigned long long wf = 0;
-        if (in_k) {
-          const float w = __expf(key_value(key) * inv_t - xmax);
-          wf = static_cast<unsigned long long>(static_cast<double>(w) * kFix + 0.5);
-        }
+        const unsigned long long wf =
+            in_k ? fixed_weight(key, inv_t, key_value(kmax) * inv_t) : 0ull;
         unsigned long long mass;
         const unsigned long long before = block_scan_u64(wf, mass, sh);
-        const double limit = static_cast<double>(fmaxf(pcut, 0.f)) * static_cast<double>(mass);
+        const double limit =
+            nucleus ? nucleus_limit
+                    : static_cast<double>(fmaxf(pcut, 0.f)) * static_cast<double>(mass);
         kept = in_k && static_cast<double>(before) <= limit;
+        // top-p alone: a cut past the lists' tokens needs the row
+        if (__builtin_expect(nucleus, 0) && !(static_cast<double>(mass) > limit))
+          sorted = from_list = false;
       }
-      unsigned long long best = 0;
-      if (kept && key != 0) {  // as pass E's offer
-        const float sc = key_value(key) * inv_t + gumbel_of(draws4(seed, row, idx >> 2)[idx & 3]);
-        const uint32_t sb = __float_as_uint(sc);
-        const uint32_t so = (sb & 0x80000000u) ? ~sb : (sb | 0x80000000u);
-        best = (static_cast<unsigned long long>(so) << 32) | (~idx);
+      if (sorted) {  // uniform
+        unsigned long long best = 0;
+        if (kept && key != 0) best = draw_candidate(key, idx, draws4(seed, row, idx >> 2)[idx & 3], inv_t);
+        best = block_max_u64(best, sh);
+        if (tid == 0) out[row] = best ? static_cast<int64_t>(~static_cast<uint32_t>(best)) : 0;
+        return;
       }
-      best = block_max_u64(best, sh);
-      if (tid == 0) out[row] = best ? static_cast<int64_t>(~static_cast<uint32_t>(best)) : 0;
-      return;
     }
     if (from_list) {
       for (int i = tid; i < kHiBins; i += kThreads) sh.cnt[i] = 0;
       if (tid < kLoBins) sh.lo_cnt[tid] = 0;
       __syncthreads();
+      unsigned long long listed = 0;
       // entry e of the concatenated lists: part c's run starts at the sum
       // of the runs before it
       for (int e = tid; e < total; e += kThreads) {
@@ -933,15 +1070,28 @@ __global__ __launch_bounds__(kThreads) void sample_kernel(const uint16_t* logits
         }
         const unsigned long long cd = rp[c].cand[e - before];
         sh.cand[e] = cd;
-        atomicAdd(&sh.cnt[static_cast<uint32_t>(cd >> 32) >> kLoBits], 1u);
+        const uint32_t key = static_cast<uint32_t>(cd >> 32);
+        if (!nucleus)
+          atomicAdd(&sh.cnt[key >> kLoBits], 1u);
+        else if (key >= t_all)
+          listed += fixed_weight(key, inv_t, key_value(kmax) * inv_t);
       }
       ncand = total;
       __syncthreads();
-    } else {
-      kmax = 0;
+      if (nucleus) {  // top-p alone: a cut past the lists' tokens needs the row
+        unsigned long long mass;
+        block_scan_u64(listed, mass, sh);
+        if (!(static_cast<double>(mass) > nucleus_limit)) {
+          from_list = false;
+          ncand = -1;
+        }
+      }
     }
   }
   if (!from_list) {
+    nucleus = false;
+    kmax = 0;
+    __syncthreads();
     for (int i = tid; i < kHiBins; i += kThreads) sh.cnt[i] = 0;
     if (tid < kLoBins) sh.lo_cnt[tid] = 0;
     if (tid == 0) sh.ncand = 0;
@@ -1014,6 +1164,7 @@ __global__ __launch_bounds__(kThreads) void sample_kernel(const uint16_t* logits
   // ---- C, D: the top-p cut over the top-k list ---------------------------
   // kc / tc: the final cut (key and ties kept at it); the kept list is the
   // first min(k, n_p) positions of the sorted top-k list.
+  if (nucleus) kk = t_all;  // nothing below it can be kept: the cut is above
   uint32_t kc = kk;
   int64_t tc = tk, cties = kties;
   if (use_p) {
@@ -1026,31 +1177,25 @@ __global__ __launch_bounds__(kThreads) void sample_kernel(const uint16_t* logits
     }
     __syncthreads();
     const bool partial_k = k < vocab && tk < kties;
-    const float wk = __expf(key_value(kk) * inv_t - xmax);
     visit([&](uint32_t key, int64_t) {
       if (key < kk || (partial_k && key == kk)) return;
-      const float w = __expf(key_value(key) * inv_t - xmax);
-      atomicAdd(&sh.mass[key >> kLoBits],
-                static_cast<unsigned long long>(static_cast<double>(w) * kFix + 0.5));
+      atomicAdd(&sh.mass[key >> kLoBits], fixed_weight(key, inv_t, xmax));
     });
     __syncthreads();
-    const unsigned long long wk_fix =
-        static_cast<unsigned long long>(static_cast<double>(wk) * kFix + 0.5);
+    const unsigned long long wk_fix = fixed_weight(kk, inv_t, xmax);
     if (partial_k && tid == 0) sh.mass[kk >> kLoBits] += wk_fix * static_cast<unsigned long long>(tk);
     __syncthreads();
     // high bins of the cut: the bin holding the first position whose mass
     // before it exceeds the limit
-    double limit;
+    double limit = nucleus_limit;
     unsigned long long above_hi;
-    const int hb = find_mass_bin_block(sh.mass, pcut, limit, above_hi, sh);
+    const int hb = find_mass_bin_block(sh.mass, pcut, limit, above_hi, sh, nucleus);
     if (hb >= 0) {  // else a row without mass (all NaN): no cut
       auto lo_hist = [&](uint32_t key, int64_t) {
         if (static_cast<int>(key >> kLoBits) != hb || key < kk) return;
         atomicAdd(&sh.lo_cnt[key & (kLoBins - 1)], 1u);
         if (partial_k && key == kk) return;
-        const float w = __expf(key_value(key) * inv_t - xmax);
-        atomicAdd(&sh.lo_mass[key & (kLoBins - 1)],
-                  static_cast<unsigned long long>(static_cast<double>(w) * kFix + 0.5));
+        atomicAdd(&sh.lo_mass[key & (kLoBins - 1)], fixed_weight(key, inv_t, xmax));
       };
       if (ncand >= 0) {
         visit(lo_hist);
@@ -1099,8 +1244,9 @@ __global__ __launch_bounds__(kThreads) void sample_kernel(const uint16_t* logits
           if (keep == 0) keep = 1;  // cannot happen unless rounding: keep the first
           // the top-p cut is inside the top-k list (its key >= kk)
           kc = key;
-          cties = key == kk ? kties : sh.lo_cnt[bin];
-          tc = key == kk ? (keep < tk ? keep : tk) : keep;
+          const bool at_k = key == kk && !nucleus;
+          cties = at_k ? kties : sh.lo_cnt[bin];
+          tc = at_k ? (keep < tk ? keep : tk) : keep;
           break;
         }
         r2 += m;
@@ -1114,11 +1260,7 @@ __global__ __launch_bounds__(kThreads) void sample_kernel(const uint16_t* logits
   const bool need_rank = tc < cties;
   unsigned long long bestk = 0;  // (ordered score, complemented index)
   auto offer = [&](uint32_t key, int64_t idx, uint32_t draw) {
-    const float sc = key_value(key) * inv_t + gumbel_of(draw);
-    const uint32_t sb = __float_as_uint(sc);
-    const uint32_t so = (sb & 0x80000000u) ? ~sb : (sb | 0x80000000u);
-    const unsigned long long c =
-        (static_cast<unsigned long long>(so) << 32) | (~static_cast<uint32_t>(idx));
+    const unsigned long long c = draw_candidate(key, idx, draw, inv_t);
     bestk = c > bestk ? c : bestk;
   };
   if (ncand >= 0 && (!need_rank || cties <= kThreads)) {
@@ -1252,7 +1394,8 @@ void launch_parts(const uint16_t* lg, int64_t row_stride, int64_t rows, int64_t 
                   const float* temperature, const int32_t* top_k, const float* top_p,
                   uint64_t seed, int64_t* out, int P, PartOut* parts, hipStream_t s) {
   hipLaunchKernelGGL(sample_part_kernel<kVec>, dim3(static_cast<unsigned>(rows * P)),
-                     dim3(kThreads), 0, s, lg, row_stride, vocab, temperature, top_k, P, parts);
+                     dim3(kThreads), 0, s, lg, row_stride, vocab, temperature, top_k, top_p,
+                     seed, P, parts);
   hipLaunchKernelGGL((sample_kernel<kVec, true>), dim3(static_cast<unsigned>(rows)),
                      dim3(kThreads), 0, s, lg, row_stride, vocab, temperature, top_k, top_p, seed,
                      out, P, parts);

@@ -214,3 +214,46 @@ def test_parallel_form_draws_the_same_tokens(gpu, B, V, stride):
     for seed in (1, 2):
         one, par = _both_forms(x, t, k, p, seed)
         assert torch.equal(one, par), f"B={B} V={V} seed={seed}: rows {(one != par).nonzero().view(-1)[:8].tolist()} differ"
+
+
+@pytest.mark.parametrize("B,V", [(1, 151936), (8, 151936), (64, 151936), (65, 40000), (24, 16390),
+                                 (9, 8193), (5, 9000)])
+def test_parallel_form_draws_uncut_rows_the_same(gpu, B, V):
+    """Rows that top-k does not cut, drawn part by part: the single form's
+    tokens exactly.  Nucleus sets inside the parts' lists (a short union of
+    few finite logits, the usual one) and past them (flat rows), ties at and
+    around the cut and across parts, top_p 0, below 0 and at 1, parts and
+    rows of -inf and NaN, +inf logits, a temperature whose inverse is inf."""
+    g = torch.Generator().manual_seed(B * 31 + V)
+    a = torch.rand(B, 1, generator=g) * 2.5 + 0.3          # from flat to peaked
+    x = a * -torch.log(torch.rand(B, V, generator=g))      # Zipf-like rows
+    t = torch.rand(B, generator=g) * 0.8 + 0.5
+    p = torch.tensor([[0.9, 0.5, 1.0, 0.99, 0.0, 0.75, -1.0][r % 7] for r in range(B)])
+    inf, nan = float("inf"), float("nan")
+    special = [
+        lambda r: r.fill_(1.25),                            # all tied: the cut is inside
+        lambda r: r[: V // 2].fill_(-inf),                  # whole parts without mass
+        lambda r: (r.fill_(-inf), r[5 :: V // 100].copy_(torch.arange(len(r[5 :: V // 100])) / 16)),
+        lambda r: r.fill_(-inf),
+        lambda r: r.fill_(nan),
+        lambda r: r[::7].fill_(nan),
+        lambda r: r[V - 3 :].fill_(inf),
+        lambda r: r.round_(),                               # few distinct values
+        lambda r: r.copy_((r > 3).float() * 4),             # two values
+    ]
+    # each special row beside ordinary ones, at top_p 0.5 and others
+    for i, f in enumerate(special):
+        if 3 * i + 1 < B:
+            f(x[3 * i + 1])
+    if B > 40:
+        t[40] = 1e-39
+    if B == 5:
+        special[0](x[1]), special[7](x[3])
+    xd, td, pd = x.to(torch.bfloat16).to(gpu), t.to(gpu), p.to(gpu)
+    announce(f"sampling uncut rows B={B} V={V}")
+    for seed in (3, 4, 5):
+        for k in (0, V):
+            kd = torch.full((B,), k, dtype=torch.int32, device=gpu)
+            one, par = _both_forms(xd, td, kd, pd, seed)
+            assert torch.equal(one, par), \
+                f"seed={seed}: rows {(one != par).nonzero().view(-1)[:8].tolist()} differ"
