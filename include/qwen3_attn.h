@@ -189,6 +189,25 @@ int qwen3_paged_decode_noalloc_bf16(const void* q, const int64_t q_strides[2],
                                     int B, int num_heads, int num_kv_heads, int head_dim,
                                     int block_size, float scale, void* stream);
 
+/* qwen3_paged_decode_bf16 without its merge launch, for B <= 2048: sequence-heads
+ * split across waves are left as partial results in the workspace, for
+ * qwen3_decode_chain_bf16 (qwen3_model_ops.h) to combine; the others are
+ * written to out.  qwen3_paged_decode_partials_waves(): the waves the
+ * workspace is laid out for on the current device (0: cannot be queried). */
+int64_t qwen3_paged_decode_partials_waves(void);
+int qwen3_paged_decode_partials_bf16(const void* q, const int64_t q_strides[2],
+                                    const void* k_cache, const int64_t k_strides[3],
+                                    const void* v_cache, const int64_t v_strides[3],
+                                    int64_t num_blocks,
+                                    const int32_t* block_table, int64_t bt_row_stride,
+                                    int64_t max_rows, int64_t max_pages,
+                                    const int32_t* seq_lens, int seq_len_bias,
+                                    const int32_t* row_ids,
+                                    void* out, const int64_t out_strides[2],
+                                    int B, int num_heads, int num_kv_heads, int head_dim,
+                                    int block_size, float scale, void* workspace,
+                                    size_t workspace_bytes, void* stream);
+
 /* ------------------------------------------------------------------------
  * Decode-form K/V slot write.
  *

@@ -34,6 +34,7 @@
 //    workgroup per partition of tiles) with the same tile math.
 #include <mutex>
 
+#include "paged_decode_merge.hpp"
 #include "paged_decode_tile.hpp"
 
 namespace {
@@ -52,6 +53,10 @@ __device__ __forceinline__ float finish_l(SoftmaxState& st) {
 
 // ---------------------------------------------------------------------------
 // Stream path: persistent waves over the flat tile list.
+
+__device__ __forceinline__ StreamPartials partials_of(const DecodeArgs& a) {
+  return {a.s_po, a.s_plse, a.s_pref, a.s_meta, a.Hkv, a.G};
+}
 
 // Load-side cursor of a wave: the next tile to fetch in the flat list.
 struct Cursor {
@@ -79,12 +84,13 @@ void paged_decode_stream_kernel(DecodeArgs a) {
   const int64_t T = static_cast<int64_t>(a.Hkv) * total;
   const int64_t W = static_cast<int64_t>(gridDim.x) * kWaves;
   int64_t pw = q3::cdiv(T, W);
-  pw = pw < kMinTilesPerWave ? kMinTilesPerWave : pw;
+  const int64_t least = T <= kChunk * gridDim.x ? kChunk : kMinTilesPerWave;
+  pw = pw < least ? least : pw;
   if (blockIdx.x == 0) {
     for (int b = tid; b <= B; b += kWaves * 64) a.s_pref[b] = s_pref[b];
     if (tid == 0) a.s_meta[0] = static_cast<int32_t>(pw);
   }
-  const int64_t w = static_cast<int64_t>(blockIdx.x) * kWaves + wave;
+  const int64_t w = wave_index(T, W, pw, wave);
   const int64_t g0 = w * pw;
   if (g0 >= T) return;
 
@@ -216,72 +222,16 @@ void paged_decode_stream_kernel(DecodeArgs a) {
 
 // Combines the partials of every sequence-head split across waves and
 // writes zeros for empty contexts.  One workgroup per (kv head, batch entry)
-// with one wave per query head of the group: lanes first fetch the LSEs of up
-// to 64 covering waves at once, then every lane owns two output dims and sums
-// the weighted partials kBatch waves at a time.
+// with one wave per query head of the group.
 __global__ __launch_bounds__(kMaxG * 64) void paged_decode_stream_merge_kernel(DecodeArgs a) {
-  constexpr int kBatch = 8;
-  const int hkv = blockIdx.x;
-  const int b = blockIdx.y;
-  const int lane = threadIdx.x & 63;
-  const int g = threadIdx.x >> 6;  // query head within the group
-  const int G = a.G;
-  if (g >= G) return;
-  const int64_t pref_b = a.s_pref[b];
-  const int n = a.s_pref[b + 1] - static_cast<int32_t>(pref_b);
-  const int64_t hq = static_cast<int64_t>(hkv) * G + g;
-  uint32_t* op = reinterpret_cast<uint32_t*>(a.out + b * a.o_sb + hq * a.o_sh + 2 * lane);
-  if (n == 0) {
-    *op = 0u;
-    return;
-  }
-  const int64_t pw = a.s_meta[0];
-  const int64_t S = static_cast<int64_t>(a.Hkv) * pref_b + static_cast<int64_t>(hkv) * n;
-  const int64_t E = S + n;
-  const int64_t wf = S / pw, wl = (E - 1) / pw;
-  if (wf == wl) return;  // written whole by its wave
-  const int nw = static_cast<int>(wl - wf + 1);
-  auto slot_of = [&](int i) -> int64_t {
-    const int64_t wv = wf + i;
-    const int half = (i == 0 && wv * pw != S) ? 1 : 0;
-    return (wv * 2 + half) * G + g;
-  };
-  // Pass 1: global max of the partial LSEs.
-  float M = q3::kNegInf;
-  for (int i0 = 0; i0 < nw; i0 += 64)
-    if (i0 + lane < nw) M = fmaxf(M, a.s_plse[slot_of(i0 + lane)]);
-#pragma unroll
-  for (int o = 32; o >= 1; o >>= 1) M = fmaxf(M, q3::shfl_xor(M, o));
-  const float M_use = M == q3::kNegInf ? 0.f : M;
-  // Pass 2: weighted sum of the partial outputs (lane owns dims 2*lane, 2*lane+1).
-  float sw = 0.f, o0 = 0.f, o1 = 0.f;
-  for (int i0 = 0; i0 < nw; i0 += 64) {
-    const float wl_lane = (i0 + lane < nw) ? q3::fast_exp2(a.s_plse[slot_of(i0 + lane)] - M_use) : 0.f;
-    float wsum = wl_lane;
-#pragma unroll
-    for (int o = 32; o >= 1; o >>= 1) wsum += q3::shfl_xor(wsum, o);
-    sw += wsum;
-    const int cnt = nw - i0 < 64 ? nw - i0 : 64;
-    for (int j0 = 0; j0 < cnt; j0 += kBatch) {
-      float2 ov[kBatch];
-      float wt[kBatch];
-#pragma unroll
-      for (int j = 0; j < kBatch; ++j) {
-        const bool ok = j0 + j < cnt;
-        wt[j] = __shfl(wl_lane, ok ? j0 + j : 0, 64);
-        ov[j] = ok ? *reinterpret_cast<const float2*>(a.s_po + slot_of(i0 + j0 + j) * kD + 2 * lane)
-                   : float2{0.f, 0.f};
-        wt[j] = ok ? wt[j] : 0.f;
-      }
-#pragma unroll
-      for (int j = 0; j < kBatch; ++j) {
-        o0 += wt[j] * ov[j].x;
-        o1 += wt[j] * ov[j].y;
-      }
-    }
-  }
-  const float inv = sw > 0.f ? 1.f / sw : 0.f;
-  *op = q3::pack_bf16x2(o0 * inv, o1 * inv);
+  // query head within the group (uniform: the addresses stay scalar)
+  const int g = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+  if (g >= a.G) return;
+  const int64_t hq = static_cast<int64_t>(blockIdx.x) * a.G + g;
+  const int b = blockIdx.y, lane = threadIdx.x & 63;
+  uint32_t y;
+  if (merge_partials(partials_of(a), b, hq, lane, y))
+    *reinterpret_cast<uint32_t*>(a.out + b * a.o_sb + hq * a.o_sh + 2 * lane) = y;
 }
 
 // ---------------------------------------------------------------------------
@@ -467,22 +417,6 @@ __global__ __launch_bounds__(kD) void paged_decode_grid_merge_kernel(DecodeArgs 
 // ---------------------------------------------------------------------------
 // Host side.
 
-struct StreamLayout {
-  int64_t po, plse, pref, meta, total;
-};
-
-// Workspace layout of the stream path for `waves` persistent waves and
-// groups of G query heads.
-StreamLayout stream_layout(int B, int64_t waves, int G) {
-  StreamLayout s;
-  s.po = 0;
-  s.plse = s.po + align256(waves * 2 * G * kD * 4);
-  s.pref = s.plse + align256(waves * 2 * G * 4);
-  s.meta = s.pref + align256((static_cast<int64_t>(B) + 1) * 4);
-  s.total = s.meta + 256;
-  return s;
-}
-
 int64_t grid_parts(int64_t max_pages, int block_size) {
   return q3::cdiv(q3::cdiv(max_pages * block_size, kTile), kGridTilesPerPart);
 }
@@ -492,8 +426,10 @@ int64_t grid_bytes(int B, int num_heads, int64_t max_pages, int block_size) {
   return align256(slots * kD * 4) + align256(slots * 4);
 }
 
-// Launches the stream path (attention pass + merge) with its workspace at ws.
-int launch_stream(DecodeArgs& a, char* ws, int wgs, hipStream_t s, const char* who) {
+// Launches the stream path (attention pass + merge, unless the caller merges)
+// with its workspace at ws.
+int launch_stream(DecodeArgs& a, char* ws, int wgs, hipStream_t s, const char* who,
+                  bool merge = true) {
   const StreamLayout L = stream_layout(a.B, int64_t(wgs) * kWaves, a.G);
   a.s_po = reinterpret_cast<float*>(ws + L.po);
   a.s_plse = reinterpret_cast<float*>(ws + L.plse);
@@ -502,7 +438,7 @@ int launch_stream(DecodeArgs& a, char* ws, int wgs, hipStream_t s, const char* w
   q3::clear_error();
   hipLaunchKernelGGL(paged_decode_stream_kernel, dim3(wgs), dim3(kWaves * 64), 0, s, a);
   int rc = q3::launch_status(who);
-  if (rc) return rc;
+  if (rc || !merge) return rc;
   hipLaunchKernelGGL(paged_decode_stream_merge_kernel, dim3(a.Hkv, a.B), dim3(64 * a.G), 0, s,
                      a);
   return q3::launch_status(who);
@@ -554,14 +490,15 @@ extern "C" size_t qwen3_paged_decode_workspace_bytes(int B, int num_heads, int n
   return static_cast<size_t>(grid_bytes(B, num_heads, max_pages, block_size));
 }
 
-extern "C" int qwen3_paged_decode_bf16(
+namespace {
+int decode_impl(
+    const char* who, bool merge,
     const void* q, const int64_t q_strides[2], const void* k_cache, const int64_t k_strides[3],
     const void* v_cache, const int64_t v_strides[3], int64_t num_blocks,
     const int32_t* block_table, int64_t bt_row_stride, int64_t max_rows, int64_t max_pages,
     const int32_t* seq_lens, int seq_len_bias, const int32_t* row_ids, void* out,
     const int64_t out_strides[2], int B, int num_heads, int num_kv_heads, int head_dim,
     int block_size, float scale, void* workspace, size_t workspace_bytes, void* stream) {
-  const char* who = "qwen3_paged_decode_bf16";
   DecodeArgs a;
   if (int rc = prepare(a, who, q, q_strides, k_cache, k_strides, v_cache, v_strides, num_blocks,
                        block_table, bt_row_stride, max_rows, max_pages, seq_lens,
@@ -582,8 +519,10 @@ extern "C" int qwen3_paged_decode_bf16(
   if (B <= kStreamMaxB) {
     const int wgs = stream_workgroups();
     if (wgs <= 0) return q3::fail(QWEN3_EINVAL, "%s: cannot query the device's CU count", who);
-    return launch_stream(a, ws, wgs, s, who);
+    return launch_stream(a, ws, wgs, s, who, merge);
   }
+  if (!merge)
+    return q3::fail(QWEN3_EUNSUPPORTED, "%s: batch %d exceeds %d", who, B, kStreamMaxB);
   const int64_t parts = grid_parts(max_pages, block_size);
   if (parts > 0x7fffffff) return q3::fail(QWEN3_EINVAL, "%s: max_pages too large", who);
   a.max_parts = static_cast<int>(parts);
@@ -598,6 +537,39 @@ extern "C" int qwen3_paged_decode_bf16(
   if (rc || parts == 1) return rc;
   hipLaunchKernelGGL(paged_decode_grid_merge_kernel, dim3(num_heads, B), dim3(kD), 0, s, a);
   return q3::launch_status(who);
+}
+}  // namespace
+
+extern "C" int qwen3_paged_decode_bf16(
+    const void* q, const int64_t q_strides[2], const void* k_cache, const int64_t k_strides[3],
+    const void* v_cache, const int64_t v_strides[3], int64_t num_blocks,
+    const int32_t* block_table, int64_t bt_row_stride, int64_t max_rows, int64_t max_pages,
+    const int32_t* seq_lens, int seq_len_bias, const int32_t* row_ids, void* out,
+    const int64_t out_strides[2], int B, int num_heads, int num_kv_heads, int head_dim,
+    int block_size, float scale, void* workspace, size_t workspace_bytes, void* stream) {
+  return decode_impl("qwen3_paged_decode_bf16", true, q, q_strides, k_cache, k_strides, v_cache,
+                     v_strides, num_blocks, block_table, bt_row_stride, max_rows, max_pages,
+                     seq_lens, seq_len_bias, row_ids, out, out_strides, B, num_heads,
+                     num_kv_heads, head_dim, block_size, scale, workspace, workspace_bytes,
+                     stream);
+}
+
+extern "C" int64_t qwen3_paged_decode_partials_waves(void) {
+  return int64_t(stream_workgroups()) * kWaves;
+}
+
+extern "C" int qwen3_paged_decode_partials_bf16(
+    const void* q, const int64_t q_strides[2], const void* k_cache, const int64_t k_strides[3],
+    const void* v_cache, const int64_t v_strides[3], int64_t num_blocks,
+    const int32_t* block_table, int64_t bt_row_stride, int64_t max_rows, int64_t max_pages,
+    const int32_t* seq_lens, int seq_len_bias, const int32_t* row_ids, void* out,
+    const int64_t out_strides[2], int B, int num_heads, int num_kv_heads, int head_dim,
+    int block_size, float scale, void* workspace, size_t workspace_bytes, void* stream) {
+  return decode_impl("qwen3_paged_decode_partials_bf16", false, q, q_strides, k_cache,
+                     k_strides, v_cache, v_strides, num_blocks, block_table, bt_row_stride,
+                     max_rows, max_pages, seq_lens, seq_len_bias, row_ids, out, out_strides, B,
+                     num_heads, num_kv_heads, head_dim, block_size, scale, workspace,
+                     workspace_bytes, stream);
 }
 
 extern "C" int qwen3_paged_decode_noalloc_bf16(

@@ -5,6 +5,7 @@
 #pragma once
 
 #include "common.hpp"
+#include "paged_decode_merge.hpp"
 
 namespace {
 
@@ -19,7 +20,9 @@ constexpr int kStreamMaxB = 2048;       // batch entries tabulated in LDS
 constexpr int kStreamWgPerCu = 2;       // resident workgroups per CU (2 waves/SIMD)
 constexpr int kStreamMaxWgs = 1024;     // persistent grid cap (512 CUs)
 // Fewest tiles a wave streams: its two load batches, both issued before the
-// first is computed, so a small batch costs one tile round trip per wave.
+// first is computed, so a small batch costs one tile round trip per wave; one
+// batch when that gives no workgroup more than one wave (one sequence of 250
+// tokens, 16/8 heads, with its merge: 10.4 -> 8.8 us; 900 tokens 11.8 -> 11.1).
 constexpr int kMinTilesPerWave = 2 * kChunk;
 
 struct DecodeArgs {
@@ -143,6 +146,18 @@ __device__ __forceinline__ int tabulate(const DecodeArgs& a, int32_t* s_pref, in
   if (tid == 0) s_pref[B] = run;
   __syncthreads();
   return run;
+}
+
+// Index of this wave's range of pw tiles among T tiles and W waves.  A batch
+// too small for every wave (pw at its minimum) is dealt one wave per workgroup
+// first: four streaming waves of one workgroup share a CU's load path, about
+// 46 GB/s, while most CUs idle (16 sequences of 400-800 tokens, 16/8 heads,
+// with their merge: 21.1 -> 16.9 us; 64 of 100-200: 21.5 -> 17.5).  The ranges,
+// and so the bits, do not depend on it.
+__device__ __forceinline__ int64_t wave_index(int64_t T, int64_t W, int64_t pw, int wave) {
+  const bool spread = T <= (W - 1) * pw;
+  return spread ? static_cast<int64_t>(wave) * gridDim.x + blockIdx.x
+                : static_cast<int64_t>(blockIdx.x) * kWaves + wave;
 }
 
 // ---------------------------------------------------------------------------
@@ -359,8 +374,6 @@ int cu_count() {
   }
   return cached[dev];
 }
-
-int64_t align256(int64_t x) { return (x + 255) / 256 * 256; }
 
 // Validates the arguments shared by both decode entry points and fills `a`
 // (everything but the workspace pointers).

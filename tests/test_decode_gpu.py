@@ -283,3 +283,24 @@ def test_decode_batch_sizes_around_tabulation_rounds(gpu, B, invariant):
                                 rows_d[ok.to(gpu)], 16)
     assert_close_attn(out[ok.to(gpu)], ref, f"B={B}")
     assert not out[bad.to(gpu)].any()
+
+
+@pytest.mark.parametrize("lens", [
+    [1], [33],                       # fewer tiles than workgroups
+    [2048], [2049],                  # 1,024 tiles on 512 workgroups: two per wave, then four
+    [16352], [16368], [16385],       # the last range short of, at and past the grid's waves
+    [700, 1, 300, 2000],
+])
+def test_decode_small_batches_around_wave_spreading(gpu, lens):
+    """Small batches run one wave per workgroup first, with one load batch
+    per wave while that covers the tiles: lengths at both edges (16/8 heads
+    on a 256-CU grid), against the fp32 reference."""
+    from qwen3_engine_from_scratch_amd.kernels.paged_attention import paged_attention_decode_hip
+
+    announce(f"decode small batch {lens}")
+    t = make_device_decode(lens, 16, 8, gpu, seed=sum(lens), slack=0.1)
+    out = paged_attention_decode_hip(t["q"], t["k"], t["v"], t["bt"], t["seq_lens"], t["row_ids"],
+                                     16)
+    torch.cuda.synchronize()
+    ref = gpu_dense_decode_fp32(t["q"], t["k"], t["v"], t["bt"], t["seq_lens"], t["row_ids"], 16)
+    assert_close_attn(out, ref, f"lens={lens}")
