@@ -140,6 +140,68 @@ int qwen3_decode_qkv_rope_bf16(const void* h, int64_t h_row_stride,
                                int64_t bt_row_stride, int64_t max_rows, int64_t max_pages,
                                const int32_t* row_ids, int block_size, void* stream);
 
+/* The dense work of a decode step between two attention launches, for M <=
+ * 16 rows, in one launch whose workgroups hand the layer's phases on through
+ * device memory: with the same results, bit for bit,
+ *   the merge of qwen3_paged_decode_partials_bf16 (attn_workspace not NULL) into o,
+ *   qwen3_decode_linear_bf16 residual (o_weight: h_mid, ss_mid from h_in), silu
+ *   (gate_up_weight, norm post_norm_weight) and residual (down_weight: h_out,
+ *   ss_out from h_mid), and qwen3_decode_qkv_rope_bf16 of the next layer
+ *   (qkv_weight not NULL).
+ * h_in, h_mid, h_out (M x hidden), act (M x intermediate), ss_mid, ss_out
+ * (M x hidden / 16) are contiguous; h_out may be h_in.  sync:
+ * qwen3_decode_chain_sync_bytes() bytes, zero before the first launch; every
+ * launch leaves it zero; launches that share one must not overlap.  Shapes:
+ * qwen3_decode_chain_supported() (its launch must fit the device at once). */
+typedef struct {
+  int M, hidden, intermediate, num_heads, num_kv_heads;
+  float eps, head_eps;
+  const void* attn_workspace; /* nullable: o is complete */
+  size_t attn_workspace_bytes;
+  int64_t attn_waves; /* qwen3_paged_decode_partials_waves() */
+  void* o;            /* (M x num_heads * 128) */
+  int64_t o_row_stride;
+  const void* o_weight;
+  int64_t o_weight_row_stride;
+  const void* h_in;
+  void* h_mid;
+  void* h_out;
+  float* ss_mid;
+  float* ss_out;
+  const void* post_norm_weight;
+  const void* gate_up_weight;
+  int64_t gate_up_row_stride;
+  void* act;
+  const void* down_weight;
+  int64_t down_row_stride;
+  uint32_t* sync;
+  const void* in_norm_weight; /* the next layer's, from here on */
+  const void* qkv_weight;     /* nullable: none */
+  int64_t qkv_row_stride;
+  const void* q_norm_weight;
+  const void* k_norm_weight;
+  const float* cos_table;
+  const float* sin_table;
+  int64_t table_row_stride, table_rows;
+  const int64_t* positions; /* nullable */
+  void* q_out;
+  int64_t q_out_strides[2];
+  void* k_cache;
+  void* v_cache;
+  int64_t k_cache_strides[4], v_cache_strides[4];
+  int64_t num_blocks;
+  const int32_t* seq_lens;
+  const int32_t* block_table;
+  int64_t bt_row_stride, max_rows, max_pages;
+  const int32_t* row_ids; /* nullable */
+  int layer_idx, num_layers, block_size;
+} qwen3_decode_chain_args;
+
+size_t qwen3_decode_chain_sync_bytes(void);
+int qwen3_decode_chain_supported(int M, int hidden, int intermediate, int num_heads,
+                                 int num_kv_heads);
+int qwen3_decode_chain_bf16(const qwen3_decode_chain_args* args, void* stream);
+
 /* h_out[r] = embedding[ids[r]] (zero row for an id outside [0, vocab)) and
  * ss_out[r * (hidden / 16) + t] = sum of h^2 over columns 16t .. 16t + 15:
  * the input of the first decode_linear with a norm prologue. */

@@ -19,6 +19,28 @@ _vp = ctypes.c_void_p
 _i = ctypes.c_int
 _i64 = ctypes.c_int64
 
+class DecodeChainArgs(ctypes.Structure):
+    """qwen3_decode_chain_args of include/qwen3_model_ops.h."""
+
+    _fields_ = [
+        ("M", _i), ("hidden", _i), ("intermediate", _i), ("num_heads", _i), ("num_kv_heads", _i),
+        ("eps", ctypes.c_float), ("head_eps", ctypes.c_float),
+        ("attn_workspace", _vp), ("attn_workspace_bytes", ctypes.c_size_t), ("attn_waves", _i64),
+        ("o", _vp), ("o_row_stride", _i64), ("o_weight", _vp), ("o_weight_row_stride", _i64),
+        ("h_in", _vp), ("h_mid", _vp), ("h_out", _vp), ("ss_mid", _vp), ("ss_out", _vp),
+        ("post_norm_weight", _vp), ("gate_up_weight", _vp), ("gate_up_row_stride", _i64),
+        ("act", _vp), ("down_weight", _vp), ("down_row_stride", _i64), ("sync", _vp),
+        ("in_norm_weight", _vp), ("qkv_weight", _vp), ("qkv_row_stride", _i64),
+        ("q_norm_weight", _vp), ("k_norm_weight", _vp), ("cos_table", _vp), ("sin_table", _vp),
+        ("table_row_stride", _i64), ("table_rows", _i64), ("positions", _vp),
+        ("q_out", _vp), ("q_out_strides", _i64 * 2), ("k_cache", _vp), ("v_cache", _vp),
+        ("k_cache_strides", _i64 * 4), ("v_cache_strides", _i64 * 4), ("num_blocks", _i64),
+        ("seq_lens", _vp), ("block_table", _vp), ("bt_row_stride", _i64), ("max_rows", _i64),
+        ("max_pages", _i64), ("row_ids", _vp),
+        ("layer_idx", _i), ("num_layers", _i), ("block_size", _i),
+    ]
+
+
 # name -> (restype, argtypes)
 _SIGNATURES = {
     "qwen3_attn_last_error": (ctypes.c_char_p, []),
@@ -38,6 +60,16 @@ _SIGNATURES = {
     "qwen3_paged_decode_invariant_workspace_bytes": (ctypes.c_size_t,
                                                      [_i, _i, _i, _i, _i64, _i]),
     "qwen3_paged_decode_invariant_bf16": (
+        _i,
+        [_vp, _c_i64p, _vp, _c_i64p, _vp, _c_i64p, _i64,
+         _vp, _i64, _i64, _i64,
+         _vp, _i, _vp,
+         _vp, _c_i64p,
+         _i, _i, _i, _i, _i, ctypes.c_float,
+         _vp, ctypes.c_size_t, _vp],
+    ),
+    "qwen3_paged_decode_partials_waves": (_i64, []),
+    "qwen3_paged_decode_partials_bf16": (
         _i,
         [_vp, _c_i64p, _vp, _c_i64p, _vp, _c_i64p, _i64,
          _vp, _i64, _i64, _i64,
@@ -122,6 +154,9 @@ _SIGNATURES = {
         [_vp, _i64, _vp, _i, _vp, ctypes.c_float, _vp, _i64, _i, _i, _i, _i,
          _vp, _i64, _vp, _i64, _vp, _i64, _vp, _i, _vp],
     ),
+    "qwen3_decode_chain_sync_bytes": (ctypes.c_size_t, []),
+    "qwen3_decode_chain_supported": (_i, [_i, _i, _i, _i, _i]),
+    "qwen3_decode_chain_bf16": (_i, [ctypes.POINTER(DecodeChainArgs), _vp]),
     "qwen3_embed_ss_bf16": (_i, [_vp, _vp, _i64, _i64, _i, _i, _vp, _i64, _vp, _vp]),
     "qwen3_decode_qkv_rope_bf16": (
         _i,

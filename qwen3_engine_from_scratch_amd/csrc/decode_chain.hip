@@ -1,0 +1,664 @@
+// The dense work between two attention launches of a decode step, for at most
+// 16 rows, in one launch:
+//   merge     the streaming attention's partial results -> o     (paged_decode_merge.hpp)
+//   o_proj    h_mid = h + o @ W_o^T                              (qwen3/attention.py:187, decoder.py:49)
+//   gate_up   act = SwiGLU(RMSNorm(h_mid) @ W_gu^T)              (qwen3/mlp.py:31-36)
+//   down      h = h_mid + act @ W_down^T                         (qwen3/decoder.py:55)
+//   qkv       the next layer's q, k, v: RMSNorm, projection, QK-norm, RoPE and
+//             the K/V pool write (as decode_qkv.hip)
+// with the arithmetic, K splits and summation orders of the separate kernels
+// (decode_linear.hip, decode_qkv.hip), so the same bits.
+//
+// Why: with few rows each of these is a few microseconds of latency -- about
+// 2.3 us of launch and end-of-kernel write-back, then weights, activations and
+// the cross-wave sum waited for in turn -- and five of them make up most of a
+// small batch's step.  Here every workgroup issues its weight loads first and
+// then waits for the phase before its own, so the layer's 30 MB stream in while
+// the first phases run and each further phase costs its hand-off instead of a
+// launch.
+//
+// Hand-off: the blocks of a phase are numbered after those of the phase
+// before it.  A block publishes its results with device-scope (sc1) stores,
+// waits until they are complete, and sets its own flag words; a block of the
+// next phase polls that phase's flags, 256 at a time, and then reads the
+// results with device-scope loads.  (Counters instead of flags: an add takes
+// about 80 ns on its line, 2.4 us for 192 blocks on eight lines.  Eight copies
+// of the flags, each polled by an eighth of the blocks: device-scope loads of
+// one line are served about 10 ns apart, 2.5 us a round for 192 blocks.)  No fence: those write back and invalidate the whole
+// L2.  The host launches at most as many blocks as are resident at once, and a
+// block waits only for lower-numbered ones, which the dispatcher starts
+// first.  Before it waits, a block runs its phase once without storing
+// anything: the weights passing through have evicted the code since the last
+// launch, and a first pass over a phase's instructions takes a microsecond or
+// more longer than the second.  A wait also ends, with the launch's results invalid, if it is ever
+// not answered within kSpinTicks, and then at once for every other wait.
+// The blocks of the last phase put the flags back to zero.
+#include "decode_head.hpp"
+#include "paged_decode_merge.hpp"
+
+namespace {
+
+constexpr int kThreads = 512;
+constexpr int kWaves = kThreads / 64;
+constexpr int kKStep = 32;      // k per MFMA
+constexpr int kMaxSteps = 12;   // k-steps of a wave's weights held in registers
+constexpr int kAhead = 8;       // activation k-steps in flight
+constexpr int kRows = 16;
+constexpr int kQkvSteps = 32;   // k-steps of a qkv wave, at most
+constexpr int kQkvHeld = 20;    // of them, held in registers while it waits
+constexpr int kMaxHidden = kQkvSteps * kKStep;  // 1024
+constexpr int kMaxBlocks = 1024;
+constexpr int kSc1 = 16;        // buffer cache policy: device scope
+constexpr uint64_t kSpinTicks = 400000000ull;  // of the 100 MHz clock: 4 s
+
+enum Phase : int { kMerge = 0, kO = 1, kGateUp = 2, kDown = 3, kQkv = 4, kPhases = 5 };
+// Sync words: kCopies flags per block, then (on lines of their own) the count of
+// last-phase blocks past their wait and the word a timed-out wait sets.
+constexpr int kCopies = 8;
+constexpr int kDoneWord = kCopies * kMaxBlocks;
+constexpr int kFailWord = kDoneWord + 32;
+constexpr int kSyncWords = kFailWord + 32;
+
+struct ChainArgs {
+  int M, K, I, KO;          // rows, hidden, intermediate, Hq * 128
+  int first[kPhases + 1];   // first block of each phase
+  int last_phase;           // kQkv, or kDown for the last layer
+  float eps;
+  StreamPartials parts;     // merge phase (its block count may be 0)
+  uint16_t* o;              // M x KO, row stride o_s
+  int64_t o_s;
+  const uint16_t* o_w;
+  int64_t o_ws;
+  const uint16_t* h_in;     // residual streams (M x K, contiguous)
+  uint16_t* h_mid;
+  uint16_t* h_out;
+  float* ss_mid;            // (M x K / 16) sums of squares
+  float* ss_out;
+  const uint16_t* post_w;
+  const uint16_t* gu_w;     // gate rows 0.., up rows I..
+  int64_t gu_ws;
+  uint16_t* act;            // M x I, contiguous
+  const uint16_t* down_w;
+  int64_t down_ws;
+  const uint16_t* in_w;     // next layer
+  const uint16_t* qkv_w;
+  int64_t qkv_ws;
+  HeadArgs hd;
+  uint32_t* sync;           // kSyncWords, zero between launches
+};
+
+__device__ __forceinline__ __amdgpu_buffer_rsrc_t rsrc_of(const void* p, int64_t bytes) {
+  return __builtin_amdgcn_make_buffer_rsrc(const_cast<void*>(p), 0, static_cast<int>(bytes),
+                                           0x00020000);
+}
+__device__ __forceinline__ q3::u32x4 ld16_dev(__amdgpu_buffer_rsrc_t r, uint32_t off) {
+  return __builtin_bit_cast(q3::u32x4, __builtin_amdgcn_raw_buffer_load_b128(r, off, 0, kSc1));
+}
+// k-step `step` of a lane's row: the row and k-group in `off`.  Steps past the
+// last lie outside every descriptor and read as zero, so that they add
+// nothing and need no branch.
+__device__ __forceinline__ uint32_t step_off(uint32_t off, int step, int steps) {
+  return step < steps ? off + step * kKStep * 2 : 0x80000000u;
+}
+__device__ __forceinline__ q3::u32x4 ld_weight(__amdgpu_buffer_rsrc_t r, uint32_t off) {
+  return __builtin_bit_cast(q3::u32x4, __builtin_amdgcn_raw_buffer_load_b128(r, off, 0, 0));
+}
+__device__ __forceinline__ void st16b_dev(uint16_t* p, uint16_t v) {
+  __hip_atomic_store(p, v, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+}
+
+// Waits for the blocks of phase `ph`.  Every thread of the block calls it.
+__device__ __forceinline__ void wait_phase(const ChainArgs& a, int ph) {
+  if (threadIdx.x < 64) {
+    const uint32_t* flags = a.sync + blockIdx.x % kCopies * kMaxBlocks;
+    const int end = a.first[ph + 1];
+    int at = a.first[ph] + static_cast<int>(threadIdx.x);
+    const uint64_t t0 = wall_clock64();
+    int polls = 0;
+    while (__any(at < end)) {  // the flags below `at` are set
+      uint32_t flag[4];  // of 256 blocks, in one round trip
+#pragma unroll
+      for (int i = 0; i < 4; ++i)
+        flag[i] = at + 64 * i < end ? __hip_atomic_load(flags + at + 64 * i, __ATOMIC_RELAXED,
+                                                        __HIP_MEMORY_SCOPE_AGENT)
+                                    : 1u;
+      if (__all((flag[0] & flag[1] & flag[2] & flag[3]) != 0u)) {
+        at += 256;
+        continue;
+      }
+      if ((++polls & 63) != 0) continue;
+      uint32_t* fail = a.sync + kFailWord;
+      if (wall_clock64() - t0 > kSpinTicks)
+        __hip_atomic_store(fail, 1u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+      if (__hip_atomic_load(fail, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) != 0u) break;
+    }
+  }
+  __syncthreads();
+}
+
+// One wave of the block, after the block's stores to device memory: they are
+// complete before the flag shows the block.
+__device__ __forceinline__ void set_flag(const ChainArgs& a) {
+  asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
+  const int lane = threadIdx.x & 63;
+  if (lane < kCopies)
+    __hip_atomic_store(a.sync + lane * kMaxBlocks + blockIdx.x, 1u, __ATOMIC_RELAXED,
+                       __HIP_MEMORY_SCOPE_AGENT);
+}
+
+// The last phase's blocks, after their wait: by then every wait of the
+// earlier phases has ended, and when all of these blocks are past theirs the
+// last of them puts the flags back to zero.  Wave 0's ticket is drawn right
+// after the wait and looked at when the block's work is done.
+__device__ __forceinline__ uint32_t past_wait(const ChainArgs& a) {
+  return threadIdx.x == 0 ? __hip_atomic_fetch_add(a.sync + kDoneWord, 1u, __ATOMIC_RELAXED,
+                                                   __HIP_MEMORY_SCOPE_AGENT)
+                          : 0u;
+}
+__device__ __forceinline__ void reset_flags(const ChainArgs& a, uint32_t ticket) {  // wave 0
+  const int end = a.first[a.last_phase];
+  if (__shfl(ticket, 0, 64) != static_cast<uint32_t>(a.first[a.last_phase + 1] - end - 1)) return;
+  for (int i = threadIdx.x; i < end; i += 64)
+#pragma unroll
+    for (int c = 0; c < kCopies; ++c)
+      __hip_atomic_store(a.sync + c * kMaxBlocks + i, 0u, __ATOMIC_RELAXED,
+                         __HIP_MEMORY_SCOPE_AGENT);
+  if (threadIdx.x == 0)
+    __hip_atomic_store(a.sync + kDoneWord, 0u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+}
+
+// rms of this lane's MFMA row (row lane % 16 of the block's rows) from the
+// producer's partial sums: four lanes per row take every fourth group of
+// tiles, then the butterfly of the separate kernels, so the same bits.
+__device__ __forceinline__ float row_rms(const ChainArgs& a, const float* ss, int lane) {
+  const int tiles = a.K / 16;
+  const int row = min(lane >> 2, a.M - 1), part = lane & 3;
+  const __amdgpu_buffer_rsrc_t r = rsrc_of(ss, static_cast<int64_t>(a.M) * tiles * 4);
+  float s = 0.f;
+  if (tiles == 64) {
+    q3::u32x4 f[4];
+#pragma unroll
+    for (int j = 0; j < 4; ++j) f[j] = ld16_dev(r, (row * 64 + 16 * part + 4 * j) * 4);
+#pragma unroll
+    for (int j = 0; j < 4; ++j)
+      s += ((__uint_as_float(f[j][0]) + __uint_as_float(f[j][1])) + __uint_as_float(f[j][2])) +
+           __uint_as_float(f[j][3]);
+  } else {
+    for (int t = part; t < tiles; t += 4)
+      s += __uint_as_float(__builtin_amdgcn_raw_buffer_load_b32(r, (row * tiles + t) * 4, 0, kSc1));
+  }
+  s += q3::dpp_f32<q3::kDppXor1>(s);  // lane ^ 1
+  s += q3::dpp_f32<q3::kDppXor2>(s);  // lane ^ 2
+  const float rms = 1.f / sqrtf(s / static_cast<float>(a.K) + a.eps);
+  return __shfl(rms, 4 * (lane & 15), 64);
+}
+
+// x, unknown to the compiler: what is derived from it is computed where it is
+// used (hoisted out of the pass loops, the offsets of all k-steps would need
+// more registers than there are).
+__device__ __forceinline__ uint32_t fresh(uint32_t x) {
+  asm volatile("" : "+v"(x));
+  return x;
+}
+
+// 2, unknown to the compiler: the dry pass and the real one share their code.
+__device__ __forceinline__ int two() {
+  int n = 2;
+  asm volatile("" : "+s"(n));
+  return n;
+}
+
+__device__ __forceinline__ q3::u32x4 to_mfma(q3::u32x4 v, int perm_addr) {
+  q3::u32x4 o;
+#pragma unroll
+  for (int e = 0; e < 4; ++e)
+    o[e] = static_cast<uint32_t>(__builtin_amdgcn_ds_bpermute(perm_addr, static_cast<int>(v[e])));
+  return o;
+}
+
+__device__ __forceinline__ q3::u32x4 normed(q3::u32x4 h, q3::u32x4 w, float rms) {
+  q3::u32x4 o;
+#pragma unroll
+  for (int e = 0; e < 4; ++e)
+    o[e] = q3::pack_bf16x2((q3::bf16_lo(h[e]) * rms) * q3::bf16_lo(w[e]),
+                           (q3::bf16_hi(h[e]) * rms) * q3::bf16_hi(w[e]));
+  return o;
+}
+
+// One 16-column tile of o_proj, gate_up or down.  Each wave holds its share of
+// the tile's weights before it waits: an eighth of K of the one weight tile
+// (o_proj, down), or a quarter of K of the gate or of the up tile (gate_up).
+template <int kPh>
+__device__ __forceinline__ void linear_phase(const ChainArgs& a, int tile, q3::f32x4 (*red)[64],
+                                             uint16_t* nw_s) {
+  constexpr bool kNorm = kPh == kGateUp;
+  constexpr int kSteps = kNorm ? kMaxHidden / 4 / kKStep : kMaxSteps;
+  constexpr int kParts = kNorm ? kWaves / 2 : kWaves;  // waves sharing one weight tile's K
+  const int tid = threadIdx.x, lane = tid & 63;
+  const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+  const int r16 = lane & 15, kg = 8 * (lane >> 4);
+  const int lrow = lane >> 2, lkg = 8 * (lane & 3);
+  const int perm_addr = 4 * (4 * r16 + (lane >> 4));
+  const int n0 = tile * 16;
+  const int K = kPh == kO ? a.KO : kPh == kGateUp ? a.K : a.I;
+  const int kw = K / kParts;
+  const int k0 = (wave % kParts) * kw;
+  const int steps = kw / kKStep;  // at most kSteps
+  const uint16_t* w = kPh == kO ? a.o_w : kPh == kGateUp ? a.gu_w : a.down_w;
+  const int64_t ws = kPh == kO ? a.o_ws : kPh == kGateUp ? a.gu_ws : a.down_ws;
+  const __amdgpu_buffer_rsrc_t wr =
+      rsrc_of(w + (n0 + (kNorm && wave >= kParts ? a.I : 0)) * ws, (15 * ws + K) * 2);
+  const uint32_t woff = static_cast<uint32_t>((lrow * ws + lkg + k0) * 2);
+  q3::u32x4 b[kSteps];
+#pragma unroll
+  for (int u = 0; u < kSteps; ++u)
+    b[u] = ld_weight(wr, step_off(woff, u, steps));
+  uint32_t res[4] = {0u, 0u, 0u, 0u};
+  if constexpr (kPh == kO) {  // the residual comes from the launch before this one
+    if (wave == 0) {
+#pragma unroll
+      for (int i = 0; i < 4; ++i) {
+        const int row = 4 * (lane >> 4) + i;
+        if (row < a.M) res[i] = a.h_in[static_cast<int64_t>(row) * a.K + n0 + r16];
+      }
+    }
+  }
+  if constexpr (kNorm) {
+    for (int i = tid; i < a.K / 8; i += kThreads)
+      *reinterpret_cast<q3::u32x4*>(nw_s + 8 * i) = q3::ld16(a.post_w + 8 * i);
+  }
+  // into the operand layout while there is nothing else to do
+#pragma unroll
+  for (int u = 0; u < kSteps; ++u) b[u] = to_mfma(b[u], perm_addr);
+  const uint16_t* x = kPh == kO ? a.o : kPh == kGateUp ? a.h_mid : a.act;
+  const int64_t xs = kPh == kO ? a.o_s : K;
+  const __amdgpu_buffer_rsrc_t xr = rsrc_of(x, (a.M - 1) * xs * 2 + static_cast<int64_t>(K) * 2);
+  // straight into the operand layout (few rows: there is little to coalesce,
+  // and a permute here would be on the critical path); rows past M repeat
+  // the last
+  const uint32_t xoff0 = static_cast<uint32_t>((min(r16, a.M - 1) * xs + kg + k0) * 2);
+  for (int pass = 0; pass < two(); ++pass) {
+    if (pass) wait_phase(a, kPh - 1);
+    const uint32_t xoff = fresh(xoff0);
+    const uint16_t* nwp = nw_s + fresh(k0 + kg);
+    q3::u32x4 xv[kAhead];
+#pragma unroll
+    for (int u = 0; u < kAhead; ++u) xv[u] = ld16_dev(xr, step_off(xoff, u, steps));
+    if constexpr (kPh == kDown) {
+      if (wave == 0) {
+        const __amdgpu_buffer_rsrc_t hr = rsrc_of(a.h_mid, static_cast<int64_t>(a.M) * a.K * 2);
+#pragma unroll
+        for (int i = 0; i < 4; ++i) {
+          const int row = min(4 * (lane >> 4) + i, a.M - 1);
+          res[i] = __builtin_amdgcn_raw_buffer_load_b16(hr, (row * a.K + n0 + r16) * 2, 0, kSc1);
+        }
+      }
+    }
+    float rms = 0.f;
+    if constexpr (kNorm) rms = row_rms(a, a.ss_mid, lane);
+    q3::f32x4 acc = {0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+    for (int u = 0; u < kSteps; ++u) {
+      q3::u32x4 av = xv[u % kAhead];
+      if (u + kAhead < kSteps) xv[u % kAhead] = ld16_dev(xr, step_off(xoff, u + kAhead, steps));
+      if constexpr (kNorm)  // (a step past the last: 0 x a weight of step 0)
+        av = normed(av, *reinterpret_cast<const q3::u32x4*>(nwp + (u < steps ? u : 0) * kKStep), rms);
+      acc = q3::mfma16x16x32(q3::as_bf16x8(av), q3::as_bf16x8(b[u]), acc);
+    }
+    // Cross-wave sum in wave order; wave 0 runs the epilogue.
+    red[wave][lane] = acc;
+    __syncthreads();
+    if (wave == 0) {
+      q3::f32x4 v = red[0][lane], up = {0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+      for (int w2 = 1; w2 < kParts; ++w2) v += red[w2][lane];
+      if constexpr (kNorm) {
+        up = red[kParts][lane];
+#pragma unroll
+        for (int w2 = kParts + 1; w2 < kWaves; ++w2) up += red[w2][lane];
+      }
+      const int col = n0 + r16;
+#pragma unroll
+      for (int i = 0; i < 4; ++i) {
+        const int row = 4 * (lane >> 4) + i;
+        const bool live = pass && row < a.M;
+        if constexpr (kNorm) {
+          const float g = round_bf16(v[i]);
+          const float u = round_bf16(up[i]);
+          const float sg = round_bf16(g / (1.f + expf(-g)));
+          if (live) st16b_dev(a.act + static_cast<int64_t>(row) * a.I + col, q3::bf16_bits(sg * u));
+        } else {
+          uint16_t* dst = kPh == kO ? a.h_mid : a.h_out;
+          float* ss = kPh == kO ? a.ss_mid : a.ss_out;
+          float h = 0.f;
+          if (live) {
+            h = round_bf16(__uint_as_float(res[i] << 16) + round_bf16(v[i]));
+            st16b_dev(dst + static_cast<int64_t>(row) * a.K + col, q3::bf16_bits(h));
+          }
+          float sq = __fmul_rn(h, h);
+          sq = q3::row16_sum(sq);
+          if (live && r16 == 0)
+            __hip_atomic_store(ss + static_cast<int64_t>(row) * (a.K / 16) + tile, sq,
+                               __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+        }
+      }
+      if (!pass) continue;
+      if (kPh != a.last_phase)
+        set_flag(a);
+      else
+        reset_flags(a, past_wait(a));
+    }
+  }
+}
+
+// One head of the next layer's q, k, v.  Wave w has the head's weight rows
+// 16 w .. 16 w + 15, all of K: 20 of at most 32 k-steps are held in registers
+// while the block waits (a head's 256 KB take a CU about 5 us to read), the
+// rest is read as they are used up.
+__device__ __forceinline__ void qkv_phase(const ChainArgs& a, int head, uint16_t* a_s,
+                                          uint16_t* nw_s) {
+  __shared__ float rms_s[kRows];
+  __shared__ uint16_t y_s[kRows][kHeadD];
+  __shared__ int64_t pos_s[kRows], phys_s[kRows];
+  __shared__ int off_s[kRows];
+  const int tid = threadIdx.x, lane = tid & 63;
+  const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+  const int r16 = lane & 15;
+  const int lrow = lane >> 2, lkg = 8 * (lane & 3);
+  const int perm_addr = 4 * (4 * r16 + (lane >> 4));
+  const int steps = a.K / kKStep;  // a multiple of 4, at most kQkvSteps
+  const int pitch = a.K + 8;
+  const __amdgpu_buffer_rsrc_t wr =
+      rsrc_of(a.qkv_w + static_cast<int64_t>(head * kHeadD + wave * 16) * a.qkv_ws,
+              (15 * a.qkv_ws + a.K) * 2);
+  // coalesced, moved into the operand layout
+  const uint32_t woff = static_cast<uint32_t>((lrow * a.qkv_ws + lkg) * 2);
+  q3::u32x4 b[kQkvHeld];
+#pragma unroll
+  for (int u = 0; u < kQkvHeld; ++u) b[u] = ld_weight(wr, step_off(woff, u, steps));
+  if (wave == 1 && lane < kRows) {
+    int64_t pos, phys;
+    int off;
+    locate_token(a.hd, lane, pos, phys, off);
+    pos_s[lane] = pos;
+    phys_s[lane] = phys;
+    off_s[lane] = off;
+  }
+  for (int i = tid; i < a.K / 8; i += kThreads)
+    *reinterpret_cast<q3::u32x4*>(nw_s + 8 * i) = q3::ld16(a.in_w + 8 * i);
+#pragma unroll
+  for (int u = 0; u < kQkvHeld; ++u) b[u] = to_mfma(b[u], perm_addr);
+  uint32_t ticket = 0;
+  for (int pass = 0; pass < two(); ++pass) {
+    const int tp = static_cast<int>(fresh(tid));
+    if (pass) {
+      wait_phase(a, kDown);
+      ticket = past_wait(a);
+    }
+
+    // The rows of h: chunk c = tid + i * threads of the M x K / 8 16-byte
+    // chunks, at most four per thread.  Rows past M stay unwritten: a row of the
+    // product depends on its own row only.
+    constexpr int kPer = kRows * kMaxHidden / 8 / kThreads;
+    const int cpr = a.K >> 3, nch = a.M * cpr;
+    q3::u32x4 hv[kPer];
+    const __amdgpu_buffer_rsrc_t hr = rsrc_of(a.h_out, static_cast<int64_t>(a.M) * a.K * 2);
+#pragma unroll
+    for (int i = 0; i < kPer; ++i) {
+      const int c = tp + i * kThreads;
+      if (c < nch) hv[i] = ld16_dev(hr, c * 16);
+    }
+    if (wave == 0) {
+      const float rms = row_rms(a, a.ss_out, tp & 63);
+      if (lane < kRows) rms_s[lane] = rms;
+    }
+    __syncthreads();
+#pragma unroll
+    for (int i = 0; i < kPer; ++i) {
+      const int c = tp + i * kThreads;
+      if (c >= nch) continue;
+      const int r = c / cpr, cc = c - r * cpr;
+      *reinterpret_cast<q3::u32x4*>(a_s + r * pitch + 8 * cc) =
+          normed(hv[i], *reinterpret_cast<const q3::u32x4*>(nw_s + 8 * cc), rms_s[r]);
+    }
+    __syncthreads();
+    // the two halves of K summed apart, then first + second, as decode_qkv.hip
+    const uint16_t* arow = a_s + (tp & 15) * pitch + 8 * ((tp & 63) >> 4);
+    // straight in the operand layout
+    const uint32_t wdir = static_cast<uint32_t>(((tp & 15) * a.qkv_ws + 8 * ((tp & 63) >> 4)) * 2);
+    const int half = steps / 2;
+    q3::f32x4 acc0 = {0.f, 0.f, 0.f, 0.f}, acc1 = acc0;
+    constexpr int kLate = kQkvSteps - kQkvHeld;  // b[u] is used for step u, then for step kQkvHeld + u
+#pragma unroll
+    for (int u = 0; u < kQkvSteps; ++u) {
+      const q3::u32x4 av = *reinterpret_cast<const q3::u32x4*>(arow + (u < steps ? u : 0) * kKStep);
+      if (u == half) {
+        acc0 = acc1;
+        acc1 = q3::f32x4{0.f, 0.f, 0.f, 0.f};
+      }
+      acc1 = q3::mfma16x16x32(q3::as_bf16x8(av),
+                              q3::as_bf16x8(b[u % kQkvHeld]), acc1);
+      if (u < kLate) b[u] = ld_weight(wr, step_off(wdir, u + kQkvHeld, steps));
+      if (u % 4 == 3) __builtin_amdgcn_sched_barrier(0);
+    }
+#pragma unroll
+    for (int u = 0; u < kLate; ++u)  // for the pass to come (none after the second)
+      b[u] = ld_weight(wr, step_off(wdir, u, pass ? 0 : steps));
+#pragma unroll
+    for (int i = 0; i < 4; ++i)
+      y_s[4 * ((tp & 63) >> 4) + i][wave * 16 + (tp & 15)] = q3::bf16_bits(acc0[i] + acc1[i]);
+    __syncthreads();
+  }
+  const int r = tid >> 4, j = tid & 15;
+  if (r < a.M)  // whole 16-lane groups
+    finish_head(a.hd, head, r, j, *reinterpret_cast<const q3::u32x4*>(&y_s[r][8 * j]), pos_s[r],
+                phys_s[r], off_s[r]);
+  if (wave == 0) reset_flags(a, ticket);
+}
+
+// Two blocks per CU (the largest grid the host launches is what fits).
+__global__ __launch_bounds__(kThreads) __attribute__((amdgpu_waves_per_eu(4, 4)))
+void decode_chain_kernel(ChainArgs a) {
+  __shared__ q3::f32x4 red[kWaves][64];
+  __shared__ __attribute__((aligned(16))) uint16_t a_s[kRows * (kMaxHidden + 8)];
+  __shared__ __attribute__((aligned(16))) uint16_t nw_s[kMaxHidden];
+  const int blk = blockIdx.x;
+  if (blk < a.first[kO]) {  // merge: one wave per (row, query head)
+    const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6), lane = threadIdx.x & 63;
+    const int hq_n = a.KO / kHeadD;
+    const int task = blk * kWaves + wave;
+    const int b = task / hq_n, hq = task - b * hq_n;
+    uint32_t y;
+    if (b < a.M && merge_partials<8>(a.parts, b, hq, lane, y))
+      __hip_atomic_store(reinterpret_cast<uint32_t*>(a.o + b * a.o_s + hq * kHeadD + 2 * lane), y,
+                         __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+    asm volatile("s_waitcnt vmcnt(0)" ::: "memory");  // this wave's stores are complete
+    __syncthreads();
+    if (wave == 0) set_flag(a);
+  } else if (blk < a.first[kGateUp]) {
+    linear_phase<kO>(a, blk - a.first[kO], red, nw_s);
+  } else if (blk < a.first[kDown]) {
+    linear_phase<kGateUp>(a, blk - a.first[kGateUp], red, nw_s);
+  } else if (blk < a.first[kQkv]) {
+    linear_phase<kDown>(a, blk - a.first[kDown], red, nw_s);
+  } else {
+    qkv_phase(a, blk - a.first[kQkv], a_s, nw_s);
+  }
+}
+
+// Blocks resident at once on the current device (0: unknown).
+int resident_blocks() {
+  static int cached[64] = {0};
+  int dev = -1;
+  if (hipGetDevice(&dev) != hipSuccess || dev < 0 || dev >= 64) return 0;
+  if (cached[dev] == 0) {
+    int cus = 0, per = 0;
+    if (hipDeviceGetAttribute(&cus, hipDeviceAttributeMultiprocessorCount, dev) != hipSuccess ||
+        hipOccupancyMaxActiveBlocksPerMultiprocessor(
+            &per, reinterpret_cast<const void*>(decode_chain_kernel), kThreads, 0) != hipSuccess)
+      return 0;
+    cached[dev] = cus * per;
+  }
+  return cached[dev];
+}
+
+// Blocks per phase; false for shapes the kernel does not hold.
+bool phase_blocks(int M, int hidden, int inter, int num_heads, int num_kv_heads, bool merge,
+                  bool qkv, int (&first)[kPhases + 1]) {
+  const int64_t KO = static_cast<int64_t>(num_heads) * kHeadD;
+  if (M < 1 || M > kRows || hidden <= 0 || inter <= 0 || num_heads <= 0 || num_kv_heads <= 0 ||
+      num_heads % num_kv_heads != 0)
+    return false;
+  // whole k-steps per wave, held in registers; rows of one head staged in
+  // LDS; o_proj and down split K over eight waves, as decode_linear does from
+  // 2048 on (fewer would sum in another order)
+  if (hidden % (4 * kKStep) != 0 || hidden > kMaxHidden || hidden / 4 / kKStep > kMaxSteps ||
+      KO < 2048 || KO % (kWaves * kKStep) != 0 || KO / kWaves / kKStep > kMaxSteps ||
+      inter < 2048 || inter % (kWaves * kKStep) != 0 || inter / kWaves / kKStep > kMaxSteps)
+    return false;
+  const int n[kPhases] = {merge ? (M * num_heads + kWaves - 1) / kWaves : 0, hidden / 16,
+                          inter / 16, hidden / 16, qkv ? num_heads + 2 * num_kv_heads : 0};
+  first[0] = 0;
+  for (int p = 0; p < kPhases; ++p) first[p + 1] = first[p] + n[p];
+  return first[kPhases] <= kMaxBlocks;
+}
+
+}  // namespace
+
+extern "C" size_t qwen3_decode_chain_sync_bytes(void) { return kSyncWords * sizeof(uint32_t); }
+
+extern "C" int qwen3_decode_chain_supported(int M, int hidden, int intermediate, int num_heads,
+                                            int num_kv_heads) {
+  int first[kPhases + 1];
+  return phase_blocks(M, hidden, intermediate, num_heads, num_kv_heads, true, true, first) &&
+                 first[kPhases] <= resident_blocks()
+             ? 1
+             : 0;
+}
+
+extern "C" int qwen3_decode_chain_bf16(const qwen3_decode_chain_args* c, void* stream) {
+  const char* who = "qwen3_decode_chain_bf16";
+  if (!c || !c->o || !c->o_weight || !c->h_in || !c->h_mid || !c->h_out || !c->ss_mid ||
+      !c->ss_out || !c->post_norm_weight || !c->gate_up_weight || !c->act || !c->down_weight ||
+      !c->sync)
+    return q3::fail(QWEN3_EINVAL, "%s: null pointer argument", who);
+  if (c->M == 0) return QWEN3_OK;
+  const bool merge = c->attn_workspace != nullptr, qkv = c->qkv_weight != nullptr;
+  ChainArgs a{};
+  if (!phase_blocks(c->M, c->hidden, c->intermediate, c->num_heads, c->num_kv_heads, merge, qkv,
+                    a.first))
+    return q3::fail(QWEN3_EUNSUPPORTED, "%s: %d rows, hidden %d, intermediate %d, heads %d / %d "
+                    "not supported", who, c->M, c->hidden, c->intermediate, c->num_heads,
+                    c->num_kv_heads);
+  if (a.first[kPhases] > resident_blocks())
+    return q3::fail(QWEN3_EUNSUPPORTED, "%s: %d blocks cannot be resident at once", who,
+                    a.first[kPhases]);
+  if (c->h_in == c->h_mid || c->h_mid == c->h_out || !(c->eps >= 0.f))
+    return q3::fail(QWEN3_EINVAL, "%s: h_mid must be a buffer of its own, eps >= 0", who);
+  bool ok = q3::aligned16(c->o) && q3::aligned16(c->o_weight) && q3::aligned16(c->h_in) &&
+            q3::aligned16(c->h_mid) && q3::aligned16(c->h_out) && q3::aligned16(c->ss_mid) &&
+            q3::aligned16(c->ss_out) && q3::aligned16(c->post_norm_weight) &&
+            q3::aligned16(c->gate_up_weight) && q3::aligned16(c->act) &&
+            q3::aligned16(c->down_weight) && q3::aligned16(c->sync) && c->o_row_stride % 8 == 0 &&
+            c->o_weight_row_stride % 8 == 0 && c->gate_up_row_stride % 8 == 0 &&
+            c->down_row_stride % 8 == 0;
+  a.M = c->M;
+  a.K = c->hidden;
+  a.I = c->intermediate;
+  a.KO = c->num_heads * kHeadD;
+  a.last_phase = qkv ? kQkv : kDown;
+  a.eps = c->eps;
+  if (merge) {
+    const int64_t waves = c->attn_waves;
+    const StreamLayout L = stream_layout(c->M, waves, c->num_heads / c->num_kv_heads);
+    if (waves <= 0 || static_cast<size_t>(L.total) > c->attn_workspace_bytes)
+      return q3::fail(QWEN3_EWORKSPACE, "%s: attention workspace of %lld bytes needed, %zu given",
+                      who, static_cast<long long>(L.total), c->attn_workspace_bytes);
+    const char* ws = static_cast<const char*>(c->attn_workspace);
+    ok = ok && q3::aligned16(ws);
+    a.parts = {reinterpret_cast<const float*>(ws + L.po),
+               reinterpret_cast<const float*>(ws + L.plse),
+               reinterpret_cast<const int32_t*>(ws + L.pref),
+               reinterpret_cast<const int32_t*>(ws + L.meta), c->num_kv_heads,
+               c->num_heads / c->num_kv_heads};
+  }
+  a.o = static_cast<uint16_t*>(c->o);
+  a.o_s = c->o_row_stride;
+  a.o_w = static_cast<const uint16_t*>(c->o_weight);
+  a.o_ws = c->o_weight_row_stride;
+  a.h_in = static_cast<const uint16_t*>(c->h_in);
+  a.h_mid = static_cast<uint16_t*>(c->h_mid);
+  a.h_out = static_cast<uint16_t*>(c->h_out);
+  a.ss_mid = c->ss_mid;
+  a.ss_out = c->ss_out;
+  a.post_w = static_cast<const uint16_t*>(c->post_norm_weight);
+  a.gu_w = static_cast<const uint16_t*>(c->gate_up_weight);
+  a.gu_ws = c->gate_up_row_stride;
+  a.act = static_cast<uint16_t*>(c->act);
+  a.down_w = static_cast<const uint16_t*>(c->down_weight);
+  a.down_ws = c->down_row_stride;
+  a.sync = c->sync;
+  if (qkv) {
+    if (!c->in_norm_weight || !c->q_norm_weight || !c->k_norm_weight || !c->cos_table ||
+        !c->sin_table || !c->q_out || !c->k_cache || !c->v_cache || !c->seq_lens ||
+        !c->block_table)
+      return q3::fail(QWEN3_EINVAL, "%s: null pointer argument", who);
+    if (c->block_size <= 0 || c->num_blocks <= 0 || c->layer_idx < 0 ||
+        c->layer_idx >= c->num_layers || c->table_rows < 0 || c->max_rows <= 0 ||
+        c->max_pages <= 0 || c->bt_row_stride < c->max_pages || !(c->head_eps >= 0.f))
+      return q3::fail(QWEN3_EINVAL, "%s: bad sizes", who);
+    ok = ok && q3::aligned16(c->in_norm_weight) && q3::aligned16(c->qkv_weight) &&
+         q3::aligned16(c->q_norm_weight) && q3::aligned16(c->k_norm_weight) &&
+         q3::aligned16(c->cos_table) && q3::aligned16(c->sin_table) && q3::aligned16(c->q_out) &&
+         q3::aligned16(c->k_cache) && q3::aligned16(c->v_cache) && c->qkv_row_stride % 8 == 0 &&
+         c->table_row_stride % 4 == 0 && c->q_out_strides[0] % 8 == 0 &&
+         c->q_out_strides[1] % 8 == 0;
+    HeadArgs& hd = a.hd;
+    for (int i = 0; i < 4; ++i) {
+      ok = ok && c->k_cache_strides[i] % 8 == 0 && c->v_cache_strides[i] % 8 == 0;
+      hd.kc[i] = c->k_cache_strides[i];
+      hd.vc[i] = c->v_cache_strides[i];
+    }
+    a.in_w = static_cast<const uint16_t*>(c->in_norm_weight);
+    a.qkv_w = static_cast<const uint16_t*>(c->qkv_weight);
+    a.qkv_ws = c->qkv_row_stride;
+    hd.M = c->M;
+    hd.Hq = c->num_heads;
+    hd.Hkv = c->num_kv_heads;
+    hd.q_w = static_cast<const uint16_t*>(c->q_norm_weight);
+    hd.k_w = static_cast<const uint16_t*>(c->k_norm_weight);
+    hd.head_eps = c->head_eps;
+    hd.cos_t = c->cos_table;
+    hd.sin_t = c->sin_table;
+    hd.tab_stride = c->table_row_stride;
+    hd.tab_rows = c->table_rows;
+    hd.positions = c->positions;
+    hd.q_out = static_cast<uint16_t*>(c->q_out);
+    hd.qo_s0 = c->q_out_strides[0];
+    hd.qo_s1 = c->q_out_strides[1];
+    hd.k_cache = static_cast<uint16_t*>(c->k_cache);
+    hd.v_cache = static_cast<uint16_t*>(c->v_cache);
+    hd.num_blocks = c->num_blocks;
+    hd.layer = c->layer_idx;
+    hd.seq_lens = c->seq_lens;
+    hd.block_table = c->block_table;
+    hd.bt_stride = c->bt_row_stride;
+    hd.max_rows = c->max_rows;
+    hd.max_pages = c->max_pages;
+    hd.row_ids = c->row_ids;
+    hd.bs = c->block_size;
+  }
+  if (!ok) return q3::fail(QWEN3_EALIGN, "%s: tensors need 16-byte aligned rows", who);
+  // rows of a weight tile inside 32-bit offsets, and not overlapping
+  const int64_t strides[4][2] = {{c->o_weight_row_stride, a.KO}, {c->gate_up_row_stride, a.K},
+                                 {c->down_row_stride, a.I},
+                                 {qkv ? c->qkv_row_stride : a.K, a.K}};
+  for (const auto& st : strides)
+    if (st[0] < st[1] || st[0] > (int64_t{1} << 24))
+      return q3::fail(QWEN3_EINVAL, "%s: weight row stride %lld", who,
+                      static_cast<long long>(st[0]));
+  q3::clear_error();
+  hipLaunchKernelGGL(decode_chain_kernel, dim3(static_cast<unsigned>(a.first[kPhases])),
+                     dim3(kThreads), 0, static_cast<hipStream_t>(stream), a);
+  return q3::launch_status(who);
+}

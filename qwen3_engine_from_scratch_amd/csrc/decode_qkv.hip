@@ -21,7 +21,7 @@
 // summation order, so the same bits).  The 16-token blocks of one head run
 // on one XCD (workgroups are dealt round-robin), so its weights come from
 // HBM once.
-#include "common.hpp"
+#include "decode_head.hpp"
 
 namespace {
 
@@ -46,31 +46,9 @@ struct QkvArgs {
   float eps;
   const uint16_t* w;  // fused qkv weight ((Hq + 2 Hkv) * 128 x K)
   int64_t w_s;
-  int M, K, Hq, Hkv;
-  const uint16_t* q_w;  // QK-norm weights (128)
-  const uint16_t* k_w;
-  float head_eps;
-  const float* cos_t;
-  const float* sin_t;
-  int64_t tab_stride, tab_rows;
-  const int64_t* positions;  // nullable: RoPE at seq_lens[row]
-  uint16_t* q_out;
-  int64_t qo_s0, qo_s1;
-  uint16_t* k_cache;
-  uint16_t* v_cache;
-  int64_t kc[4], vc[4];
-  int64_t num_blocks;
-  int layer;
-  const int32_t* seq_lens;
-  const int32_t* block_table;
-  int64_t bt_stride, max_rows, max_pages;
-  const int32_t* row_ids;  // nullable: identity
-  int bs;
+  int M, K;
+  HeadArgs hd;
 };
-
-__device__ __forceinline__ float round_bf16(float x) {
-  return __uint_as_float(static_cast<uint32_t>(q3::bf16_bits(x)) << 16);
-}
 
 __global__ __launch_bounds__(kThreadsQ) void qkv_rope_kernel(QkvArgs a) {
   // The block's 16 normalised A rows, staged once: row r at a_s + r * pitch.
@@ -81,7 +59,7 @@ __global__ __launch_bounds__(kThreadsQ) void qkv_rope_kernel(QkvArgs a) {
   __shared__ int64_t pos_s[kRowsPerBlock], phys_s[kRowsPerBlock];
   __shared__ int off_s[kRowsPerBlock];
 
-  const int heads = a.Hq + 2 * a.Hkv;
+  const int heads = a.hd.Hq + 2 * a.hd.Hkv;
   const int rbc = (a.M + 15) >> 4;
   const int b = blockIdx.x;
   const int slot = b >> 3;
@@ -163,23 +141,12 @@ __global__ __launch_bounds__(kThreadsQ) void qkv_rope_kernel(QkvArgs a) {
     s += q3::dpp_f32<q3::kDppXor2>(s);  // lane ^ 2
     if (part == 0) rms_s[lane >> 2] = 1.f / sqrtf(s / static_cast<float>(a.K) + a.eps);
   } else if (wave == 1 && lane < kRowsPerBlock) {
-    const int t = rb * 16 + lane;
-    int64_t pos = -1, phys = -1, off = 0;
-    if (t < a.M) {
-      const int64_t row = a.row_ids ? a.row_ids[t] : t;
-      if (row >= 0 && row < a.max_rows) {
-        const int64_t wpos = a.seq_lens[row];
-        const int64_t pg = wpos >= 0 ? wpos / a.bs : -1;
-        if (pg >= 0 && pg < a.max_pages) {
-          phys = a.block_table[row * a.bt_stride + pg];
-          off = wpos % a.bs;
-        }
-        pos = a.positions ? a.positions[t] : wpos;
-      }
-    }
+    int64_t pos, phys;
+    int off;
+    locate_token(a.hd, rb * 16 + lane, pos, phys, off);
     pos_s[lane] = pos;
     phys_s[lane] = phys;
-    off_s[lane] = static_cast<int>(off);
+    off_s[lane] = off;
   }
   __syncthreads();
   // a = bf16((h * rms) * w), the input RMSNorm (qwen3/norm.py:22-26)
@@ -242,81 +209,7 @@ __global__ __launch_bounds__(kThreadsQ) void qkv_rope_kernel(QkvArgs a) {
   const int t = rb * 16 + r;
   if (t >= a.M) return;  // whole 16-lane groups
   const q3::u32x4 xw = *reinterpret_cast<const q3::u32x4*>(&y_s[r][8 * j]);
-  const int64_t pos = pos_s[r], phys = phys_s[r];
-  const int off = off_s[r];
-  const bool ok_pos = pos >= 0 && pos < a.tab_rows;
-  const bool write_pool = ok_pos && phys >= 0 && phys < a.num_blocks;
-  const int kv_base = a.Hq + a.Hkv;
-  if (head >= kv_base) {  // v: a bit-exact copy into the pool
-    if (write_pool)
-      q3::st16(a.v_cache + phys * a.vc[0] + static_cast<int64_t>(a.layer) * a.vc[1] +
-                   static_cast<int64_t>(head - kv_base) * a.vc[2] + off * a.vc[3] + 8 * j,
-               xw);
-    return;
-  }
-  const uint16_t* wn = head < a.Hq ? a.q_w : a.k_w;
-  const q3::u32x4 ww = q3::ld16(wn + 8 * j);
-  float x[8], w[8];
-#pragma unroll
-  for (int e = 0; e < 4; ++e) {
-    x[2 * e] = q3::bf16_lo(xw[e]);
-    x[2 * e + 1] = q3::bf16_hi(xw[e]);
-    w[2 * e] = q3::bf16_lo(ww[e]);
-    w[2 * e + 1] = q3::bf16_hi(ww[e]);
-  }
-  float cv[8], sv[8];
-  if (ok_pos) {
-    const float* cr = a.cos_t + pos * a.tab_stride + 8 * j;
-    const float* sr = a.sin_t + pos * a.tab_stride + 8 * j;
-    const float4 c0 = *reinterpret_cast<const float4*>(cr);
-    const float4 c1 = *reinterpret_cast<const float4*>(cr + 4);
-    const float4 s0 = *reinterpret_cast<const float4*>(sr);
-    const float4 s1 = *reinterpret_cast<const float4*>(sr + 4);
-    const float cc[8] = {c0.x, c0.y, c0.z, c0.w, c1.x, c1.y, c1.z, c1.w};
-    const float ss_[8] = {s0.x, s0.y, s0.z, s0.w, s1.x, s1.y, s1.z, s1.w};
-#pragma unroll
-    for (int e = 0; e < 8; ++e) {
-      cv[e] = round_bf16(cc[e]);  // cos / sin .to(q.dtype)
-      sv[e] = round_bf16(ss_[e]);
-    }
-  }
-  // Squares rounded, then summed (no fused multiply-add), as x.pow(2).mean().
-  float ss = 0.f;
-#pragma unroll
-  for (int e = 0; e < 8; ++e) ss = __fadd_rn(ss, __fmul_rn(x[e], x[e]));
-  ss = q3::row16_sum(ss);
-  const float rmsh = 1.f / sqrtf(ss / static_cast<float>(kD) + a.head_eps);
-  uint32_t np[4], pp[4];
-#pragma unroll
-  for (int e = 0; e < 4; ++e)
-    np[e] = q3::pack_bf16x2((x[2 * e] * rmsh) * w[2 * e], (x[2 * e + 1] * rmsh) * w[2 * e + 1]);
-#pragma unroll
-  for (int e = 0; e < 4; ++e) pp[e] = q3::dpp_u32<q3::kDppRor8>(np[e]);  // lane j ^ 8
-  const float sign = j < 8 ? -1.f : 1.f;  // rotate_half: (-x2, x1)
-  q3::u32x4 out = {0u, 0u, 0u, 0u};
-  if (ok_pos) {
-#pragma unroll
-    for (int e = 0; e < 4; ++e) {
-      float o[2];
-#pragma unroll
-      for (int hl = 0; hl < 2; ++hl) {
-        const int el = 2 * e + hl;
-        const float n = hl ? q3::bf16_hi(np[e]) : q3::bf16_lo(np[e]);
-        const float rh = sign * (hl ? q3::bf16_hi(pp[e]) : q3::bf16_lo(pp[e]));
-        o[hl] = round_bf16(n * cv[el]) + round_bf16(rh * sv[el]);
-      }
-      out[e] = q3::pack_bf16x2(o[0], o[1]);
-    }
-  }
-  if (head < a.Hq) {
-    q3::st16(a.q_out + static_cast<int64_t>(t) * a.qo_s0 + static_cast<int64_t>(head) * a.qo_s1 +
-                 8 * j,
-             out);
-  } else if (write_pool) {
-    q3::st16(a.k_cache + phys * a.kc[0] + static_cast<int64_t>(a.layer) * a.kc[1] +
-                 static_cast<int64_t>(head - a.Hq) * a.kc[2] + off * a.kc[3] + 8 * j,
-             out);
-  }
+  finish_head(a.hd, head, t, j, xw, pos_s[r], phys_s[r], off_s[r]);
 }
 
 }  // namespace
@@ -374,34 +267,36 @@ extern "C" int qwen3_decode_qkv_rope_bf16(
   a.w_s = weight_row_stride;
   a.M = M;
   a.K = K;
-  a.Hq = num_heads;
-  a.Hkv = num_kv_heads;
-  a.q_w = static_cast<const uint16_t*>(q_norm_weight);
-  a.k_w = static_cast<const uint16_t*>(k_norm_weight);
-  a.head_eps = head_eps;
-  a.cos_t = cos_table;
-  a.sin_t = sin_table;
-  a.tab_stride = table_row_stride;
-  a.tab_rows = table_rows;
-  a.positions = positions;
-  a.q_out = static_cast<uint16_t*>(q_out);
-  a.qo_s0 = q_out_strides[0];
-  a.qo_s1 = q_out_strides[1];
-  a.k_cache = static_cast<uint16_t*>(k_cache);
-  a.v_cache = static_cast<uint16_t*>(v_cache);
+  HeadArgs& hd = a.hd;
+  hd.M = M;
+  hd.Hq = num_heads;
+  hd.Hkv = num_kv_heads;
+  hd.q_w = static_cast<const uint16_t*>(q_norm_weight);
+  hd.k_w = static_cast<const uint16_t*>(k_norm_weight);
+  hd.head_eps = head_eps;
+  hd.cos_t = cos_table;
+  hd.sin_t = sin_table;
+  hd.tab_stride = table_row_stride;
+  hd.tab_rows = table_rows;
+  hd.positions = positions;
+  hd.q_out = static_cast<uint16_t*>(q_out);
+  hd.qo_s0 = q_out_strides[0];
+  hd.qo_s1 = q_out_strides[1];
+  hd.k_cache = static_cast<uint16_t*>(k_cache);
+  hd.v_cache = static_cast<uint16_t*>(v_cache);
   for (int i = 0; i < 4; ++i) {
-    a.kc[i] = k_cache_strides[i];
-    a.vc[i] = v_cache_strides[i];
+    hd.kc[i] = k_cache_strides[i];
+    hd.vc[i] = v_cache_strides[i];
   }
-  a.num_blocks = num_blocks;
-  a.layer = layer_idx;
-  a.seq_lens = seq_lens;
-  a.block_table = block_table;
-  a.bt_stride = bt_row_stride;
-  a.max_rows = max_rows;
-  a.max_pages = max_pages;
-  a.row_ids = row_ids;
-  a.bs = block_size;
+  hd.num_blocks = num_blocks;
+  hd.layer = layer_idx;
+  hd.seq_lens = seq_lens;
+  hd.block_table = block_table;
+  hd.bt_stride = bt_row_stride;
+  hd.max_rows = max_rows;
+  hd.max_pages = max_pages;
+  hd.row_ids = row_ids;
+  hd.bs = block_size;
   const int heads = num_heads + 2 * num_kv_heads;
   const int64_t blocks = q3::cdiv(heads, kXcds) * kXcds * ((M + 15) / 16);
   q3::clear_error();

@@ -10,13 +10,16 @@ qwen3/sampling.py:256-258, qwen3/PagedKVcache.py:216-219.
 """
 from __future__ import annotations
 
+import ctypes
+
 import torch
 
 from .. import _lib
 
 __all__ = ["add_rms_norm", "embed_rms_norm", "silu_mul", "argmax", "advance_seq_lens",
            "lm_head_argmax", "LM_HEAD_ARGMAX_MAX_K",
-           "decode_linear", "decode_qkv_rope", "embed_ss", "DECODE_LINEAR_MAX_ROWS"]
+           "decode_linear", "decode_qkv_rope", "decode_chain", "decode_chain_ok",
+           "decode_chain_sync", "embed_ss", "DECODE_LINEAR_MAX_ROWS", "DECODE_CHAIN_MAX_ROWS"]
 
 DECODE_LINEAR_MAX_ROWS = 64
 LM_HEAD_ARGMAX_MAX_K = 1024
@@ -231,6 +234,96 @@ def embed_ss(ids: torch.Tensor, embed_weight: torch.Tensor, *, h_out: torch.Tens
                                          h_out.stride(0), ss_out.data_ptr(), _lib.stream_of(dev))
     _lib.check(rc, "qwen3_embed_ss_bf16")
     return h_out, ss_out
+
+
+DECODE_CHAIN_MAX_ROWS = 16
+
+
+def decode_chain_ok(batch: int, hidden: int, intermediate: int, num_heads: int,
+                    num_kv_heads: int) -> bool:
+    """Whether decode_chain serves `batch` rows of these widths on the
+    current device."""
+    return (0 < batch <= DECODE_CHAIN_MAX_ROWS
+            and bool(_lib.load().qwen3_decode_chain_supported(batch, hidden, intermediate,
+                                                              num_heads, num_kv_heads)))
+
+
+def decode_chain_sync(device) -> torch.Tensor:
+    """The hand-off counters of decode_chain, zeroed once (every launch leaves
+    them zero); launches that may overlap need their own."""
+    return torch.zeros(int(_lib.load().qwen3_decode_chain_sync_bytes()), dtype=torch.uint8,
+                       device=device)
+
+
+def decode_chain(o: torch.Tensor, h: torch.Tensor, h_mid: torch.Tensor, ss: torch.Tensor,
+                 ss_mid: torch.Tensor, layer, eps: float, num_heads: int, num_kv_heads: int,
+                 sync: torch.Tensor, *, attn_workspace: torch.Tensor | None = None,
+                 next_layer=None, head_eps: float = 0.0, cos_table: torch.Tensor | None = None,
+                 sin_table: torch.Tensor | None = None, pool=None, next_idx: int = 0,
+                 row_ids: torch.Tensor | None = None,
+                 positions: torch.Tensor | None = None) -> torch.Tensor | None:
+    """o_proj, gate_up and down of `layer` and, with next_layer, its qkv
+    projection up to attention, in one launch for at most 16 rows: the
+    results of decode_linear and decode_qkv_rope bit for bit.  o (M, Hq, 128)
+    is the attention output, completed here from attn_workspace when
+    paged_attention_decode_partials_hip left partial results there; the
+    residual stream h and its sums of squares ss are updated in place through
+    h_mid and ss_mid.  Returns the next layer's q."""
+    M, hidden = h.shape
+    mlp = layer.mlp
+    wo, wg, wd = layer.self_attn.o_proj.weight, mlp.gate_up_proj.weight, mlp.down_proj.weight
+    inter = wd.shape[1]
+    assert o.shape == (M, num_heads, 128) and o.stride(2) == 1 and o.stride(1) == 128
+    assert wo.shape == (hidden, num_heads * 128) and wg.shape == (2 * inter, hidden) \
+        and wd.shape == (hidden, inter)
+    for t in (h, h_mid):
+        assert t.shape == h.shape and t.dtype == torch.bfloat16 and t.is_contiguous()
+    for t in (ss, ss_mid):
+        assert t.shape == (M, hidden // 16) and t.dtype == torch.float32 and t.is_contiguous()
+    assert all(w.dtype == torch.bfloat16 and w.stride(1) == 1 for w in (wo, wg, wd))
+    lib = _lib.load()
+    dev = _lib.require_hip(o, h, h_mid, ss, ss_mid, wo, wg, wd, sync, attn_workspace, row_ids,
+                           positions)
+    act = torch.empty(M, inter, dtype=h.dtype, device=h.device)
+    a = _lib.DecodeChainArgs(
+        M=M, hidden=hidden, intermediate=inter, num_heads=num_heads, num_kv_heads=num_kv_heads,
+        eps=eps, head_eps=head_eps, o=o.data_ptr(), o_row_stride=o.stride(0),
+        o_weight=wo.data_ptr(), o_weight_row_stride=wo.stride(0), h_in=h.data_ptr(),
+        h_mid=h_mid.data_ptr(), h_out=h.data_ptr(), ss_mid=ss_mid.data_ptr(),
+        ss_out=ss.data_ptr(), post_norm_weight=layer.post_attention_layernorm.weight.data_ptr(),
+        gate_up_weight=wg.data_ptr(), gate_up_row_stride=wg.stride(0), act=act.data_ptr(),
+        down_weight=wd.data_ptr(), down_row_stride=wd.stride(0), sync=sync.data_ptr())
+    if attn_workspace is not None:
+        a.attn_workspace = attn_workspace.data_ptr()
+        a.attn_workspace_bytes = attn_workspace.numel()
+        a.attn_waves = lib.qwen3_paged_decode_partials_waves()
+    q = None
+    if next_layer is not None:
+        at, kb, vb, bt = next_layer.self_attn, pool.k_buffer, pool.v_buffer, pool.block_table_2d
+        wq = at.qkv_proj.weight
+        assert wq.shape == ((num_heads + 2 * num_kv_heads) * 128, hidden) and wq.stride(1) == 1
+        assert cos_table.dtype == sin_table.dtype == torch.float32 and cos_table.stride(1) == 1
+        assert row_ids is None or (row_ids.dtype == torch.int32 and row_ids.is_contiguous()
+                                   and row_ids.numel() == M)
+        assert positions is None or (positions.dtype == torch.int64 and positions.is_contiguous()
+                                     and positions.numel() == M)
+        q = torch.empty(M, num_heads, 128, dtype=h.dtype, device=h.device)
+        a.in_norm_weight = next_layer.input_layernorm.weight.data_ptr()
+        a.qkv_weight, a.qkv_row_stride = wq.data_ptr(), wq.stride(0)
+        a.q_norm_weight, a.k_norm_weight = at.q_norm.weight.data_ptr(), at.k_norm.weight.data_ptr()
+        a.cos_table, a.sin_table = cos_table.data_ptr(), sin_table.data_ptr()
+        a.table_row_stride, a.table_rows = cos_table.stride(0), cos_table.shape[0]
+        a.positions, a.row_ids = _lib.ptr(positions), _lib.ptr(row_ids)
+        a.q_out, a.q_out_strides = q.data_ptr(), _lib.strides(q, (0, 1))
+        a.k_cache, a.k_cache_strides = kb.data_ptr(), _lib.strides(kb, (0, 1, 2, 3))
+        a.v_cache, a.v_cache_strides = vb.data_ptr(), _lib.strides(vb, (0, 1, 2, 3))
+        a.num_blocks, a.num_layers, a.block_size = kb.shape[0], kb.shape[1], kb.shape[3]
+        a.layer_idx = next_idx
+        a.seq_lens, a.block_table = pool.seq_lens.data_ptr(), bt.data_ptr()
+        a.bt_row_stride, a.max_rows, a.max_pages = bt.stride(0), bt.shape[0], bt.shape[1]
+    rc = lib.qwen3_decode_chain_bf16(ctypes.byref(a), _lib.stream_of(dev))
+    _lib.check(rc, "qwen3_decode_chain_bf16")
+    return q
 
 
 def decode_qkv_rope(h: torch.Tensor, ss_in: torch.Tensor, norm_weight: torch.Tensor, eps: float,

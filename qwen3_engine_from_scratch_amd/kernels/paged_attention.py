@@ -94,6 +94,22 @@ def paged_attention_decode_hip(q, k_buffer, v_buffer, block_table_2d,
     (default kernel) or one per device, stream and KV-head count kept by this
     module (batch-invariant kernel).
     """
+    name = "qwen3_paged_decode_invariant_bf16" if batch_invariant else "qwen3_paged_decode_bf16"
+    return _decode(name, q, k_buffer, v_buffer, block_table_2d, seq_lens_full, row_ids, block_size,
+                   seq_len_bias, scale, out, workspace, batch_invariant)
+
+
+def paged_attention_decode_partials_hip(q, k_buffer, v_buffer, block_table_2d, seq_lens_full,
+                                        row_ids, block_size, workspace: torch.Tensor):
+    """paged_attention_decode_hip (default kernel) without its merge launch:
+    sequence-heads split across waves are left as partial results in
+    `workspace`, for decode_chain to combine.  At most 2,048 rows."""
+    return _decode("qwen3_paged_decode_partials_bf16", q, k_buffer, v_buffer, block_table_2d,
+                   seq_lens_full, row_ids, block_size, 1, None, None, workspace, False)
+
+
+def _decode(name, q, k_buffer, v_buffer, block_table_2d, seq_lens_full, row_ids, block_size,
+            seq_len_bias, scale, out, workspace, batch_invariant):
     B, num_heads, head_dim = q.shape
     num_blocks, num_kv_heads, block_size_check, head_dim_check = k_buffer.shape
     assert block_size_check == block_size
@@ -129,8 +145,7 @@ def paged_attention_decode_hip(q, k_buffer, v_buffer, block_table_2d,
         else:
             workspace = torch.empty(max(need, 1), dtype=torch.uint8, device=dev)
     lib = _lib.load()
-    fn = lib.qwen3_paged_decode_invariant_bf16 if batch_invariant else lib.qwen3_paged_decode_bf16
-    rc = fn(
+    rc = getattr(lib, name)(
         q.data_ptr(), _lib.strides(q, (0, 1)),
         k_buffer.data_ptr(), _lib.strides(k_buffer, (0, 1, 2)),
         v_buffer.data_ptr(), _lib.strides(v_buffer, (0, 1, 2)),
@@ -140,8 +155,7 @@ def paged_attention_decode_hip(q, k_buffer, v_buffer, block_table_2d,
         out.data_ptr(), _lib.strides(out, (0, 1)),
         B, num_heads, num_kv_heads, head_dim, block_size, float(scale),
         workspace.data_ptr(), workspace.numel(), _lib.stream_of(dev))
-    _lib.check(rc, "qwen3_paged_decode_invariant_bf16" if batch_invariant
-               else "qwen3_paged_decode_bf16")
+    _lib.check(rc, name)
     return out
 
 

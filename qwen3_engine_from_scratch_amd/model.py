@@ -33,11 +33,14 @@ import torch.nn.functional as F
 
 from .config import Qwen3Config
 from .kernels.flash_attention_varlen import flash_attention_prefill
-from .kernels.model_ops import (DECODE_LINEAR_MAX_ROWS, add_rms_norm, argmax, decode_linear,
+from .kernels.model_ops import (DECODE_LINEAR_MAX_ROWS, add_rms_norm, argmax, decode_chain,
+                                decode_chain_ok, decode_chain_sync, decode_linear,
                                 decode_qkv_rope, embed_rms_norm, embed_ss, lm_head_argmax,
                                 lm_head_argmax_ok, silu_mul)
 from . import _lib
-from .kernels.paged_attention import paged_attention_decode_hip, paged_decode_workspace_bytes
+from .kernels.paged_attention import (paged_attention_decode_hip,
+                                      paged_attention_decode_partials_hip,
+                                      paged_decode_workspace_bytes)
 from .kernels.pre_attention import qk_norm_rope_decode, qk_norm_rope_prefill, rope_tables
 
 __all__ = ["Qwen3ForCausalLM", "Qwen3Model", "init_random_weights"]
@@ -138,6 +141,7 @@ class Qwen3ForCausalLM(nn.Module):
         self._ws_mode = None
         self._superseded = []
         self._head_ws = None
+        self._chain_sync = None
         # Decode attention with the batch-invariant kernel: each sequence's
         # tokens independent of the rest of the batch (batched == serial),
         # at some HBM time where sequences are split across waves.
@@ -188,6 +192,8 @@ class Qwen3ForCausalLM(nn.Module):
             self._workspace = torch.zeros(max(need, 1), dtype=torch.uint8,
                                           device=pool.k_buffer.device)
             self._ws_mode = inv
+        if self._chain_sync is None:
+            self._chain_sync = decode_chain_sync(pool.k_buffer.device)
         if self._head_ws is None:
             self._head_ws = torch.empty(int(_lib.load().qwen3_lm_head_argmax_workspace_bytes()),
                                         dtype=torch.uint8, device=pool.k_buffer.device)
@@ -226,6 +232,27 @@ class Qwen3ForCausalLM(nn.Module):
         h_a, ss_a = embed_ss(ids, self.model.embed_tokens.weight)
         h_b = torch.empty_like(h_a)
         ss_b = torch.empty_like(ss_a)
+        chain = decode_chain_ok(B, cfg.hidden_size, cfg.intermediate_size, Hq, Hkv)
+        if chain:
+            # at most 16 rows: the dense work between two attention launches is
+            # one launch (with separate ones, launch and load latency is most
+            # of such a step)
+            pos = None if positions is None else positions.reshape(-1).contiguous()
+            at0 = layers[0].self_attn
+            q = decode_qkv_rope(h_a, ss_a, layers[0].input_layernorm.weight, eps,
+                                at0.qkv_proj.weight, Hq, Hkv, at0.q_norm.weight,
+                                at0.k_norm.weight, eps, cos, sin, pool, 0, row_ids, pos)
+            for i, layer in enumerate(layers):
+                kv = (q, pool.k_buffer[:, i], pool.v_buffer[:, i], pool.block_table_2d,
+                      pool.seq_lens, row_ids, pool.block_size)
+                o = (paged_attention_decode_hip(*kv, workspace=ws, batch_invariant=True)
+                     if self._ws_mode else paged_attention_decode_partials_hip(*kv, ws))
+                q = decode_chain(o, h_a, h_b, ss_a, ss_b, layer, eps, Hq, Hkv, self._chain_sync,
+                                 attn_workspace=None if self._ws_mode else ws,
+                                 next_layer=layers[i + 1] if i + 1 < len(layers) else None,
+                                 head_eps=eps, cos_table=cos, sin_table=sin, pool=pool,
+                                 next_idx=i + 1, row_ids=row_ids, positions=pos)
+            return h_a, ss_a
         for i, layer in enumerate(layers):
             at = layer.self_attn
             q = decode_qkv_rope(h_a, ss_a, layer.input_layernorm.weight, eps, at.qkv_proj.weight,
