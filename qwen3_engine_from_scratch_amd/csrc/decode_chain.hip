@@ -94,15 +94,25 @@ __device__ __forceinline__ __amdgpu_buffer_rsrc_t rsrc_of(const void* p, int64_t
 __device__ __forceinline__ q3::u32x4 ld16_dev(__amdgpu_buffer_rsrc_t r, uint32_t off) {
   return __builtin_bit_cast(q3::u32x4, __builtin_amdgcn_raw_buffer_load_b128(r, off, 0, kSc1));
 }
-// k-step `step` of a lane's row: the row and k-group in `off`.  Steps past the
-// last lie outside every descriptor and read as zero, so that they add
-// nothing and need no branch.
-__device__ __forceinline__ uint32_t step_off(uint32_t off, int step, int steps) {
-  return step < steps ? off + step * kKStep * 2 : 0x80000000u;
-}
-__device__ __forceinline__ q3::u32x4 ld_weight(__amdgpu_buffer_rsrc_t r, uint32_t off) {
-  return __builtin_bit_cast(q3::u32x4, __builtin_amdgcn_raw_buffer_load_b128(r, off, 0, 0));
-}
+// k-step u of a lane's row (the row and k-group in `off`, so that the step is
+// the instruction's own offset).  Steps past the last go through an empty
+// descriptor and read as zero: they add nothing and need no branch.
+struct Rows {
+  const void* p;
+  int bytes, steps;
+  __device__ __forceinline__ __amdgpu_buffer_rsrc_t at(int u) const {
+    return __builtin_amdgcn_make_buffer_rsrc(const_cast<void*>(p), 0, u < steps ? bytes : 0,
+                                             0x00020000);
+  }
+  __device__ __forceinline__ q3::u32x4 weight(uint32_t off, int u) const {
+    return __builtin_bit_cast(q3::u32x4, __builtin_amdgcn_raw_buffer_load_b128(
+                                             at(u), off + u * kKStep * 2, 0, 0));
+  }
+  __device__ __forceinline__ q3::u32x4 activation(uint32_t off, int u) const {
+    return __builtin_bit_cast(q3::u32x4, __builtin_amdgcn_raw_buffer_load_b128(
+                                             at(u), off + u * kKStep * 2, 0, kSc1));
+  }
+};
 __device__ __forceinline__ void st16b_dev(uint16_t* p, uint16_t v) {
   __hip_atomic_store(p, v, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
 }
@@ -246,13 +256,21 @@ __device__ __forceinline__ void linear_phase(const ChainArgs& a, int tile, q3::f
   const int steps = kw / kKStep;  // at most kSteps
   const uint16_t* w = kPh == kO ? a.o_w : kPh == kGateUp ? a.gu_w : a.down_w;
   const int64_t ws = kPh == kO ? a.o_ws : kPh == kGateUp ? a.gu_ws : a.down_ws;
-  const __amdgpu_buffer_rsrc_t wr =
-      rsrc_of(w + (n0 + (kNorm && wave >= kParts ? a.I : 0)) * ws, (15 * ws + K) * 2);
+  const Rows wr{w + (n0 + (kNorm && wave >= kParts ? a.I : 0)) * ws,
+                static_cast<int>((15 * ws + K) * 2), steps};
   const uint32_t woff = static_cast<uint32_t>((lrow * ws + lkg + k0) * 2);
   q3::u32x4 b[kSteps];
+  auto load_weights = [&]() {
 #pragma unroll
-  for (int u = 0; u < kSteps; ++u)
-    b[u] = ld_weight(wr, step_off(woff, u, steps));
+    for (int u = 0; u < kSteps; ++u) b[u] = wr.weight(woff, u);
+  };
+  // gate_up and down ask for theirs after the dry pass: 26 MB asked for at
+  // once would hold up the merge's loads and o_proj's
+  if constexpr (kPh == kO)
+    load_weights();
+  else
+#pragma unroll
+    for (int u = 0; u < kSteps; ++u) b[u] = q3::u32x4{0u, 0u, 0u, 0u};
   uint32_t res[4] = {0u, 0u, 0u, 0u};
   if constexpr (kPh == kO) {  // the residual comes from the launch before this one
     if (wave == 0) {
@@ -267,23 +285,26 @@ __device__ __forceinline__ void linear_phase(const ChainArgs& a, int tile, q3::f
     for (int i = tid; i < a.K / 8; i += kThreads)
       *reinterpret_cast<q3::u32x4*>(nw_s + 8 * i) = q3::ld16(a.post_w + 8 * i);
   }
-  // into the operand layout while there is nothing else to do
-#pragma unroll
-  for (int u = 0; u < kSteps; ++u) b[u] = to_mfma(b[u], perm_addr);
   const uint16_t* x = kPh == kO ? a.o : kPh == kGateUp ? a.h_mid : a.act;
   const int64_t xs = kPh == kO ? a.o_s : K;
-  const __amdgpu_buffer_rsrc_t xr = rsrc_of(x, (a.M - 1) * xs * 2 + static_cast<int64_t>(K) * 2);
+  const Rows xr{x, static_cast<int>(((a.M - 1) * xs + K) * 2), steps};
   // straight into the operand layout (few rows: there is little to coalesce,
   // and a permute here would be on the critical path); rows past M repeat
   // the last
   const uint32_t xoff0 = static_cast<uint32_t>((min(r16, a.M - 1) * xs + kg + k0) * 2);
   for (int pass = 0; pass < two(); ++pass) {
-    if (pass) wait_phase(a, kPh - 1);
+    if (pass) {
+      if constexpr (kPh != kO) load_weights();
+      // into the operand layout while there is nothing else to do
+#pragma unroll
+      for (int u = 0; u < kSteps; ++u) b[u] = to_mfma(b[u], perm_addr);
+      wait_phase(a, kPh - 1);
+    }
     const uint32_t xoff = fresh(xoff0);
     const uint16_t* nwp = nw_s + fresh(k0 + kg);
     q3::u32x4 xv[kAhead];
 #pragma unroll
-    for (int u = 0; u < kAhead; ++u) xv[u] = ld16_dev(xr, step_off(xoff, u, steps));
+    for (int u = 0; u < kAhead; ++u) xv[u] = xr.activation(xoff, u);
     if constexpr (kPh == kDown) {
       if (wave == 0) {
         const __amdgpu_buffer_rsrc_t hr = rsrc_of(a.h_mid, static_cast<int64_t>(a.M) * a.K * 2);
@@ -300,7 +321,7 @@ __device__ __forceinline__ void linear_phase(const ChainArgs& a, int tile, q3::f
 #pragma unroll
     for (int u = 0; u < kSteps; ++u) {
       q3::u32x4 av = xv[u % kAhead];
-      if (u + kAhead < kSteps) xv[u % kAhead] = ld16_dev(xr, step_off(xoff, u + kAhead, steps));
+      if (u + kAhead < kSteps) xv[u % kAhead] = xr.activation(xoff, u + kAhead);
       if constexpr (kNorm)  // (a step past the last: 0 x a weight of step 0)
         av = normed(av, *reinterpret_cast<const q3::u32x4*>(nwp + (u < steps ? u : 0) * kKStep), rms);
       acc = q3::mfma16x16x32(q3::as_bf16x8(av), q3::as_bf16x8(b[u]), acc);
@@ -368,14 +389,13 @@ __device__ __forceinline__ void qkv_phase(const ChainArgs& a, int head, uint16_t
   const int perm_addr = 4 * (4 * r16 + (lane >> 4));
   const int steps = a.K / kKStep;  // a multiple of 4, at most kQkvSteps
   const int pitch = a.K + 8;
-  const __amdgpu_buffer_rsrc_t wr =
-      rsrc_of(a.qkv_w + static_cast<int64_t>(head * kHeadD + wave * 16) * a.qkv_ws,
-              (15 * a.qkv_ws + a.K) * 2);
+  const Rows wr{a.qkv_w + static_cast<int64_t>(head * kHeadD + wave * 16) * a.qkv_ws,
+                static_cast<int>((15 * a.qkv_ws + a.K) * 2), steps};
   // coalesced, moved into the operand layout
   const uint32_t woff = static_cast<uint32_t>((lrow * a.qkv_ws + lkg) * 2);
   q3::u32x4 b[kQkvHeld];
 #pragma unroll
-  for (int u = 0; u < kQkvHeld; ++u) b[u] = ld_weight(wr, step_off(woff, u, steps));
+  for (int u = 0; u < kQkvHeld; ++u) b[u] = q3::u32x4{0u, 0u, 0u, 0u};
   if (wave == 1 && lane < kRows) {
     int64_t pos, phys;
     int off;
@@ -386,12 +406,14 @@ __device__ __forceinline__ void qkv_phase(const ChainArgs& a, int head, uint16_t
   }
   for (int i = tid; i < a.K / 8; i += kThreads)
     *reinterpret_cast<q3::u32x4*>(nw_s + 8 * i) = q3::ld16(a.in_w + 8 * i);
-#pragma unroll
-  for (int u = 0; u < kQkvHeld; ++u) b[u] = to_mfma(b[u], perm_addr);
   uint32_t ticket = 0;
   for (int pass = 0; pass < two(); ++pass) {
     const int tp = static_cast<int>(fresh(tid));
     if (pass) {
+#pragma unroll
+      for (int u = 0; u < kQkvHeld; ++u) b[u] = wr.weight(woff, u);
+#pragma unroll
+      for (int u = 0; u < kQkvHeld; ++u) b[u] = to_mfma(b[u], perm_addr);
       wait_phase(a, kDown);
       ticket = past_wait(a);
     }
@@ -405,8 +427,7 @@ __device__ __forceinline__ void qkv_phase(const ChainArgs& a, int head, uint16_t
     const __amdgpu_buffer_rsrc_t hr = rsrc_of(a.h_out, static_cast<int64_t>(a.M) * a.K * 2);
 #pragma unroll
     for (int i = 0; i < kPer; ++i) {
-      const int c = tp + i * kThreads;
-      if (c < nch) hv[i] = ld16_dev(hr, c * 16);
+      hv[i] = ld16_dev(hr, (tp + i * kThreads) * 16);  // (past the rows: zero)
     }
     if (wave == 0) {
       const float rms = row_rms(a, a.ss_out, tp & 63);
@@ -438,12 +459,9 @@ __device__ __forceinline__ void qkv_phase(const ChainArgs& a, int head, uint16_t
       }
       acc1 = q3::mfma16x16x32(q3::as_bf16x8(av),
                               q3::as_bf16x8(b[u % kQkvHeld]), acc1);
-      if (u < kLate) b[u] = ld_weight(wr, step_off(wdir, u + kQkvHeld, steps));
+      if (u < kLate) b[u] = wr.weight(wdir, u + kQkvHeld);
       if (u % 4 == 3) __builtin_amdgcn_sched_barrier(0);
     }
-#pragma unroll
-    for (int u = 0; u < kLate; ++u)  // for the pass to come (none after the second)
-      b[u] = ld_weight(wr, step_off(wdir, u, pass ? 0 : steps));
 #pragma unroll
     for (int i = 0; i < 4; ++i)
       y_s[4 * ((tp & 63) >> 4) + i][wave * 16 + (tp & 15)] = q3::bf16_bits(acc0[i] + acc1[i]);
@@ -469,7 +487,7 @@ void decode_chain_kernel(ChainArgs a) {
     const int task = blk * kWaves + wave;
     const int b = task / hq_n, hq = task - b * hq_n;
     uint32_t y;
-    if (b < a.M && merge_partials<8>(a.parts, b, hq, lane, y))
+    if (b < a.M && merge_partials<32>(a.parts, b, hq, lane, y))
       __hip_atomic_store(reinterpret_cast<uint32_t*>(a.o + b * a.o_s + hq * kHeadD + 2 * lane), y,
                          __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
     asm volatile("s_waitcnt vmcnt(0)" ::: "memory");  // this wave's stores are complete

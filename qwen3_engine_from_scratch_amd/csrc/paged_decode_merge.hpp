@@ -60,46 +60,50 @@ __device__ __forceinline__ bool merge_partials(const StreamPartials& p, int b, i
   if (wf == wl) return false;  // written whole by its wave
   const int nw = static_cast<int>(wl - wf + 1);
   const int slot0 = static_cast<int>(wf) * 2 * G + g;  // fewer than 2^18 slots
-  const int half0 = wf * pw != S ? G : 0;
-  auto slot_of = [&](int i) -> int { return slot0 + i * 2 * G + (i == 0 ? half0 : 0); };
-  // The partials kBatch at a time; the first ones are fetched with the LSEs.
-  float2 ov[kBatch];
+  const int half0 = wf * pw != S ? G : 0;              // the first wave's second slot
+  // The partials kBatch at a time, the first ones fetched with the LSEs; one
+  // past the last lies outside the descriptor and reads as zero.
+  const int stride = 2 * G * kD * 4;  // bytes from one wave's partial to the next
+  const __amdgpu_buffer_rsrc_t po = __builtin_amdgcn_make_buffer_rsrc(
+      const_cast<float*>(p.po + static_cast<int64_t>(slot0) * kD), 0, (nw - 1) * stride + kD * 4,
+      0x00020000);
+  q3::u32x2 ov[kBatch];
   auto fetch = [&](int i0) {
+    const int off = i0 * stride + 8 * lane;
 #pragma unroll
     for (int j = 0; j < kBatch; ++j)
-      ov[j] = i0 + j < nw ? *reinterpret_cast<const float2*>(p.po + slot_of(i0 + j) * kD + 2 * lane)
-                          : float2{0.f, 0.f};
+      ov[j] = __builtin_bit_cast(
+          q3::u32x2, __builtin_amdgcn_raw_buffer_load_b64(
+                         po, off + j * stride + (j == 0 && i0 == 0 ? half0 * kD * 4 : 0), 0, 0));
+  };
+  auto lse_at = [&](int i) -> float {
+    return i < nw ? p.plse[slot0 + i * 2 * G + (i == 0 ? half0 : 0)] : q3::kNegInf;
   };
   fetch(0);
   // Pass 1: global max of the partial LSEs.
-  float M = q3::kNegInf;
-  for (int i0 = 0; i0 < nw; i0 += 64)
-    if (i0 + lane < nw) M = fmaxf(M, p.plse[slot_of(i0 + lane)]);
+  const float lse0 = lse_at(lane);
+  float M = lse0;
+  for (int i0 = 64; i0 < nw; i0 += 64) M = fmaxf(M, lse_at(i0 + lane));
 #pragma unroll
   for (int o = 32; o >= 1; o >>= 1) M = fmaxf(M, q3::shfl_xor(M, o));
   const float M_use = M == q3::kNegInf ? 0.f : M;
   // Pass 2: weighted sum of the partial outputs (lane owns dims 2*lane, 2*lane+1).
   float sw = 0.f, o0 = 0.f, o1 = 0.f;
   for (int i0 = 0; i0 < nw; i0 += 64) {
-    const float wl_lane = (i0 + lane < nw) ? q3::fast_exp2(p.plse[slot_of(i0 + lane)] - M_use) : 0.f;
+    const float wl_lane = q3::fast_exp2((i0 == 0 ? lse0 : lse_at(i0 + lane)) - M_use);
     float wsum = wl_lane;
 #pragma unroll
     for (int o = 32; o >= 1; o >>= 1) wsum += q3::shfl_xor(wsum, o);
     sw += wsum;
     const int cnt = nw - i0 < 64 ? nw - i0 : 64;
     for (int j0 = 0; j0 < cnt; j0 += kBatch) {
-      float wt[kBatch];
-#pragma unroll
-      for (int j = 0; j < kBatch; ++j) {
-        const bool ok = j0 + j < cnt;
-        wt[j] = __shfl(wl_lane, ok ? j0 + j : 0, 64);
-        wt[j] = ok ? wt[j] : 0.f;
-      }
       if (i0 + j0 > 0) fetch(i0 + j0);
 #pragma unroll
-      for (int j = 0; j < kBatch; ++j) {
-        o0 += wt[j] * ov[j].x;
-        o1 += wt[j] * ov[j].y;
+      for (int j = 0; j < kBatch; ++j) {  // weight 0 past the last
+        const float wt =
+            __uint_as_float(__builtin_amdgcn_readlane(__float_as_uint(wl_lane), j0 + j));
+        o0 += wt * __uint_as_float(ov[j][0]);
+        o1 += wt * __uint_as_float(ov[j][1]);
       }
     }
   }
