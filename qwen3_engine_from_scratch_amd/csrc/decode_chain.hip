@@ -27,7 +27,7 @@
 // one line are served about 10 ns apart, 2.5 us a round for 192 blocks.)  No fence: those write back and invalidate the whole
 // L2.  The host launches at most as many blocks as are resident at once, and a
 // block waits only for lower-numbered ones, which the dispatcher starts
-// first.  Before it waits, a block runs its phase once without storing
+// first (and the two blocks of a head, next to each other, for one another).  Before it waits, a block runs its phase once without storing
 // anything: the weights passing through have evicted the code since the last
 // launch, and a first pass over a phase's instructions takes a microsecond or
 // more longer than the second.  A wait also ends, with the launch's results invalid, if it is ever
@@ -44,20 +44,22 @@ constexpr int kKStep = 32;      // k per MFMA
 constexpr int kMaxSteps = 12;   // k-steps of a wave's weights held in registers
 constexpr int kAhead = 8;       // activation k-steps in flight
 constexpr int kRows = 16;
-constexpr int kQkvSteps = 32;   // k-steps of a qkv wave, at most
-constexpr int kQkvHeld = 20;    // of them, held in registers while it waits
-constexpr int kMaxHidden = kQkvSteps * kKStep;  // 1024
+constexpr int kQkvSteps = 16;   // k-steps of half of K, at most
+constexpr int kMaxHidden = 2 * kQkvSteps * kKStep;  // 1024
 constexpr int kMaxBlocks = 1024;
+constexpr int kMaxNormHeads = 64;  // q and k heads
 constexpr int kSc1 = 16;        // buffer cache policy: device scope
 constexpr uint64_t kSpinTicks = 400000000ull;  // of the 100 MHz clock: 4 s
 
 enum Phase : int { kMerge = 0, kO = 1, kGateUp = 2, kDown = 3, kQkv = 4, kPhases = 5 };
 // Sync words: kCopies flags per block, then (on lines of their own) the count of
-// last-phase blocks past their wait and the word a timed-out wait sets.
+// last-phase blocks past their wait and the word a timed-out wait sets, and
+// the sums that the two blocks of a q or k head exchange.
 constexpr int kCopies = 8;
 constexpr int kDoneWord = kCopies * kMaxBlocks;
 constexpr int kFailWord = kDoneWord + 32;
-constexpr int kSyncWords = kFailWord + 32;
+constexpr int kSumWord = kFailWord + 32;  // [head][half of it][row][2]
+constexpr int kSyncWords = kSumWord + kMaxNormHeads * 2 * kRows * 2;
 
 struct ChainArgs {
   int M, K, I, KO;          // rows, hidden, intermediate, Hq * 128
@@ -117,6 +119,15 @@ __device__ __forceinline__ void st16b_dev(uint16_t* p, uint16_t v) {
   __hip_atomic_store(p, v, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
 }
 
+// For a wait that has polled a while since t0: whether it, or any other wait of
+// the launch, has been too long.
+__device__ __forceinline__ bool timed_out(const ChainArgs& a, uint64_t t0) {
+  uint32_t* fail = a.sync + kFailWord;
+  if (wall_clock64() - t0 > kSpinTicks)
+    __hip_atomic_store(fail, 1u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+  return __hip_atomic_load(fail, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) != 0u;
+}
+
 // Waits for the blocks of phase `ph`.  Every thread of the block calls it.
 __device__ __forceinline__ void wait_phase(const ChainArgs& a, int ph) {
   if (threadIdx.x < 64) {
@@ -136,11 +147,7 @@ __device__ __forceinline__ void wait_phase(const ChainArgs& a, int ph) {
         at += 256;
         continue;
       }
-      if ((++polls & 63) != 0) continue;
-      uint32_t* fail = a.sync + kFailWord;
-      if (wall_clock64() - t0 > kSpinTicks)
-        __hip_atomic_store(fail, 1u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-      if (__hip_atomic_load(fail, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) != 0u) break;
+      if ((++polls & 63) == 0 && timed_out(a, t0)) break;
     }
   }
   __syncthreads();
@@ -287,12 +294,11 @@ __device__ __forceinline__ void linear_phase(const ChainArgs& a, int tile, q3::f
   }
   const uint16_t* x = kPh == kO ? a.o : kPh == kGateUp ? a.h_mid : a.act;
   const int64_t xs = kPh == kO ? a.o_s : K;
-  const Rows xr{x, static_cast<int>(((a.M - 1) * xs + K) * 2), steps};
   // straight into the operand layout (few rows: there is little to coalesce,
   // and a permute here would be on the critical path); rows past M repeat
   // the last
   const uint32_t xoff0 = static_cast<uint32_t>((min(r16, a.M - 1) * xs + kg + k0) * 2);
-  for (int pass = 0; pass < two(); ++pass) {
+  for (int pass = kPh == kO ? 1 : 0; pass < two(); ++pass) {
     if (pass) {
       if constexpr (kPh != kO) load_weights();
       // into the operand layout while there is nothing else to do
@@ -300,6 +306,8 @@ __device__ __forceinline__ void linear_phase(const ChainArgs& a, int tile, q3::f
       for (int u = 0; u < kSteps; ++u) b[u] = to_mfma(b[u], perm_addr);
       wait_phase(a, kPh - 1);
     }
+    // (the dry pass asks for nothing: an empty descriptor)
+    const Rows xr{x, static_cast<int>(((a.M - 1) * xs + K) * 2), pass ? steps : 0};
     const uint32_t xoff = fresh(xoff0);
     const uint16_t* nwp = nw_s + fresh(k0 + kg);
     q3::u32x4 xv[kAhead];
@@ -372,30 +380,67 @@ __device__ __forceinline__ void linear_phase(const ChainArgs& a, int tile, q3::f
   }
 }
 
-// One head of the next layer's q, k, v.  Wave w has the head's weight rows
-// 16 w .. 16 w + 15, all of K: 20 of at most 32 k-steps are held in registers
-// while the block waits (a head's 256 KB take a CU about 5 us to read), the
-// rest is read as they are used up.
-__device__ __forceinline__ void qkv_phase(const ChainArgs& a, int head, uint16_t* a_s,
-                                          uint16_t* nw_s) {
+// Adds up the 16 lanes of a token's head (lane j: 8 of its dims, squared and
+// summed) when this block has only quads hf and hf + 2 of them: each quad sum
+// goes to the head's other block, which has the other two.  Quads 0 + 1 and
+// 2 + 3 are added first, as row16_sum does, so the same bits in both blocks.
+// A word is the sum's bits plus one (a sum is never negative, 0 is "not
+// yet"); its one reader puts it back to zero.
+__device__ __forceinline__ float exchange_sum(const ChainArgs& a, int head, int hf, int row, int j,
+                                              float v) {
+  v += q3::dpp_f32<q3::kDppXor1>(v);
+  v += q3::dpp_f32<q3::kDppXor2>(v);
+  const bool mine = ((j >> 2) & 1) == hf;
+  uint32_t* word =
+      a.sync + kSumWord + ((head * 2 + (mine ? hf : 1 - hf)) * kRows + row) * 2 + (j >> 3);
+  const bool first = (j & 3) == 0;
+  if (first && mine)
+    __hip_atomic_store(word, __float_as_uint(v) + 1u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+  const bool reads = first && !mine;
+  uint32_t got = 1u;
+  const uint64_t t0 = wall_clock64();
+  for (int polls = 1;; ++polls) {
+    if (reads) got = __hip_atomic_load(word, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+    if (__all(got != 0u)) break;
+    if ((polls & 63) != 0) continue;
+    if (timed_out(a, t0)) break;
+  }
+  if (reads) __hip_atomic_store(word, 0u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+  constexpr int kQuadFirst = 0x00;  // quad_perm [0,0,0,0]
+  const float theirs = q3::dpp_f32<kQuadFirst>(__uint_as_float(got - 1u));
+  v = mine ? v : theirs;
+  v += q3::dpp_f32<q3::kDppHalfMirror>(v);
+  v += q3::dpp_f32<q3::kDppMirror>(v);
+  return v;
+}
+
+// Half a head of the next layer's q, k, v: dims 32 hf .. + 31 and 64 + 32 hf
+// .. + 31, so that RoPE's pairs are inside; the two halves exchange their sums
+// of squares.  Wave w has 16 of the 64 weight rows (w % 4) and a half of K (w /
+// 4), all of it in registers while it waits.  (A whole head in one block: its
+// 256 KB do not fit the registers, and what was left to read after the wait
+// took 2.5 us at the 46 GB/s of one CU.)
+__device__ __forceinline__ void qkv_phase(const ChainArgs& a, int blk, q3::f32x4 (*red)[64],
+                                          uint16_t* a_s, uint16_t* nw_s) {
   __shared__ float rms_s[kRows];
-  __shared__ uint16_t y_s[kRows][kHeadD];
+  __shared__ __attribute__((aligned(16))) uint16_t y_s[kRows][kHeadD / 2];
   __shared__ int64_t pos_s[kRows], phys_s[kRows];
   __shared__ int off_s[kRows];
+  const int head = blk >> 1, hf = blk & 1;
   const int tid = threadIdx.x, lane = tid & 63;
   const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+  const int ct = wave & 3, kh = wave >> 2;
   const int r16 = lane & 15;
   const int lrow = lane >> 2, lkg = 8 * (lane & 3);
   const int perm_addr = 4 * (4 * r16 + (lane >> 4));
-  const int steps = a.K / kKStep;  // a multiple of 4, at most kQkvSteps
+  const int steps = a.K / 2 / kKStep;  // at most kQkvSteps
   const int pitch = a.K + 8;
-  const Rows wr{a.qkv_w + static_cast<int64_t>(head * kHeadD + wave * 16) * a.qkv_ws,
-                static_cast<int>((15 * a.qkv_ws + a.K) * 2), steps};
-  // coalesced, moved into the operand layout
-  const uint32_t woff = static_cast<uint32_t>((lrow * a.qkv_ws + lkg) * 2);
-  q3::u32x4 b[kQkvHeld];
+  const int wrow = head * kHeadD + (ct < 2 ? 0 : kHeadD / 2 - 32) + 32 * hf + 16 * ct;
+  const Rows wr{a.qkv_w + wrow * a.qkv_ws, static_cast<int>((15 * a.qkv_ws + a.K) * 2), steps};
+  const uint32_t woff = static_cast<uint32_t>((lrow * a.qkv_ws + lkg + kh * (a.K / 2)) * 2);
+  q3::u32x4 b[kQkvSteps];
 #pragma unroll
-  for (int u = 0; u < kQkvHeld; ++u) b[u] = q3::u32x4{0u, 0u, 0u, 0u};
+  for (int u = 0; u < kQkvSteps; ++u) b[u] = q3::u32x4{0u, 0u, 0u, 0u};
   if (wave == 1 && lane < kRows) {
     int64_t pos, phys;
     int off;
@@ -408,27 +453,26 @@ __device__ __forceinline__ void qkv_phase(const ChainArgs& a, int head, uint16_t
     *reinterpret_cast<q3::u32x4*>(nw_s + 8 * i) = q3::ld16(a.in_w + 8 * i);
   uint32_t ticket = 0;
   for (int pass = 0; pass < two(); ++pass) {
-    const int tp = static_cast<int>(fresh(tid));
     if (pass) {
 #pragma unroll
-      for (int u = 0; u < kQkvHeld; ++u) b[u] = wr.weight(woff, u);
+      for (int u = 0; u < kQkvSteps; ++u) b[u] = wr.weight(woff, u);
 #pragma unroll
-      for (int u = 0; u < kQkvHeld; ++u) b[u] = to_mfma(b[u], perm_addr);
+      for (int u = 0; u < kQkvSteps; ++u) b[u] = to_mfma(b[u], perm_addr);
       wait_phase(a, kDown);
       ticket = past_wait(a);
     }
-
     // The rows of h: chunk c = tid + i * threads of the M x K / 8 16-byte
     // chunks, at most four per thread.  Rows past M stay unwritten: a row of the
     // product depends on its own row only.
     constexpr int kPer = kRows * kMaxHidden / 8 / kThreads;
+    const int tp = static_cast<int>(fresh(tid));
     const int cpr = a.K >> 3, nch = a.M * cpr;
     q3::u32x4 hv[kPer];
-    const __amdgpu_buffer_rsrc_t hr = rsrc_of(a.h_out, static_cast<int64_t>(a.M) * a.K * 2);
+    const __amdgpu_buffer_rsrc_t hr =
+        rsrc_of(a.h_out, pass ? static_cast<int64_t>(a.M) * a.K * 2 : 0);
 #pragma unroll
-    for (int i = 0; i < kPer; ++i) {
+    for (int i = 0; i < kPer; ++i)
       hv[i] = ld16_dev(hr, (tp + i * kThreads) * 16);  // (past the rows: zero)
-    }
     if (wave == 0) {
       const float rms = row_rms(a, a.ss_out, tp & 63);
       if (lane < kRows) rms_s[lane] = rms;
@@ -443,34 +487,36 @@ __device__ __forceinline__ void qkv_phase(const ChainArgs& a, int head, uint16_t
           normed(hv[i], *reinterpret_cast<const q3::u32x4*>(nw_s + 8 * cc), rms_s[r]);
     }
     __syncthreads();
-    // the two halves of K summed apart, then first + second, as decode_qkv.hip
-    const uint16_t* arow = a_s + (tp & 15) * pitch + 8 * ((tp & 63) >> 4);
-    // straight in the operand layout
-    const uint32_t wdir = static_cast<uint32_t>(((tp & 15) * a.qkv_ws + 8 * ((tp & 63) >> 4)) * 2);
-    const int half = steps / 2;
-    q3::f32x4 acc0 = {0.f, 0.f, 0.f, 0.f}, acc1 = acc0;
-    constexpr int kLate = kQkvSteps - kQkvHeld;  // b[u] is used for step u, then for step kQkvHeld + u
+    const uint16_t* arow = a_s + (tp & 15) * pitch + 8 * ((tp & 63) >> 4) + kh * (a.K / 2);
+    q3::f32x4 acc = {0.f, 0.f, 0.f, 0.f};
 #pragma unroll
-    for (int u = 0; u < kQkvSteps; ++u) {
-      const q3::u32x4 av = *reinterpret_cast<const q3::u32x4*>(arow + (u < steps ? u : 0) * kKStep);
-      if (u == half) {
-        acc0 = acc1;
-        acc1 = q3::f32x4{0.f, 0.f, 0.f, 0.f};
-      }
-      acc1 = q3::mfma16x16x32(q3::as_bf16x8(av),
-                              q3::as_bf16x8(b[u % kQkvHeld]), acc1);
-      if (u < kLate) b[u] = wr.weight(wdir, u + kQkvHeld);
-      if (u % 4 == 3) __builtin_amdgcn_sched_barrier(0);
+    for (int u = 0; u < kQkvSteps; ++u)
+      acc = q3::mfma16x16x32(q3::as_bf16x8(*reinterpret_cast<const q3::u32x4*>(
+                                 arow + (u < steps ? u : 0) * kKStep)),
+                             q3::as_bf16x8(b[u]), acc);
+    // first half of K + second, rounded to bf16, as decode_qkv.hip
+    if (kh == 1) red[ct][lane] = acc;
+    __syncthreads();
+    if (kh == 0) {
+      const q3::f32x4 other = red[ct][lane];
+#pragma unroll
+      for (int i = 0; i < 4; ++i)
+        y_s[4 * (lane >> 4) + i][ct * 16 + r16] = q3::bf16_bits(acc[i] + other[i]);
     }
-#pragma unroll
-    for (int i = 0; i < 4; ++i)
-      y_s[4 * ((tp & 63) >> 4) + i][wave * 16 + (tp & 15)] = q3::bf16_bits(acc0[i] + acc1[i]);
     __syncthreads();
   }
+  // 16 lanes per token as for a whole head; the quads of the other block are
+  // zero here.
   const int r = tid >> 4, j = tid & 15;
-  if (r < a.M)  // whole 16-lane groups
-    finish_head(a.hd, head, r, j, *reinterpret_cast<const q3::u32x4*>(&y_s[r][8 * j]), pos_s[r],
-                phys_s[r], off_s[r]);
+  if (r < a.M) {  // whole 16-lane groups
+    const bool mine = ((j >> 2) & 1) == hf;
+    const int at = 8 * (j & 3) + (j >> 3) * 32;
+    const q3::u32x4 xw = mine ? *reinterpret_cast<const q3::u32x4*>(&y_s[r][at])
+                              : q3::u32x4{0u, 0u, 0u, 0u};
+    if (mine || head < a.hd.Hq + a.hd.Hkv)
+      finish_head(a.hd, head, r, j, xw, pos_s[r], phys_s[r], off_s[r], mine,
+                  [&](float ss) { return exchange_sum(a, head, hf, r, j, ss); });
+  }
   if (wave == 0) reset_flags(a, ticket);
 }
 
@@ -500,7 +546,7 @@ void decode_chain_kernel(ChainArgs a) {
   } else if (blk < a.first[kQkv]) {
     linear_phase<kDown>(a, blk - a.first[kDown], red, nw_s);
   } else {
-    qkv_phase(a, blk - a.first[kQkv], a_s, nw_s);
+    qkv_phase(a, blk - a.first[kQkv], red, a_s, nw_s);
   }
 }
 
@@ -524,7 +570,7 @@ int resident_blocks() {
 bool phase_blocks(int M, int hidden, int inter, int num_heads, int num_kv_heads, bool merge,
                   bool qkv, int (&first)[kPhases + 1]) {
   const int64_t KO = static_cast<int64_t>(num_heads) * kHeadD;
-  if (M < 1 || M > kRows || hidden <= 0 || inter <= 0 || num_heads <= 0 || num_kv_heads <= 0 ||
+  if (num_heads + num_kv_heads > kMaxNormHeads || M < 1 || M > kRows || hidden <= 0 || inter <= 0 || num_heads <= 0 || num_kv_heads <= 0 ||
       num_heads % num_kv_heads != 0)
     return false;
   // whole k-steps per wave, held in registers; rows of one head staged in
@@ -535,7 +581,7 @@ bool phase_blocks(int M, int hidden, int inter, int num_heads, int num_kv_heads,
       inter < 2048 || inter % (kWaves * kKStep) != 0 || inter / kWaves / kKStep > kMaxSteps)
     return false;
   const int n[kPhases] = {merge ? (M * num_heads + kWaves - 1) / kWaves : 0, hidden / 16,
-                          inter / 16, hidden / 16, qkv ? num_heads + 2 * num_kv_heads : 0};
+                          inter / 16, hidden / 16, qkv ? 2 * (num_heads + 2 * num_kv_heads) : 0};
   first[0] = 0;
   for (int p = 0; p < kPhases; ++p) first[p + 1] = first[p] + n[p];
   return first[kPhases] <= kMaxBlocks;

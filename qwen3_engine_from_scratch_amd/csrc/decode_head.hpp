@@ -57,11 +57,13 @@ __device__ __forceinline__ void locate_token(const HeadArgs& a, int t, int64_t& 
 }
 
 // Head `head` of token t (< M): lane j of a 16-lane group holds dims 8j ..
-// 8j + 7 of the projection's output (xw).  Called by whole groups; without
-// `store` nothing is written.
+// 8j + 7 of the projection's output (xw).  Called by whole groups; a lane
+// without `store` writes nothing.  row_sum: the sum over the group's lanes
+// (q3::row16_sum, or its value by other means).
+template <typename Sum>
 __device__ __forceinline__ void finish_head(const HeadArgs& a, int head, int t, int j,
                                             q3::u32x4 xw, int64_t pos, int64_t phys, int off,
-                                            bool store = true) {
+                                            bool store, Sum&& row_sum) {
   const bool ok_pos = pos >= 0 && pos < a.tab_rows;
   const bool write_pool = store && ok_pos && phys >= 0 && phys < a.num_blocks;
   const int kv_base = a.Hq + a.Hkv;
@@ -102,7 +104,7 @@ __device__ __forceinline__ void finish_head(const HeadArgs& a, int head, int t, 
   float ss = 0.f;
 #pragma unroll
   for (int e = 0; e < 8; ++e) ss = __fadd_rn(ss, __fmul_rn(x[e], x[e]));
-  ss = q3::row16_sum(ss);
+  ss = row_sum(ss);
   const float rmsh = 1.f / sqrtf(ss / static_cast<float>(kHeadD) + a.head_eps);
   uint32_t np[4], pp[4];
 #pragma unroll
@@ -136,6 +138,11 @@ __device__ __forceinline__ void finish_head(const HeadArgs& a, int head, int t, 
                  static_cast<int64_t>(head - a.Hq) * a.kc[2] + off * a.kc[3] + 8 * j,
              out);
   }
+}
+__device__ __forceinline__ void finish_head(const HeadArgs& a, int head, int t, int j,
+                                            q3::u32x4 xw, int64_t pos, int64_t phys, int off) {
+  finish_head(a, head, t, j, xw, pos, phys, off, true,
+              [](float ss) { return q3::row16_sum(ss); });
 }
 
 }  // namespace
