@@ -202,6 +202,15 @@ int qwen3_decode_chain_supported(int M, int hidden, int intermediate, int num_he
                                  int num_kv_heads);
 int qwen3_decode_chain_bf16(const qwen3_decode_chain_args* args, void* stream);
 
+/* qwen3_decode_qkv_rope_bf16, bit for bit, on two workgroups per head that
+ * exchange their sums of squares through sync (as above), for M <= 64 rows: of
+ * args it reads M, hidden, num_heads, num_kv_heads, eps, h_out and ss_out (the
+ * residual stream, rows h_row_stride apart, and its sums), sync, and
+ * everything from in_norm_weight on. */
+int qwen3_decode_qkv_half_supported(int M, int hidden, int num_heads, int num_kv_heads);
+int qwen3_decode_qkv_half_bf16(const qwen3_decode_chain_args* args, int64_t h_row_stride,
+                               void* stream);
+
 /* h_out[r] = embedding[ids[r]] (zero row for an id outside [0, vocab)) and
  * ss_out[r * (hidden / 16) + t] = sum of h^2 over columns 16t .. 16t + 15:
  * the input of the first decode_linear with a norm prologue. */

@@ -157,6 +157,8 @@ _SIGNATURES = {
     "qwen3_decode_chain_sync_bytes": (ctypes.c_size_t, []),
     "qwen3_decode_chain_supported": (_i, [_i, _i, _i, _i, _i]),
     "qwen3_decode_chain_bf16": (_i, [ctypes.POINTER(DecodeChainArgs), _vp]),
+    "qwen3_decode_qkv_half_supported": (_i, [_i, _i, _i, _i]),
+    "qwen3_decode_qkv_half_bf16": (_i, [ctypes.POINTER(DecodeChainArgs), _i64, _vp]),
     "qwen3_embed_ss_bf16": (_i, [_vp, _vp, _i64, _i64, _i, _i, _vp, _i64, _vp, _vp]),
     "qwen3_decode_qkv_rope_bf16": (
         _i,

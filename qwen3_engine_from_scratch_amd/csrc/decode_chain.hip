@@ -59,7 +59,9 @@ constexpr int kCopies = 8;
 constexpr int kDoneWord = kCopies * kMaxBlocks;
 constexpr int kFailWord = kDoneWord + 32;
 constexpr int kSumWord = kFailWord + 32;  // [head][half of it][row][2]
-constexpr int kSyncWords = kSumWord + kMaxNormHeads * 2 * kRows * 2;
+constexpr int kSumWords = kMaxNormHeads * 2 * kRows * 2;
+constexpr int kMaxRowBlocks = 4;  // of the qkv kernel
+constexpr int kSyncWords = kSumWord + kMaxRowBlocks * kSumWords;
 
 struct ChainArgs {
   int M, K, I, KO;          // rows, hidden, intermediate, Hq * 128
@@ -82,6 +84,7 @@ struct ChainArgs {
   uint16_t* act;            // M x I, contiguous
   const uint16_t* down_w;
   int64_t down_ws;
+  int64_t h_s;              // row stride of h_out for the qkv phase
   const uint16_t* in_w;     // next layer
   const uint16_t* qkv_w;
   int64_t qkv_ws;
@@ -187,10 +190,10 @@ __device__ __forceinline__ void reset_flags(const ChainArgs& a, uint32_t ticket)
 // rms of this lane's MFMA row (row lane % 16 of the block's rows) from the
 // producer's partial sums: four lanes per row take every fourth group of
 // tiles, then the butterfly of the separate kernels, so the same bits.
-__device__ __forceinline__ float row_rms(const ChainArgs& a, const float* ss, int lane) {
+__device__ __forceinline__ float row_rms(const ChainArgs& a, const float* ss, int M, int lane) {
   const int tiles = a.K / 16;
-  const int row = min(lane >> 2, a.M - 1), part = lane & 3;
-  const __amdgpu_buffer_rsrc_t r = rsrc_of(ss, static_cast<int64_t>(a.M) * tiles * 4);
+  const int row = min(lane >> 2, M - 1), part = lane & 3;
+  const __amdgpu_buffer_rsrc_t r = rsrc_of(ss, static_cast<int64_t>(M) * tiles * 4);
   float s = 0.f;
   if (tiles == 64) {
     q3::u32x4 f[4];
@@ -324,7 +327,7 @@ __device__ __forceinline__ void linear_phase(const ChainArgs& a, int tile, q3::f
       }
     }
     float rms = 0.f;
-    if constexpr (kNorm) rms = row_rms(a, a.ss_mid, lane);
+    if constexpr (kNorm) rms = row_rms(a, a.ss_mid, a.M, lane);
     q3::f32x4 acc = {0.f, 0.f, 0.f, 0.f};
 #pragma unroll
     for (int u = 0; u < kSteps; ++u) {
@@ -386,13 +389,12 @@ __device__ __forceinline__ void linear_phase(const ChainArgs& a, int tile, q3::f
 // 2 + 3 are added first, as row16_sum does, so the same bits in both blocks.
 // A word is the sum's bits plus one (a sum is never negative, 0 is "not
 // yet"); its one reader puts it back to zero.
-__device__ __forceinline__ float exchange_sum(const ChainArgs& a, int head, int hf, int row, int j,
-                                              float v) {
+__device__ __forceinline__ float exchange_sum(const ChainArgs& a, uint32_t* words, int head, int hf,
+                                              int row, int j, float v) {
   v += q3::dpp_f32<q3::kDppXor1>(v);
   v += q3::dpp_f32<q3::kDppXor2>(v);
   const bool mine = ((j >> 2) & 1) == hf;
-  uint32_t* word =
-      a.sync + kSumWord + ((head * 2 + (mine ? hf : 1 - hf)) * kRows + row) * 2 + (j >> 3);
+  uint32_t* word = words + ((head * 2 + (mine ? hf : 1 - hf)) * kRows + row) * 2 + (j >> 3);
   const bool first = (j & 3) == 0;
   if (first && mine)
     __hip_atomic_store(word, __float_as_uint(v) + 1u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
@@ -419,14 +421,19 @@ __device__ __forceinline__ float exchange_sum(const ChainArgs& a, int head, int 
 // of squares.  Wave w has 16 of the 64 weight rows (w % 4) and a half of K (w /
 // 4), all of it in registers while it waits.  (A whole head in one block: its
 // 256 KB do not fit the registers, and what was left to read after the wait
-// took 2.5 us at the 46 GB/s of one CU.)
-__device__ __forceinline__ void qkv_phase(const ChainArgs& a, int blk, q3::f32x4 (*red)[64],
-                                          uint16_t* a_s, uint16_t* nw_s) {
+// took 2.5 us at the 46 GB/s of one CU.)  kAlone: a launch of its own, rows
+// 16 rb .. of h.
+template <bool kAlone>
+__device__ __forceinline__ void qkv_phase(const ChainArgs& a, int blk, int rb,
+                                          q3::f32x4 (*red)[64], uint16_t* a_s, uint16_t* nw_s) {
   __shared__ float rms_s[kRows];
   __shared__ __attribute__((aligned(16))) uint16_t y_s[kRows][kHeadD / 2];
   __shared__ int64_t pos_s[kRows], phys_s[kRows];
   __shared__ int off_s[kRows];
   const int head = blk >> 1, hf = blk & 1;
+  const int M = kAlone ? min(kRows, a.M - kRows * rb) : a.M;
+  const uint16_t* h = a.h_out + static_cast<int64_t>(kRows * rb) * a.h_s;
+  const float* ss = a.ss_out + kRows * rb * (a.K / 16);
   const int tid = threadIdx.x, lane = tid & 63;
   const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
   const int ct = wave & 3, kh = wave >> 2;
@@ -440,11 +447,12 @@ __device__ __forceinline__ void qkv_phase(const ChainArgs& a, int blk, q3::f32x4
   const uint32_t woff = static_cast<uint32_t>((lrow * a.qkv_ws + lkg + kh * (a.K / 2)) * 2);
   q3::u32x4 b[kQkvSteps];
 #pragma unroll
-  for (int u = 0; u < kQkvSteps; ++u) b[u] = q3::u32x4{0u, 0u, 0u, 0u};
+  for (int u = 0; u < kQkvSteps; ++u)
+    b[u] = kAlone ? wr.weight(woff, u) : q3::u32x4{0u, 0u, 0u, 0u};
   if (wave == 1 && lane < kRows) {
     int64_t pos, phys;
     int off;
-    locate_token(a.hd, lane, pos, phys, off);
+    locate_token(a.hd, kRows * rb + lane, pos, phys, off);
     pos_s[lane] = pos;
     phys_s[lane] = phys;
     off_s[lane] = off;
@@ -452,8 +460,8 @@ __device__ __forceinline__ void qkv_phase(const ChainArgs& a, int blk, q3::f32x4
   for (int i = tid; i < a.K / 8; i += kThreads)
     *reinterpret_cast<q3::u32x4*>(nw_s + 8 * i) = q3::ld16(a.in_w + 8 * i);
   uint32_t ticket = 0;
-  for (int pass = 0; pass < two(); ++pass) {
-    if (pass) {
+  for (int pass = kAlone ? 1 : 0; pass < two(); ++pass) {
+    if (!kAlone && pass) {
 #pragma unroll
       for (int u = 0; u < kQkvSteps; ++u) b[u] = wr.weight(woff, u);
 #pragma unroll
@@ -466,15 +474,17 @@ __device__ __forceinline__ void qkv_phase(const ChainArgs& a, int blk, q3::f32x4
     // product depends on its own row only.
     constexpr int kPer = kRows * kMaxHidden / 8 / kThreads;
     const int tp = static_cast<int>(fresh(tid));
-    const int cpr = a.K >> 3, nch = a.M * cpr;
+    const int cpr = a.K >> 3, nch = M * cpr;
     q3::u32x4 hv[kPer];
     const __amdgpu_buffer_rsrc_t hr =
-        rsrc_of(a.h_out, pass ? static_cast<int64_t>(a.M) * a.K * 2 : 0);
+        rsrc_of(h, pass ? ((M - 1) * a.h_s + a.K) * 2 : 0);
 #pragma unroll
-    for (int i = 0; i < kPer; ++i)
-      hv[i] = ld16_dev(hr, (tp + i * kThreads) * 16);  // (past the rows: zero)
+    for (int i = 0; i < kPer; ++i) {  // (past the rows: zero)
+      const int c = tp + i * kThreads, r = c / cpr;
+      hv[i] = ld16_dev(hr, static_cast<uint32_t>((r * a.h_s + 8 * (c - r * cpr)) * 2));
+    }
     if (wave == 0) {
-      const float rms = row_rms(a, a.ss_out, tp & 63);
+      const float rms = row_rms(a, ss, M, tp & 63);
       if (lane < kRows) rms_s[lane] = rms;
     }
     __syncthreads();
@@ -488,6 +498,9 @@ __device__ __forceinline__ void qkv_phase(const ChainArgs& a, int blk, q3::f32x4
     }
     __syncthreads();
     const uint16_t* arow = a_s + (tp & 15) * pitch + 8 * ((tp & 63) >> 4) + kh * (a.K / 2);
+    if constexpr (kAlone)
+#pragma unroll
+      for (int u = 0; u < kQkvSteps; ++u) b[u] = to_mfma(b[u], perm_addr);
     q3::f32x4 acc = {0.f, 0.f, 0.f, 0.f};
 #pragma unroll
     for (int u = 0; u < kQkvSteps; ++u)
@@ -508,16 +521,18 @@ __device__ __forceinline__ void qkv_phase(const ChainArgs& a, int blk, q3::f32x4
   // 16 lanes per token as for a whole head; the quads of the other block are
   // zero here.
   const int r = tid >> 4, j = tid & 15;
-  if (r < a.M) {  // whole 16-lane groups
+  if (r < M) {  // whole 16-lane groups
     const bool mine = ((j >> 2) & 1) == hf;
     const int at = 8 * (j & 3) + (j >> 3) * 32;
     const q3::u32x4 xw = mine ? *reinterpret_cast<const q3::u32x4*>(&y_s[r][at])
                               : q3::u32x4{0u, 0u, 0u, 0u};
     if (mine || head < a.hd.Hq + a.hd.Hkv)
-      finish_head(a.hd, head, r, j, xw, pos_s[r], phys_s[r], off_s[r], mine,
-                  [&](float ss) { return exchange_sum(a, head, hf, r, j, ss); });
+      finish_head(a.hd, head, kRows * rb + r, j, xw, pos_s[r], phys_s[r], off_s[r], mine,
+                  [&](float v) {
+                    return exchange_sum(a, a.sync + kSumWord + rb * kSumWords, head, hf, r, j, v);
+                  });
   }
-  if (wave == 0) reset_flags(a, ticket);
+  if (!kAlone && wave == 0) reset_flags(a, ticket);
 }
 
 // Two blocks per CU (the largest grid the host launches is what fits).
@@ -546,8 +561,23 @@ void decode_chain_kernel(ChainArgs a) {
   } else if (blk < a.first[kQkv]) {
     linear_phase<kDown>(a, blk - a.first[kDown], red, nw_s);
   } else {
-    qkv_phase(a, blk - a.first[kQkv], red, a_s, nw_s);
+    qkv_phase<false>(a, blk - a.first[kQkv], 0, red, a_s, nw_s);
   }
+}
+
+// The qkv phase as a launch of its own, for up to 64 rows: block (half head,
+// 16-row block), the row blocks of a half head on one XCD (blocks are dealt to
+// the eight in turn) where their weights meet in its L2.
+__global__ __launch_bounds__(kThreads) __attribute__((amdgpu_waves_per_eu(4, 4)))
+void decode_qkv_half_kernel(ChainArgs a) {
+  __shared__ q3::f32x4 red[kWaves][64];
+  __shared__ __attribute__((aligned(16))) uint16_t a_s[kRows * (kMaxHidden + 8)];
+  __shared__ __attribute__((aligned(16))) uint16_t nw_s[kMaxHidden];
+  const int rbc = (a.M + kRows - 1) / kRows;
+  const int halves = 2 * (a.hd.Hq + 2 * a.hd.Hkv);
+  const int slot = static_cast<int>(blockIdx.x >> 3);
+  const int half = (slot / rbc) * 8 + static_cast<int>(blockIdx.x & 7);
+  if (half < halves) qkv_phase<true>(a, half, slot % rbc, red, a_s, nw_s);
 }
 
 // Blocks resident at once on the current device (0: unknown).
@@ -585,6 +615,60 @@ bool phase_blocks(int M, int hidden, int inter, int num_heads, int num_kv_heads,
   first[0] = 0;
   for (int p = 0; p < kPhases; ++p) first[p + 1] = first[p] + n[p];
   return first[kPhases] <= kMaxBlocks;
+}
+
+// The next layer's part of the arguments.
+int fill_qkv(ChainArgs& a, const qwen3_decode_chain_args* c, const char* who) {
+  if (!c->in_norm_weight || !c->q_norm_weight || !c->k_norm_weight || !c->cos_table ||
+      !c->sin_table || !c->q_out || !c->k_cache || !c->v_cache || !c->seq_lens ||
+      !c->block_table)
+    return q3::fail(QWEN3_EINVAL, "%s: null pointer argument", who);
+  if (c->block_size <= 0 || c->num_blocks <= 0 || c->layer_idx < 0 ||
+      c->layer_idx >= c->num_layers || c->table_rows < 0 || c->max_rows <= 0 ||
+      c->max_pages <= 0 || c->bt_row_stride < c->max_pages || !(c->head_eps >= 0.f))
+    return q3::fail(QWEN3_EINVAL, "%s: bad sizes", who);
+  bool ok = q3::aligned16(c->in_norm_weight) && q3::aligned16(c->qkv_weight) &&
+       q3::aligned16(c->q_norm_weight) && q3::aligned16(c->k_norm_weight) &&
+       q3::aligned16(c->cos_table) && q3::aligned16(c->sin_table) && q3::aligned16(c->q_out) &&
+       q3::aligned16(c->k_cache) && q3::aligned16(c->v_cache) && c->qkv_row_stride % 8 == 0 &&
+       c->table_row_stride % 4 == 0 && c->q_out_strides[0] % 8 == 0 &&
+       c->q_out_strides[1] % 8 == 0;
+  HeadArgs& hd = a.hd;
+  for (int i = 0; i < 4; ++i) {
+    ok = ok && c->k_cache_strides[i] % 8 == 0 && c->v_cache_strides[i] % 8 == 0;
+    hd.kc[i] = c->k_cache_strides[i];
+    hd.vc[i] = c->v_cache_strides[i];
+  }
+  a.in_w = static_cast<const uint16_t*>(c->in_norm_weight);
+  a.qkv_w = static_cast<const uint16_t*>(c->qkv_weight);
+  a.qkv_ws = c->qkv_row_stride;
+  hd.M = c->M;
+  hd.Hq = c->num_heads;
+  hd.Hkv = c->num_kv_heads;
+  hd.q_w = static_cast<const uint16_t*>(c->q_norm_weight);
+  hd.k_w = static_cast<const uint16_t*>(c->k_norm_weight);
+  hd.head_eps = c->head_eps;
+  hd.cos_t = c->cos_table;
+  hd.sin_t = c->sin_table;
+  hd.tab_stride = c->table_row_stride;
+  hd.tab_rows = c->table_rows;
+  hd.positions = c->positions;
+  hd.q_out = static_cast<uint16_t*>(c->q_out);
+  hd.qo_s0 = c->q_out_strides[0];
+  hd.qo_s1 = c->q_out_strides[1];
+  hd.k_cache = static_cast<uint16_t*>(c->k_cache);
+  hd.v_cache = static_cast<uint16_t*>(c->v_cache);
+  hd.num_blocks = c->num_blocks;
+  hd.layer = c->layer_idx;
+  hd.seq_lens = c->seq_lens;
+  hd.block_table = c->block_table;
+  hd.bt_stride = c->bt_row_stride;
+  hd.max_rows = c->max_rows;
+  hd.max_pages = c->max_pages;
+  hd.row_ids = c->row_ids;
+  hd.bs = c->block_size;
+  if (!ok) return q3::fail(QWEN3_EALIGN, "%s: tensors need 16-byte aligned rows", who);
+  return QWEN3_OK;
 }
 
 }  // namespace
@@ -662,56 +746,9 @@ extern "C" int qwen3_decode_chain_bf16(const qwen3_decode_chain_args* c, void* s
   a.down_w = static_cast<const uint16_t*>(c->down_weight);
   a.down_ws = c->down_row_stride;
   a.sync = c->sync;
-  if (qkv) {
-    if (!c->in_norm_weight || !c->q_norm_weight || !c->k_norm_weight || !c->cos_table ||
-        !c->sin_table || !c->q_out || !c->k_cache || !c->v_cache || !c->seq_lens ||
-        !c->block_table)
-      return q3::fail(QWEN3_EINVAL, "%s: null pointer argument", who);
-    if (c->block_size <= 0 || c->num_blocks <= 0 || c->layer_idx < 0 ||
-        c->layer_idx >= c->num_layers || c->table_rows < 0 || c->max_rows <= 0 ||
-        c->max_pages <= 0 || c->bt_row_stride < c->max_pages || !(c->head_eps >= 0.f))
-      return q3::fail(QWEN3_EINVAL, "%s: bad sizes", who);
-    ok = ok && q3::aligned16(c->in_norm_weight) && q3::aligned16(c->qkv_weight) &&
-         q3::aligned16(c->q_norm_weight) && q3::aligned16(c->k_norm_weight) &&
-         q3::aligned16(c->cos_table) && q3::aligned16(c->sin_table) && q3::aligned16(c->q_out) &&
-         q3::aligned16(c->k_cache) && q3::aligned16(c->v_cache) && c->qkv_row_stride % 8 == 0 &&
-         c->table_row_stride % 4 == 0 && c->q_out_strides[0] % 8 == 0 &&
-         c->q_out_strides[1] % 8 == 0;
-    HeadArgs& hd = a.hd;
-    for (int i = 0; i < 4; ++i) {
-      ok = ok && c->k_cache_strides[i] % 8 == 0 && c->v_cache_strides[i] % 8 == 0;
-      hd.kc[i] = c->k_cache_strides[i];
-      hd.vc[i] = c->v_cache_strides[i];
-    }
-    a.in_w = static_cast<const uint16_t*>(c->in_norm_weight);
-    a.qkv_w = static_cast<const uint16_t*>(c->qkv_weight);
-    a.qkv_ws = c->qkv_row_stride;
-    hd.M = c->M;
-    hd.Hq = c->num_heads;
-    hd.Hkv = c->num_kv_heads;
-    hd.q_w = static_cast<const uint16_t*>(c->q_norm_weight);
-    hd.k_w = static_cast<const uint16_t*>(c->k_norm_weight);
-    hd.head_eps = c->head_eps;
-    hd.cos_t = c->cos_table;
-    hd.sin_t = c->sin_table;
-    hd.tab_stride = c->table_row_stride;
-    hd.tab_rows = c->table_rows;
-    hd.positions = c->positions;
-    hd.q_out = static_cast<uint16_t*>(c->q_out);
-    hd.qo_s0 = c->q_out_strides[0];
-    hd.qo_s1 = c->q_out_strides[1];
-    hd.k_cache = static_cast<uint16_t*>(c->k_cache);
-    hd.v_cache = static_cast<uint16_t*>(c->v_cache);
-    hd.num_blocks = c->num_blocks;
-    hd.layer = c->layer_idx;
-    hd.seq_lens = c->seq_lens;
-    hd.block_table = c->block_table;
-    hd.bt_stride = c->bt_row_stride;
-    hd.max_rows = c->max_rows;
-    hd.max_pages = c->max_pages;
-    hd.row_ids = c->row_ids;
-    hd.bs = c->block_size;
-  }
+  a.h_s = c->hidden;
+  if (qkv)
+    if (const int rc = fill_qkv(a, c, who)) return rc;
   if (!ok) return q3::fail(QWEN3_EALIGN, "%s: tensors need 16-byte aligned rows", who);
   // rows of a weight tile inside 32-bit offsets, and not overlapping
   const int64_t strides[4][2] = {{c->o_weight_row_stride, a.KO}, {c->gate_up_row_stride, a.K},
@@ -724,5 +761,46 @@ extern "C" int qwen3_decode_chain_bf16(const qwen3_decode_chain_args* c, void* s
   q3::clear_error();
   hipLaunchKernelGGL(decode_chain_kernel, dim3(static_cast<unsigned>(a.first[kPhases])),
                      dim3(kThreads), 0, static_cast<hipStream_t>(stream), a);
+  return q3::launch_status(who);
+}
+
+extern "C" int qwen3_decode_qkv_half_supported(int M, int hidden, int num_heads,
+                                               int num_kv_heads) {
+  const int64_t blocks = q3::cdiv(2 * (num_heads + 2 * num_kv_heads), 8) * 8 * ((M + 15) / 16);
+  return M >= 1 && M <= kMaxRowBlocks * kRows && num_heads > 0 && num_kv_heads > 0 &&
+                 num_heads + num_kv_heads <= kMaxNormHeads && hidden > 0 &&
+                 hidden % (2 * kKStep) == 0 && hidden <= kMaxHidden && blocks <= resident_blocks()
+             ? 1
+             : 0;
+}
+
+extern "C" int qwen3_decode_qkv_half_bf16(const qwen3_decode_chain_args* c, int64_t h_row_stride,
+                                          void* stream) {
+  const char* who = "qwen3_decode_qkv_half_bf16";
+  if (!c || !c->h_out || !c->ss_out || !c->qkv_weight || !c->sync)
+    return q3::fail(QWEN3_EINVAL, "%s: null pointer argument", who);
+  if (c->M == 0) return QWEN3_OK;
+  if (!qwen3_decode_qkv_half_supported(c->M, c->hidden, c->num_heads, c->num_kv_heads))
+    return q3::fail(QWEN3_EUNSUPPORTED, "%s: %d rows, hidden %d, heads %d / %d not supported", who,
+                    c->M, c->hidden, c->num_heads, c->num_kv_heads);
+  if (h_row_stride < c->hidden || h_row_stride > (int64_t{1} << 24) ||
+      c->qkv_row_stride < c->hidden || c->qkv_row_stride > (int64_t{1} << 24) || !(c->eps >= 0.f))
+    return q3::fail(QWEN3_EINVAL, "%s: bad row strides or eps", who);
+  ChainArgs a{};
+  a.M = c->M;
+  a.K = c->hidden;
+  a.eps = c->eps;
+  a.h_out = static_cast<uint16_t*>(c->h_out);
+  a.h_s = h_row_stride;
+  a.ss_out = c->ss_out;
+  a.sync = c->sync;
+  if (const int rc = fill_qkv(a, c, who)) return rc;
+  if (!q3::aligned16(c->h_out) || !q3::aligned16(c->ss_out) || h_row_stride % 8 != 0)
+    return q3::fail(QWEN3_EALIGN, "%s: tensors need 16-byte aligned rows", who);
+  const int64_t blocks =
+      q3::cdiv(2 * (c->num_heads + 2 * c->num_kv_heads), 8) * 8 * ((c->M + 15) / 16);
+  q3::clear_error();
+  hipLaunchKernelGGL(decode_qkv_half_kernel, dim3(static_cast<unsigned>(blocks)), dim3(kThreads), 0,
+                     static_cast<hipStream_t>(stream), a);
   return q3::launch_status(who);
 }

@@ -255,6 +255,25 @@ def decode_chain_sync(device) -> torch.Tensor:
                        device=device)
 
 
+def _set_qkv(a, norm_weight, qkv_weight, q_norm_weight, k_norm_weight, cos_table, sin_table,
+             positions, q_out, pool, layer_idx, row_ids) -> None:
+    """The qkv projection's part of a DecodeChainArgs."""
+    kb, vb, bt = pool.k_buffer, pool.v_buffer, pool.block_table_2d
+    a.in_norm_weight = norm_weight.data_ptr()
+    a.qkv_weight, a.qkv_row_stride = qkv_weight.data_ptr(), qkv_weight.stride(0)
+    a.q_norm_weight, a.k_norm_weight = q_norm_weight.data_ptr(), k_norm_weight.data_ptr()
+    a.cos_table, a.sin_table = cos_table.data_ptr(), sin_table.data_ptr()
+    a.table_row_stride, a.table_rows = cos_table.stride(0), cos_table.shape[0]
+    a.positions, a.row_ids = _lib.ptr(positions), _lib.ptr(row_ids)
+    a.q_out, a.q_out_strides = q_out.data_ptr(), _lib.strides(q_out, (0, 1))
+    a.k_cache, a.k_cache_strides = kb.data_ptr(), _lib.strides(kb, (0, 1, 2, 3))
+    a.v_cache, a.v_cache_strides = vb.data_ptr(), _lib.strides(vb, (0, 1, 2, 3))
+    a.num_blocks, a.num_layers, a.block_size = kb.shape[0], kb.shape[1], kb.shape[3]
+    a.layer_idx = layer_idx
+    a.seq_lens, a.block_table = pool.seq_lens.data_ptr(), bt.data_ptr()
+    a.bt_row_stride, a.max_rows, a.max_pages = bt.stride(0), bt.shape[0], bt.shape[1]
+
+
 def decode_chain(o: torch.Tensor, h: torch.Tensor, h_mid: torch.Tensor, ss: torch.Tensor,
                  ss_mid: torch.Tensor, layer, eps: float, num_heads: int, num_kv_heads: int,
                  sync: torch.Tensor, *, attn_workspace: torch.Tensor | None = None,
@@ -299,7 +318,7 @@ def decode_chain(o: torch.Tensor, h: torch.Tensor, h_mid: torch.Tensor, ss: torc
         a.attn_waves = lib.qwen3_paged_decode_partials_waves()
     q = None
     if next_layer is not None:
-        at, kb, vb, bt = next_layer.self_attn, pool.k_buffer, pool.v_buffer, pool.block_table_2d
+        at = next_layer.self_attn
         wq = at.qkv_proj.weight
         assert wq.shape == ((num_heads + 2 * num_kv_heads) * 128, hidden) and wq.stride(1) == 1
         assert cos_table.dtype == sin_table.dtype == torch.float32 and cos_table.stride(1) == 1
@@ -308,19 +327,8 @@ def decode_chain(o: torch.Tensor, h: torch.Tensor, h_mid: torch.Tensor, ss: torc
         assert positions is None or (positions.dtype == torch.int64 and positions.is_contiguous()
                                      and positions.numel() == M)
         q = torch.empty(M, num_heads, 128, dtype=h.dtype, device=h.device)
-        a.in_norm_weight = next_layer.input_layernorm.weight.data_ptr()
-        a.qkv_weight, a.qkv_row_stride = wq.data_ptr(), wq.stride(0)
-        a.q_norm_weight, a.k_norm_weight = at.q_norm.weight.data_ptr(), at.k_norm.weight.data_ptr()
-        a.cos_table, a.sin_table = cos_table.data_ptr(), sin_table.data_ptr()
-        a.table_row_stride, a.table_rows = cos_table.stride(0), cos_table.shape[0]
-        a.positions, a.row_ids = _lib.ptr(positions), _lib.ptr(row_ids)
-        a.q_out, a.q_out_strides = q.data_ptr(), _lib.strides(q, (0, 1))
-        a.k_cache, a.k_cache_strides = kb.data_ptr(), _lib.strides(kb, (0, 1, 2, 3))
-        a.v_cache, a.v_cache_strides = vb.data_ptr(), _lib.strides(vb, (0, 1, 2, 3))
-        a.num_blocks, a.num_layers, a.block_size = kb.shape[0], kb.shape[1], kb.shape[3]
-        a.layer_idx = next_idx
-        a.seq_lens, a.block_table = pool.seq_lens.data_ptr(), bt.data_ptr()
-        a.bt_row_stride, a.max_rows, a.max_pages = bt.stride(0), bt.shape[0], bt.shape[1]
+        _set_qkv(a, next_layer.input_layernorm.weight, wq, at.q_norm.weight, at.k_norm.weight,
+                 cos_table, sin_table, positions, q, pool, next_idx, row_ids)
     rc = lib.qwen3_decode_chain_bf16(ctypes.byref(a), _lib.stream_of(dev))
     _lib.check(rc, "qwen3_decode_chain_bf16")
     return q
@@ -331,10 +339,13 @@ def decode_qkv_rope(h: torch.Tensor, ss_in: torch.Tensor, norm_weight: torch.Ten
                     q_norm_weight: torch.Tensor, k_norm_weight: torch.Tensor, head_eps: float,
                     cos_table: torch.Tensor, sin_table: torch.Tensor, pool, layer_idx: int,
                     row_ids: torch.Tensor | None, positions: torch.Tensor | None = None,
-                    q_out: torch.Tensor | None = None) -> torch.Tensor:
+                    q_out: torch.Tensor | None = None,
+                    sync: torch.Tensor | None = None) -> torch.Tensor:
     """Input RMSNorm + qkv projection + QK-norm + RoPE + K/V pool write of a
     decode step for at most 64 tokens in one launch; returns q (M, Hq, 128)
-    for the attention kernel (k and v go into `pool` at seq_lens[row])."""
+    for the attention kernel (k and v go into `pool` at seq_lens[row]).
+    sync (decode_chain_sync): two workgroups may share a head, with the same
+    results."""
     h = _rows2d(h)
     M, K = h.shape
     D = 128
@@ -352,7 +363,20 @@ def decode_qkv_rope(h: torch.Tensor, ss_in: torch.Tensor, norm_weight: torch.Ten
         positions = positions.contiguous()
     if q_out is None:
         q_out = torch.empty(M, num_heads, D, dtype=h.dtype, device=h.device)
-    rc = _lib.load().qwen3_decode_qkv_rope_bf16(
+    lib = _lib.load()
+    # the halves wait for one another, so all of them must be resident at once
+    if sync is not None and lib.qwen3_decode_qkv_half_supported(M, K, num_heads, num_kv_heads) \
+            and ss_in.shape[1] == K // 16:
+        a = _lib.DecodeChainArgs(M=M, hidden=K, num_heads=num_heads, num_kv_heads=num_kv_heads,
+                                 eps=eps, head_eps=head_eps, h_out=h.data_ptr(),
+                                 ss_out=ss_in.data_ptr(), sync=sync.data_ptr())
+        _set_qkv(a, norm_weight, qkv_weight, q_norm_weight, k_norm_weight, cos_table, sin_table,
+                 positions, q_out, pool, int(layer_idx), row_ids)
+        _lib.check(lib.qwen3_decode_qkv_half_bf16(ctypes.byref(a), h.stride(0),
+                                                  _lib.stream_of(dev)),
+                   "qwen3_decode_qkv_half_bf16")
+        return q_out
+    rc = lib.qwen3_decode_qkv_rope_bf16(
         h.data_ptr(), h.stride(0), ss_in.data_ptr(), ss_in.shape[1], norm_weight.data_ptr(),
         float(eps), qkv_weight.data_ptr(), qkv_weight.stride(0), M, K, num_heads, num_kv_heads,
         D, q_norm_weight.data_ptr(), k_norm_weight.data_ptr(), float(head_eps),

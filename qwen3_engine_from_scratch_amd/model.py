@@ -241,7 +241,8 @@ class Qwen3ForCausalLM(nn.Module):
             at0 = layers[0].self_attn
             q = decode_qkv_rope(h_a, ss_a, layers[0].input_layernorm.weight, eps,
                                 at0.qkv_proj.weight, Hq, Hkv, at0.q_norm.weight,
-                                at0.k_norm.weight, eps, cos, sin, pool, 0, row_ids, pos)
+                                at0.k_norm.weight, eps, cos, sin, pool, 0, row_ids, pos,
+                                sync=self._chain_sync)
             for i, layer in enumerate(layers):
                 kv = (q, pool.k_buffer[:, i], pool.v_buffer[:, i], pool.block_table_2d,
                       pool.seq_lens, row_ids, pool.block_size)
@@ -257,7 +258,7 @@ class Qwen3ForCausalLM(nn.Module):
             at = layer.self_attn
             q = decode_qkv_rope(h_a, ss_a, layer.input_layernorm.weight, eps, at.qkv_proj.weight,
                                 Hq, Hkv, at.q_norm.weight, at.k_norm.weight, eps, cos, sin, pool,
-                                i, row_ids, positions)
+                                i, row_ids, positions, sync=self._chain_sync)
             o = paged_attention_decode_hip(q, pool.k_buffer[:, i], pool.v_buffer[:, i],
                                            pool.block_table_2d, pool.seq_lens, row_ids,
                                            pool.block_size, workspace=ws,

@@ -116,3 +116,51 @@ def test_chain_same_bits_as_separate_kernels(gpu, hidden, inter, hq, hkv, M, mer
                               [h, ss, mid, ss_mid, pool.k_buffer, pool.v_buffer, q], want[i]):
             assert (x is None and y is None) or torch.equal(x, y), f"launch {i}: {name}"
         assert not sync.any()
+
+
+@pytest.mark.parametrize("hidden, hq, hkv", [(1024, 16, 8), (64, 3, 1), (640, 18, 9)])
+@pytest.mark.parametrize("M", [1, 16, 17, 33, 64])
+def test_qkv_half_heads_same_bits(gpu, hidden, hq, hkv, M):
+    """decode_qkv_rope on two workgroups per head against one: rows past a
+    16-row block's end, rows outside the resident table, a row stride of the
+    residual stream that is not its width; the exchanged words are left zero."""
+    from qwen3_engine_from_scratch_amd.PagedKVcache import (KVCachePool, PagedKVCache,
+                                                            reserve_pages_bulk, set_seq_lens_bulk)
+    from qwen3_engine_from_scratch_amd.kernels.model_ops import (decode_chain_sync,
+                                                                 decode_qkv_rope, embed_ss)
+    from qwen3_engine_from_scratch_amd.kernels.pre_attention import rope_tables
+
+    g = torch.Generator(device=gpu).manual_seed(M + hidden)
+    layer = _layer(g, gpu, hidden, 128, hq, hkv)
+    at = layer.self_attn
+    lens = [(37 * i) % 200 for i in range(M)]
+    pool = KVCachePool(sum(n // 16 + 1 for n in lens) + 2, 2, 16, hkv, 128, device=gpu,
+                       dtype=torch.bfloat16, max_seq_len=256, max_requests=M + 1)
+    caches = [PagedKVCache(pool) for _ in range(M)]
+    reserve_pages_bulk(caches, [n + 1 for n in lens])
+    for c, n in zip(caches, lens):
+        c.seq_len = n
+    set_seq_lens_bulk(caches)
+    rows = torch.tensor([c.row_id for c in caches], dtype=torch.int32, device=gpu)
+    if M > 16:
+        rows[5], rows[16] = -1, 1 << 20
+    cos, sin = rope_tables(128, 1e6, 256, device=gpu)
+    h, ss = embed_ss(torch.arange(M, device=gpu),
+                     torch.randn(64, hidden, generator=g, device=gpu).bfloat16())
+    wide = torch.zeros(M, hidden + 64, dtype=h.dtype, device=gpu)
+    wide[:, :hidden] = h
+    sync = decode_chain_sync(gpu)
+    announce(f"qkv half heads M={M} hidden={hidden} heads={hq}/{hkv}")
+
+    def run(x, **kw):
+        pool.k_buffer.zero_()
+        pool.v_buffer.zero_()
+        q = decode_qkv_rope(x, ss, layer.input_layernorm.weight, 1e-6, at.qkv_proj.weight, hq, hkv,
+                            at.q_norm.weight, at.k_norm.weight, 1e-5, cos, sin, pool, 1, rows, **kw)
+        return q, pool.k_buffer.clone(), pool.v_buffer.clone()
+
+    want = run(h)
+    for x in (h, wide[:, :hidden], h):
+        for a, b in zip(run(x, sync=sync), want):
+            assert torch.equal(a, b)
+    assert not sync.any()
