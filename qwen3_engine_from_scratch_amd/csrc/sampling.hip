@@ -201,10 +201,13 @@ struct alignas(16) PartOut {
 // tokens); 1 means the single-workgroup form.
 constexpr int kMaxParts = 8;
 // Top-p alone: tokens that the parts of a row list between them (each part
-// its share, at least; ties add to it).  Nucleus sets of language-model logits are mostly
-// below a few hundred tokens; a row whose cut lies past the listed ones is
-// streamed by one workgroup as without parts.
-constexpr int kNucleusList = 512;
+// its share, at least; ties add to it).  A row whose cut lies past the listed
+// ones is streamed by one workgroup as without parts, after the lists (132 us
+// against 88), so the list is long: top-p 0.9 over logits whose softmax
+// falls as rank^-1.3 keeps 1,250 tokens (rank^-1.5: 60).  512 entries are 1-2
+// us faster where they suffice (64 rows 32 against 34 us), but one row in a
+// few hundred of such logits did not.
+constexpr int kNucleusList = 1536;
 __host__ __device__ inline int parts_for(int64_t rows, int64_t vocab) {
   int p = rows <= 32 ? kMaxParts : rows <= 64 ? 4 : rows <= 128 ? 2 : 1;
   const int64_t rounds = (vocab + kThreads * 8 - 1) / (kThreads * 8);
@@ -586,7 +589,7 @@ __device__ __forceinline__ void part_values(int P, T none, F&& get, T (&v)[kMaxP
 //
 // One workgroup per row is bound by the row's passes on one CU (about 20 us
 // each), which is why the uncut rows are split too: top-p 0.9 over 8 x 151,936
-// logits 88.0 -> 28.4 us; over 62 rows 104.6 -> 34.8; no cut at all, 44 rows, 178.6 -> 31.5.
+// logits 88 -> 27.5 us, over 64 rows 105 -> 34; no cut at all, 44 rows, 178.6 -> 31.5.
 template <bool kVec>
 __global__ __launch_bounds__(kThreads) void sample_part_kernel(const uint16_t* logits,
                                                                int64_t row_s, int64_t vocab,
@@ -932,9 +935,33 @@ __global__ __launch_bounds__(kThreads) void sample_kernel(const uint16_t* logits
   // ---- A: high-bin counts and the maximum key ----------------------------
   uint32_t kmax = 0;
   bool from_list = false;  // the parts' lists stand for the row in passes A, B
+  // The top-p cut inside the high bin whose mass above it is r2, from the
+  // low-bin histograms: the first low bin whose mass passes the limit and how
+  // many of its ties are kept: rank r while the mass before it, r2 + r * w, is
+  // within the limit (rank 0 of the list's first key is always kept since r2
+  // is then 0).  Returns the bin, or -1.
+  auto low_cut = [&](unsigned long long r2, double limit, int64_t& keep) -> int {
+    for (int bin = kLoBins - 1; bin >= 0; --bin) {
+      const unsigned long long m = sh.lo_mass[bin];
+      if (sh.lo_cnt[bin] == 0) continue;
+      if (static_cast<double>(r2 + m) > limit) {
+        const unsigned long long w = m / sh.lo_cnt[bin];
+        keep = 0;
+        while (keep < static_cast<int64_t>(sh.lo_cnt[bin]) &&
+               static_cast<double>(r2 + w * static_cast<unsigned long long>(keep)) <= limit)
+          ++keep;
+        if (keep == 0) keep = 1;  // cannot happen unless rounding: keep the first
+        return bin;
+      }
+      r2 += m;
+    }
+    return -1;
+  };
   bool nucleus = false;    // ... of a row that only top-p cuts,
   uint32_t t_all = 0;      // where the lists hold every token at or above this key
   double nucleus_limit = 0.0;  // and this is top_p x the row's whole mass
+  uint32_t kc = 0;         // the final cut: a key and
+  int64_t tc = 0, cties = 0;  // the ties kept at it, of how many
   if constexpr (kPre) {
     int nc[kMaxParts];
     int total = 0;
@@ -1052,10 +1079,17 @@ __global__ __launch_bounds__(kThreads) void sample_kernel(const uint16_t* logits
       }
     }
     if (from_list) {
-      for (int i = tid; i < kHiBins; i += kThreads) sh.cnt[i] = 0;
-      if (tid < kLoBins) sh.lo_cnt[tid] = 0;
+      // the union's counts for passes A and B, or its masses for the cut of
+      // top-p alone (whose weights are relative to the row's maximum as ever)
+      const float xm = key_value(kmax) * inv_t;
+      for (int i = tid; i < kHiBins; i += kThreads) {
+        if (nucleus) sh.mass[i] = 0ull; else sh.cnt[i] = 0;
+      }
+      if (tid < kLoBins) {
+        sh.lo_cnt[tid] = 0;
+        sh.lo_mass[tid] = 0ull;
+      }
       __syncthreads();
-      unsigned long long listed = 0;
       // entry e of the concatenated lists: part c's run starts at the sum
       // of the runs before it
       for (int e = tid; e < total; e += kThreads) {
@@ -1074,14 +1108,25 @@ __global__ __launch_bounds__(kThreads) void sample_kernel(const uint16_t* logits
         if (!nucleus)
           atomicAdd(&sh.cnt[key >> kLoBits], 1u);
         else if (key >= t_all)
-          listed += fixed_weight(key, inv_t, key_value(kmax) * inv_t);
+          atomicAdd(&sh.mass[key >> kLoBits], fixed_weight(key, inv_t, xm));
       }
       ncand = total;
       __syncthreads();
-      if (nucleus) {  // top-p alone: a cut past the lists' tokens needs the row
-        unsigned long long mass;
-        block_scan_u64(listed, mass, sh);
-        if (!(static_cast<double>(mass) > nucleus_limit)) {
+      if (nucleus) {
+        unsigned long long above;
+        const int hb = find_mass_bin_block(sh.mass, pcut, nucleus_limit, above, sh, true);
+        if (hb >= 0) {
+          for (int i = tid; i < total; i += kThreads) {
+            const uint32_t key = static_cast<uint32_t>(sh.cand[i] >> 32);
+            if (static_cast<int>(key >> kLoBits) != hb || key < t_all) continue;
+            atomicAdd(&sh.lo_cnt[key & (kLoBins - 1)], 1u);
+            atomicAdd(&sh.lo_mass[key & (kLoBins - 1)], fixed_weight(key, inv_t, xm));
+          }
+          __syncthreads();
+          const int lb = low_cut(above, nucleus_limit, tc);
+          kc = (static_cast<uint32_t>(hb) << kLoBits) | static_cast<uint32_t>(lb);
+          cties = sh.lo_cnt[lb];
+        } else {  // a cut past the lists' tokens needs the row
           from_list = false;
           ncand = -1;
         }
@@ -1162,12 +1207,13 @@ __global__ __launch_bounds__(kThreads) void sample_kernel(const uint16_t* logits
   // with rank < tk (ranks in token order)
 
   // ---- C, D: the top-p cut over the top-k list ---------------------------
-  // kc / tc: the final cut (key and ties kept at it); the kept list is the
-  // first min(k, n_p) positions of the sorted top-k list.
-  if (nucleus) kk = t_all;  // nothing below it can be kept: the cut is above
-  uint32_t kc = kk;
-  int64_t tc = tk, cties = kties;
-  if (use_p) {
+  // The kept list is the first min(k, n_p) positions of the sorted top-k list.
+  if (!nucleus) {
+    kc = kk;
+    tc = tk;
+    cties = kties;
+  }
+  if (use_p && !nucleus) {
     // masses of the top-k list; the ties at kk count only up to tk of them
     __syncthreads();
     for (int i = tid; i < kHiBins; i += kThreads) sh.mass[i] = 0ull;
@@ -1187,9 +1233,9 @@ __global__ __launch_bounds__(kThreads) void sample_kernel(const uint16_t* logits
     __syncthreads();
     // high bins of the cut: the bin holding the first position whose mass
     // before it exceeds the limit
-    double limit = nucleus_limit;
+    double limit;
     unsigned long long above_hi;
-    const int hb = find_mass_bin_block(sh.mass, pcut, limit, above_hi, sh, nucleus);
+    const int hb = find_mass_bin_block(sh.mass, pcut, limit, above_hi, sh);
     if (hb >= 0) {  // else a row without mass (all NaN): no cut
       auto lo_hist = [&](uint32_t key, int64_t) {
         if (static_cast<int>(key >> kLoBits) != hb || key < kk) return;
@@ -1227,29 +1273,13 @@ __global__ __launch_bounds__(kThreads) void sample_kernel(const uint16_t* logits
         sh.lo_cnt[kk & (kLoBins - 1)] = static_cast<uint32_t>(tk);
       }
       __syncthreads();
-      unsigned long long r2 = above_hi;
-      for (int bin = kLoBins - 1; bin >= 0; --bin) {
-        const unsigned long long m = sh.lo_mass[bin];
-        if (sh.lo_cnt[bin] == 0) continue;
-        if (static_cast<double>(r2 + m) > limit) {
-          // ties at this key: keep rank r while the mass before it, r2 +
-          // r * w, is within the limit (rank 0 of the list's first key is
-          // always kept since r2 is then 0)
-          const uint32_t key = (static_cast<uint32_t>(hb) << kLoBits) | static_cast<uint32_t>(bin);
-          const unsigned long long w = m / sh.lo_cnt[bin];
-          int64_t keep = 0;
-          while (keep < static_cast<int64_t>(sh.lo_cnt[bin]) &&
-                 static_cast<double>(r2 + w * static_cast<unsigned long long>(keep)) <= limit)
-            ++keep;
-          if (keep == 0) keep = 1;  // cannot happen unless rounding: keep the first
-          // the top-p cut is inside the top-k list (its key >= kk)
-          kc = key;
-          const bool at_k = key == kk && !nucleus;
-          cties = at_k ? kties : sh.lo_cnt[bin];
-          tc = at_k ? (keep < tk ? keep : tk) : keep;
-          break;
-        }
-        r2 += m;
+      int64_t keep;
+      const int lb = low_cut(above_hi, limit, keep);
+      if (lb >= 0) {  // the cut is inside the top-k list (its key >= kk)
+        const uint32_t key = (static_cast<uint32_t>(hb) << kLoBits) | static_cast<uint32_t>(lb);
+        kc = key;
+        cties = key == kk ? kties : sh.lo_cnt[lb];
+        tc = key == kk ? (keep < tk ? keep : tk) : keep;
       }
     }
   }
