@@ -94,22 +94,6 @@ def paged_attention_decode_hip(q, k_buffer, v_buffer, block_table_2d,
     (default kernel) or one per device, stream and KV-head count kept by this
     module (batch-invariant kernel).
     """
-    name = "qwen3_paged_decode_invariant_bf16" if batch_invariant else "qwen3_paged_decode_bf16"
-    return _decode(name, q, k_buffer, v_buffer, block_table_2d, seq_lens_full, row_ids, block_size,
-                   seq_len_bias, scale, out, workspace, batch_invariant)
-
-
-def paged_attention_decode_partials_hip(q, k_buffer, v_buffer, block_table_2d, seq_lens_full,
-                                        row_ids, block_size, workspace: torch.Tensor):
-    """paged_attention_decode_hip (default kernel) without its merge launch:
-    sequence-heads split across waves are left as partial results in
-    `workspace`, for decode_chain to combine.  At most 2,048 rows."""
-    return _decode("qwen3_paged_decode_partials_bf16", q, k_buffer, v_buffer, block_table_2d,
-                   seq_lens_full, row_ids, block_size, 1, None, None, workspace, False)
-
-
-def _decode(name, q, k_buffer, v_buffer, block_table_2d, seq_lens_full, row_ids, block_size,
-            seq_len_bias, scale, out, workspace, batch_invariant):
     B, num_heads, head_dim = q.shape
     num_blocks, num_kv_heads, block_size_check, head_dim_check = k_buffer.shape
     assert block_size_check == block_size
@@ -145,7 +129,8 @@ def _decode(name, q, k_buffer, v_buffer, block_table_2d, seq_lens_full, row_ids,
         else:
             workspace = torch.empty(max(need, 1), dtype=torch.uint8, device=dev)
     lib = _lib.load()
-    rc = getattr(lib, name)(
+    fn = lib.qwen3_paged_decode_invariant_bf16 if batch_invariant else lib.qwen3_paged_decode_bf16
+    rc = fn(
         q.data_ptr(), _lib.strides(q, (0, 1)),
         k_buffer.data_ptr(), _lib.strides(k_buffer, (0, 1, 2)),
         v_buffer.data_ptr(), _lib.strides(v_buffer, (0, 1, 2)),
@@ -155,7 +140,41 @@ def _decode(name, q, k_buffer, v_buffer, block_table_2d, seq_lens_full, row_ids,
         out.data_ptr(), _lib.strides(out, (0, 1)),
         B, num_heads, num_kv_heads, head_dim, block_size, float(scale),
         workspace.data_ptr(), workspace.numel(), _lib.stream_of(dev))
-    _lib.check(rc, name)
+    _lib.check(rc, "qwen3_paged_decode_invariant_bf16" if batch_invariant
+               else "qwen3_paged_decode_bf16")
+    return out
+
+
+def paged_attention_decode_partials_hip(q, k_buffer, v_buffer, block_table_2d, seq_lens_full,
+                                        row_ids, block_size, workspace: torch.Tensor):
+    """paged_attention_decode_hip (default kernel, bias 1, scale
+    1/sqrt(head_dim)) without its merge launch: sequence-heads split across
+    waves are left as partial results in `workspace`
+    (paged_decode_workspace_bytes), for decode_chain to combine.  At most 2,048
+    rows; q, row_ids and seq_lens_full contiguous."""
+    B, num_heads, head_dim = q.shape
+    num_blocks, num_kv_heads, block_size_check, head_dim_check = k_buffer.shape
+    assert block_size_check == block_size and head_dim_check == head_dim
+    assert v_buffer.shape == k_buffer.shape
+    assert q.dtype == k_buffer.dtype == v_buffer.dtype == torch.bfloat16
+    assert block_table_2d.dtype == seq_lens_full.dtype == row_ids.dtype == torch.int32
+    assert q.is_contiguous() and row_ids.is_contiguous() and seq_lens_full.is_contiguous()
+    assert row_ids.numel() == B and block_table_2d.stride(1) == 1
+    assert k_buffer.stride(3) == 1 and v_buffer.stride(3) == 1
+    dev = _lib.require_hip(q, k_buffer, v_buffer, block_table_2d, seq_lens_full, row_ids,
+                           workspace)
+    out = torch.empty_like(q)
+    rc = _lib.load().qwen3_paged_decode_partials_bf16(
+        q.data_ptr(), _lib.strides(q, (0, 1)),
+        k_buffer.data_ptr(), _lib.strides(k_buffer, (0, 1, 2)),
+        v_buffer.data_ptr(), _lib.strides(v_buffer, (0, 1, 2)),
+        num_blocks,
+        block_table_2d.data_ptr(), block_table_2d.stride(0), *block_table_2d.shape,
+        seq_lens_full.data_ptr(), 1, row_ids.data_ptr(),
+        out.data_ptr(), _lib.strides(out, (0, 1)),
+        B, num_heads, num_kv_heads, head_dim, block_size, 1.0 / math.sqrt(head_dim),
+        workspace.data_ptr(), workspace.numel(), _lib.stream_of(dev))
+    _lib.check(rc, "qwen3_paged_decode_partials_bf16")
     return out
 
 

@@ -221,7 +221,9 @@ class Qwen3ForCausalLM(nn.Module):
         the linear after it and every residual add the epilogue of the
         linear before it; the qkv projection also applies QK-norm and RoPE
         and writes K/V into the pool, leaving one attention launch (plus its
-        merge) per layer.  Returns the last residual stream and its sums."""
+        merge) per layer.  At most 16 rows: everything between two attention
+        launches is one (decode_chain), with the same results.  Returns the last
+        residual stream and its sums."""
         cfg = self.config
         eps = cfg.rms_norm_eps
         layers = self.model.layers
