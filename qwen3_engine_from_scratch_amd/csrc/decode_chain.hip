@@ -24,15 +24,27 @@
 // results with device-scope loads.  (Counters instead of flags: an add takes
 // about 80 ns on its line, 2.4 us for 192 blocks on eight lines.  Eight copies
 // of the flags, each polled by an eighth of the blocks: device-scope loads of
-// one line are served about 10 ns apart, 2.5 us a round for 192 blocks.)  No fence: those write back and invalidate the whole
-// L2.  The host launches at most as many blocks as are resident at once, and a
-// block waits only for lower-numbered ones, which the dispatcher starts
-// first (and the two blocks of a head, next to each other, for one another).  Before it waits, a block runs its phase once without storing
-// anything: the weights passing through have evicted the code since the last
-// launch, and a first pass over a phase's instructions takes a microsecond or
-// more longer than the second.  A wait also ends, with the launch's results invalid, if it is ever
-// not answered within kSpinTicks, and then at once for every other wait.
-// The blocks of the last phase put the flags back to zero.
+// one line are served about 10 ns apart, 2.5 us a round for 192 blocks.)  No
+// fence: those write back and invalidate the whole L2.
+//
+// The host launches at most as many blocks as are resident at once, and a
+// block waits only for lower-numbered ones, which the dispatcher starts first
+// (and the two blocks of a head, next to each other, for one another).  A wait
+// also ends, with the launch's results invalid, if it is ever not answered
+// within kSpinTicks, and then at once for every other wait.  The blocks of the
+// last phase put the flags back to zero.
+//
+// Before they wait, gate_up, down and qkv blocks run their phase once without
+// data and without storing anything: the weights passing through have evicted
+// the code since the last launch, and a first pass over a phase's
+// instructions takes a microsecond or more longer than the second.  They ask
+// for their weights after that, when the merge's loads and o_proj's are out.
+// (o_proj has no such pass: it would end after the merge.)
+//
+// Qwen3-0.6B, one row at 900 tokens: merge done 6.2 us after the start, o_proj
+// 9.9, gate_up 14, down 17.5, qkv 22.5; as separate launches 5.0, 5.9, 7.4,
+// 5.9 and 13.5 each.  A step with them: 1445 -> 958 us, the attention's change
+// for small batches included.
 #include "decode_head.hpp"
 #include "paged_decode_merge.hpp"
 

@@ -45,11 +45,14 @@
 // at or above the row's k-th largest key is then kept: a part holding one
 // below its own threshold holds k tokens above it, more than the row has.
 // One workgroup per row then runs passes A to E over the concatenated lists
-// instead of the row (or over the row when a list overflowed or top-k cuts
-// nothing).  The lists hold the whole top-k list and every tie at its
-// boundary, and no step depends on the order of the candidates, so the
-// draws are the single workgroup's.  Greedy rows take each part's first
-// maximum and then the first among the parts.
+// instead of the row (or over the row when a list overflowed).  The lists hold
+// the whole top-k list and every tie at its boundary, and no step depends on
+// the order of the candidates, so the draws are the single workgroup's.
+// Greedy rows take each part's first maximum and then the first among the
+// parts; rows that nothing cuts each part's draw and then the best; rows that
+// only top-p cuts list a fixed share of tokens per part beside the part's
+// softmax mass, and the cut is made in the union (or over the row when it lies
+// past the listed tokens).
 //
 // The VALU is the limit of every pass (a wave64 instruction occupies its
 // SIMD four cycles), so the per-token work is kept small: whole rounds of
