@@ -84,8 +84,7 @@ void paged_decode_stream_kernel(DecodeArgs a) {
   const int64_t T = static_cast<int64_t>(a.Hkv) * total;
   const int64_t W = static_cast<int64_t>(gridDim.x) * kWaves;
   int64_t pw = q3::cdiv(T, W);
-  const int64_t least = T <= kChunk * gridDim.x ? kChunk : kMinTilesPerWave;
-  pw = pw < least ? least : pw;
+  pw = pw < kMinTilesPerWave ? kMinTilesPerWave : pw;
   if (blockIdx.x == 0) {
     for (int b = tid; b <= B; b += kWaves * 64) a.s_pref[b] = s_pref[b];
     if (tid == 0) a.s_meta[0] = static_cast<int32_t>(pw);

@@ -20,9 +20,11 @@ constexpr int kStreamMaxB = 2048;       // batch entries tabulated in LDS
 constexpr int kStreamWgPerCu = 2;       // resident workgroups per CU (2 waves/SIMD)
 constexpr int kStreamMaxWgs = 1024;     // persistent grid cap (512 CUs)
 // Fewest tiles a wave streams: its two load batches, both issued before the
-// first is computed, so a small batch costs one tile round trip per wave; one
-// batch when that gives no workgroup more than one wave (one sequence of 250
-// tokens, 16/8 heads, with its merge: 10.4 -> 8.8 us; 900 tokens 11.8 -> 11.1).
+// first is computed, so a small batch costs one tile round trip per wave.  Part
+// of the output's bits (a head is split where a range ends), so not a choice
+// made by the batch: with one load batch per wave for the smallest ones, a
+// decode step of one sequence would differ by 1.4% (one of 250 tokens, 16/8
+// heads, with its merge: 8.8 us against 10.4).
 constexpr int kMinTilesPerWave = 2 * kChunk;
 
 struct DecodeArgs {

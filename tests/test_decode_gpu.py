@@ -287,14 +287,13 @@ def test_decode_batch_sizes_around_tabulation_rounds(gpu, B, invariant):
 
 @pytest.mark.parametrize("lens", [
     [1], [33],                       # fewer tiles than workgroups
-    [2048], [2049],                  # 1,024 tiles on 512 workgroups: two per wave, then four
+    [2048], [2049],
     [16352], [16368], [16385],       # the last range short of, at and past the grid's waves
     [700, 1, 300, 2000],
 ])
 def test_decode_small_batches_around_wave_spreading(gpu, lens):
-    """Small batches run one wave per workgroup first, with one load batch
-    per wave while that covers the tiles: lengths at both edges (16/8 heads
-    on a 256-CU grid), against the fp32 reference."""
+    """Small batches run one wave per workgroup first: lengths at both edges
+    (16/8 heads on a 256-CU grid), against the fp32 reference."""
     from qwen3_engine_from_scratch_amd.kernels.paged_attention import paged_attention_decode_hip
 
     announce(f"decode small batch {lens}")
@@ -304,3 +303,20 @@ def test_decode_small_batches_around_wave_spreading(gpu, lens):
     torch.cuda.synchronize()
     ref = gpu_dense_decode_fp32(t["q"], t["k"], t["v"], t["bt"], t["seq_lens"], t["row_ids"], 16)
     assert_close_attn(out, ref, f"lens={lens}")
+
+
+@pytest.mark.parametrize("n", [1, 3, 16])
+def test_decode_small_batch_ranges_are_whole_load_pairs(gpu, n):
+    """The smallest range of a wave is its two load batches, four tiles: a
+    head of 64 tokens is one wave's whole, so it has the bits of the large
+    batch whose waves hold several heads each."""
+    from qwen3_engine_from_scratch_amd.kernels.paged_attention import paged_attention_decode_hip
+
+    announce(f"decode ranges of a small batch n={n}")
+    t = make_device_decode([64] * 512, 16, 8, gpu, seed=3, slack=0.1)
+
+    def run(rows):
+        return paged_attention_decode_hip(t["q"][:rows].contiguous(), t["k"], t["v"], t["bt"],
+                                          t["seq_lens"], t["row_ids"][:rows].contiguous(), 16)
+
+    assert torch.equal(run(n), run(512)[:n])
