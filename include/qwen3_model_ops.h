@@ -150,9 +150,13 @@ int qwen3_decode_qkv_rope_bf16(const void* h, int64_t h_row_stride,
  *   (qkv_weight not NULL).
  * h_in, h_mid, h_out (M x hidden), act (M x intermediate), ss_mid, ss_out
  * (M x hidden / 16) are contiguous; h_out may be h_in.  sync:
- * qwen3_decode_chain_sync_bytes() bytes, zero before the first launch; every
- * launch leaves it zero; launches that share one must not overlap.  Shapes:
- * qwen3_decode_chain_supported() (its launch must fit the device at once). */
+ * qwen3_decode_chain_sync_bytes() bytes, zero before the first launch and the
+ * launches' own from then on (their number, flags that carry it); launches that
+ * share one must not overlap.  Any number of launches with a sync each may
+ * overlap, with one another and with other work: a block that waits longer
+ * than wait_ticks for others runs their part itself, so every launch ends with
+ * the same results wherever its blocks are started.  Shapes:
+ * qwen3_decode_chain_supported() (grids that fit the device at once). */
 typedef struct {
   int M, hidden, intermediate, num_heads, num_kv_heads;
   float eps, head_eps;
@@ -195,6 +199,7 @@ typedef struct {
   int64_t bt_row_stride, max_rows, max_pages;
   const int32_t* row_ids; /* nullable */
   int layer_idx, num_layers, block_size;
+  int64_t wait_ticks; /* of the 100 MHz clock; 0: the default, 200 us; below: none */
 } qwen3_decode_chain_args;
 
 size_t qwen3_decode_chain_sync_bytes(void);

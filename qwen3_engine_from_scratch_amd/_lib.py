@@ -37,7 +37,7 @@ class DecodeChainArgs(ctypes.Structure):
         ("k_cache_strides", _i64 * 4), ("v_cache_strides", _i64 * 4), ("num_blocks", _i64),
         ("seq_lens", _vp), ("block_table", _vp), ("bt_row_stride", _i64), ("max_rows", _i64),
         ("max_pages", _i64), ("row_ids", _vp),
-        ("layer_idx", _i), ("num_layers", _i), ("block_size", _i),
+        ("layer_idx", _i), ("num_layers", _i), ("block_size", _i), ("wait_ticks", _i64),
     ]
 
 

@@ -16,6 +16,17 @@ void clear_error();
 // Converts the launch status of the kernel just enqueued into a return code.
 int launch_status(const char* what);
 
+// A pointer to device memory as a field of a kernel's argument: accesses
+// through it are global ones also where the compiler cannot see that the
+// field comes from the argument.
+template <typename T>
+struct GlobalPtr {
+  __attribute__((address_space(1))) T* p;
+  GlobalPtr() = default;
+  __host__ __device__ GlobalPtr(T* x) : p((__attribute__((address_space(1))) T*)x) {}
+  __host__ __device__ operator T*() const { return (T*)p; }
+};
+
 // ---- register types ------------------------------------------------------
 typedef __bf16 bf16x8 __attribute__((__vector_size__(8 * sizeof(__bf16))));
 typedef __bf16 bf16x4 __attribute__((__vector_size__(4 * sizeof(__bf16))));

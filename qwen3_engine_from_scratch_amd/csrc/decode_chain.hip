@@ -19,20 +19,29 @@
 //
 // Hand-off: the blocks of a phase are numbered after those of the phase
 // before it.  A block publishes its results with device-scope (sc1) stores,
-// waits until they are complete, and sets its own flag words; a block of the
-// next phase polls that phase's flags, 256 at a time, and then reads the
-// results with device-scope loads.  (Counters instead of flags: an add takes
-// about 80 ns on its line, 2.4 us for 192 blocks on eight lines.  Eight copies
-// of the flags, each polled by an eighth of the blocks: device-scope loads of
-// one line are served about 10 ns apart, 2.5 us a round for 192 blocks.)  No
-// fence: those write back and invalidate the whole L2.
+// waits until they are complete, and sets its own flag words to the launch's
+// number; a block of the next phase polls that phase's flags, 256 at a time, and
+// then reads the results with device-scope loads.  (Counters instead of flags:
+// an add takes about 80 ns on its line, 2.4 us for 192 blocks on eight lines.
+// Eight copies of the flags, each polled by an eighth of the blocks: device-scope
+// loads of one line are served about 10 ns apart, 2.5 us a round for 192
+// blocks.)  No fence: those write back and invalidate the whole L2.
 //
-// The host launches at most as many blocks as are resident at once, and a
-// block waits only for lower-numbered ones, which the dispatcher starts first
-// (and the two blocks of a head, next to each other, for one another).  A wait
-// also ends, with the launch's results invalid, if it is ever not answered
-// within kSpinTicks, and then at once for every other wait.  The blocks of the
-// last phase put the flags back to zero.
+// Progress: a block never depends on another one being resident.  The dispatcher
+// starts the blocks in order on each XCD, but not across XCDs, and other work
+// (another such launch on another stream, another process, a CU mask) may hold
+// the slots that a waited-for block needs.  So a wait that is not answered within
+// wait_ticks ends, and the block runs the missing blocks' work itself, lowest
+// phase first, and then its own again (next_item).  That is sound because every
+// block's work is a function of its number whose inputs do not change while
+// anyone may still need them: running it twice, even at the same time, stores
+// the same bits.  (The one input that the launch overwrites, h_in where h_out is
+// the same buffer: an o_proj block first loads its residual and then looks at its
+// own flag; unset, what it loaded is from before any down block could store;
+// set, its work is done and it stores nothing.)  Nothing is put back to zero for
+// the next launch, which would have to know that no late block still comes:
+// flags and exchanged sums carry the launch's number, which the last block to
+// arrive advances.
 //
 // Before they wait, gate_up, down and qkv blocks run their phase once without
 // data and without storing anything: the weights passing through have evicted
@@ -43,8 +52,11 @@
 //
 // Qwen3-0.6B, one row at 900 tokens: merge done 6.2 us after the start, o_proj
 // 9.9, gate_up 14, down 17.5, qkv 22.5; as separate launches 5.0, 5.9, 7.4,
-// 5.9 and 13.5 each.  A step with them: 1445 -> 958 us, the attention's change
-// for small batches included.
+// 5.9 and 13.5 each (24.5 for the launch as a kernel trace counts it).  A step
+// with them: 1448 -> 1033 us, of which a flag that carries the launch's number,
+// where the flags were put back to zero and a wait could fail for good, is
+// 10.  The rare path is code of its own behind the usual one: a loop around both
+// would hold what it shares in more registers than there are.
 #include "decode_head.hpp"
 #include "paged_decode_merge.hpp"
 
@@ -61,19 +73,27 @@ constexpr int kMaxHidden = 2 * kQkvSteps * kKStep;  // 1024
 constexpr int kMaxBlocks = 1024;
 constexpr int kMaxNormHeads = 64;  // q and k heads
 constexpr int kSc1 = 16;        // buffer cache policy: device scope
-constexpr uint64_t kSpinTicks = 400000000ull;  // of the 100 MHz clock: 4 s
+// A wait's limit, in ticks of the 100 MHz clock: 200 us, ten times the longest
+// wait of a launch that has the device to itself.
+constexpr int64_t kWaitTicks = 20000;
 
 enum Phase : int { kMerge = 0, kO = 1, kGateUp = 2, kDown = 3, kQkv = 4, kPhases = 5 };
-// Sync words: kCopies flags per block, then (on lines of their own) the count of
-// last-phase blocks past their wait and the word a timed-out wait sets, and
-// the sums that the two blocks of a q or k head exchange.
+// Sync words, each part on lines (128 bytes) of its own: the number of launches
+// so far, the counts of blocks that have arrived (kArriveLines lines, then
+// the lines that are complete), kCopies flags per block, and the sums that the
+// two blocks of a q or k head exchange (8 bytes: launch number, sum).
 constexpr int kCopies = 8;
-constexpr int kDoneWord = kCopies * kMaxBlocks;
-constexpr int kFailWord = kDoneWord + 32;
-constexpr int kSumWord = kFailWord + 32;  // [head][half of it][row][2]
-constexpr int kSumWords = kMaxNormHeads * 2 * kRows * 2;
+constexpr int kLine = 32;
+constexpr int kArriveLines = 32;
+constexpr int kArriveWord = kLine;
+constexpr int kFlagWord = kArriveWord + (kArriveLines + 1) * kLine;
+constexpr int kSumWord = kFlagWord + kCopies * kMaxBlocks;  // [head][half of it][row][2]
+constexpr int kSums = kMaxNormHeads * 2 * kRows * 2;
 constexpr int kMaxRowBlocks = 4;  // of the qkv kernel
-constexpr int kSyncWords = kSumWord + kMaxRowBlocks * kSumWords;
+constexpr int kSyncWords = kSumWord + 2 * kMaxRowBlocks * kSums;
+
+// How a run of one block's work ended: stored, or a wait was not answered.
+enum Run : int { kDone = 0, kPhaseMissing = 1, kPartnerMissing = 2 };
 
 struct ChainArgs {
   int M, K, I, KO;          // rows, hidden, intermediate, Hq * 128
@@ -81,27 +101,36 @@ struct ChainArgs {
   int last_phase;           // kQkv, or kDown for the last layer
   float eps;
   StreamPartials parts;     // merge phase (its block count may be 0)
-  uint16_t* o;              // M x KO, row stride o_s
+  q3::GlobalPtr<uint16_t> o;              // M x KO, row stride o_s
   int64_t o_s;
-  const uint16_t* o_w;
+  q3::GlobalPtr<const uint16_t> o_w;
   int64_t o_ws;
-  const uint16_t* h_in;     // residual streams (M x K, contiguous)
-  uint16_t* h_mid;
-  uint16_t* h_out;
-  float* ss_mid;            // (M x K / 16) sums of squares
-  float* ss_out;
-  const uint16_t* post_w;
-  const uint16_t* gu_w;     // gate rows 0.., up rows I..
+  q3::GlobalPtr<const uint16_t> h_in;     // residual streams (M x K, contiguous)
+  q3::GlobalPtr<uint16_t> h_mid;
+  q3::GlobalPtr<uint16_t> h_out;
+  q3::GlobalPtr<float> ss_mid;            // (M x K / 16) sums of squares
+  q3::GlobalPtr<float> ss_out;
+  q3::GlobalPtr<const uint16_t> post_w;
+  q3::GlobalPtr<const uint16_t> gu_w;     // gate rows 0.., up rows I..
   int64_t gu_ws;
-  uint16_t* act;            // M x I, contiguous
-  const uint16_t* down_w;
+  q3::GlobalPtr<uint16_t> act;            // M x I, contiguous
+  q3::GlobalPtr<const uint16_t> down_w;
   int64_t down_ws;
   int64_t h_s;              // row stride of h_out for the qkv phase
-  const uint16_t* in_w;     // next layer
-  const uint16_t* qkv_w;
+  q3::GlobalPtr<const uint16_t> in_w;     // next layer
+  q3::GlobalPtr<const uint16_t> qkv_w;
   int64_t qkv_ws;
   HeadArgs hd;
-  uint32_t* sync;           // kSyncWords, zero between launches
+  q3::GlobalPtr<uint32_t> sync;           // kSyncWords, zero before the first launch
+  int64_t wait_ticks;
+};
+
+// Of one workgroup, in LDS.
+struct Shared {
+  uint32_t launch;  // this launch's number
+  bool arrived;     // of wave kTagWave's own
+  int run;          // of the current run: its Run so far
+  int item;         // the next item to run
 };
 
 __device__ __forceinline__ __amdgpu_buffer_rsrc_t rsrc_of(const void* p, int64_t bytes) {
@@ -134,69 +163,139 @@ __device__ __forceinline__ void st16b_dev(uint16_t* p, uint16_t v) {
   __hip_atomic_store(p, v, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
 }
 
-// For a wait that has polled a while since t0: whether it, or any other wait of
-// the launch, has been too long.
-__device__ __forceinline__ bool timed_out(const ChainArgs& a, uint64_t t0) {
-  uint32_t* fail = a.sync + kFailWord;
-  if (wall_clock64() - t0 > kSpinTicks)
-    __hip_atomic_store(fail, 1u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-  return __hip_atomic_load(fail, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) != 0u;
+__device__ __forceinline__ uint32_t ld_dev(const uint32_t* p) {
+  return __hip_atomic_load(p, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+}
+__device__ __forceinline__ void st_dev(uint32_t* p, uint32_t v) {
+  __hip_atomic_store(p, v, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+}
+__device__ __forceinline__ uint32_t add_dev(uint32_t* p) {
+  return __hip_atomic_fetch_add(p, 1u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
 }
 
-// Waits for the blocks of phase `ph`.  Every thread of the block calls it.
-__device__ __forceinline__ void wait_phase(const ChainArgs& a, int ph) {
-  if (threadIdx.x < 64) {
-    const uint32_t* flags = a.sync + blockIdx.x % kCopies * kMaxBlocks;
+// x, unknown to the compiler: what is derived from it is computed where it is
+// used (hoisted out of the pass loops, the offsets of all k-steps would need
+// more registers than there are).
+__device__ __forceinline__ uint32_t fresh(uint32_t x) {
+  asm volatile("" : "+v"(x));
+  return x;
+}
+
+// The wave that reads the launch's number and reports the block's arrival: it
+// has nothing to do while wave 0 waits, stores or polls.
+constexpr int kTagWave = kWaves - 1;
+
+// The launch's number, never 0, read once per block, by wave kTagWave into LDS;
+// the other waves use it after the block's next barrier.  (It comes round after
+// 2^32 - 1 launches, days of decoding; a word is then taken for set only if no
+// launch since has used it.)
+__device__ __forceinline__ uint32_t read_launch(const uint32_t* sync) {
+  return threadIdx.x == kTagWave * 64 ? max(ld_dev(sync) + 1u, 1u) : 0u;
+}
+__device__ __forceinline__ void share_launch(Shared& sh, uint32_t launch) {
+  if (launch != 0u) {
+    sh.launch = launch;
+    sh.arrived = false;
+  }
+}
+
+// Reports that this block has read the launch's number (wave kTagWave, after
+// share_launch; once).  The last of all blocks advances the number: no block of
+// this launch can read it any more, and the next launch begins after all of
+// them have ended.
+__device__ __forceinline__ void arrive(const ChainArgs& a, Shared& sh) {
+  if (threadIdx.x != kTagWave * 64 || sh.arrived) return;
+  sh.arrived = true;
+  const int line = blockIdx.x % kArriveLines;
+  const int lines = min(static_cast<int>(gridDim.x), kArriveLines);
+  const int n = (static_cast<int>(gridDim.x) - line + kArriveLines - 1) / kArriveLines;
+  uint32_t* count = a.sync + kArriveWord + line * kLine;
+  uint32_t* all = a.sync + kArriveWord + kArriveLines * kLine;
+  if (add_dev(count) == static_cast<uint32_t>(n - 1)) {
+    st_dev(count, 0u);
+    if (add_dev(all) == static_cast<uint32_t>(lines - 1)) {
+      st_dev(all, 0u);
+      st_dev(a.sync, sh.launch);
+    }
+  }
+}
+
+__device__ __forceinline__ const uint32_t* flags_of(const ChainArgs& a) {
+  return a.sync + kFlagWord + blockIdx.x % kCopies * kMaxBlocks;
+}
+
+// Whether a wait since t0 is over, after `polls` that were not answered (a
+// negative limit: after the first).
+__device__ __forceinline__ bool too_long(const ChainArgs& a, uint64_t t0, int polls) {
+  return ((polls & 3) == 0 || a.wait_ticks < 0) &&
+         static_cast<int64_t>(wall_clock64() - t0) > a.wait_ticks;
+}
+
+// Waits for the blocks of phase `ph`; afterwards sh.run tells whether it was
+// answered.  Every thread of the block calls it.
+template <bool kFirst>
+__device__ __forceinline__ void wait_phase(const ChainArgs& a, Shared& sh, int ph) {
+  const int tid = static_cast<int>(fresh(threadIdx.x));
+  if (tid < 64) {
+    const uint32_t* flags = flags_of(a);
+    const uint32_t tag = sh.launch;
     const int end = a.first[ph + 1];
-    int at = a.first[ph] + static_cast<int>(threadIdx.x);
+    int at = a.first[ph] + tid;
     const uint64_t t0 = wall_clock64();
     int polls = 0;
     while (__any(at < end)) {  // the flags below `at` are set
-      uint32_t flag[4];  // of 256 blocks, in one round trip
+      uint32_t off = 0u;       // of 256 blocks, in one round trip
 #pragma unroll
       for (int i = 0; i < 4; ++i)
-        flag[i] = at + 64 * i < end ? __hip_atomic_load(flags + at + 64 * i, __ATOMIC_RELAXED,
-                                                        __HIP_MEMORY_SCOPE_AGENT)
-                                    : 1u;
-      if (__all((flag[0] & flag[1] & flag[2] & flag[3]) != 0u)) {
+        off |= at + 64 * i < end ? ld_dev(flags + at + 64 * i) ^ tag : 0u;
+      if (__all(off == 0u)) {
         at += 256;
         continue;
       }
-      if ((++polls & 63) == 0 && timed_out(a, t0)) break;
+      if (too_long(a, t0, ++polls)) break;
     }
+    const bool answered = !__any(at < end);
+    if (tid == 0) sh.run = answered ? kDone : kPhaseMissing;
+  } else if (kFirst && ph > kMerge) {  // (o_proj may not have that long to wait)
+    arrive(a, sh);
   }
   __syncthreads();
 }
 
 // One wave of the block, after the block's stores to device memory: they are
-// complete before the flag shows the block.
-__device__ __forceinline__ void set_flag(const ChainArgs& a) {
+// complete before the flag shows the item.
+__device__ __forceinline__ void set_flag(const ChainArgs& a, const Shared& sh, int item) {
   asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
-  const int lane = threadIdx.x & 63;
-  if (lane < kCopies)
-    __hip_atomic_store(a.sync + lane * kMaxBlocks + blockIdx.x, 1u, __ATOMIC_RELAXED,
-                       __HIP_MEMORY_SCOPE_AGENT);
+  const int lane = static_cast<int>(fresh(threadIdx.x)) & 63;
+  if (lane < kCopies) st_dev(a.sync + kFlagWord + lane * kMaxBlocks + item, sh.launch);
 }
 
-// The last phase's blocks, after their wait: by then every wait of the
-// earlier phases has ended, and when all of these blocks are past theirs the
-// last of them puts the flags back to zero.  Wave 0's ticket is drawn right
-// after the wait and looked at when the block's work is done.
-__device__ __forceinline__ uint32_t past_wait(const ChainArgs& a) {
-  return threadIdx.x == 0 ? __hip_atomic_fetch_add(a.sync + kDoneWord, 1u, __ATOMIC_RELAXED,
-                                                   __HIP_MEMORY_SCOPE_AGENT)
-                          : 0u;
-}
-__device__ __forceinline__ void reset_flags(const ChainArgs& a, uint32_t ticket) {  // wave 0
-  const int end = a.first[a.last_phase];
-  if (__shfl(ticket, 0, 64) != static_cast<uint32_t>(a.first[a.last_phase + 1] - end - 1)) return;
-  for (int i = threadIdx.x; i < end; i += 64)
+// What a block runs next after a wait that was not answered (or after such a
+// missing item): the other half of its head (`partner`), or an item without a
+// flag in the first incomplete phase before its own -- all its inputs are there
+// -- and otherwise its own again.  The blocks look from different places, so
+// that they help with different items.  Called by every thread of the block.
+__device__ __forceinline__ int next_item(const ChainArgs& a, Shared& sh, int own, bool partner) {
+  __syncthreads();  // the run before this is over in every wave
+  if (partner) return a.first[kQkv] + ((own - a.first[kQkv]) ^ 1);
+  const int lane = static_cast<int>(fresh(threadIdx.x));
+  if (lane < 64) {
+    const uint32_t* flags = flags_of(a);
+    int next = own;
 #pragma unroll
-    for (int c = 0; c < kCopies; ++c)
-      __hip_atomic_store(a.sync + c * kMaxBlocks + i, 0u, __ATOMIC_RELAXED,
-                         __HIP_MEMORY_SCOPE_AGENT);
-  if (threadIdx.x == 0)
-    __hip_atomic_store(a.sync + kDoneWord, 0u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+    for (int ph = 0; ph < kPhases - 1; ++ph) {
+      if (own < a.first[ph + 1]) break;  // not before its own
+      const int n = a.first[ph + 1] - a.first[ph];
+      for (int i = 0; i < n && next == own; i += 64) {
+        const int item = a.first[ph] + (i + lane + own) % n;
+        const uint64_t missing = __ballot(i + lane < n && ld_dev(flags + item) != sh.launch);
+        if (missing) next = __shfl(item, __ffsll(static_cast<unsigned long long>(missing)) - 1, 64);
+      }
+    }
+    if (lane == 0) sh.item = next;
+  }
+  __syncthreads();
+  return __builtin_amdgcn_readfirstlane(sh.item);
 }
 
 // rms of this lane's MFMA row (row lane % 16 of the block's rows) from the
@@ -223,14 +322,6 @@ __device__ __forceinline__ float row_rms(const ChainArgs& a, const float* ss, in
   s += q3::dpp_f32<q3::kDppXor2>(s);  // lane ^ 2
   const float rms = 1.f / sqrtf(s / static_cast<float>(a.K) + a.eps);
   return __shfl(rms, 4 * (lane & 15), 64);
-}
-
-// x, unknown to the compiler: what is derived from it is computed where it is
-// used (hoisted out of the pass loops, the offsets of all k-steps would need
-// more registers than there are).
-__device__ __forceinline__ uint32_t fresh(uint32_t x) {
-  asm volatile("" : "+v"(x));
-  return x;
 }
 
 // 2, unknown to the compiler: the dry pass and the real one share their code.
@@ -260,13 +351,14 @@ __device__ __forceinline__ q3::u32x4 normed(q3::u32x4 h, q3::u32x4 w, float rms)
 // One 16-column tile of o_proj, gate_up or down.  Each wave holds its share of
 // the tile's weights before it waits: an eighth of K of the one weight tile
 // (o_proj, down), or a quarter of K of the gate or of the up tile (gate_up).
-template <int kPh>
-__device__ __forceinline__ void linear_phase(const ChainArgs& a, int tile, q3::f32x4 (*red)[64],
-                                             uint16_t* nw_s) {
+template <int kPh, bool kFirst>
+__device__ __forceinline__ int linear_phase(const ChainArgs& a, Shared& sh, int tile,
+                                            uint32_t launch, q3::f32x4 (*red)[64],
+                                            uint16_t* nw_s) {
   constexpr bool kNorm = kPh == kGateUp;
   constexpr int kSteps = kNorm ? kMaxHidden / 4 / kKStep : kMaxSteps;
   constexpr int kParts = kNorm ? kWaves / 2 : kWaves;  // waves sharing one weight tile's K
-  const int tid = threadIdx.x, lane = tid & 63;
+  const int tid = static_cast<int>(fresh(threadIdx.x)), lane = tid & 63;
   const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
   const int r16 = lane & 15, kg = 8 * (lane >> 4);
   const int lrow = lane >> 2, lkg = 8 * (lane & 3);
@@ -288,12 +380,8 @@ __device__ __forceinline__ void linear_phase(const ChainArgs& a, int tile, q3::f
   };
   // gate_up and down ask for theirs after the dry pass: 26 MB asked for at
   // once would hold up the merge's loads and o_proj's
-  if constexpr (kPh == kO)
-    load_weights();
-  else
-#pragma unroll
-    for (int u = 0; u < kSteps; ++u) b[u] = q3::u32x4{0u, 0u, 0u, 0u};
   uint32_t res[4] = {0u, 0u, 0u, 0u};
+  bool done = false;  // o_proj: by another block already
   if constexpr (kPh == kO) {  // the residual comes from the launch before this one
     if (wave == 0) {
 #pragma unroll
@@ -302,6 +390,21 @@ __device__ __forceinline__ void linear_phase(const ChainArgs& a, int tile, q3::f
         if (row < a.M) res[i] = a.h_in[static_cast<int64_t>(row) * a.K + n0 + r16];
       }
     }
+    load_weights();
+    if constexpr (kFirst) share_launch(sh, launch);
+    uint32_t flag = 0u;
+    if (wave == 0) {  // the residual is here; after that, whether it still was h_in
+#pragma unroll
+      for (int i = 0; i < 4; ++i) asm volatile("" : "+v"(res[i])::"memory");
+      const uint32_t* flags = a.sync + kFlagWord + a.first[kO] + tile;  // every copy
+      flag = ld_dev(flags + (lane % kCopies) * kMaxBlocks);
+    }
+    __syncthreads();  // sh.launch
+    done = __any(flag == sh.launch);
+  } else {
+#pragma unroll
+    for (int u = 0; u < kSteps; ++u) b[u] = q3::u32x4{0u, 0u, 0u, 0u};
+    if constexpr (kFirst) share_launch(sh, launch);  // (the dry pass has a barrier)
   }
   if constexpr (kNorm) {
     for (int i = tid; i < a.K / 8; i += kThreads)
@@ -319,7 +422,7 @@ __device__ __forceinline__ void linear_phase(const ChainArgs& a, int tile, q3::f
       // into the operand layout while there is nothing else to do
 #pragma unroll
       for (int u = 0; u < kSteps; ++u) b[u] = to_mfma(b[u], perm_addr);
-      wait_phase(a, kPh - 1);
+      wait_phase<kFirst>(a, sh, kPh - 1);
     }
     // (the dry pass asks for nothing: an empty descriptor)
     const Rows xr{x, static_cast<int>(((a.M - 1) * xs + K) * 2), pass ? steps : 0};
@@ -353,6 +456,7 @@ __device__ __forceinline__ void linear_phase(const ChainArgs& a, int tile, q3::f
     red[wave][lane] = acc;
     __syncthreads();
     if (wave == 0) {
+      const bool stores = pass && sh.run == kDone && !done;
       q3::f32x4 v = red[0][lane], up = {0.f, 0.f, 0.f, 0.f};
 #pragma unroll
       for (int w2 = 1; w2 < kParts; ++w2) v += red[w2][lane];
@@ -365,7 +469,7 @@ __device__ __forceinline__ void linear_phase(const ChainArgs& a, int tile, q3::f
 #pragma unroll
       for (int i = 0; i < 4; ++i) {
         const int row = 4 * (lane >> 4) + i;
-        const bool live = pass && row < a.M;
+        const bool live = stores && row < a.M;
         if constexpr (kNorm) {
           const float g = round_bf16(v[i]);
           const float u = round_bf16(up[i]);
@@ -386,42 +490,42 @@ __device__ __forceinline__ void linear_phase(const ChainArgs& a, int tile, q3::f
                                __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
         }
       }
-      if (!pass) continue;
-      if (kPh != a.last_phase)
-        set_flag(a);
-      else
-        reset_flags(a, past_wait(a));
+      if (stores && kPh != a.last_phase) set_flag(a, sh, a.first[kPh] + tile);
     }
   }
+  return sh.run;
 }
 
 // Adds up the 16 lanes of a token's head (lane j: 8 of its dims, squared and
 // summed) when this block has only quads hf and hf + 2 of them: each quad sum
 // goes to the head's other block, which has the other two.  Quads 0 + 1 and
 // 2 + 3 are added first, as row16_sum does, so the same bits in both blocks.
-// A word is the sum's bits plus one (a sum is never negative, 0 is "not
-// yet"); its one reader puts it back to zero.
-__device__ __forceinline__ float exchange_sum(const ChainArgs& a, uint32_t* words, int head, int hf,
-                                              int row, int j, float v) {
+// `late` is set where they do not come in time.
+__device__ __forceinline__ float exchange_sum(const ChainArgs& a, uint32_t tag, int rb, int head,
+                                              int hf, int row, int j, float v, bool& late) {
   v += q3::dpp_f32<q3::kDppXor1>(v);
   v += q3::dpp_f32<q3::kDppXor2>(v);
   const bool mine = ((j >> 2) & 1) == hf;
-  uint32_t* word = words + ((head * 2 + (mine ? hf : 1 - hf)) * kRows + row) * 2 + (j >> 3);
+  uint64_t* word = reinterpret_cast<uint64_t*>(a.sync + kSumWord) + rb * kSums +
+                   ((head * 2 + (mine ? hf : 1 - hf)) * kRows + row) * 2 + (j >> 3);
   const bool first = (j & 3) == 0;
   if (first && mine)
-    __hip_atomic_store(word, __float_as_uint(v) + 1u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+    __hip_atomic_store(word, static_cast<uint64_t>(tag) << 32 | __float_as_uint(v),
+                       __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
   const bool reads = first && !mine;
-  uint32_t got = 1u;
+  uint64_t got = static_cast<uint64_t>(tag) << 32;
   const uint64_t t0 = wall_clock64();
   for (int polls = 1;; ++polls) {
     if (reads) got = __hip_atomic_load(word, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-    if (__all(got != 0u)) break;
-    if ((polls & 63) != 0) continue;
-    if (timed_out(a, t0)) break;
+    if (__all(static_cast<uint32_t>(got >> 32) == tag)) break;
+    if (too_long(a, t0, polls)) {
+      late = true;
+      break;
+    }
   }
-  if (reads) __hip_atomic_store(word, 0u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
   constexpr int kQuadFirst = 0x00;  // quad_perm [0,0,0,0]
-  const float theirs = q3::dpp_f32<kQuadFirst>(__uint_as_float(got - 1u));
+  const float theirs =
+      q3::dpp_f32<kQuadFirst>(__uint_as_float(static_cast<uint32_t>(got)));
   v = mine ? v : theirs;
   v += q3::dpp_f32<q3::kDppHalfMirror>(v);
   v += q3::dpp_f32<q3::kDppMirror>(v);
@@ -435,9 +539,10 @@ __device__ __forceinline__ float exchange_sum(const ChainArgs& a, uint32_t* word
 // 256 KB do not fit the registers, and what was left to read after the wait
 // took 2.5 us at the 46 GB/s of one CU.)  kAlone: a launch of its own, rows
 // 16 rb .. of h.
-template <bool kAlone>
-__device__ __forceinline__ void qkv_phase(const ChainArgs& a, int blk, int rb,
-                                          q3::f32x4 (*red)[64], uint16_t* a_s, uint16_t* nw_s) {
+template <bool kAlone, bool kFirst>
+__device__ __forceinline__ int qkv_phase(const ChainArgs& a, Shared& sh, int blk, int rb,
+                                         uint32_t launch, q3::f32x4 (*red)[64], uint16_t* a_s,
+                                         uint16_t* nw_s) {
   __shared__ float rms_s[kRows];
   __shared__ __attribute__((aligned(16))) uint16_t y_s[kRows][kHeadD / 2];
   __shared__ int64_t pos_s[kRows], phys_s[kRows];
@@ -446,7 +551,7 @@ __device__ __forceinline__ void qkv_phase(const ChainArgs& a, int blk, int rb,
   const int M = kAlone ? min(kRows, a.M - kRows * rb) : a.M;
   const uint16_t* h = a.h_out + static_cast<int64_t>(kRows * rb) * a.h_s;
   const float* ss = a.ss_out + kRows * rb * (a.K / 16);
-  const int tid = threadIdx.x, lane = tid & 63;
+  const int tid = static_cast<int>(fresh(threadIdx.x)), lane = tid & 63;
   const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
   const int ct = wave & 3, kh = wave >> 2;
   const int r16 = lane & 15;
@@ -471,15 +576,15 @@ __device__ __forceinline__ void qkv_phase(const ChainArgs& a, int blk, int rb,
   }
   for (int i = tid; i < a.K / 8; i += kThreads)
     *reinterpret_cast<q3::u32x4*>(nw_s + 8 * i) = q3::ld16(a.in_w + 8 * i);
-  uint32_t ticket = 0;
+  if constexpr (kFirst) share_launch(sh, launch);  // (there are barriers before its use)
+  if (kAlone && tid == 0) sh.run = kDone;
   for (int pass = kAlone ? 1 : 0; pass < two(); ++pass) {
     if (!kAlone && pass) {
 #pragma unroll
       for (int u = 0; u < kQkvSteps; ++u) b[u] = wr.weight(woff, u);
 #pragma unroll
       for (int u = 0; u < kQkvSteps; ++u) b[u] = to_mfma(b[u], perm_addr);
-      wait_phase(a, kDown);
-      ticket = past_wait(a);
+      wait_phase<kFirst>(a, sh, kDown);
     }
     // The rows of h: chunk c = tid + i * threads of the M x K / 8 16-byte
     // chunks, at most four per thread.  Rows past M stay unwritten: a row of the
@@ -532,64 +637,115 @@ __device__ __forceinline__ void qkv_phase(const ChainArgs& a, int blk, int rb,
   }
   // 16 lanes per token as for a whole head; the quads of the other block are
   // zero here.
-  const int r = tid >> 4, j = tid & 15;
-  if (r < M) {  // whole 16-lane groups
-    const bool mine = ((j >> 2) & 1) == hf;
-    const int at = 8 * (j & 3) + (j >> 3) * 32;
-    const q3::u32x4 xw = mine ? *reinterpret_cast<const q3::u32x4*>(&y_s[r][at])
-                              : q3::u32x4{0u, 0u, 0u, 0u};
-    if (mine || head < a.hd.Hq + a.hd.Hkv)
-      finish_head(a.hd, head, kRows * rb + r, j, xw, pos_s[r], phys_s[r], off_s[r], mine,
-                  [&](float v) {
-                    return exchange_sum(a, a.sync + kSumWord + rb * kSumWords, head, hf, r, j, v);
-                  });
+  if (sh.run == kDone) {  // uniform
+    const int r = tid >> 4, j = tid & 15;
+    if (r < M) {  // whole 16-lane groups
+      const bool mine = ((j >> 2) & 1) == hf;
+      const int at = 8 * (j & 3) + (j >> 3) * 32;
+      const q3::u32x4 xw = mine ? *reinterpret_cast<const q3::u32x4*>(&y_s[r][at])
+                                : q3::u32x4{0u, 0u, 0u, 0u};
+      bool late = false;
+      if (mine || head < a.hd.Hq + a.hd.Hkv)
+        finish_head(a.hd, head, kRows * rb + r, j, xw, pos_s[r], phys_s[r], off_s[r],
+                    [&]() { return mine && !late; }, [&](float v) {
+                      return exchange_sum(a, sh.launch, rb, head, hf, r, j, v, late);
+                    });
+      if (late && (tid & 63) == 0) sh.run = kPartnerMissing;
+    }
+    if constexpr (kAlone && kFirst) arrive(a, sh);  // (this wave has no rows)
+    __syncthreads();  // sh.run
   }
-  if (!kAlone && wave == 0) reset_flags(a, ticket);
+  return sh.run;
 }
 
-// Two blocks per CU (the largest grid the host launches is what fits).
+template <bool kFirst>
+__device__ __forceinline__ int merge_phase(const ChainArgs& a, Shared& sh, int item,
+                                           uint32_t launch) {
+  const int tid = static_cast<int>(fresh(threadIdx.x)), lane = tid & 63;
+  const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+  const int hq_n = a.KO / kHeadD;
+  const int task = item * kWaves + wave;  // one wave per (row, query head)
+  const int b = task / hq_n, hq = task - b * hq_n;
+  uint32_t y;
+  if (b < a.M && merge_partials<32>(a.parts, b, hq, lane, y))
+    st_dev(reinterpret_cast<uint32_t*>(a.o + b * a.o_s + hq * kHeadD + 2 * lane), y);
+  if constexpr (kFirst) share_launch(sh, launch);
+  asm volatile("s_waitcnt vmcnt(0)" ::: "memory");  // this wave's stores are complete
+  __syncthreads();
+  if (wave == 0) set_flag(a, sh, item);
+  return kDone;
+}
+
+// kFirst: a block's first run, of its own item.
+template <bool kFirst>
+__device__ __forceinline__ int run_item(const ChainArgs& a, Shared& sh, int item,
+                                        uint32_t launch, q3::f32x4 (*red)[64], uint16_t* a_s,
+                                        uint16_t* nw_s) {
+  if (item < a.first[kO]) return merge_phase<kFirst>(a, sh, item, launch);
+  if (item < a.first[kGateUp])
+    return linear_phase<kO, kFirst>(a, sh, item - a.first[kO], launch, red, nw_s);
+  if (item < a.first[kDown])
+    return linear_phase<kGateUp, kFirst>(a, sh, item - a.first[kGateUp], launch, red, nw_s);
+  if (item < a.first[kQkv])
+    return linear_phase<kDown, kFirst>(a, sh, item - a.first[kDown], launch, red, nw_s);
+  return qkv_phase<false, kFirst>(a, sh, item - a.first[kQkv], 0, launch, red, a_s, nw_s);
+}
+
+// The kernel's argument (the first, at offset 0), read anew: the rare path that
+// runs another block's work keeps nothing in registers across the usual one.
+__device__ __forceinline__ const ChainArgs& item_args() {
+  typedef const __attribute__((address_space(4))) ChainArgs kernarg;
+  kernarg* p = (kernarg*)__builtin_amdgcn_kernarg_segment_ptr();
+  asm volatile("" : "+s"(p));
+  return *(const ChainArgs*)p;
+}
+
+// Two blocks per CU.
 __global__ __launch_bounds__(kThreads) __attribute__((amdgpu_waves_per_eu(4, 4)))
-void decode_chain_kernel(ChainArgs a) {
+void decode_chain_kernel(ChainArgs args) {
   __shared__ q3::f32x4 red[kWaves][64];
   __shared__ __attribute__((aligned(16))) uint16_t a_s[kRows * (kMaxHidden + 8)];
   __shared__ __attribute__((aligned(16))) uint16_t nw_s[kMaxHidden];
-  const int blk = blockIdx.x;
-  if (blk < a.first[kO]) {  // merge: one wave per (row, query head)
-    const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6), lane = threadIdx.x & 63;
-    const int hq_n = a.KO / kHeadD;
-    const int task = blk * kWaves + wave;
-    const int b = task / hq_n, hq = task - b * hq_n;
-    uint32_t y;
-    if (b < a.M && merge_partials<32>(a.parts, b, hq, lane, y))
-      __hip_atomic_store(reinterpret_cast<uint32_t*>(a.o + b * a.o_s + hq * kHeadD + 2 * lane), y,
-                         __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-    asm volatile("s_waitcnt vmcnt(0)" ::: "memory");  // this wave's stores are complete
-    __syncthreads();
-    if (wave == 0) set_flag(a);
-  } else if (blk < a.first[kGateUp]) {
-    linear_phase<kO>(a, blk - a.first[kO], red, nw_s);
-  } else if (blk < a.first[kDown]) {
-    linear_phase<kGateUp>(a, blk - a.first[kGateUp], red, nw_s);
-  } else if (blk < a.first[kQkv]) {
-    linear_phase<kDown>(a, blk - a.first[kDown], red, nw_s);
-  } else {
-    qkv_phase<false>(a, blk - a.first[kQkv], 0, red, a_s, nw_s);
+  __shared__ Shared sh;
+  const int own = blockIdx.x;
+  const uint32_t launch = read_launch(args.sync);
+  int item = own, run = run_item<true>(args, sh, item, launch, red, a_s, nw_s);
+  while (__builtin_expect(run != kDone || item != own, 0)) {
+    const ChainArgs& a = item_args();
+    // the other half of the head, or what the phases before this one lack
+    item = next_item(a, sh, own, run == kPartnerMissing && item == own);
+    run = run_item<false>(a, sh, item, 0u, red, a_s, nw_s);
   }
+  arrive(args, sh);  // (where it has not waited)
 }
 
 // The qkv phase as a launch of its own, for up to 64 rows: block (half head,
 // 16-row block), the row blocks of a half head on one XCD (blocks are dealt to
 // the eight in turn) where their weights meet in its L2.
 __global__ __launch_bounds__(kThreads) __attribute__((amdgpu_waves_per_eu(4, 4)))
-void decode_qkv_half_kernel(ChainArgs a) {
+void decode_qkv_half_kernel(ChainArgs args) {
   __shared__ q3::f32x4 red[kWaves][64];
   __shared__ __attribute__((aligned(16))) uint16_t a_s[kRows * (kMaxHidden + 8)];
   __shared__ __attribute__((aligned(16))) uint16_t nw_s[kMaxHidden];
-  const int rbc = (a.M + kRows - 1) / kRows;
-  const int halves = 2 * (a.hd.Hq + 2 * a.hd.Hkv);
+  __shared__ Shared sh;
+  const int rbc = (args.M + kRows - 1) / kRows;
+  const int halves = 2 * (args.hd.Hq + 2 * args.hd.Hkv);
   const int slot = static_cast<int>(blockIdx.x >> 3);
   const int half = (slot / rbc) * 8 + static_cast<int>(blockIdx.x & 7);
-  if (half < halves) qkv_phase<true>(a, half, slot % rbc, red, a_s, nw_s);
+  const uint32_t launch = read_launch(args.sync);
+  if (half < halves) {
+    int item = half;
+    int run = qkv_phase<true, true>(args, sh, item, slot % rbc, launch, red, a_s, nw_s);
+    while (__builtin_expect(run != kDone || item != half, 0)) {
+      const ChainArgs& a = item_args();
+      item = run == kPartnerMissing && item == half ? half ^ 1 : half;
+      __syncthreads();  // the run before this is over in every wave
+      run = qkv_phase<true, false>(a, sh, item, slot % rbc, 0u, red, a_s, nw_s);
+    }
+  } else {
+    share_launch(sh, launch);
+  }
+  arrive(args, sh);
 }
 
 // Blocks resident at once on the current device (0: unknown).
@@ -758,6 +914,7 @@ extern "C" int qwen3_decode_chain_bf16(const qwen3_decode_chain_args* c, void* s
   a.down_w = static_cast<const uint16_t*>(c->down_weight);
   a.down_ws = c->down_row_stride;
   a.sync = c->sync;
+  a.wait_ticks = c->wait_ticks ? c->wait_ticks : kWaitTicks;
   a.h_s = c->hidden;
   if (qkv)
     if (const int rc = fill_qkv(a, c, who)) return rc;
@@ -806,6 +963,7 @@ extern "C" int qwen3_decode_qkv_half_bf16(const qwen3_decode_chain_args* c, int6
   a.h_s = h_row_stride;
   a.ss_out = c->ss_out;
   a.sync = c->sync;
+  a.wait_ticks = c->wait_ticks ? c->wait_ticks : kWaitTicks;
   if (const int rc = fill_qkv(a, c, who)) return rc;
   if (!q3::aligned16(c->h_out) || !q3::aligned16(c->ss_out) || h_row_stride % 8 != 0)
     return q3::fail(QWEN3_EALIGN, "%s: tensors need 16-byte aligned rows", who);

@@ -12,24 +12,24 @@ constexpr int kHeadD = 128;
 
 struct HeadArgs {
   int M, Hq, Hkv;
-  const uint16_t* q_w;  // QK-norm weights (128)
-  const uint16_t* k_w;
+  q3::GlobalPtr<const uint16_t> q_w;  // QK-norm weights (128)
+  q3::GlobalPtr<const uint16_t> k_w;
   float head_eps;
-  const float* cos_t;
-  const float* sin_t;
+  q3::GlobalPtr<const float> cos_t;
+  q3::GlobalPtr<const float> sin_t;
   int64_t tab_stride, tab_rows;
-  const int64_t* positions;  // nullable: RoPE at seq_lens[row]
-  uint16_t* q_out;
+  q3::GlobalPtr<const int64_t> positions;  // nullable: RoPE at seq_lens[row]
+  q3::GlobalPtr<uint16_t> q_out;
   int64_t qo_s0, qo_s1;
-  uint16_t* k_cache;
-  uint16_t* v_cache;
+  q3::GlobalPtr<uint16_t> k_cache;
+  q3::GlobalPtr<uint16_t> v_cache;
   int64_t kc[4], vc[4];
   int64_t num_blocks;
   int layer;
-  const int32_t* seq_lens;
-  const int32_t* block_table;
+  q3::GlobalPtr<const int32_t> seq_lens;
+  q3::GlobalPtr<const int32_t> block_table;
   int64_t bt_stride, max_rows, max_pages;
-  const int32_t* row_ids;  // nullable: identity
+  q3::GlobalPtr<const int32_t> row_ids;  // nullable: identity
   int bs;
 };
 
@@ -58,17 +58,17 @@ __device__ __forceinline__ void locate_token(const HeadArgs& a, int t, int64_t& 
 
 // Head `head` of token t (< M): lane j of a 16-lane group holds dims 8j ..
 // 8j + 7 of the projection's output (xw).  Called by whole groups; a lane
-// without `store` writes nothing.  row_sum: the sum over the group's lanes
-// (q3::row16_sum, or its value by other means).
-template <typename Sum>
+// whose stores() is false writes nothing (asked for after row_sum).  row_sum: the
+// sum over the group's lanes (q3::row16_sum, or its value by other means).
+template <typename Stores, typename Sum>
 __device__ __forceinline__ void finish_head(const HeadArgs& a, int head, int t, int j,
                                             q3::u32x4 xw, int64_t pos, int64_t phys, int off,
-                                            bool store, Sum&& row_sum) {
+                                            Stores&& stores, Sum&& row_sum) {
   const bool ok_pos = pos >= 0 && pos < a.tab_rows;
-  const bool write_pool = store && ok_pos && phys >= 0 && phys < a.num_blocks;
+  const bool write_pool = ok_pos && phys >= 0 && phys < a.num_blocks;
   const int kv_base = a.Hq + a.Hkv;
   if (head >= kv_base) {  // v: a bit-exact copy into the pool
-    if (write_pool)
+    if (write_pool && stores())
       q3::st16(a.v_cache + phys * a.vc[0] + static_cast<int64_t>(a.layer) * a.vc[1] +
                    static_cast<int64_t>(head - kv_base) * a.vc[2] + off * a.vc[3] + 8 * j,
                xw);
@@ -128,11 +128,11 @@ __device__ __forceinline__ void finish_head(const HeadArgs& a, int head, int t, 
       out[e] = q3::pack_bf16x2(o[0], o[1]);
     }
   }
+  if (!stores()) return;
   if (head < a.Hq) {
-    if (store)
-      q3::st16(a.q_out + static_cast<int64_t>(t) * a.qo_s0 +
-                   static_cast<int64_t>(head) * a.qo_s1 + 8 * j,
-               out);
+    q3::st16(a.q_out + static_cast<int64_t>(t) * a.qo_s0 +
+                 static_cast<int64_t>(head) * a.qo_s1 + 8 * j,
+             out);
   } else if (write_pool) {
     q3::st16(a.k_cache + phys * a.kc[0] + static_cast<int64_t>(a.layer) * a.kc[1] +
                  static_cast<int64_t>(head - a.Hq) * a.kc[2] + off * a.kc[3] + 8 * j,
@@ -141,7 +141,7 @@ __device__ __forceinline__ void finish_head(const HeadArgs& a, int head, int t, 
 }
 __device__ __forceinline__ void finish_head(const HeadArgs& a, int head, int t, int j,
                                             q3::u32x4 xw, int64_t pos, int64_t phys, int off) {
-  finish_head(a, head, t, j, xw, pos, phys, off, true,
+  finish_head(a, head, t, j, xw, pos, phys, off, []() { return true; },
               [](float ss) { return q3::row16_sum(ss); });
 }
 

@@ -26,10 +26,10 @@ inline StreamLayout stream_layout(int B, int64_t waves, int G) {
 }
 
 struct StreamPartials {
-  const float* po;      // [W][2][G][128] normalised partial outputs
-  const float* plse;    // [W][2][G] log2-sum-exp of each
-  const int32_t* pref;  // [B + 1] exclusive prefix of tiles per sequence
-  const int32_t* meta;  // [0] tiles per wave
+  q3::GlobalPtr<const float> po;      // [W][2][G][128] normalised partial outputs
+  q3::GlobalPtr<const float> plse;    // [W][2][G] log2-sum-exp of each
+  q3::GlobalPtr<const int32_t> pref;  // [B + 1] exclusive prefix of tiles per sequence
+  q3::GlobalPtr<const int32_t> meta;  // [0] tiles per wave
   int Hkv, G;
 };
 

@@ -249,8 +249,8 @@ def decode_chain_ok(batch: int, hidden: int, intermediate: int, num_heads: int,
 
 
 def decode_chain_sync(device) -> torch.Tensor:
-    """The hand-off counters of decode_chain, zeroed once (every launch leaves
-    them zero); launches that may overlap need their own."""
+    """The hand-off words of decode_chain, zeroed once and the launches' own from
+    then on; launches that may overlap need their own."""
     return torch.zeros(int(_lib.load().qwen3_decode_chain_sync_bytes()), dtype=torch.uint8,
                        device=device)
 
@@ -280,14 +280,17 @@ def decode_chain(o: torch.Tensor, h: torch.Tensor, h_mid: torch.Tensor, ss: torc
                  next_layer=None, head_eps: float = 0.0, cos_table: torch.Tensor | None = None,
                  sin_table: torch.Tensor | None = None, pool=None, next_idx: int = 0,
                  row_ids: torch.Tensor | None = None,
-                 positions: torch.Tensor | None = None) -> torch.Tensor | None:
+                 positions: torch.Tensor | None = None,
+                 wait_ticks: int = 0) -> torch.Tensor | None:
     """o_proj, gate_up and down of `layer` and, with next_layer, its qkv
     projection up to attention, in one launch for at most 16 rows: the
     results of decode_linear and decode_qkv_rope bit for bit.  o (M, Hq, 128)
     is the attention output, completed here from attn_workspace when
     paged_attention_decode_partials_hip left partial results there; the
     residual stream h and its sums of squares ss are updated in place through
-    h_mid and ss_mid.  Returns the next layer's q."""
+    h_mid and ss_mid.  wait_ticks (10 ns each; 0: 200 us; below: none): how long
+    a workgroup waits for others before it does their part itself.  Returns
+    the next layer's q."""
     M, hidden = h.shape
     mlp = layer.mlp
     wo, wg, wd = layer.self_attn.o_proj.weight, mlp.gate_up_proj.weight, mlp.down_proj.weight
@@ -311,7 +314,8 @@ def decode_chain(o: torch.Tensor, h: torch.Tensor, h_mid: torch.Tensor, ss: torc
         h_mid=h_mid.data_ptr(), h_out=h.data_ptr(), ss_mid=ss_mid.data_ptr(),
         ss_out=ss.data_ptr(), post_norm_weight=layer.post_attention_layernorm.weight.data_ptr(),
         gate_up_weight=wg.data_ptr(), gate_up_row_stride=wg.stride(0), act=act.data_ptr(),
-        down_weight=wd.data_ptr(), down_row_stride=wd.stride(0), sync=sync.data_ptr())
+        down_weight=wd.data_ptr(), down_row_stride=wd.stride(0), sync=sync.data_ptr(),
+        wait_ticks=wait_ticks)
     if attn_workspace is not None:
         a.attn_workspace = attn_workspace.data_ptr()
         a.attn_workspace_bytes = attn_workspace.numel()
@@ -339,13 +343,13 @@ def decode_qkv_rope(h: torch.Tensor, ss_in: torch.Tensor, norm_weight: torch.Ten
                     q_norm_weight: torch.Tensor, k_norm_weight: torch.Tensor, head_eps: float,
                     cos_table: torch.Tensor, sin_table: torch.Tensor, pool, layer_idx: int,
                     row_ids: torch.Tensor | None, positions: torch.Tensor | None = None,
-                    q_out: torch.Tensor | None = None,
-                    sync: torch.Tensor | None = None) -> torch.Tensor:
+                    q_out: torch.Tensor | None = None, sync: torch.Tensor | None = None,
+                    wait_ticks: int = 0) -> torch.Tensor:
     """Input RMSNorm + qkv projection + QK-norm + RoPE + K/V pool write of a
     decode step for at most 64 tokens in one launch; returns q (M, Hq, 128)
     for the attention kernel (k and v go into `pool` at seq_lens[row]).
     sync (decode_chain_sync): two workgroups may share a head, with the same
-    results."""
+    results; wait_ticks as decode_chain."""
     h = _rows2d(h)
     M, K = h.shape
     D = 128
@@ -364,12 +368,13 @@ def decode_qkv_rope(h: torch.Tensor, ss_in: torch.Tensor, norm_weight: torch.Ten
     if q_out is None:
         q_out = torch.empty(M, num_heads, D, dtype=h.dtype, device=h.device)
     lib = _lib.load()
-    # the halves wait for one another, so all of them must be resident at once
+    # the halves wait for one another: where all of them are resident at once
     if sync is not None and lib.qwen3_decode_qkv_half_supported(M, K, num_heads, num_kv_heads) \
             and ss_in.shape[1] == K // 16:
         a = _lib.DecodeChainArgs(M=M, hidden=K, num_heads=num_heads, num_kv_heads=num_kv_heads,
                                  eps=eps, head_eps=head_eps, h_out=h.data_ptr(),
-                                 ss_out=ss_in.data_ptr(), sync=sync.data_ptr())
+                                 ss_out=ss_in.data_ptr(), sync=sync.data_ptr(),
+                                 wait_ticks=wait_ticks)
         _set_qkv(a, norm_weight, qkv_weight, q_norm_weight, k_norm_weight, cos_table, sin_table,
                  positions, q_out, pool, int(layer_idx), row_ids)
         _lib.check(lib.qwen3_decode_qkv_half_bf16(ctypes.byref(a), h.stride(0),

@@ -26,6 +26,14 @@ def _layer(g, dev, hidden, inter, hq, hkv):
         input_layernorm=norm(hidden), post_attention_layernorm=norm(hidden))
 
 
+def _launches(sync):
+    """The launches counted in the hand-off words (their first word; the
+    blocks' arrivals, on the 33 lines after it, are put back to zero)."""
+    words = sync.view(torch.int32)
+    assert not words[1:34 * 32].any()
+    return words[0].item()
+
+
 @pytest.mark.parametrize("hidden, inter, hq, hkv", [
     (1024, 3072, 16, 8),   # Qwen3-0.6B: every register of the weight slabs used
     (128, 2048, 16, 8),    # one k-step per wave of gate_up
@@ -37,8 +45,8 @@ def _layer(g, dev, hidden, inter, hq, hkv):
 def test_chain_same_bits_as_separate_kernels(gpu, hidden, inter, hq, hkv, M, merge):
     """Lengths from 1 token to thousands (heads written whole by one wave and
     split over many), a row outside the resident table, with and without the
-    merge and the next layer; the counters are left at zero; three launches
-    in a row."""
+    merge and the next layer; three launches in a row, each of which advances
+    the launch number."""
     from qwen3_engine_from_scratch_amd.PagedKVcache import (KVCachePool, PagedKVCache,
                                                             reserve_pages_bulk, set_seq_lens_bulk)
     from qwen3_engine_from_scratch_amd.kernels.model_ops import (
@@ -48,7 +56,8 @@ def test_chain_same_bits_as_separate_kernels(gpu, hidden, inter, hq, hkv, M, mer
         paged_decode_workspace_bytes)
     from qwen3_engine_from_scratch_amd.kernels.pre_attention import rope_tables
 
-    assert decode_chain_ok(M, hidden, inter, hq, hkv)
+    if not decode_chain_ok(M, hidden, inter, hq, hkv):
+        pytest.skip("the grid does not fit this device at once")
     assert not decode_chain_ok(17, hidden, inter, hq, hkv)
     g = torch.Generator(device=gpu).manual_seed(M + hidden)
     a, b = (_layer(g, gpu, hidden, inter, hq, hkv) for _ in range(2))
@@ -115,7 +124,7 @@ def test_chain_same_bits_as_separate_kernels(gpu, hidden, inter, hq, hkv, M, mer
         for name, x, y in zip("h ss mid ss_mid k v q".split(),
                               [h, ss, mid, ss_mid, pool.k_buffer, pool.v_buffer, q], want[i]):
             assert (x is None and y is None) or torch.equal(x, y), f"launch {i}: {name}"
-        assert not sync.any()
+        assert _launches(sync) == i + 1
 
 
 @pytest.mark.parametrize("hidden, hq, hkv", [(1024, 16, 8), (64, 3, 1), (640, 18, 9)])
@@ -123,7 +132,7 @@ def test_chain_same_bits_as_separate_kernels(gpu, hidden, inter, hq, hkv, M, mer
 def test_qkv_half_heads_same_bits(gpu, hidden, hq, hkv, M):
     """decode_qkv_rope on two workgroups per head against one: rows past a
     16-row block's end, rows outside the resident table, a row stride of the
-    residual stream that is not its width; the exchanged words are left zero."""
+    residual stream that is not its width; every launch is counted."""
     from qwen3_engine_from_scratch_amd.PagedKVcache import (KVCachePool, PagedKVCache,
                                                             reserve_pages_bulk, set_seq_lens_bulk)
     from qwen3_engine_from_scratch_amd.kernels.model_ops import (decode_chain_sync,
@@ -163,4 +172,184 @@ def test_qkv_half_heads_same_bits(gpu, hidden, hq, hkv, M):
     for x in (h, wide[:, :hidden], h):
         for a, b in zip(run(x, sync=sync), want):
             assert torch.equal(a, b)
-    assert not sync.any()
+    assert _launches(sync) == 3
+
+
+class _Chain:
+    """A layer's dense work after an attention over M sequences, with the next
+    layer's qkv, on a pool, a residual stream and hand-off words of its own."""
+
+    def __init__(self, gpu, M, hidden=1024, inter=3072, hq=16, hkv=8, seed=0):
+        from qwen3_engine_from_scratch_amd.PagedKVcache import (KVCachePool, PagedKVCache,
+                                                                reserve_pages_bulk,
+                                                                set_seq_lens_bulk)
+        from qwen3_engine_from_scratch_amd.kernels.model_ops import (decode_chain_ok,
+                                                                     decode_chain_sync, embed_ss)
+        from qwen3_engine_from_scratch_amd.kernels.paged_attention import (
+            paged_decode_workspace_bytes)
+        from qwen3_engine_from_scratch_amd.kernels.pre_attention import rope_tables
+
+        if not decode_chain_ok(M, hidden, inter, hq, hkv):
+            pytest.skip("the grid does not fit this device at once")
+        g = torch.Generator(device=gpu).manual_seed(seed)
+        self.M, self.hq, self.hkv = M, hq, hkv
+        self.a, self.b = (_layer(g, gpu, hidden, inter, hq, hkv) for _ in range(2))
+        lens = [(331 * i + 900) % 1500 + 1 for i in range(M)]
+        self.pool = pool = KVCachePool(sum(n // 16 + 1 for n in lens) + 2, 2, 16, hkv, 128,
+                                       device=gpu, dtype=torch.bfloat16, max_seq_len=2048,
+                                       max_requests=M + 1)
+        caches = [PagedKVCache(pool) for _ in range(M)]
+        reserve_pages_bulk(caches, [n + 1 for n in lens])
+        for c, n in zip(caches, lens):
+            c.seq_len = n
+        set_seq_lens_bulk(caches)
+        self.rows = torch.tensor([c.row_id for c in caches], dtype=torch.int32, device=gpu)
+        pool.k_buffer.normal_(generator=g)
+        pool.v_buffer.normal_(generator=g)
+        self.tables = rope_tables(128, 1e6, 2048, device=gpu)
+        self.h0, self.ss0 = embed_ss(
+            torch.arange(M, device=gpu),
+            torch.randn(64, hidden, generator=g, device=gpu).bfloat16())
+        self.q0 = torch.randn(M, hq, 128, generator=g, device=gpu).bfloat16()
+        self.ws = torch.zeros(
+            paged_decode_workspace_bytes(M, hq, hkv, 128, pool.block_table_2d.shape[1], 16),
+            dtype=torch.uint8, device=gpu)
+        self.sync = decode_chain_sync(gpu)
+
+    def run(self, merge=True, nxt=True, **kw):
+        """One pass from the same inputs, with no synchronisation."""
+        from qwen3_engine_from_scratch_amd.kernels.model_ops import decode_chain
+        from qwen3_engine_from_scratch_amd.kernels.paged_attention import (
+            paged_attention_decode_hip, paged_attention_decode_partials_hip)
+
+        kv = (self.q0, self.pool.k_buffer[:, 0], self.pool.v_buffer[:, 0],
+              self.pool.block_table_2d, self.pool.seq_lens, self.rows, 16)
+        o = (paged_attention_decode_partials_hip(*kv, self.ws) if merge
+             else paged_attention_decode_hip(*kv, workspace=self.ws))
+        h, ss = self.h0.clone(), self.ss0.clone()
+        mid, ss_mid = torch.empty_like(h), torch.empty_like(ss)
+        q = decode_chain(o, h, mid, ss, ss_mid, self.a, 1e-6, self.hq, self.hkv, self.sync,
+                         attn_workspace=self.ws if merge else None,
+                         next_layer=self.b if nxt else None, head_eps=1e-6,
+                         cos_table=self.tables[0], sin_table=self.tables[1], pool=self.pool,
+                         next_idx=1, row_ids=self.rows, **kw)
+        out = [o, h, ss, mid, ss_mid, self.pool.k_buffer[:, 1].clone(),
+               self.pool.v_buffer[:, 1].clone()]
+        return out + ([q] if nxt else [])
+
+
+def _same(x, y):
+    """Bit for bit (NaNs too)."""
+    return all(torch.equal(a.view(torch.int16), b.view(torch.int16)) for a, b in zip(x, y))
+
+
+@pytest.mark.parametrize("M", [1, 7, 16])
+@pytest.mark.parametrize("merge, nxt", [(True, True), (False, True), (True, False)])
+@pytest.mark.parametrize("ticks", [-1, 1, 500])
+def test_chain_waits_that_are_not_answered(gpu, M, merge, nxt, ticks):
+    """Every wait gives up at its first unanswered poll, or soon after it: the
+    blocks run one another's work, several of them the same, with the same
+    bits, in place, launch after launch."""
+    c = _Chain(gpu, M, seed=M)
+    announce(f"decode chain unanswered waits M={M} merge={merge} next={nxt} ticks={ticks}")
+    want = c.run(merge, nxt)
+    for i in range(4):
+        assert _same(c.run(merge, nxt, wait_ticks=ticks), want), f"launch {i}"
+    assert _same(c.run(merge, nxt), want)
+    assert _launches(c.sync) == 6
+
+
+@pytest.mark.parametrize("hidden, hq, hkv", [(1024, 16, 8), (64, 3, 1)])
+@pytest.mark.parametrize("M", [1, 17, 64])
+@pytest.mark.parametrize("ticks", [-1, 1])
+def test_qkv_halves_that_do_not_come(gpu, hidden, hq, hkv, M, ticks):
+    """The sums of a head's other half do not come in time: a block runs that
+    half itself, with the same bits."""
+    from types import SimpleNamespace as NS
+
+    from qwen3_engine_from_scratch_amd.kernels.model_ops import (decode_chain_sync,
+                                                                 decode_qkv_rope, embed_ss)
+    from qwen3_engine_from_scratch_amd.kernels.pre_attention import rope_tables
+
+    g = torch.Generator(device=gpu).manual_seed(M)
+    layer = _layer(g, gpu, hidden, 128, hq, hkv)
+    at = layer.self_attn
+    pool = NS(k_buffer=torch.zeros(M, 1, hkv, 16, 128, dtype=torch.bfloat16, device=gpu),
+              v_buffer=torch.zeros(M, 1, hkv, 16, 128, dtype=torch.bfloat16, device=gpu),
+              block_table_2d=torch.arange(M, dtype=torch.int32, device=gpu).view(M, 1),
+              seq_lens=(torch.arange(M, device=gpu) % 16).to(torch.int32))
+    cos, sin = rope_tables(128, 1e6, 64, device=gpu)
+    h, ss = embed_ss(torch.arange(M, device=gpu),
+                     torch.randn(64, hidden, generator=g, device=gpu).bfloat16())
+    sync = decode_chain_sync(gpu)
+    announce(f"qkv halves that do not come M={M} hidden={hidden} ticks={ticks}")
+
+    def run(**kw):
+        pool.k_buffer.zero_()
+        pool.v_buffer.zero_()
+        q = decode_qkv_rope(h, ss, layer.input_layernorm.weight, 1e-6, at.qkv_proj.weight, hq, hkv,
+                            at.q_norm.weight, at.k_norm.weight, 1e-6, cos, sin, pool, 0, None, **kw)
+        return q, pool.k_buffer.clone(), pool.v_buffer.clone()
+
+    want = run()
+    for _ in range(3):
+        assert _same(run(sync=sync, wait_ticks=ticks), want)
+    assert _launches(sync) == 3
+
+
+def test_chain_launches_that_overlap(gpu):
+    """Four models' launches in flight at once, each with hand-off words of its
+    own (together more blocks than are resident), waiting as long as they like
+    and giving up at once: every one has its own bits."""
+    chains = [_Chain(gpu, M, seed=20 + M) for M in (16, 1, 7, 16)]
+    want = [c.run() for c in chains]
+    streams = [torch.cuda.Stream() for _ in chains]
+    torch.cuda.synchronize()
+    announce("decode chain: four launches in flight")
+    for ticks in (0, -1):
+        got = [[] for _ in chains]
+        for _ in range(6):
+            for c, s, out in zip(chains, streams, got):
+                with torch.cuda.stream(s):
+                    out.append(c.run(wait_ticks=ticks))
+        torch.cuda.synchronize()
+        for i, (outs, w) in enumerate(zip(got, want)):
+            assert all(_same(x, w) for x in outs), f"stream {i}, ticks {ticks}"
+    assert [_launches(c.sync) for c in chains] == [13] * 4
+
+
+@pytest.mark.parametrize("value", ["nan", "-nan", "inf", "big"])
+def test_chain_non_finite_activations(gpu, value):
+    """A residual row that is not finite (or whose squares are not) goes through
+    the handed-on sums as through the separate kernels: NaN sums of either
+    sign are sums, and the other rows have their bits."""
+    from qwen3_engine_from_scratch_amd.kernels.model_ops import decode_qkv_rope
+
+    c = _Chain(gpu, 7, seed=5)
+    announce(f"decode chain: {value} in the residual stream")
+    x = {"nan": float("nan"), "-nan": float("nan"), "inf": float("inf"), "big": 3e38}[value]
+    want = c.run()
+    c.h0[2, 5] = x
+    if value == "-nan":
+        c.h0.view(torch.int16)[2, 5] = -1  # every bit set
+    c.ss0[2] = c.h0[2].float().square().view(-1, 16).sum(-1)
+    got = c.run(nxt=False)
+    h, ss = got[1], got[2]
+    assert not torch.isfinite(ss[2]).all()
+    keep = [0, 1, 3, 4, 5, 6]
+    assert _same([h[keep], ss[keep]], [want[1][keep], want[2][keep]])
+    # the next layer's heads from that stream, in one workgroup each and in two
+    at = c.b.self_attn
+
+    def qkv(**kw):
+        q = decode_qkv_rope(h, ss, c.b.input_layernorm.weight, 1e-6, at.qkv_proj.weight, 16, 8,
+                            at.q_norm.weight, at.k_norm.weight, 1e-6, *c.tables, c.pool, 1, c.rows,
+                            **kw)
+        return q, c.pool.k_buffer[:, 1].clone(), c.pool.v_buffer[:, 1].clone()
+
+    one, two = qkv(), qkv(sync=c.sync)
+    for a, b in zip(one, two):
+        assert torch.equal(a.isnan(), b.isnan()) and torch.equal(a.nan_to_num(), b.nan_to_num())
+    q = c.run()[-1]
+    assert torch.equal(q.isnan(), one[0].isnan())
+    assert torch.equal(q.nan_to_num(), one[0].nan_to_num())
