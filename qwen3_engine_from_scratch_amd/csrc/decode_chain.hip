@@ -748,20 +748,28 @@ void decode_qkv_half_kernel(ChainArgs args) {
   arrive(args, sh);
 }
 
-// Blocks resident at once on the current device (0: unknown).
-int resident_blocks() {
-  static int cached[64] = {0};
+// Blocks of the kernel resident at once on the current device (0: unknown).
+int resident_blocks(void (*kernel)(ChainArgs), int (&cached)[64]) {
   int dev = -1;
   if (hipGetDevice(&dev) != hipSuccess || dev < 0 || dev >= 64) return 0;
   if (cached[dev] == 0) {
     int cus = 0, per = 0;
     if (hipDeviceGetAttribute(&cus, hipDeviceAttributeMultiprocessorCount, dev) != hipSuccess ||
         hipOccupancyMaxActiveBlocksPerMultiprocessor(
-            &per, reinterpret_cast<const void*>(decode_chain_kernel), kThreads, 0) != hipSuccess)
+            &per, reinterpret_cast<const void*>(kernel), kThreads, 0) != hipSuccess)
       return 0;
     cached[dev] = cus * per;
   }
   return cached[dev];
+}
+// Larger grids would be answered too, but their waits would run out.
+int chain_blocks() {
+  static int cached[64] = {0};
+  return resident_blocks(decode_chain_kernel, cached);
+}
+int qkv_half_blocks() {
+  static int cached[64] = {0};
+  return resident_blocks(decode_qkv_half_kernel, cached);
 }
 
 // Blocks per phase; false for shapes the kernel does not hold.
@@ -847,7 +855,7 @@ extern "C" int qwen3_decode_chain_supported(int M, int hidden, int intermediate,
                                             int num_kv_heads) {
   int first[kPhases + 1];
   return phase_blocks(M, hidden, intermediate, num_heads, num_kv_heads, true, true, first) &&
-                 first[kPhases] <= resident_blocks()
+                 first[kPhases] <= chain_blocks()
              ? 1
              : 0;
 }
@@ -866,7 +874,7 @@ extern "C" int qwen3_decode_chain_bf16(const qwen3_decode_chain_args* c, void* s
     return q3::fail(QWEN3_EUNSUPPORTED, "%s: %d rows, hidden %d, intermediate %d, heads %d / %d "
                     "not supported", who, c->M, c->hidden, c->intermediate, c->num_heads,
                     c->num_kv_heads);
-  if (a.first[kPhases] > resident_blocks())
+  if (a.first[kPhases] > chain_blocks())
     return q3::fail(QWEN3_EUNSUPPORTED, "%s: %d blocks cannot be resident at once", who,
                     a.first[kPhases]);
   if (c->h_in == c->h_mid || c->h_mid == c->h_out || !(c->eps >= 0.f))
@@ -938,7 +946,7 @@ extern "C" int qwen3_decode_qkv_half_supported(int M, int hidden, int num_heads,
   const int64_t blocks = q3::cdiv(2 * (num_heads + 2 * num_kv_heads), 8) * 8 * ((M + 15) / 16);
   return M >= 1 && M <= kMaxRowBlocks * kRows && num_heads > 0 && num_kv_heads > 0 &&
                  num_heads + num_kv_heads <= kMaxNormHeads && hidden > 0 &&
-                 hidden % (2 * kKStep) == 0 && hidden <= kMaxHidden && blocks <= resident_blocks()
+                 hidden % (2 * kKStep) == 0 && hidden <= kMaxHidden && blocks <= qkv_half_blocks()
              ? 1
              : 0;
 }
