@@ -370,7 +370,8 @@ def decode_qkv_rope(h: torch.Tensor, ss_in: torch.Tensor, norm_weight: torch.Ten
     lib = _lib.load()
     # the halves wait for one another: where all of them are resident at once
     if sync is not None and lib.qwen3_decode_qkv_half_supported(M, K, num_heads, num_kv_heads) \
-            and ss_in.shape[1] == K // 16:
+            and ss_in.shape[1] == K // 16 and K <= h.stride(0) <= 1 << 24 \
+            and K <= qkv_weight.stride(0) <= 1 << 24:
         a = _lib.DecodeChainArgs(M=M, hidden=K, num_heads=num_heads, num_kv_heads=num_kv_heads,
                                  eps=eps, head_eps=head_eps, h_out=h.data_ptr(),
                                  ss_out=ss_in.data_ptr(), sync=sync.data_ptr(),

@@ -353,3 +353,20 @@ def test_chain_non_finite_activations(gpu, value):
     q = c.run()[-1]
     assert torch.equal(q.isnan(), one[0].isnan())
     assert torch.equal(q.nan_to_num(), one[0].nan_to_num())
+
+
+def test_qkv_rows_that_coincide(gpu):
+    """Rows that are one row (stride 0) go to the one-workgroup form, hand-off
+    words or not."""
+    from qwen3_engine_from_scratch_amd.kernels.model_ops import decode_qkv_rope
+
+    c = _Chain(gpu, 3)
+    at = c.b.self_attn
+    h, ss = c.h0[:1].expand(3, -1), c.ss0[:1].expand(3, -1).contiguous()
+
+    def qkv(x, **kw):
+        return decode_qkv_rope(x, ss, c.b.input_layernorm.weight, 1e-6, at.qkv_proj.weight, 16, 8,
+                               at.q_norm.weight, at.k_norm.weight, 1e-6, *c.tables, c.pool, 1,
+                               c.rows, **kw)
+
+    assert torch.equal(qkv(h, sync=c.sync), qkv(h.contiguous()))
