@@ -874,9 +874,6 @@ extern "C" int qwen3_decode_chain_bf16(const qwen3_decode_chain_args* c, void* s
     return q3::fail(QWEN3_EUNSUPPORTED, "%s: %d rows, hidden %d, intermediate %d, heads %d / %d "
                     "not supported", who, c->M, c->hidden, c->intermediate, c->num_heads,
                     c->num_kv_heads);
-  if (a.first[kPhases] > chain_blocks())
-    return q3::fail(QWEN3_EUNSUPPORTED, "%s: %d blocks cannot be resident at once", who,
-                    a.first[kPhases]);
   if (c->h_in == c->h_mid || c->h_mid == c->h_out || !(c->eps >= 0.f))
     return q3::fail(QWEN3_EINVAL, "%s: h_mid must be a buffer of its own, eps >= 0", who);
   bool ok = q3::aligned16(c->o) && q3::aligned16(c->o_weight) && q3::aligned16(c->h_in) &&
@@ -927,28 +924,39 @@ extern "C" int qwen3_decode_chain_bf16(const qwen3_decode_chain_args* c, void* s
   if (qkv)
     if (const int rc = fill_qkv(a, c, who)) return rc;
   if (!ok) return q3::fail(QWEN3_EALIGN, "%s: tensors need 16-byte aligned rows", who);
-  // rows of a weight tile inside 32-bit offsets, and not overlapping
-  const int64_t strides[4][2] = {{c->o_weight_row_stride, a.KO}, {c->gate_up_row_stride, a.K},
+  // rows of o and of a weight tile inside 32-bit offsets, and not overlapping
+  const int64_t strides[5][2] = {{c->o_weight_row_stride, a.KO}, {c->gate_up_row_stride, a.K},
                                  {c->down_row_stride, a.I},
-                                 {qkv ? c->qkv_row_stride : a.K, a.K}};
+                                 {qkv ? c->qkv_row_stride : a.K, a.K},
+                                 {c->M > 1 ? c->o_row_stride : a.KO, a.KO}};
   for (const auto& st : strides)
     if (st[0] < st[1] || st[0] > (int64_t{1} << 24))
-      return q3::fail(QWEN3_EINVAL, "%s: weight row stride %lld", who,
-                      static_cast<long long>(st[0]));
+      return q3::fail(QWEN3_EINVAL, "%s: row stride %lld of %lld columns", who,
+                      static_cast<long long>(st[0]), static_cast<long long>(st[1]));
+  if (a.first[kPhases] > chain_blocks())
+    return q3::fail(QWEN3_EUNSUPPORTED, "%s: %d blocks cannot be resident at once", who,
+                    a.first[kPhases]);
   q3::clear_error();
   hipLaunchKernelGGL(decode_chain_kernel, dim3(static_cast<unsigned>(a.first[kPhases])),
                      dim3(kThreads), 0, static_cast<hipStream_t>(stream), a);
   return q3::launch_status(who);
 }
 
+namespace {
+// Blocks of the half-head launch; 0 for shapes the kernel does not hold.
+int64_t half_blocks(int M, int hidden, int num_heads, int num_kv_heads) {
+  if (M < 1 || M > kMaxRowBlocks * kRows || num_heads <= 0 || num_kv_heads <= 0 ||
+      num_heads + num_kv_heads > kMaxNormHeads || hidden <= 0 || hidden % (2 * kKStep) != 0 ||
+      hidden > kMaxHidden)
+    return 0;
+  return q3::cdiv(2 * (num_heads + 2 * num_kv_heads), 8) * 8 * ((M + kRows - 1) / kRows);
+}
+}  // namespace
+
 extern "C" int qwen3_decode_qkv_half_supported(int M, int hidden, int num_heads,
                                                int num_kv_heads) {
-  const int64_t blocks = q3::cdiv(2 * (num_heads + 2 * num_kv_heads), 8) * 8 * ((M + 15) / 16);
-  return M >= 1 && M <= kMaxRowBlocks * kRows && num_heads > 0 && num_kv_heads > 0 &&
-                 num_heads + num_kv_heads <= kMaxNormHeads && hidden > 0 &&
-                 hidden % (2 * kKStep) == 0 && hidden <= kMaxHidden && blocks <= qkv_half_blocks()
-             ? 1
-             : 0;
+  const int64_t blocks = half_blocks(M, hidden, num_heads, num_kv_heads);
+  return blocks > 0 && blocks <= qkv_half_blocks() ? 1 : 0;
 }
 
 extern "C" int qwen3_decode_qkv_half_bf16(const qwen3_decode_chain_args* c, int64_t h_row_stride,
@@ -957,7 +965,8 @@ extern "C" int qwen3_decode_qkv_half_bf16(const qwen3_decode_chain_args* c, int6
   if (!c || !c->h_out || !c->ss_out || !c->qkv_weight || !c->sync)
     return q3::fail(QWEN3_EINVAL, "%s: null pointer argument", who);
   if (c->M == 0) return QWEN3_OK;
-  if (!qwen3_decode_qkv_half_supported(c->M, c->hidden, c->num_heads, c->num_kv_heads))
+  const int64_t blocks = half_blocks(c->M, c->hidden, c->num_heads, c->num_kv_heads);
+  if (blocks == 0)
     return q3::fail(QWEN3_EUNSUPPORTED, "%s: %d rows, hidden %d, heads %d / %d not supported", who,
                     c->M, c->hidden, c->num_heads, c->num_kv_heads);
   if (h_row_stride < c->hidden || h_row_stride > (int64_t{1} << 24) ||
@@ -973,10 +982,12 @@ extern "C" int qwen3_decode_qkv_half_bf16(const qwen3_decode_chain_args* c, int6
   a.sync = c->sync;
   a.wait_ticks = c->wait_ticks ? c->wait_ticks : kWaitTicks;
   if (const int rc = fill_qkv(a, c, who)) return rc;
-  if (!q3::aligned16(c->h_out) || !q3::aligned16(c->ss_out) || h_row_stride % 8 != 0)
+  if (!q3::aligned16(c->h_out) || !q3::aligned16(c->ss_out) || !q3::aligned16(c->sync) ||
+      h_row_stride % 8 != 0)
     return q3::fail(QWEN3_EALIGN, "%s: tensors need 16-byte aligned rows", who);
-  const int64_t blocks =
-      q3::cdiv(2 * (c->num_heads + 2 * c->num_kv_heads), 8) * 8 * ((c->M + 15) / 16);
+  if (blocks > qkv_half_blocks())
+    return q3::fail(QWEN3_EUNSUPPORTED, "%s: %lld blocks cannot be resident at once", who,
+                    static_cast<long long>(blocks));
   q3::clear_error();
   hipLaunchKernelGGL(decode_qkv_half_kernel, dim3(static_cast<unsigned>(blocks)), dim3(kThreads), 0,
                      static_cast<hipStream_t>(stream), a);

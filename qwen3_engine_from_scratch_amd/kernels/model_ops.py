@@ -255,6 +255,15 @@ def decode_chain_sync(device) -> torch.Tensor:
                        device=device)
 
 
+def _check_norm(weight: torch.Tensor, n: int) -> None:
+    assert weight.dtype == torch.bfloat16 and weight.is_contiguous() and weight.numel() == n
+
+
+def _check_sync(sync: torch.Tensor, lib) -> None:
+    assert sync.is_contiguous() and sync.numel() * sync.element_size() >= \
+        int(lib.qwen3_decode_chain_sync_bytes()), "sync must be decode_chain_sync(device)"
+
+
 def _set_qkv(a, norm_weight, qkv_weight, q_norm_weight, k_norm_weight, cos_table, sin_table,
              positions, q_out, pool, layer_idx, row_ids) -> None:
     """The qkv projection's part of a DecodeChainArgs."""
@@ -302,17 +311,21 @@ def decode_chain(o: torch.Tensor, h: torch.Tensor, h_mid: torch.Tensor, ss: torc
         assert t.shape == h.shape and t.dtype == torch.bfloat16 and t.is_contiguous()
     for t in (ss, ss_mid):
         assert t.shape == (M, hidden // 16) and t.dtype == torch.float32 and t.is_contiguous()
+    assert o.dtype == torch.bfloat16
     assert all(w.dtype == torch.bfloat16 and w.stride(1) == 1 for w in (wo, wg, wd))
+    post = layer.post_attention_layernorm.weight
+    _check_norm(post, hidden)
     lib = _lib.load()
-    dev = _lib.require_hip(o, h, h_mid, ss, ss_mid, wo, wg, wd, sync, attn_workspace, row_ids,
-                           positions)
+    _check_sync(sync, lib)
+    dev = _lib.require_hip(o, h, h_mid, ss, ss_mid, wo, wg, wd, post, sync, attn_workspace,
+                           row_ids, positions)
     act = torch.empty(M, inter, dtype=h.dtype, device=h.device)
     a = _lib.DecodeChainArgs(
         M=M, hidden=hidden, intermediate=inter, num_heads=num_heads, num_kv_heads=num_kv_heads,
         eps=eps, head_eps=head_eps, o=o.data_ptr(), o_row_stride=o.stride(0),
         o_weight=wo.data_ptr(), o_weight_row_stride=wo.stride(0), h_in=h.data_ptr(),
         h_mid=h_mid.data_ptr(), h_out=h.data_ptr(), ss_mid=ss_mid.data_ptr(),
-        ss_out=ss.data_ptr(), post_norm_weight=layer.post_attention_layernorm.weight.data_ptr(),
+        ss_out=ss.data_ptr(), post_norm_weight=post.data_ptr(),
         gate_up_weight=wg.data_ptr(), gate_up_row_stride=wg.stride(0), act=act.data_ptr(),
         down_weight=wd.data_ptr(), down_row_stride=wd.stride(0), sync=sync.data_ptr(),
         wait_ticks=wait_ticks)
@@ -324,7 +337,13 @@ def decode_chain(o: torch.Tensor, h: torch.Tensor, h_mid: torch.Tensor, ss: torc
     if next_layer is not None:
         at = next_layer.self_attn
         wq = at.qkv_proj.weight
-        assert wq.shape == ((num_heads + 2 * num_kv_heads) * 128, hidden) and wq.stride(1) == 1
+        assert wq.shape == ((num_heads + 2 * num_kv_heads) * 128, hidden) and wq.stride(1) == 1 \
+            and wq.dtype == torch.bfloat16
+        norms = (next_layer.input_layernorm.weight, at.q_norm.weight, at.k_norm.weight)
+        for w, n in zip(norms, (hidden, 128, 128)):
+            _check_norm(w, n)
+        _lib.require_hip(h, wq, *norms, cos_table, sin_table, pool.k_buffer, pool.v_buffer,
+                         pool.seq_lens, pool.block_table_2d)
         assert cos_table.dtype == sin_table.dtype == torch.float32 and cos_table.stride(1) == 1
         assert row_ids is None or (row_ids.dtype == torch.int32 and row_ids.is_contiguous()
                                    and row_ids.numel() == M)
@@ -372,6 +391,8 @@ def decode_qkv_rope(h: torch.Tensor, ss_in: torch.Tensor, norm_weight: torch.Ten
     if sync is not None and lib.qwen3_decode_qkv_half_supported(M, K, num_heads, num_kv_heads) \
             and ss_in.shape[1] == K // 16 and K <= h.stride(0) <= 1 << 24 \
             and K <= qkv_weight.stride(0) <= 1 << 24:
+        _check_sync(sync, lib)
+        _lib.require_hip(h, sync)
         a = _lib.DecodeChainArgs(M=M, hidden=K, num_heads=num_heads, num_kv_heads=num_kv_heads,
                                  eps=eps, head_eps=head_eps, h_out=h.data_ptr(),
                                  ss_out=ss_in.data_ptr(), sync=sync.data_ptr(),

@@ -318,3 +318,97 @@ def test_mfma_rate_reference_rejects_bad_arguments():
     assert lib.qwen3_mfma_rate_reference(10, None, ctypes.byref(flops), None) == -1
     assert lib.qwen3_mfma_rate_reference(10, FAKE, None, None) == -1
     assert lib.qwen3_mfma_rate_reference(10, FAKE + 4, ctypes.byref(flops), None) == -2
+
+
+def _decode_chain_args(**kw):
+    """Sound arguments of a four-row launch of Qwen3-0.6B's widths, but `kw`."""
+    a = _lib.DecodeChainArgs(
+        M=4, hidden=1024, intermediate=3072, num_heads=16, num_kv_heads=8, eps=1e-6, head_eps=1e-6,
+        o=FAKE, o_row_stride=2048, o_weight=FAKE, o_weight_row_stride=2048, h_in=FAKE,
+        h_mid=FAKE + 4096, h_out=FAKE, ss_mid=FAKE, ss_out=FAKE, post_norm_weight=FAKE,
+        gate_up_weight=FAKE, gate_up_row_stride=1024, act=FAKE, down_weight=FAKE,
+        down_row_stride=3072, sync=FAKE, in_norm_weight=FAKE, qkv_weight=FAKE, qkv_row_stride=1024,
+        q_norm_weight=FAKE, k_norm_weight=FAKE, cos_table=FAKE, sin_table=FAKE,
+        table_row_stride=128, table_rows=64, q_out=FAKE, q_out_strides=_s(2048, 128), k_cache=FAKE,
+        v_cache=FAKE, k_cache_strides=_s(1 << 16, 1 << 14, 2048, 128),
+        v_cache_strides=_s(1 << 16, 1 << 14, 2048, 128), num_blocks=16, seq_lens=FAKE,
+        block_table=FAKE, bt_row_stride=8, max_rows=8, max_pages=8, layer_idx=1, num_layers=28,
+        block_size=16)
+    for k, v in kw.items():
+        setattr(a, k, v)
+    return ctypes.byref(a)
+
+
+@pytest.mark.parametrize("code, kw", [
+    (-1, dict(o=None)), (-1, dict(sync=None)), (-1, dict(act=None)), (-1, dict(post_norm_weight=None)),
+    (-1, dict(in_norm_weight=None)), (-1, dict(k_cache=None)), (-1, dict(block_table=None)),
+    (-3, dict(M=17)), (-3, dict(hidden=1000)), (-3, dict(hidden=2048)), (-3, dict(intermediate=1024)),
+    (-3, dict(num_heads=12)), (-3, dict(num_heads=8)),
+    (-1, dict(h_mid=FAKE)), (-1, dict(eps=-1.0)), (-1, dict(head_eps=-1.0)),
+    (-4, dict(attn_workspace=FAKE, attn_waves=2048, attn_workspace_bytes=1 << 16)),
+    (-4, dict(attn_workspace=FAKE, attn_waves=0, attn_workspace_bytes=1 << 30)),
+    (-2, dict(attn_workspace=FAKE + 4, attn_waves=64, attn_workspace_bytes=1 << 30)),
+    (-1, dict(o_row_stride=1024)), (-1, dict(o_row_stride=1 << 25)), (-2, dict(o_row_stride=2052)),
+    (-1, dict(o_weight_row_stride=1024)), (-1, dict(gate_up_row_stride=1 << 25)),
+    (-1, dict(down_row_stride=1024)), (-1, dict(qkv_row_stride=512)),
+    (-2, dict(sync=FAKE + 4)), (-2, dict(h_out=FAKE + 2)), (-2, dict(gate_up_weight=FAKE + 2)),
+    (-2, dict(cos_table=FAKE + 4)), (-2, dict(k_cache_strides=_s(1 << 16, 1 << 14, 2048, 129))),
+    (-1, dict(layer_idx=28)), (-1, dict(bt_row_stride=4)), (-1, dict(block_size=0)),
+    (0, dict(M=0)),
+])
+def test_decode_chain_rejects_bad_arguments(code, kw):
+    lib = _lib.load()
+    assert lib.qwen3_decode_chain_bf16(_decode_chain_args(**kw), None) == code
+
+
+@pytest.mark.parametrize("code, kw, stride", [
+    (-1, dict(h_out=None), 1024), (-1, dict(ss_out=None), 1024), (-1, dict(qkv_weight=None), 1024),
+    (-1, dict(sync=None), 1024), (-3, dict(M=65), 1024), (-3, dict(hidden=1000), 1024),
+    (-3, dict(hidden=2048), 2048), (-3, dict(num_heads=60, num_kv_heads=5), 1024),
+    (-1, {}, 1016), (-1, {}, 1 << 25), (-2, {}, 1028), (-1, dict(qkv_row_stride=1 << 25), 1024),
+    (-1, dict(eps=-1.0), 1024), (-1, dict(q_out=None), 1024), (-2, dict(q_out=FAKE + 2), 1024),
+    (-2, dict(h_out=FAKE + 2), 1024), (-2, dict(sync=FAKE + 4), 1024), (0, dict(M=0), 1024),
+])
+def test_decode_qkv_half_rejects_bad_arguments(code, kw, stride):
+    lib = _lib.load()
+    assert lib.qwen3_decode_qkv_half_bf16(_decode_chain_args(**kw), stride, None) == code
+
+
+def test_paged_decode_partials_rejects_bad_arguments():
+    lib = _lib.load()
+
+    def call(q=FAKE, qs=_s(4096, 128), B=4, D=128, bts=8, ws=FAKE, wsb=1 << 40):
+        return lib.qwen3_paged_decode_partials_bf16(
+            q, qs, FAKE, _s(1 << 14, 2048, 128), FAKE, _s(1 << 14, 2048, 128), 64, FAKE, bts, 4096,
+            8, FAKE, 1, FAKE, FAKE, _s(4096, 128), B, 32, 8, D, 16, 0.088, ws, wsb, None)
+
+    assert call(q=None) == -1 and call(bts=4) == -1
+    assert call(D=64) == -3
+    assert call(q=FAKE + 2) == -2 and call(qs=_s(4097, 128)) == -2 and call(ws=FAKE + 8) == -2
+    assert call(ws=None) == -4 and call(wsb=4096) == -4
+    assert call(B=2049) == -3          # no partial results on the grid path
+    assert call(B=0) == 0
+
+
+def test_decode_chain_args_match_the_header(tmp_path):
+    """The ctypes mirror of qwen3_decode_chain_args has the C struct's size and
+    field offsets."""
+    import shutil
+    import subprocess
+
+    gcc = shutil.which("gcc") or shutil.which("cc")
+    if not gcc:
+        pytest.skip("no C compiler")
+    names = [f[0] for f in _lib.DecodeChainArgs._fields_]
+    src = tmp_path / "layout.c"
+    src.write_text('#include <stddef.h>\n#include <stdio.h>\n#include "qwen3_model_ops.h"\n'
+                   "int main(void) {\n"
+                   + "".join(f'  printf("%zu\\n", offsetof(qwen3_decode_chain_args, {n}));\n'
+                             for n in names)
+                   + '  printf("%zu\\n", sizeof(qwen3_decode_chain_args));\n  return 0;\n}\n')
+    exe = tmp_path / "layout"
+    subprocess.run([gcc, "-I", str(HEADERS[0].parent), str(src), "-o", str(exe)], check=True)
+    got = [int(x) for x in subprocess.run([str(exe)], check=True, capture_output=True,
+                                          text=True).stdout.split()]
+    assert got == [getattr(_lib.DecodeChainArgs, n).offset for n in names] + [
+        ctypes.sizeof(_lib.DecodeChainArgs)]

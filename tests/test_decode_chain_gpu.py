@@ -355,6 +355,29 @@ def test_chain_non_finite_activations(gpu, value):
     assert torch.equal(q.nan_to_num(), one[0].nan_to_num())
 
 
+def test_chain_refuses_wrong_tensors(gpu):
+    """What the separate wrappers refuse: a norm of another length or type, and
+    hand-off words that are too few."""
+    from types import SimpleNamespace as NS
+
+    c = _Chain(gpu, 2)
+    norm = c.a.post_attention_layernorm
+    for bad in (norm.weight[:512], norm.weight.float(), torch.stack([norm.weight] * 2, 1)[:, 0]):
+        c.a.post_attention_layernorm = NS(weight=bad)
+        with pytest.raises(AssertionError):
+            c.run()
+    c.a.post_attention_layernorm = norm
+    c.b.self_attn.q_norm, q_norm = NS(weight=c.b.self_attn.q_norm.weight[:64]), c.b.self_attn.q_norm
+    with pytest.raises(AssertionError):
+        c.run()
+    c.b.self_attn.q_norm = q_norm
+    c.sync, sync = c.sync[:-16], c.sync
+    with pytest.raises(AssertionError):
+        c.run()
+    c.sync = sync
+    c.run()
+
+
 def test_qkv_rows_that_coincide(gpu):
     """Rows that are one row (stride 0) go to the one-workgroup form, hand-off
     words or not."""
