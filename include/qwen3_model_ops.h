@@ -257,8 +257,8 @@ int qwen3_sample_bf16(const void* logits, int64_t row_stride, int64_t rows, int6
  * and keeps the tokens at or above it, and a second launch draws from the
  * union of those lists (it holds every token of the row's top k), falling
  * back to streaming the row when the lists overflow.  Rows that top-k does not
- * cut list the parts' largest tokens and masses (top-p alone) or draw part by
- * part.  The launches meet in
+ * cut list the parts' largest tokens and add the parts' masses up (top-p
+ * alone) or draw part by part.  The launches meet in
  * a caller workspace of qwen3_sample_workspace_bytes(rows, vocab) bytes
  * (device, 16-byte aligned, no initialisation; calls that share one must
  * not overlap); 0 bytes means one part per row, and then, or with a NULL

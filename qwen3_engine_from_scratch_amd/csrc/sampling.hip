@@ -49,10 +49,12 @@
 // the whole top-k list and every tie at its boundary, and no step depends on
 // the order of the candidates, so the draws are the single workgroup's.
 // Greedy rows take each part's first maximum and then the first among the
-// parts; rows that nothing cuts each part's draw and then the best; rows that
-// only top-p cuts list a fixed share of tokens per part beside the part's
-// softmax mass, and the cut is made in the union (or over the row when it lies
-// past the listed tokens).
+// parts; rows that nothing cuts each part's draw and then the best.  Rows that
+// only top-p cuts need the row's maximum before any weight: their parts list a
+// fixed share of tokens first, and in the second launch one workgroup per part
+// adds its masses to the row's bins; the one that comes last has the single
+// workgroup's bins, whole numbers, and cuts in the lists (or over the row where
+// the cut lies past the listed tokens).
 //
 // The VALU is the limit of every pass (a wave64 instruction occupies its
 // SIMD four cycles), so the per-token work is kept small: whole rounds of
@@ -189,13 +191,18 @@ struct Shared {
 // workspace).
 struct alignas(16) PartOut {
   uint32_t kmax;                  // the part's largest key (kmax, ncand: one 8-byte load);
-                                  // top-p alone: t_lo << 16 above it, every token with
-                                  // key >= t_lo is listed
+                                  // rows that top-k does not cut: t_lo << 16 above it, every
+                                  // token with key >= t_lo is listed
   int32_t ncand;                  // candidates written, -1 none
   unsigned long long best;        // greedy rows: (key + 1) << 32 | ~index, the first maximum;
-                                  // rows drawn uncut: the part's draw (score, ~index);
-                                  // top-p alone: the part's mass (a double)
+                                  // rows drawn uncut: the part's draw (score, ~index)
   unsigned long long cand[kCap];  // (key << 32) | token index
+};
+// A row that only top-p cuts: its bins' masses over all parts, and how many
+// parts have added theirs.  Cleared by the first launch.
+struct alignas(16) RowMass {
+  unsigned long long bin[kHiBins];
+  uint32_t arrived;
 };
 
 // Parts per row of the parallel form: about one workgroup per CU over the
@@ -203,13 +210,13 @@ struct alignas(16) PartOut {
 // 55 for two and 65 for eight), each part at least one round (kThreads * 8
 // tokens); 1 means the single-workgroup form.
 constexpr int kMaxParts = 8;
-// Top-p alone: tokens that the parts of a row list between them (each part
-// its share, at least; ties add to it).  A row whose cut lies past the listed
-// ones is streamed by one workgroup as without parts, after the lists (132 us
-// against 88), so the list is long: top-p 0.9 over logits whose softmax
-// falls as rank^-1.3 keeps 1,250 tokens (rank^-1.5: 60).  512 entries are 1-2
-// us faster where they suffice (64 rows 32 against 34 us), but one row in a
-// few hundred of such logits did not.
+// Top-p alone: tokens that the parts of a row list between them (each part its
+// share, at least; ties add to it).  About 1,200 of them lie above the largest
+// of the parts' thresholds and can be cut in: top-p 0.9 over logits whose
+// softmax falls as rank^-1.5 keeps 60 tokens, rank^-1.3 1,250.  A row whose cut
+// lies past them is passed over twice more by one workgroup (8 x 151,936
+// logits, rank^-2.2 and -1.6: 30 us; -1.3: 76; -1: 203; one workgroup per row
+// for everything: 89, 90, 126 and 242).
 constexpr int kNucleusList = 1536;
 __host__ __device__ inline int parts_for(int64_t rows, int64_t vocab) {
   int p = rows <= 32 ? kMaxParts : rows <= 64 ? 4 : rows <= 128 ? 2 : 1;
@@ -248,21 +255,6 @@ __device__ __forceinline__ unsigned long long block_max_u64(unsigned long long v
   return __shfl(v, 0, 64);
 }
 
-// Block-wide sum in a fixed order; every thread gets the result.
-__device__ __forceinline__ double block_sum_f64(double v, Shared& sh) {
-#pragma unroll
-  for (int m = 1; m < 64; m <<= 1) v += __shfl_xor(v, m, 64);
-  __syncthreads();
-  double* part = reinterpret_cast<double*>(sh.wmass);
-  if ((threadIdx.x & 63) == 0) part[threadIdx.x >> 6] = v;
-  __syncthreads();
-  const int lane = threadIdx.x & 63;
-  v = lane < kWaves ? part[lane] : 0.0;
-#pragma unroll
-  for (int m = 1; m < kWaves; m <<= 1) v += __shfl_xor(v, m, 64);
-  return __shfl(v, 0, 64);
-}
-
 // Gumbel-max candidate of one token: (ordered score, complemented index).
 __device__ __forceinline__ unsigned long long draw_candidate(uint32_t key, int64_t idx,
                                                              uint32_t draw, float inv_t) {
@@ -272,10 +264,14 @@ __device__ __forceinline__ unsigned long long draw_candidate(uint32_t key, int64
   return (static_cast<unsigned long long>(so) << 32) | (~static_cast<uint32_t>(idx));
 }
 
-// Softmax weight relative to the maximum, in fixed point.
-__device__ __forceinline__ unsigned long long fixed_weight(uint32_t key, float inv_t, float xmax) {
-  const float w = __expf(key_value(key) * inv_t - xmax);
+// Softmax weight relative to the maximum, in fixed point: the same bits wherever
+// it is computed (the multiply-add is not left to the compiler).
+__device__ __forceinline__ unsigned long long fixed_weight_of(float x, float inv_t, float xmax) {
+  const float w = __expf(fmaf(x, inv_t, -xmax));
   return static_cast<unsigned long long>(static_cast<double>(w) * kFix + 0.5);
+}
+__device__ __forceinline__ unsigned long long fixed_weight(uint32_t key, float inv_t, float xmax) {
+  return fixed_weight_of(key_value(key), inv_t, xmax);
 }
 
 // Appends (key, index) of the lanes where q holds to the block's candidate
@@ -538,11 +534,10 @@ __device__ __forceinline__ int find_count_bin_block(const uint32_t* h, int64_t n
 // converted to double, exceeds it (there is one when top_p < 1 and the total
 // is positive).  Returns the bin, or -1, and sets `run` to the mass above
 // it.  The same block-wide scan as find_count_bin_block; the caller has
-// passed a barrier since the last read of sh.sel_bin.  given_limit: the
-// limit is the caller's (the bins hold only the tokens that can be kept).
+// passed a barrier since the last read of sh.sel_bin.
 __device__ __forceinline__ int find_mass_bin_block(const unsigned long long* m, float top_p,
                                                    double& limit, unsigned long long& run,
-                                                   Shared& sh, bool given_limit = false) {
+                                                   Shared& sh) {
   const int top = kHiBins - 1 - kBinsPerThread * static_cast<int>(threadIdx.x);
   unsigned long long mine = 0;
 #pragma unroll
@@ -550,7 +545,7 @@ __device__ __forceinline__ int find_mass_bin_block(const unsigned long long* m, 
   if (threadIdx.x == 0) sh.sel_bin = -1;  // before the scan's barriers
   unsigned long long total;
   unsigned long long r = block_scan_u64(mine, total, sh);
-  if (!given_limit) limit = static_cast<double>(fmaxf(top_p, 0.f)) * static_cast<double>(total);
+  limit = static_cast<double>(fmaxf(top_p, 0.f)) * static_cast<double>(total);
   if (static_cast<double>(r) <= limit && static_cast<double>(r + mine) > limit) {
 #pragma unroll
     for (int j = 0; j < kBinsPerThread; ++j) {
@@ -583,23 +578,23 @@ __device__ __forceinline__ void part_values(int P, T none, F&& get, T (&v)[kMaxP
 // the part's first maximum; for a row that top-k cuts, the part's largest
 // key and its tokens at or above its own threshold (a list of -1 entries:
 // more than kCap); for a row that only top-p cuts, the same with a threshold
-// that the part's share of kNucleusList tokens reach, and the part's softmax
-// mass relative to its own maximum (one pass instead of the row's maximum
-// first: the merge rescales the parts' sums, whose relative error, that of
-// the weights' 32-bit exponentials, stays); for a row that nothing cuts, the
-// draw itself over the part.  A part of at most 8 rounds is held in
+// that the part's share of kNucleusList tokens reach; for a row that nothing
+// cuts, the draw itself over the part.  A part of at most 8 rounds is held in
 // registers for all of its passes.
+//
 //
 // One workgroup per row is bound by the row's passes on one CU (about 20 us
 // each), which is why the uncut rows are split too: top-p 0.9 over 8 x 151,936
-// logits 88 -> 27.5 us, over 64 rows 105 -> 34; no cut at all, 44 rows, 178.6 -> 31.5.
+// peaked logits 89 -> 30 us, over 64 rows 89 -> 41; no cut at all, 44 rows,
+// 178.6 -> 31.5.
 template <bool kVec>
 __global__ __launch_bounds__(kThreads) void sample_part_kernel(const uint16_t* logits,
                                                                int64_t row_s, int64_t vocab,
                                                                const float* temperature,
                                                                const int32_t* top_k,
                                                                const float* top_p, uint64_t seed,
-                                                               int P, PartOut* parts) {
+                                                               int P, PartOut* parts,
+                                                               RowMass* mass) {
   __shared__ Shared sh;
   const int64_t row = blockIdx.x / P;
   const int c = static_cast<int>(blockIdx.x % P);
@@ -637,7 +632,11 @@ __global__ __launch_bounds__(kThreads) void sample_part_kernel(const uint16_t* l
       if (tid == 0) po.best = best;
       return;
     }
-    if (uncut) kreq = kNucleusList / P;  // top-p alone: the tokens this part lists
+    if (uncut) {
+      kreq = kNucleusList / P;  // top-p alone: the tokens this part lists
+      for (int i = c * kThreads + tid; i < kHiBins; i += P * kThreads) mass[row].bin[i] = 0ull;
+      if (c == 0 && tid == 0) mass[row].arrived = 0u;
+    }
     if (!greedy) {
       for (int i = tid; i < kHiBins; i += kThreads) sh.cnt[i] = 0;
       if (tid == 0) sh.ncand = 0;
@@ -718,29 +717,15 @@ __global__ __launch_bounds__(kThreads) void sample_part_kernel(const uint16_t* l
       t_lo = static_cast<uint32_t>(find_count_bin_block(sh.cnt, kreq, above, sh)) << kLoBits;
     }
     if (__builtin_expect(uncut, 0)) {
-      // the part's mass: numbers only (a NaN's weight is 0), in doubles; a
-      // part of nothing but -inf and NaN has none, and where the maximum is
-      // not finite the row goes to the single workgroup
-      const float xm = key_value(kmax) * inv_t;
-      const bool none = kmax <= 0x7Fu;
-      double m = 0.0;
-      if (!none && xm < INFINITY && xm > -INFINITY)
-        visit([&](int64_t i0, const uint32_t* b, auto full) {
-#pragma unroll
-          for (int e = 0; e < 8; ++e) {
-            const float w = __expf(__uint_as_float(b[e] << 16) * inv_t - xm);
-            if (full || i0 + e < hi) m += static_cast<double>(fmaxf(w, 0.f));
-          }
-        });
-      m = block_sum_f64(m, sh);
-      if (tid == 0) po.best = static_cast<unsigned long long>(__double_as_longlong(m));
-      if (none || !(xm < INFINITY && xm > -INFINITY)) {
+      // -inf (key 0x7F) and NaN have no mass and are never listed
+      if (kmax <= 0x7Fu) {
         if (tid == 0) {
           po.kmax = kmax;
-          po.ncand = none ? 0 : -1;
+          po.ncand = 0;
         }
         return;
       }
+      t_lo = max(t_lo, 0x80u);
     }
     visit([&](int64_t i0, const uint32_t* b, auto full) {
       bool q[8], any = false;
@@ -809,20 +794,22 @@ __global__ __launch_bounds__(kThreads) void sample_part_kernel(const uint16_t* l
   }
 }
 
-// One workgroup per row.  kPre: greedy rows, rows drawn uncut and, when every
-// part kept its list, passes A to E run over the parts' results instead of
-// the row; otherwise the workgroup streams the row for them itself.  For
-// top-p alone the union of the lists is every token at or above the largest
-// of the parts' thresholds, and the cut must lie among those.
+// One workgroup per row.  kPre: workgroup (row, part), of which part 0 does the
+// row: for greedy rows, rows drawn uncut and, when every part kept its list,
+// passes A to E run over the parts' results instead of the row; otherwise the
+// workgroup streams the row for them itself.  A row that only top-p cuts takes
+// all its workgroups: each adds its part's masses to the row's bins, and the
+// last to arrive (nobody waits) goes on from pass C's bins.
 template <bool kVec, bool kPre>
 __global__ __launch_bounds__(kThreads) void sample_kernel(const uint16_t* logits, int64_t row_s,
                                                           int64_t vocab, const float* temperature,
                                                           const int32_t* top_k,
                                                           const float* top_p, uint64_t seed,
                                                           int64_t* out, int P,
-                                                          const PartOut* parts) {
+                                                          const PartOut* parts, RowMass* mass) {
   __shared__ Shared sh;
   const int64_t row = blockIdx.x;
+  const int part = kPre ? static_cast<int>(blockIdx.y) : 0;
   const uint16_t* p = logits + row * row_s;
   const float temp = temperature ? temperature[row] : 0.f;
   const int64_t kreq = top_k ? top_k[row] : 0;
@@ -840,7 +827,7 @@ __global__ __launch_bounds__(kThreads) void sample_kernel(const uint16_t* logits
   unsigned long long spec = 0;
   unsigned long long hdr[kMaxParts];
   if constexpr (kPre) {
-    spec = rp[cpart].cand[coff];
+    if (part == 0) spec = rp[cpart].cand[coff];
     part_values(P, 0ull, [&](int c) {
       return *reinterpret_cast<const unsigned long long*>(&rp[c].kmax);
     }, hdr);
@@ -848,6 +835,11 @@ __global__ __launch_bounds__(kThreads) void sample_kernel(const uint16_t* logits
     // branches that use them, after the parameters' round trip)
     asm volatile("" ::"v"(spec), "v"(hdr[0]));
   }
+
+  const bool uncut = kreq <= 0 || kreq >= vocab;  // by top-k, as the part kernel
+  // cut by top-p alone: every part's workgroup has a share
+  const bool split = kPre && temp > 0.f && uncut && pcut < 1.f;
+  if (part > 0 && !split) return;
 
   // ---- greedy -----------------------------------------------------------
   if (kPre && !(temp > 0.f)) {
@@ -886,7 +878,6 @@ __global__ __launch_bounds__(kThreads) void sample_kernel(const uint16_t* logits
   const int64_t k = (kreq <= 0 || kreq > vocab) ? vocab : kreq;
   const bool use_p = pcut < 1.f;
   const float inv_t = 1.f / temp;
-  const bool uncut = kreq <= 0 || kreq >= vocab;  // as the part kernel
 
   if (kPre && __builtin_expect(uncut && !use_p, 0)) {  // the best of the parts' draws
     if (tid == 0) {
@@ -938,36 +929,25 @@ __global__ __launch_bounds__(kThreads) void sample_kernel(const uint16_t* logits
   // ---- A: high-bin counts and the maximum key ----------------------------
   uint32_t kmax = 0;
   bool from_list = false;  // the parts' lists stand for the row in passes A, B
-  // The top-p cut inside the high bin whose mass above it is r2, from the
-  // low-bin histograms: the first low bin whose mass passes the limit and how
-  // many of its ties are kept: rank r while the mass before it, r2 + r * w, is
-  // within the limit (rank 0 of the list's first key is always kept since r2
-  // is then 0).  Returns the bin, or -1.
-  auto low_cut = [&](unsigned long long r2, double limit, int64_t& keep) -> int {
-    for (int bin = kLoBins - 1; bin >= 0; --bin) {
-      const unsigned long long m = sh.lo_mass[bin];
-      if (sh.lo_cnt[bin] == 0) continue;
-      if (static_cast<double>(r2 + m) > limit) {
-        const unsigned long long w = m / sh.lo_cnt[bin];
-        keep = 0;
-        while (keep < static_cast<int64_t>(sh.lo_cnt[bin]) &&
-               static_cast<double>(r2 + w * static_cast<unsigned long long>(keep)) <= limit)
-          ++keep;
-        if (keep == 0) keep = 1;  // cannot happen unless rounding: keep the first
-        return bin;
+  bool have_mass = false;  // sh.mass holds the row's masses (pass C)
+  int nc[kMaxParts] = {0};
+  int total = 0;
+  uint32_t t_all = 0;      // the lists hold every token at or above this key (top-p alone)
+  // entry e of the concatenated lists: part c's run starts at the sum of the
+  // runs before it
+  auto list_entry = [&](int e) -> unsigned long long {
+    int c = 0, before = 0, start = 0;  // the last part whose run starts at or before e
+#pragma unroll
+    for (int j = 0; j < kMaxParts; ++j) {
+      if (e >= start) {
+        c = j;
+        before = start;
       }
-      r2 += m;
+      start += nc[j];
     }
-    return -1;
+    return rp[c].cand[e - before];
   };
-  bool nucleus = false;    // ... of a row that only top-p cuts,
-  uint32_t t_all = 0;      // where the lists hold every token at or above this key
-  double nucleus_limit = 0.0;  // and this is top_p x the row's whole mass
-  uint32_t kc = 0;         // the final cut: a key and
-  int64_t tc = 0, cties = 0;  // the ties kept at it, of how many
   if constexpr (kPre) {
-    int nc[kMaxParts];
-    int total = 0;
     from_list = true;
     bool short_list = true;
 #pragma unroll
@@ -979,26 +959,54 @@ __global__ __launch_bounds__(kThreads) void sample_kernel(const uint16_t* logits
       total += nc[c] > 0 ? nc[c] : 0;
       kmax = km > kmax ? km : kmax;
     }
-    from_list = from_list && total <= kCap;
-    if (__builtin_expect(uncut && from_list, 0)) {  // uniform
-      unsigned long long mass[kMaxParts];
-      part_values(P, 0ull, [&](int c) { return rp[c].best; }, mass);
+    if (__builtin_expect(split, 0)) {  // uniform
       const float xm = key_value(kmax) * inv_t;
-      from_list = kmax > 0x7Fu && xm < INFINITY && xm > -INFINITY;
-      nucleus = from_list;
-      double whole = 0.0;
+      // (without a finite maximum there are no masses: part 0 streams the row)
+      have_mass = kmax > 0x7Fu && xm < INFINITY && xm > -INFINITY;
+      if (!have_mass && part > 0) return;
+      if (have_mass) {
 #pragma unroll
-      for (int c = 0; c < kMaxParts; ++c) {
-        const uint32_t tl = static_cast<uint32_t>(hdr[c]) >> 16;
-        t_all = tl > t_all ? tl : t_all;
-        const float xc = key_value(static_cast<uint32_t>(hdr[c]) & 0xFFFFu) * inv_t;
-        const double m = __longlong_as_double(static_cast<long long>(mass[c]));
-        if (m > 0.0) whole += m * exp(static_cast<double>(xc) - static_cast<double>(xm));
+        for (int c = 0; c < kMaxParts; ++c) {
+          const uint32_t tl = c < P ? static_cast<uint32_t>(hdr[c]) >> 16 : 0u;
+          t_all = tl > t_all ? tl : t_all;
+        }
+        if (!from_list) t_all = 0xFFFFu;  // a list is missing
+        for (int i = tid; i < kHiBins; i += kThreads) sh.mass[i] = 0ull;
+        __syncthreads();
+        int64_t lo, hi;
+        part_range(vocab, P, part, lo, hi);
+        for_each_round_in<kVec>(p, lo, hi, [&](int64_t i0, const uint32_t* b, auto full) {
+          unsigned long long w[8];  // a NaN's is 0, whatever its bin
+#pragma unroll
+          for (int e = 0; e < 8; ++e)
+            w[e] = full || i0 + e < hi ? fixed_weight_of(__uint_as_float(b[e] << 16), inv_t, xm) : 0ull;
+#pragma unroll
+          for (int j = 0; j < 4; ++j) {
+            const uint32_t k2 = raw_keys2(b[2 * j] | (b[2 * j + 1] << 16));
+            atomicAdd(&sh.mass[(k2 & 0xFFFFu) >> kLoBits], w[2 * j]);
+            atomicAdd(&sh.mass[k2 >> (16 + kLoBits)], w[2 * j + 1]);
+          }
+        });
+        __syncthreads();
+        RowMass& rm = mass[row];
+        for (int i = tid; i < kHiBins; i += kThreads)
+          if (sh.mass[i])
+            __hip_atomic_fetch_add(&rm.bin[i], sh.mass[i], __ATOMIC_RELAXED,
+                                   __HIP_MEMORY_SCOPE_AGENT);
+        asm volatile("s_waitcnt vmcnt(0)" ::: "memory");  // this wave's sums are in
+        __syncthreads();
+        if (tid == 0)
+          sh.sel_bin = static_cast<int>(__hip_atomic_fetch_add(
+              &rm.arrived, 1u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT));
+        __syncthreads();
+        if (sh.sel_bin != P - 1) return;
+        for (int i = tid; i < kHiBins; i += kThreads)
+          sh.mass[i] = __hip_atomic_load(&rm.bin[i], __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+        __syncthreads();
       }
-      nucleus_limit = static_cast<double>(fmaxf(pcut, 0.f)) * (whole * kFix);
     }
-    bool sorted = from_list && short_list && (!nucleus || total <= kThreads / 4);
-    if (sorted) {  // uniform
+    from_list = from_list && total <= kCap && !split;
+    if (from_list && short_list) {  // uniform
       // A short union (the usual case: k plus a few per part): one entry
       // per thread, sorted by key (descending) and token index (ascending)
       // with a bitonic network; the top-k list is then its first k
@@ -1058,86 +1066,36 @@ __global__ __launch_bounds__(kThreads) void sample_kernel(const uint16_t* logits
       }
       const uint32_t key = static_cast<uint32_t>(x >> 32);
       const uint32_t idx = ~static_cast<uint32_t>(x);
-      const bool in_k = tid < k && tid < total && key >= t_all;
+      const bool in_k = tid < k && tid < total;
       bool kept = in_k;
       if (use_p) {
         const unsigned long long wf =
             in_k ? fixed_weight(key, inv_t, key_value(kmax) * inv_t) : 0ull;
         unsigned long long mass;
         const unsigned long long before = block_scan_u64(wf, mass, sh);
-        const double limit =
-            nucleus ? nucleus_limit
-                    : static_cast<double>(fmaxf(pcut, 0.f)) * static_cast<double>(mass);
+        const double limit = static_cast<double>(fmaxf(pcut, 0.f)) * static_cast<double>(mass);
         kept = in_k && static_cast<double>(before) <= limit;
-        // top-p alone: a cut past the lists' tokens needs the row
-        if (__builtin_expect(nucleus, 0) && !(static_cast<double>(mass) > limit))
-          sorted = from_list = false;
       }
-      if (sorted) {  // uniform
-        unsigned long long best = 0;
-        if (kept && key != 0) best = draw_candidate(key, idx, draws4(seed, row, idx >> 2)[idx & 3], inv_t);
-        best = block_max_u64(best, sh);
-        if (tid == 0) out[row] = best ? static_cast<int64_t>(~static_cast<uint32_t>(best)) : 0;
-        return;
-      }
+      unsigned long long best = 0;
+      if (kept && key != 0) best = draw_candidate(key, idx, draws4(seed, row, idx >> 2)[idx & 3], inv_t);
+      best = block_max_u64(best, sh);
+      if (tid == 0) out[row] = best ? static_cast<int64_t>(~static_cast<uint32_t>(best)) : 0;
+      return;
     }
-    if (from_list) {
-      // the union's counts for passes A and B, or its masses for the cut of
-      // top-p alone (whose weights are relative to the row's maximum as ever)
-      const float xm = key_value(kmax) * inv_t;
-      for (int i = tid; i < kHiBins; i += kThreads) {
-        if (nucleus) sh.mass[i] = 0ull; else sh.cnt[i] = 0;
-      }
-      if (tid < kLoBins) {
-        sh.lo_cnt[tid] = 0;
-        sh.lo_mass[tid] = 0ull;
-      }
+    if (from_list) {  // the union's counts for passes A and B
+      for (int i = tid; i < kHiBins; i += kThreads) sh.cnt[i] = 0;
+      if (tid < kLoBins) sh.lo_cnt[tid] = 0;
       __syncthreads();
-      // entry e of the concatenated lists: part c's run starts at the sum
-      // of the runs before it
       for (int e = tid; e < total; e += kThreads) {
-        int c = 0, before = 0, start = 0;  // the last part whose run starts at or before e
-#pragma unroll
-        for (int j = 0; j < kMaxParts; ++j) {
-          if (e >= start) {
-            c = j;
-            before = start;
-          }
-          start += nc[j];
-        }
-        const unsigned long long cd = rp[c].cand[e - before];
+        const unsigned long long cd = list_entry(e);
         sh.cand[e] = cd;
-        const uint32_t key = static_cast<uint32_t>(cd >> 32);
-        if (!nucleus)
-          atomicAdd(&sh.cnt[key >> kLoBits], 1u);
-        else if (key >= t_all)
-          atomicAdd(&sh.mass[key >> kLoBits], fixed_weight(key, inv_t, xm));
+        atomicAdd(&sh.cnt[static_cast<uint32_t>(cd >> 32) >> kLoBits], 1u);
       }
       ncand = total;
       __syncthreads();
-      if (nucleus) {
-        unsigned long long above;
-        const int hb = find_mass_bin_block(sh.mass, pcut, nucleus_limit, above, sh, true);
-        if (hb >= 0) {
-          for (int i = tid; i < total; i += kThreads) {
-            const uint32_t key = static_cast<uint32_t>(sh.cand[i] >> 32);
-            if (static_cast<int>(key >> kLoBits) != hb || key < t_all) continue;
-            atomicAdd(&sh.lo_cnt[key & (kLoBins - 1)], 1u);
-            atomicAdd(&sh.lo_mass[key & (kLoBins - 1)], fixed_weight(key, inv_t, xm));
-          }
-          __syncthreads();
-          const int lb = low_cut(above, nucleus_limit, tc);
-          kc = (static_cast<uint32_t>(hb) << kLoBits) | static_cast<uint32_t>(lb);
-          cties = sh.lo_cnt[lb];
-        } else {  // a cut past the lists' tokens needs the row
-          from_list = false;
-          ncand = -1;
-        }
-      }
     }
   }
-  if (!from_list) {
-    nucleus = false;
+  if (!from_list && !have_mass) {
     kmax = 0;
     __syncthreads();
     for (int i = tid; i < kHiBins; i += kThreads) sh.cnt[i] = 0;
@@ -1209,27 +1167,51 @@ __global__ __launch_bounds__(kThreads) void sample_kernel(const uint16_t* logits
   // membership in the top-k list before tie ranks: key > kk, or key == kk
   // with rank < tk (ranks in token order)
 
+  // The top-p cut inside the high bin whose mass above it is r2, from the
+  // low-bin histograms: the first low bin whose mass passes the limit and how
+  // many of its ties are kept: rank r while the mass before it, r2 + r * w, is
+  // within the limit (rank 0 of the list's first key is always kept since r2
+  // is then 0).  Returns the bin, or -1.
+  auto low_cut = [&](unsigned long long r2, double limit, int64_t& keep) -> int {
+    for (int bin = kLoBins - 1; bin >= 0; --bin) {
+      const unsigned long long m = sh.lo_mass[bin];
+      if (sh.lo_cnt[bin] == 0) continue;
+      if (static_cast<double>(r2 + m) > limit) {
+        const unsigned long long w = m / sh.lo_cnt[bin];
+        keep = 0;
+        while (keep < static_cast<int64_t>(sh.lo_cnt[bin]) &&
+               static_cast<double>(r2 + w * static_cast<unsigned long long>(keep)) <= limit)
+          ++keep;
+        if (keep == 0) keep = 1;  // cannot happen unless rounding: keep the first
+        return bin;
+      }
+      r2 += m;
+    }
+    return -1;
+  };
+
   // ---- C, D: the top-p cut over the top-k list ---------------------------
-  // The kept list is the first min(k, n_p) positions of the sorted top-k list.
-  if (!nucleus) {
-    kc = kk;
-    tc = tk;
-    cties = kties;
-  }
-  if (use_p && !nucleus) {
+  // kc / tc: the final cut (key and ties kept at it); the kept list is the
+  // first min(k, n_p) positions of the sorted top-k list.
+  uint32_t kc = kk;
+  int64_t tc = tk, cties = kties;
+  if (use_p) {
     // masses of the top-k list; the ties at kk count only up to tk of them
     __syncthreads();
-    for (int i = tid; i < kHiBins; i += kThreads) sh.mass[i] = 0ull;
+    if (!have_mass)
+      for (int i = tid; i < kHiBins; i += kThreads) sh.mass[i] = 0ull;
     if (tid < kLoBins) {
       sh.lo_mass[tid] = 0ull;
       sh.lo_cnt[tid] = 0;
     }
+    if (have_mass && tid == 0) sh.ncand = 0;
     __syncthreads();
     const bool partial_k = k < vocab && tk < kties;
-    visit([&](uint32_t key, int64_t) {
-      if (key < kk || (partial_k && key == kk)) return;
-      atomicAdd(&sh.mass[key >> kLoBits], fixed_weight(key, inv_t, xmax));
-    });
+    if (!have_mass)
+      visit([&](uint32_t key, int64_t) {
+        if (key < kk || (partial_k && key == kk)) return;
+        atomicAdd(&sh.mass[key >> kLoBits], fixed_weight(key, inv_t, xmax));
+      });
     __syncthreads();
     const unsigned long long wk_fix = fixed_weight(kk, inv_t, xmax);
     if (partial_k && tid == 0) sh.mass[kk >> kLoBits] += wk_fix * static_cast<unsigned long long>(tk);
@@ -1246,27 +1228,42 @@ __global__ __launch_bounds__(kThreads) void sample_kernel(const uint16_t* logits
         if (partial_k && key == kk) return;
         atomicAdd(&sh.lo_mass[key & (kLoBins - 1)], fixed_weight(key, inv_t, xmax));
       };
+      // the parts' lists hold all of these tokens where none was left out of them
+      // above the bin's lowest key
+      if (have_mass && (static_cast<uint32_t>(hb) << kLoBits) >= t_all) {
+        for (int e0 = 0; e0 < total; e0 += kThreads) {
+          const unsigned long long cd = e0 + tid < total ? list_entry(e0 + tid) : 0ull;
+          const uint32_t key = static_cast<uint32_t>(cd >> 32);
+          compact(e0 + tid < total && static_cast<int>(key >> kLoBits) >= hb, key,
+                  static_cast<int64_t>(static_cast<uint32_t>(cd)));
+        }
+        finish_compaction();
+        __syncthreads();
+        if (ncand < 0 && tid == 0) sh.ncand = 0;  // more than fit: as without lists
+        __syncthreads();
+      }
       if (ncand >= 0) {
         visit(lo_hist);
       } else {
         // the tokens that can be kept lie in bins >= hb: keep them when they fit
-        const bool keep_list = count_from(hb) <= kCap;
+        // (with the parts' masses there are no counts: until they don't)
+        const bool keep_list = have_mass || count_from(hb) <= kCap;
         for_each_round<kVec>(p, vocab, [&](int64_t i0, const uint32_t* b, auto full) {
           bool q[8], any = false;  // tokens that can still be kept
+          uint32_t keys[8];
 #pragma unroll
           for (int e = 0; e < 8; ++e) {
-            const uint32_t key = okey(b[e]);
-            q[e] = (full || i0 + e < vocab) && static_cast<int>(key >> kLoBits) >= hb &&
-                   key >= kk;
+            keys[e] = okey(b[e]);
+            q[e] = (full || i0 + e < vocab) && static_cast<int>(keys[e] >> kLoBits) >= hb &&
+                   keys[e] >= kk;
             any = any || q[e];
           }
           if (__ballot(any) == 0ull) return;  // most rounds: none in the wave
 #pragma unroll
-          for (int e = 0; e < 8; ++e) {
-            const uint32_t key = okey(b[e]);
-            if (q[e]) lo_hist(key, i0 + e);
-            if (keep_list) compact(q[e], key, i0 + e);
-          }
+          for (int e = 0; e < 8; ++e)
+            if (q[e]) lo_hist(keys[e], i0 + e);
+          if (keep_list && *static_cast<volatile int*>(&sh.ncand) <= kCap)
+            append_round(q, keys, i0, sh);
         });
         if (keep_list) finish_compaction();
       }
@@ -1407,18 +1404,18 @@ extern "C" int qwen3_sample_bf16(const void* logits, int64_t row_stride, int64_t
   if (q3::aligned16(logits) && row_stride % 8 == 0)
     hipLaunchKernelGGL((sample_kernel<true, false>), dim3(static_cast<unsigned>(rows)),
                        dim3(kThreads), 0, s, lg, row_stride, vocab, temperature, top_k, top_p,
-                       seed, out, 0, nullptr);
+                       seed, out, 0, nullptr, nullptr);
   else
     hipLaunchKernelGGL((sample_kernel<false, false>), dim3(static_cast<unsigned>(rows)),
                        dim3(kThreads), 0, s, lg, row_stride, vocab, temperature, top_k, top_p,
-                       seed, out, 0, nullptr);
+                       seed, out, 0, nullptr, nullptr);
   return q3::launch_status(who);
 }
 
 extern "C" size_t qwen3_sample_workspace_bytes(int64_t rows, int64_t vocab) {
   if (rows <= 0 || vocab <= 0) return 0;
   const int P = parts_for(rows, vocab);
-  return P > 1 ? static_cast<size_t>(rows) * P * sizeof(PartOut) : 0;
+  return P > 1 ? static_cast<size_t>(rows) * (P * sizeof(PartOut) + sizeof(RowMass)) : 0;
 }
 
 namespace {
@@ -1426,12 +1423,13 @@ template <bool kVec>
 void launch_parts(const uint16_t* lg, int64_t row_stride, int64_t rows, int64_t vocab,
                   const float* temperature, const int32_t* top_k, const float* top_p,
                   uint64_t seed, int64_t* out, int P, PartOut* parts, hipStream_t s) {
+  RowMass* mass = reinterpret_cast<RowMass*>(parts + rows * P);
   hipLaunchKernelGGL(sample_part_kernel<kVec>, dim3(static_cast<unsigned>(rows * P)),
                      dim3(kThreads), 0, s, lg, row_stride, vocab, temperature, top_k, top_p,
-                     seed, P, parts);
-  hipLaunchKernelGGL((sample_kernel<kVec, true>), dim3(static_cast<unsigned>(rows)),
+                     seed, P, parts, mass);
+  hipLaunchKernelGGL((sample_kernel<kVec, true>), dim3(static_cast<unsigned>(rows), P),
                      dim3(kThreads), 0, s, lg, row_stride, vocab, temperature, top_k, top_p, seed,
-                     out, P, parts);
+                     out, P, parts, mass);
 }
 }  // namespace
 

@@ -257,3 +257,82 @@ def test_parallel_form_draws_uncut_rows_the_same(gpu, B, V):
             one, par = _both_forms(xd, td, kd, pd, seed)
             assert torch.equal(one, par), \
                 f"seed={seed}: rows {(one != par).nonzero().view(-1)[:8].tolist()} differ"
+
+
+def _ulps(p, n):
+    """The float32 n steps above p."""
+    return (torch.tensor([p], dtype=torch.float32).view(torch.int32) + n).view(torch.float32)
+
+
+@pytest.mark.parametrize("B,V", [(32, 20000), (32, 151936), (64, 40000)])
+def test_top_p_cut_decided_by_rounding_is_the_same_in_both_forms(gpu, B, V):
+    """Kept sets of a few equally likely tokens, whose last one stays or goes
+    with the last bits of the row's mass: top_p in steps of one float32 ulp
+    across the place where the mass before that token reaches the limit, the
+    parts' own maxima apart.  A mass that differed by 1e-7 between the forms
+    would keep another set in some of the rows, and one draw in five shows it."""
+    announce(f"sampling: cuts at the limit B={B} V={V}")
+    g = torch.Generator().manual_seed(V)
+    for trial in range(4):
+        n = 4 + trial
+        row = torch.full((V,), -9.0) + torch.randn(V, generator=g)
+        lo = torch.randperm(V // 3, generator=g)
+        row[lo[:1] + 2 * (V // 3)] = 4.0 + trial / 8               # the maximum, in a late part
+        row[lo[1 : 1 + n]] = 3.0                                   # the tied ones, in the first
+        row[lo[1 + n : 400] + V // 3] = (torch.rand(399 - n, generator=g) * 4 - 3)  # the tail
+        row = row.to(torch.bfloat16)
+        t = 0.7 + 0.1 * trial
+        w = torch.exp(row.double() / torch.tensor(t, dtype=torch.float32).double())
+        w = w / w.max()
+        p0 = float((1 + (n - 1) * w[lo[1]]) / w.sum())             # the last tied token's own limit
+        p = torch.cat([_ulps(p0, i - B // 2) for i in range(B)]).to(gpu)
+        x = row.expand(B, V).contiguous().to(gpu)
+        td = torch.full((B,), t, device=gpu)
+        kd = torch.zeros(B, dtype=torch.int32, device=gpu)
+        for seed in range(24):
+            one, par = _both_forms(x, td, kd, p, seed)
+            assert torch.equal(one, par), \
+                f"trial={trial} seed={seed}: rows {(one != par).nonzero().view(-1)[:8].tolist()} differ"
+
+
+@pytest.mark.parametrize("B,V", [(3, 151936), (33, 20000), (128, 16385)])
+def test_split_top_p_rows_share_nothing_between_calls(gpu, B, V):
+    """Rows that all parts' workgroups work on: masked rows (the lowest finite
+    value and -inf), kept sets longer than a candidate list, and a workspace
+    used again by batches of other sizes, eager and in a replayed graph."""
+    from qwen3_engine_from_scratch_amd import _lib
+
+    announce(f"sampling: split rows B={B} V={V}")
+    lib = _lib.load()
+    g = torch.Generator().manual_seed(B)
+    x = torch.randn(B, V, generator=g) * 0.3                     # nearly flat: > 4,096 kept
+    x[0, ::2] = torch.finfo(torch.bfloat16).min
+    x[1, 1::2] = float("-inf")
+    x[2, 40:] = float("-inf")
+    xd = x.to(torch.bfloat16).to(gpu)
+    t, p = torch.ones(B, device=gpu), torch.full((B,), 0.9, device=gpu)
+    k = torch.zeros(B, dtype=torch.int32, device=gpu)
+    need = int(lib.qwen3_sample_workspace_bytes(B, V))
+    ws = torch.full((need,), 0x5A, dtype=torch.uint8, device=gpu)
+    out = torch.empty(B, dtype=torch.int64, device=gpu)
+
+    def call(rows):
+        _lib.check(lib.qwen3_sample_ws_bf16(
+            xd.data_ptr(), V, rows, V, t.data_ptr(), k.data_ptr(), p.data_ptr(), 11,
+            out.data_ptr(), ws.data_ptr(), need, torch.cuda.current_stream().cuda_stream),
+            "qwen3_sample_ws_bf16")
+
+    one, _ = _both_forms(xd, t, k, p, 11)
+    for rows in (B, 1, 2, B):
+        out.fill_(-7)
+        call(rows)
+        assert torch.equal(out[:rows].cpu(), one[:rows]), rows
+    graph = torch.cuda.CUDAGraph()
+    with torch.cuda.graph(graph):
+        call(B)
+    for _ in range(4):
+        out.fill_(-7)
+        graph.replay()
+        torch.cuda.synchronize()
+        assert torch.equal(out.cpu(), one)
+        call(2)
