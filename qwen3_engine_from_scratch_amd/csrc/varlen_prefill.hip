@@ -1735,7 +1735,7 @@ extern "C" int qwen3_padded_prefill_bf16(const void* q, const int64_t q_strides[
     return q3::fail(QWEN3_EINVAL, "%s: null pointer argument", who);
   if (const int rc = check_heads(num_heads, num_kv_heads, head_dim, who)) return rc;
   if (num_seqs < 0 || padded_len < 0 ||
-      static_cast<int64_t>(kMaxSeqs) * padded_len > 0x7fffffff)
+      static_cast<int64_t>(num_seqs < kMaxSeqs ? num_seqs : kMaxSeqs) * padded_len > 0x7fffffff)
     return q3::fail(QWEN3_EINVAL, "%s: bad sizes", who);
   for (int i = 0; i < num_seqs; ++i)
     if (lens[i] <= 0 || lens[i] > padded_len)

@@ -148,7 +148,9 @@ def test_padded_prefill_rejects_bad_arguments():
     assert call(q=None) == -1
     assert call(lens=(64, 0)) == -1
     assert call(lens=(65, 1)) == -1
-    assert call(S=1 << 24) == -1       # rows of a launch past 32 bits
+    assert call(S=1 << 30) == -1       # rows of a launch past 31 bits
+    # ... of its own sequences: two long ones pass (on to the alignment check)
+    assert call(S=1 << 29, qs=_s(64 * 2048, 2049, 128)) == -2
     assert call(qs=_s(64 * 2048, 2049, 128)) == -2
     assert call(ks=_s(64, 64, 1 << 16)) == -3       # overlapping rows
     assert call(ks=_s(64, 1 << 24, 128)) == -3      # a tile's rows past 32-bit offsets
