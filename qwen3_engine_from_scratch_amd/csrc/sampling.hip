@@ -195,15 +195,19 @@ struct alignas(16) PartOut {
                                   // token with key >= t_lo is listed
   int32_t ncand;                  // candidates written, -1 none
   unsigned long long best;        // greedy rows: (key + 1) << 32 | ~index, the first maximum;
-                                  // rows drawn uncut: the part's draw (score, ~index)
+                                  // rows drawn uncut: the part's draw (score, ~index);
+                                  // top-p alone: in part 0, the parts that are in
   unsigned long long cand[kCap];  // (key << 32) | token index
 };
-// A row that only top-p cuts: its bins' masses over all parts, and how many
-// parts have added theirs.  Cleared by the first launch.
-struct alignas(16) RowMass {
-  unsigned long long bin[kHiBins];
-  uint32_t arrived;
-};
+// A row that only top-p cuts keeps its bins' masses over all parts at the ends of
+// its first parts' lists, which are that much shorter, and in part 0's `best`
+// how many parts have added theirs.  Cleared by the first launch.
+__device__ __forceinline__ int bins_log2(int P) { return P >= 8 ? 9 : P >= 4 ? 10 : 11; }
+__device__ __forceinline__ int nucleus_cap(int P) { return kCap - (1 << bins_log2(P)); }
+__device__ __forceinline__ unsigned long long* row_bin(PartOut* rp, int P, int i) {
+  const int sl = bins_log2(P);
+  return &rp[i >> sl].cand[kCap - (1 << sl) + (i & ((1 << sl) - 1))];
+}
 
 // Parts per row of the parallel form: about one workgroup per CU over the
 // batch (four parts for 64 rows measured best on 256 CUs: 44 us against
@@ -593,8 +597,7 @@ __global__ __launch_bounds__(kThreads) void sample_part_kernel(const uint16_t* l
                                                                const float* temperature,
                                                                const int32_t* top_k,
                                                                const float* top_p, uint64_t seed,
-                                                               int P, PartOut* parts,
-                                                               RowMass* mass) {
+                                                               int P, PartOut* parts) {
   __shared__ Shared sh;
   const int64_t row = blockIdx.x / P;
   const int c = static_cast<int>(blockIdx.x % P);
@@ -634,8 +637,10 @@ __global__ __launch_bounds__(kThreads) void sample_part_kernel(const uint16_t* l
     }
     if (uncut) {
       kreq = kNucleusList / P;  // top-p alone: the tokens this part lists
-      for (int i = c * kThreads + tid; i < kHiBins; i += P * kThreads) mass[row].bin[i] = 0ull;
-      if (c == 0 && tid == 0) mass[row].arrived = 0u;
+      const int cap = nucleus_cap(P);
+      if (c < kHiBins / (kCap - cap))
+        for (int i = cap + tid; i < kCap; i += kThreads) po.cand[i] = 0ull;
+      if (c == 0 && tid == 0) po.best = 0ull;
     }
     if (!greedy) {
       for (int i = tid; i < kHiBins; i += kThreads) sh.cnt[i] = 0;
@@ -771,7 +776,7 @@ __global__ __launch_bounds__(kThreads) void sample_part_kernel(const uint16_t* l
     });
     __syncthreads();
     const int n = sh.ncand;
-    const bool ok = n <= kCap;
+    const bool ok = n <= (uncut ? nucleus_cap(P) : kCap);
     if (tid == 0) {
       po.kmax = uncut ? kmax | (t_lo << 16) : kmax;
       po.ncand = ok ? n : -1;
@@ -806,7 +811,7 @@ __global__ __launch_bounds__(kThreads) void sample_kernel(const uint16_t* logits
                                                           const int32_t* top_k,
                                                           const float* top_p, uint64_t seed,
                                                           int64_t* out, int P,
-                                                          const PartOut* parts, RowMass* mass) {
+                                                          PartOut* parts) {
   __shared__ Shared sh;
   const int64_t row = blockIdx.x;
   const int part = kPre ? static_cast<int>(blockIdx.y) : 0;
@@ -816,7 +821,7 @@ __global__ __launch_bounds__(kThreads) void sample_kernel(const uint16_t* logits
   const float pcut = top_p ? top_p[row] : 1.f;
   const int tid = threadIdx.x;
   const int lane = tid & 63, wave = tid >> 6;
-  const PartOut* rp = kPre ? parts + row * P : nullptr;
+  PartOut* rp = kPre ? parts + row * P : nullptr;
 
   // One round trip with the row's parameters: every part's (kmax, ncand) and,
   // ahead of knowing the counts, entry tid % L of part tid / L (L = kThreads
@@ -988,20 +993,20 @@ __global__ __launch_bounds__(kThreads) void sample_kernel(const uint16_t* logits
           }
         });
         __syncthreads();
-        RowMass& rm = mass[row];
         for (int i = tid; i < kHiBins; i += kThreads)
           if (sh.mass[i])
-            __hip_atomic_fetch_add(&rm.bin[i], sh.mass[i], __ATOMIC_RELAXED,
+            __hip_atomic_fetch_add(row_bin(rp, P, i), sh.mass[i], __ATOMIC_RELAXED,
                                    __HIP_MEMORY_SCOPE_AGENT);
         asm volatile("s_waitcnt vmcnt(0)" ::: "memory");  // this wave's sums are in
         __syncthreads();
         if (tid == 0)
           sh.sel_bin = static_cast<int>(__hip_atomic_fetch_add(
-              &rm.arrived, 1u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT));
+              &rp[0].best, 1ull, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT));
         __syncthreads();
         if (sh.sel_bin != P - 1) return;
         for (int i = tid; i < kHiBins; i += kThreads)
-          sh.mass[i] = __hip_atomic_load(&rm.bin[i], __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+          sh.mass[i] = __hip_atomic_load(row_bin(rp, P, i), __ATOMIC_RELAXED,
+                                         __HIP_MEMORY_SCOPE_AGENT);
         __syncthreads();
       }
     }
@@ -1404,18 +1409,18 @@ extern "C" int qwen3_sample_bf16(const void* logits, int64_t row_stride, int64_t
   if (q3::aligned16(logits) && row_stride % 8 == 0)
     hipLaunchKernelGGL((sample_kernel<true, false>), dim3(static_cast<unsigned>(rows)),
                        dim3(kThreads), 0, s, lg, row_stride, vocab, temperature, top_k, top_p,
-                       seed, out, 0, nullptr, nullptr);
+                       seed, out, 0, nullptr);
   else
     hipLaunchKernelGGL((sample_kernel<false, false>), dim3(static_cast<unsigned>(rows)),
                        dim3(kThreads), 0, s, lg, row_stride, vocab, temperature, top_k, top_p,
-                       seed, out, 0, nullptr, nullptr);
+                       seed, out, 0, nullptr);
   return q3::launch_status(who);
 }
 
 extern "C" size_t qwen3_sample_workspace_bytes(int64_t rows, int64_t vocab) {
   if (rows <= 0 || vocab <= 0) return 0;
   const int P = parts_for(rows, vocab);
-  return P > 1 ? static_cast<size_t>(rows) * (P * sizeof(PartOut) + sizeof(RowMass)) : 0;
+  return P > 1 ? static_cast<size_t>(rows) * P * sizeof(PartOut) : 0;
 }
 
 namespace {
@@ -1423,13 +1428,12 @@ template <bool kVec>
 void launch_parts(const uint16_t* lg, int64_t row_stride, int64_t rows, int64_t vocab,
                   const float* temperature, const int32_t* top_k, const float* top_p,
                   uint64_t seed, int64_t* out, int P, PartOut* parts, hipStream_t s) {
-  RowMass* mass = reinterpret_cast<RowMass*>(parts + rows * P);
   hipLaunchKernelGGL(sample_part_kernel<kVec>, dim3(static_cast<unsigned>(rows * P)),
                      dim3(kThreads), 0, s, lg, row_stride, vocab, temperature, top_k, top_p,
-                     seed, P, parts, mass);
+                     seed, P, parts);
   hipLaunchKernelGGL((sample_kernel<kVec, true>), dim3(static_cast<unsigned>(rows), P),
                      dim3(kThreads), 0, s, lg, row_stride, vocab, temperature, top_k, top_p, seed,
-                     out, P, parts, mass);
+                     out, P, parts);
 }
 }  // namespace
 

@@ -264,7 +264,7 @@ def _ulps(p, n):
     return (torch.tensor([p], dtype=torch.float32).view(torch.int32) + n).view(torch.float32)
 
 
-@pytest.mark.parametrize("B,V", [(32, 20000), (32, 151936), (64, 40000)])
+@pytest.mark.parametrize("B,V", [(32, 20000), (32, 151936), (64, 40000), (16, 57000)])
 def test_top_p_cut_decided_by_rounding_is_the_same_in_both_forms(gpu, B, V):
     """Kept sets of a few equally likely tokens, whose last one stays or goes
     with the last bits of the row's mass: top_p in steps of one float32 ulp
