@@ -69,6 +69,23 @@ __device__ __forceinline__ uint16_t bf16_bits(float x) {
   return __builtin_bit_cast(uint16_t, static_cast<__bf16>(x));
 }
 
+__device__ __forceinline__ float round_bf16(float x) {
+  return __uint_as_float(static_cast<uint32_t>(bf16_bits(x)) << 16);
+}
+
+// The ends of the decode linears, with the roundings of separate bf16 operations,
+// in one place so that every kernel gives the same bits.
+// SwiGLU of the two projections' sums: bf16(bf16(silu(gate)) * up).
+__device__ __forceinline__ uint16_t swiglu_bf16(float gate, float up) {
+  const float g = round_bf16(gate);
+  const float u = round_bf16(up);
+  return bf16_bits(round_bf16(g / (1.f + expf(-g))) * u);
+}
+// bf16(residual + bf16(sum)), the residual as its bits.
+__device__ __forceinline__ float add_residual(uint32_t res, float sum) {
+  return round_bf16(__uint_as_float(res << 16) + round_bf16(sum));
+}
+
 __device__ __forceinline__ float bf16_lo(uint32_t w) {
   return __builtin_bit_cast(float, w << 16);
 }

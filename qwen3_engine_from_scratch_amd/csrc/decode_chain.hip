@@ -471,16 +471,14 @@ __device__ __forceinline__ int linear_phase(const ChainArgs& a, Shared& sh, int 
         const int row = 4 * (lane >> 4) + i;
         const bool live = stores && row < a.M;
         if constexpr (kNorm) {
-          const float g = round_bf16(v[i]);
-          const float u = round_bf16(up[i]);
-          const float sg = round_bf16(g / (1.f + expf(-g)));
-          if (live) st16b_dev(a.act + static_cast<int64_t>(row) * a.I + col, q3::bf16_bits(sg * u));
+          const uint16_t y = q3::swiglu_bf16(v[i], up[i]);
+          if (live) st16b_dev(a.act + static_cast<int64_t>(row) * a.I + col, y);
         } else {
           uint16_t* dst = kPh == kO ? a.h_mid : a.h_out;
           float* ss = kPh == kO ? a.ss_mid : a.ss_out;
           float h = 0.f;
           if (live) {
-            h = round_bf16(__uint_as_float(res[i] << 16) + round_bf16(v[i]));
+            h = q3::add_residual(res[i], v[i]);
             st16b_dev(dst + static_cast<int64_t>(row) * a.K + col, q3::bf16_bits(h));
           }
           float sq = __fmul_rn(h, h);
@@ -776,8 +774,8 @@ int qkv_half_blocks() {
 bool phase_blocks(int M, int hidden, int inter, int num_heads, int num_kv_heads, bool merge,
                   bool qkv, int (&first)[kPhases + 1]) {
   const int64_t KO = static_cast<int64_t>(num_heads) * kHeadD;
-  if (num_heads + num_kv_heads > kMaxNormHeads || M < 1 || M > kRows || hidden <= 0 || inter <= 0 || num_heads <= 0 || num_kv_heads <= 0 ||
-      num_heads % num_kv_heads != 0)
+  if (M < 1 || M > kRows || hidden <= 0 || inter <= 0 || num_heads <= 0 || num_kv_heads <= 0 ||
+      num_heads % num_kv_heads != 0 || num_heads + num_kv_heads > kMaxNormHeads)
     return false;
   // whole k-steps per wave, held in registers; rows of one head staged in
   // LDS; o_proj and down split K over eight waves, as decode_linear does from

@@ -33,10 +33,6 @@ struct HeadArgs {
   int bs;
 };
 
-__device__ __forceinline__ float round_bf16(float x) {
-  return __uint_as_float(static_cast<uint32_t>(q3::bf16_bits(x)) << 16);
-}
-
 // RoPE position, pool block and slot in it of token t; -1 where the tables
 // have none.
 __device__ __forceinline__ void locate_token(const HeadArgs& a, int t, int64_t& pos,
@@ -96,8 +92,8 @@ __device__ __forceinline__ void finish_head(const HeadArgs& a, int head, int t, 
     const float ss_[8] = {s0.x, s0.y, s0.z, s0.w, s1.x, s1.y, s1.z, s1.w};
 #pragma unroll
     for (int e = 0; e < 8; ++e) {
-      cv[e] = round_bf16(cc[e]);  // cos / sin .to(q.dtype)
-      sv[e] = round_bf16(ss_[e]);
+      cv[e] = q3::round_bf16(cc[e]);  // cos / sin .to(q.dtype)
+      sv[e] = q3::round_bf16(ss_[e]);
     }
   }
   // Squares rounded, then summed (no fused multiply-add), as x.pow(2).mean().
@@ -123,7 +119,7 @@ __device__ __forceinline__ void finish_head(const HeadArgs& a, int head, int t, 
         const int el = 2 * e + hl;
         const float n = hl ? q3::bf16_hi(np[e]) : q3::bf16_lo(np[e]);
         const float rh = sign * (hl ? q3::bf16_hi(pp[e]) : q3::bf16_lo(pp[e]));
-        o[hl] = round_bf16(n * cv[el]) + round_bf16(rh * sv[el]);
+        o[hl] = q3::round_bf16(n * cv[el]) + q3::round_bf16(rh * sv[el]);
       }
       out[e] = q3::pack_bf16x2(o[0], o[1]);
     }

@@ -57,9 +57,6 @@ struct LinArgs {
   int up_row;  // kSilu: first weight row of the up half
 };
 
-__device__ __forceinline__ float round_bf16(float x) {
-  return __uint_as_float(static_cast<uint32_t>(q3::bf16_bits(x)) << 16);
-}
 __device__ __forceinline__ uint16_t to_bf16(float x) { return q3::bf16_bits(x); }
 
 template <bool kNorm, int kEpi, int kWaves>
@@ -225,16 +222,12 @@ __global__ __launch_bounds__(kWaves * 64) void decode_linear_kernel(LinArgs a) {
     if constexpr (kEpi == kStore) {
       if (live) a.y[static_cast<int64_t>(row) * a.y_s + col] = to_bf16(v[0][i]);
     } else if constexpr (kEpi == kSilu) {
-      const float g = round_bf16(v[0][i]);
-      const float u = round_bf16(v[1][i]);
-      const float sg = round_bf16(g / (1.f + expf(-g)));
-      if (live) a.y[static_cast<int64_t>(row) * a.y_s + col] = to_bf16(sg * u);
+      const uint16_t y = q3::swiglu_bf16(v[0][i], v[1][i]);
+      if (live) a.y[static_cast<int64_t>(row) * a.y_s + col] = y;
     } else {
       float h = 0.f;
       if (live) {
-        const float o = round_bf16(v[0][i]);
-        const float r = __uint_as_float(res_pre[i] << 16);
-        h = round_bf16(r + o);
+        h = q3::add_residual(res_pre[i], v[0][i]);
         a.res_out[static_cast<int64_t>(row) * a.res_out_s + col] = to_bf16(h);
       }
       float sq = __fmul_rn(h, h);
@@ -384,12 +377,7 @@ __global__ __launch_bounds__(kWaves64 * 64) void gate_up64_kernel(LinArgs a) {
       usum += red[(((w * 4 + rb) * 2 + 1) * 4 + i) * 64 + lane];
     }
     const int row = 16 * rb + 4 * (lane >> 4) + i;
-    if (row < a.M) {
-      const float g = round_bf16(gsum);
-      const float u = round_bf16(usum);
-      const float sg = round_bf16(g / (1.f + expf(-g)));
-      a.y[static_cast<int64_t>(row) * a.y_s + col] = to_bf16(sg * u);
-    }
+    if (row < a.M) a.y[static_cast<int64_t>(row) * a.y_s + col] = q3::swiglu_bf16(gsum, usum);
   }
 }
 

@@ -15,10 +15,6 @@ namespace {
 
 constexpr int kWave = 64;
 
-__device__ __forceinline__ float round_bf16(float x) {
-  return __uint_as_float(static_cast<uint32_t>(q3::bf16_bits(x)) << 16);
-}
-
 // ---------------------------------------------------------------------------
 // Residual add + RMSNorm: one wave per output row, 16-byte chunks, CPL chunks
 // per lane (hidden <= 512 * CPL).
@@ -119,8 +115,8 @@ __global__ __launch_bounds__(256) void silu_mul_kernel(SiluArgs a) {
   q3::u32x4 o;
 #pragma unroll
   for (int e = 0; e < 4; ++e)
-    o[e] = q3::pack_bf16x2(round_bf16(silu(q3::bf16_lo(g[e]))) * q3::bf16_lo(u[e]),
-                           round_bf16(silu(q3::bf16_hi(g[e]))) * q3::bf16_hi(u[e]));
+    o[e] = q3::pack_bf16x2(q3::round_bf16(silu(q3::bf16_lo(g[e]))) * q3::bf16_lo(u[e]),
+                           q3::round_bf16(silu(q3::bf16_hi(g[e]))) * q3::bf16_hi(u[e]));
   q3::st16(a.out + r * a.out_s + 8 * ch, o);
 }
 

@@ -66,9 +66,6 @@ struct PreAttnArgs {
 
 __device__ __forceinline__ float bf_lo(uint32_t w) { return __uint_as_float(w << 16); }
 __device__ __forceinline__ float bf_hi(uint32_t w) { return __uint_as_float(w & 0xffff0000u); }
-__device__ __forceinline__ float round_bf16(float x) {
-  return __uint_as_float(static_cast<uint32_t>(q3::bf16_bits(x)) << 16);
-}
 
 // Rows of one token handled by one 16-lane group: their loads are issued
 // together, and the token's position, slot and cos/sin row are fetched
@@ -152,8 +149,8 @@ __global__ __launch_bounds__(256) void pre_attention_kernel(PreAttnArgs a) {
     const float ss_[8] = {s0.x, s0.y, s0.z, s0.w, s1.x, s1.y, s1.z, s1.w};
 #pragma unroll
     for (int e = 0; e < 8; ++e) {
-      cv[e] = round_bf16(cc[e]);  // cos / sin .to(q.dtype)
-      sv[e] = round_bf16(ss_[e]);
+      cv[e] = q3::round_bf16(cc[e]);  // cos / sin .to(q.dtype)
+      sv[e] = q3::round_bf16(ss_[e]);
     }
   }
   // rotate_half: (-x2, x1).  The sign goes into this lane's sin values once
