@@ -823,6 +823,15 @@ __global__ __launch_bounds__(kThreads) void sample_kernel(const uint16_t* logits
   const int lane = tid & 63, wave = tid >> 6;
   PartOut* rp = kPre ? parts + row * P : nullptr;
 
+  // cut by top-p alone: every part's workgroup has a share
+  auto split_row = [&]() {
+    return kPre && temp > 0.f && (kreq <= 0 || kreq >= vocab) && pcut < 1.f;
+  };
+  if (part > 0) {
+    asm volatile("");  // (a branch of its own: part 0 does not wait for the parameters here)
+    if (!split_row()) return;
+  }
+
   // One round trip with the row's parameters: every part's (kmax, ncand) and,
   // ahead of knowing the counts, entry tid % L of part tid / L (L = kThreads
   // / P entries per part: all of a short list).
@@ -842,9 +851,7 @@ __global__ __launch_bounds__(kThreads) void sample_kernel(const uint16_t* logits
   }
 
   const bool uncut = kreq <= 0 || kreq >= vocab;  // by top-k, as the part kernel
-  // cut by top-p alone: every part's workgroup has a share
-  const bool split = kPre && temp > 0.f && uncut && pcut < 1.f;
-  if (part > 0 && !split) return;
+  const bool split = split_row();
 
   // ---- greedy -----------------------------------------------------------
   if (kPre && !(temp > 0.f)) {
@@ -918,7 +925,7 @@ __global__ __launch_bounds__(kThreads) void sample_kernel(const uint16_t* logits
   };
   // Tokens of the high bins >= hb, from the pass-A histogram (every thread
   // gets the sum).
-  auto count_from = [&](int hb) {
+  auto count_from = [&](int hb) __attribute__((always_inline)) {
     const int top = kHiBins - 1 - kBinsPerThread * tid;
     int c = 0;
 #pragma unroll
