@@ -839,15 +839,14 @@ __global__ __launch_bounds__(kThreads) void sample_kernel(const uint16_t* logits
   const int cpart = kPre ? (tid / L < P ? tid / L : P - 1) : 0;
   const int coff = kPre ? tid - (tid / L) * L : 0;
   unsigned long long spec = 0;
-  unsigned long long hdr[kMaxParts];
+  unsigned long long hdr_lane = 0;  // of part lane % 8: one load for all of them
   if constexpr (kPre) {
     if (part == 0) spec = rp[cpart].cand[coff];
-    part_values(P, 0ull, [&](int c) {
-      return *reinterpret_cast<const unsigned long long*>(&rp[c].kmax);
-    }, hdr);
+    hdr_lane = *reinterpret_cast<const unsigned long long*>(
+        &rp[min(lane & (kMaxParts - 1), P - 1)].kmax);
     // the loads stay here (the compiler would otherwise move them into the
     // branches that use them, after the parameters' round trip)
-    asm volatile("" ::"v"(spec), "v"(hdr[0]));
+    asm volatile("" ::"v"(spec), "v"(hdr_lane));
   }
 
   const bool uncut = kreq <= 0 || kreq >= vocab;  // by top-k, as the part kernel
@@ -964,8 +963,9 @@ __global__ __launch_bounds__(kThreads) void sample_kernel(const uint16_t* logits
     bool short_list = true;
 #pragma unroll
     for (int c = 0; c < kMaxParts; ++c) {
-      nc[c] = static_cast<int>(hdr[c] >> 32);
-      const uint32_t km = static_cast<uint32_t>(hdr[c]) & 0xFFFFu;
+      const uint32_t h = __builtin_amdgcn_readlane(static_cast<uint32_t>(hdr_lane), c);
+      nc[c] = c < P ? __builtin_amdgcn_readlane(static_cast<uint32_t>(hdr_lane >> 32), c) : 0;
+      const uint32_t km = h & 0xFFFFu;  // (past the parts: the last part's again)
       from_list = from_list && nc[c] >= 0;
       short_list = short_list && nc[c] <= L;
       total += nc[c] > 0 ? nc[c] : 0;
@@ -979,8 +979,8 @@ __global__ __launch_bounds__(kThreads) void sample_kernel(const uint16_t* logits
       if (have_mass) {
 #pragma unroll
         for (int c = 0; c < kMaxParts; ++c) {
-          const uint32_t tl = c < P ? static_cast<uint32_t>(hdr[c]) >> 16 : 0u;
-          t_all = tl > t_all ? tl : t_all;
+          const uint32_t h = __builtin_amdgcn_readlane(static_cast<uint32_t>(hdr_lane), c);
+          t_all = max(t_all, h >> 16);
         }
         if (!from_list) t_all = 0xFFFFu;  // a list is missing
         for (int i = tid; i < kHiBins; i += kThreads) sh.mass[i] = 0ull;
