@@ -52,7 +52,7 @@
 //
 // Qwen3-0.6B, one row at 900 tokens: merge done 6.2 us after the start, o_proj
 // 9.9, gate_up 14, down 17.5, qkv 22.5; as separate launches 5.0, 5.9, 7.4,
-// 5.9 and 13.5 each (24.5 for the launch as a kernel trace counts it).  A step
+// 5.9 and 13.5 each (24.4 for the launch as a kernel trace counts it).  A step
 // with them: 1448 -> 1033 us, of which a flag that carries the launch's number,
 // where the flags were put back to zero and a wait could fail for good, is
 // 10.  The rare path is code of its own behind the usual one: a loop around both
